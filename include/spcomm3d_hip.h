@@ -502,7 +502,8 @@ SPC3D_API int spc3d_sddmm_host(spc3d_ctx *ctx, int dtype, uint32_t m, uint32_t n
 SPC3D_API int spc3d_spmm_host(spc3d_ctx *ctx, int dtype, uint32_t ncols, uint32_t nrows, uint32_t k,
                     const void *X, uint64_t nnz, const uint32_t *ii, const uint32_t *jj,
                     const void *avv, void *Y);
-/* Frees what the one-shot calls keep (no counterpart in the reference, whose operands
+/* Frees what the one-shot calls keep, and the device memory that the context keeps for the plans to
+ * come (at most 1/64 of the device's) (no counterpart in the reference, whose operands
  * live in host vectors). */
 SPC3D_API int spc3d_host_cache_clear(spc3d_ctx *ctx);
 /* What the last one-shot call on this context moved: bytes sent to the device, bytes of

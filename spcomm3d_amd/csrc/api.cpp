@@ -152,6 +152,14 @@ int spc3d_ctx_create_ex(int device, const spc3d_ctx_opts *opts, spc3d_ctx **out)
         (void)hipGetLastError();
         c->cu_count = 256;
     }
+    // What the pool may keep: 1/64 of the device's memory (4.5 of 288 GB), enough for the plan
+    // of a pattern of about 100 M entries and its construction.
+    size_t mem_free = 0, mem_total = 0;
+    if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess) {
+        (void)hipGetLastError();
+        mem_total = 0;
+    }
+    c->pool.set_limit(mem_total / 64);
     if (!(o.flags & SPC3D_CTX_NO_AUX_STREAM)) {
         e = hipStreamCreateWithFlags(&c->aux_stream, hipStreamNonBlocking);
         if (e == hipSuccess)
@@ -341,7 +349,7 @@ int spc3d_ctx_probe_xcd(spc3d_ctx *ctx, uint32_t nblocks, uint32_t *xcd)
     if (rc)
         return rc;
     uint32_t *dev = nullptr;
-    rc = dev_alloc(&dev, (size_t)nblocks);
+    rc = dev_alloc(ctx, &dev, (size_t)nblocks);
     if (rc)
         return rc;
     hipError_t e = launch_xcc_probe(dev, nblocks, ctx->stream);
@@ -401,7 +409,7 @@ int spc3d_panel_create(spc3d_ctx *ctx, int dtype, uint32_t m, uint32_t n, spc3d_
     p->dtype = dtype;
     p->m = m;
     p->n = n;
-    rc = dev_alloc_bytes(&p->dev, (size_t)m * n * elem_size(dtype));
+    rc = dev_alloc_bytes(ctx, &p->dev, (size_t)m * n * elem_size(dtype));
     if (rc) {
         delete p;
         return rc;
@@ -569,7 +577,7 @@ int spc3d_vals_create(spc3d_ctx *ctx, int dtype, uint64_t n, spc3d_vals **out)
     v->ctx = ctx;
     v->dtype = dtype;
     v->n = n;
-    rc = dev_alloc_bytes(&v->dev, (size_t)n * elem_size(dtype));
+    rc = dev_alloc_bytes(ctx, &v->dev, (size_t)n * elem_size(dtype));
     if (rc) {
         delete v;
         return rc;
@@ -1025,10 +1033,10 @@ int spc3d_rowmap_create(spc3d_ctx *ctx, uint32_t panel_rows, uint64_t n, const u
     m->panel_rows = panel_rows;
     m->nslots = (uint32_t)n;
     m->nuniq = (uint32_t)urows.size();
-    rc = dev_alloc(&m->rows, (size_t)n);
-    if (!rc) rc = dev_alloc(&m->urows, urows.size());
-    if (!rc) rc = dev_alloc(&m->ptr, n ? ptr.size() : 0);
-    if (!rc) rc = dev_alloc(&m->slots, (size_t)n);
+    rc = dev_alloc(ctx, &m->rows, (size_t)n);
+    if (!rc) rc = dev_alloc(ctx, &m->urows, urows.size());
+    if (!rc) rc = dev_alloc(ctx, &m->ptr, n ? ptr.size() : 0);
+    if (!rc) rc = dev_alloc(ctx, &m->slots, (size_t)n);
     if (!rc) rc = copy_h2d(ctx, m->rows, rows, (size_t)n * 4);
     if (!rc) rc = copy_h2d(ctx, m->urows, urows.data(), urows.size() * 4);
     if (!rc && n) rc = copy_h2d(ctx, m->ptr, ptr.data(), ptr.size() * 4);

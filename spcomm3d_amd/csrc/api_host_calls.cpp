@@ -368,10 +368,12 @@ int spc3d_host_cache_clear(spc3d_ctx *ctx)
     if (!live(ctx))
         return fail(SPC3D_ERR_INVALID_ARG, "context is NULL or destroyed");
     std::lock_guard<std::mutex> lock(ctx->host_mutex);
-    HostCallCache *hc = ctx->host_cache;
-    if (!hc)
-        return SPC3D_OK;
     (void)hipSetDevice(ctx->device);
+    HostCallCache *hc = ctx->host_cache;
+    if (!hc) {
+        ctx->pool.trim();
+        return SPC3D_OK;
+    }
     for (CachedHostPlan &e : hc->plans)
         (void)spc3d_plan_destroy(e.plan);
     for (auto &e : hc->panels)
@@ -380,6 +382,7 @@ int spc3d_host_cache_clear(spc3d_ctx *ctx)
         (void)spc3d_vals_destroy(hc->c);
     delete hc;
     ctx->host_cache = nullptr;
+    ctx->pool.trim();
     return SPC3D_OK;
 }
 

@@ -21,6 +21,7 @@
 #include <system_error>
 #include <vector>
 
+#include "dev_pool.h"
 #include "host_cache.h"
 #include "kernels.h"
 #include "plan_device.h"
@@ -88,6 +89,7 @@ struct spc3d_ctx {
     bool use_host_cache;       // false: the one-shot calls keep nothing between calls
     unsigned host_threads;     // host threads a one-shot call may use, the caller's included
     std::mutex host_mutex;     // the one-shot calls of a context run one at a time
+    DevPool pool;              // device memory of plans and of the plan builder
 };
 
 struct spc3d_panel {
@@ -275,24 +277,29 @@ inline int use_device(const spc3d_ctx *ctx, bool capturable = false)
     return SPC3D_OK;
 }
 
-template <typename T> int dev_alloc(T **out, size_t count)
-{
-    *out = nullptr;
-    if (count == 0)
-        return SPC3D_OK;
-    if (count > SIZE_MAX / sizeof(T))
-        return fail(SPC3D_ERR_TOO_LARGE, "allocation size overflows");
-    HIP_TRY(hipMalloc((void **)out, count * sizeof(T)));
-    return SPC3D_OK;
-}
-
-inline int dev_alloc_bytes(void **out, size_t bytes)
+// Device memory that callers may see (panels, value vectors, row maps); kept blocks of the
+// context's pool give way to it.
+inline int dev_alloc_bytes(spc3d_ctx *ctx, void **out, size_t bytes)
 {
     *out = nullptr;
     if (bytes == 0)
         return SPC3D_OK;
-    HIP_TRY(hipMalloc(out, bytes));
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ctx->pool.trim();
+        e = hipMalloc(out, bytes);
+    }
+    if (e != hipSuccess)
+        return fail_hip(e, "hipMalloc");
     return SPC3D_OK;
+}
+template <typename T> int dev_alloc(spc3d_ctx *ctx, T **out, size_t count)
+{
+    *out = nullptr;
+    if (count > SIZE_MAX / sizeof(T))
+        return fail(SPC3D_ERR_TOO_LARGE, "allocation size overflows");
+    return dev_alloc_bytes(ctx, (void **)out, count * sizeof(T));
 }
 
 // Pageable-host <-> device copy ordered after everything queued on the
@@ -315,31 +322,50 @@ inline int copy_d2h(spc3d_ctx *ctx, void *dst, const void *src, size_t bytes)
     return SPC3D_OK;
 }
 
+// The same out of the context's pool: memory of plans and scratch of calls, used on the
+// context's stream only.
+template <typename T> int ctx_alloc(spc3d_ctx *ctx, T **out, size_t count)
+{
+    *out = nullptr;
+    if (count > SIZE_MAX / sizeof(T))
+        return fail(SPC3D_ERR_TOO_LARGE, "allocation size overflows");
+    HIP_TRY(ctx->pool.get((void **)out, count * sizeof(T)));
+    return SPC3D_OK;
+}
+inline int ctx_alloc_bytes(spc3d_ctx *ctx, void **out, size_t bytes)
+{
+    HIP_TRY(ctx->pool.get(out, bytes));
+    return SPC3D_OK;
+}
+inline void ctx_free(spc3d_ctx *ctx, void *p) { ctx->pool.put(p); }
+
+inline DevStream dev_stream(spc3d_ctx *ctx) { return DevStream{ctx->stream, &ctx->pool}; }
+
 inline void plan_free_device(spc3d_plan *p)
 {
-    if (p->segs) (void)hipFree(p->segs);
-    if (p->col) (void)hipFree(p->col);
-    if (p->perm) (void)hipFree(p->perm);
-    if (p->sval) (void)hipFree(p->sval);
-    if (p->splits) (void)hipFree(p->splits);
-    if (p->first_cols) (void)hipFree(p->first_cols);
-    if (p->store.perm2) (void)hipFree(p->store.perm2);
-    if (p->store.dst) (void)hipFree(p->store.dst);
-    if (p->store.src) (void)hipFree(p->store.src);
+    if (p->segs) ctx_free(p->ctx, p->segs);
+    if (p->col) ctx_free(p->ctx, p->col);
+    if (p->perm) ctx_free(p->ctx, p->perm);
+    if (p->sval) ctx_free(p->ctx, p->sval);
+    if (p->splits) ctx_free(p->ctx, p->splits);
+    if (p->first_cols) ctx_free(p->ctx, p->first_cols);
+    if (p->store.perm2) ctx_free(p->ctx, p->store.perm2);
+    if (p->store.dst) ctx_free(p->ctx, p->store.dst);
+    if (p->store.src) ctx_free(p->ctx, p->store.src);
     if ((p->store.n || p->two.n) && p->c_stage) {
-        (void)hipFree(p->c_stage);
+        ctx_free(p->ctx, p->c_stage);
         p->c_stage = nullptr;
     }
     p->store = StoreStaging();
-    if (p->two.l1) (void)hipFree(p->two.l1);
-    if (p->two.dst1) (void)hipFree(p->two.dst1);
-    if (p->two.l2) (void)hipFree(p->two.l2);
-    if (p->c_mid) (void)hipFree(p->c_mid);
+    if (p->two.l1) ctx_free(p->ctx, p->two.l1);
+    if (p->two.dst1) ctx_free(p->ctx, p->two.dst1);
+    if (p->two.l2) ctx_free(p->ctx, p->two.l2);
+    if (p->c_mid) ctx_free(p->ctx, p->c_mid);
     p->two = TwoPass();
     p->c_mid = nullptr;
-    if (p->partial) (void)hipFree(p->partial);
+    if (p->partial) ctx_free(p->ctx, p->partial);
     for (void *old : p->retired_partial)
-        (void)hipFree(old);
+        ctx_free(p->ctx, old);
     p->retired_partial.clear();
     p->retired_bytes = 0;
     p->segs = nullptr;

@@ -125,7 +125,7 @@ int spc3d_plan_build_host(int dtype, uint32_t nrows, uint32_t ncols, uint64_t nn
 static int finish_plan(spc3d_plan *p, uint32_t k0)
 {
     const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
-    int rc = dev_alloc(&p->first_cols, (size_t)nshort * kFirstCols);
+    int rc = ctx_alloc(p->ctx, &p->first_cols, (size_t)nshort * kFirstCols);
     if (rc)
         return rc;
     HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->col, p->first_cols,
@@ -173,7 +173,7 @@ static int add_store_staging(spc3d_plan *p, const StoreOpts &so)
         return SPC3D_OK;
     std::string err;
     StoreStaging st;
-    int rc = build_store_staging(p->ctx->stream, p->segs, p->info.nsegments_padded, p->perm,
+    int rc = build_store_staging(dev_stream(p->ctx), p->segs, p->info.nsegments_padded, p->perm,
                                  p->info.nnz, st, err);
     if (rc)
         return optional_path(fail(rc, err));
@@ -181,11 +181,11 @@ static int add_store_staging(spc3d_plan *p, const StoreOpts &so)
     p->info.positions_by_segment = st.consecutive ? 1 : 0;
     if (!st.n)
         return SPC3D_OK;
-    rc = dev_alloc_bytes(&p->c_stage, (size_t)st.n * elem_size(p->dtype));
+    rc = ctx_alloc_bytes(p->ctx, &p->c_stage, (size_t)st.n * elem_size(p->dtype));
     if (rc) {
-        (void)hipFree(st.perm2);
-        (void)hipFree(st.dst);
-        (void)hipFree(st.src);
+        ctx_free(p->ctx, st.perm2);
+        ctx_free(p->ctx, st.dst);
+        ctx_free(p->ctx, st.src);
         p->store = StoreStaging();
         p->info.positions_by_segment = 0;
         return optional_path(rc);
@@ -212,20 +212,20 @@ static int add_two_pass(spc3d_plan *p, const StoreOpts &so)
         return SPC3D_OK;
     std::string err;
     TwoPass tp;
-    int rc = build_two_pass(p->ctx->stream, p->perm, p->info.nnz, two_pass_tile_elems(p->dtype), tp,
+    int rc = build_two_pass(dev_stream(p->ctx), p->perm, p->info.nnz, two_pass_tile_elems(p->dtype), tp,
                             err);
     if (rc)
         return optional_path(fail(rc, err));
     if (!tp.n)
         return SPC3D_OK;
     const size_t bytes = (size_t)p->info.nnz * elem_size(p->dtype);
-    rc = dev_alloc_bytes(&p->c_stage, bytes);
-    if (!rc) rc = dev_alloc_bytes(&p->c_mid, bytes);
+    rc = ctx_alloc_bytes(p->ctx, &p->c_stage, bytes);
+    if (!rc) rc = ctx_alloc_bytes(p->ctx, &p->c_mid, bytes);
     if (rc) {
-        (void)hipFree(tp.l1);
-        (void)hipFree(tp.dst1);
-        (void)hipFree(tp.l2);
-        if (p->c_stage) (void)hipFree(p->c_stage);
+        ctx_free(p->ctx, tp.l1);
+        ctx_free(p->ctx, tp.dst1);
+        ctx_free(p->ctx, tp.l2);
+        if (p->c_stage) ctx_free(p->ctx, p->c_stage);
         p->c_stage = nullptr;
         return optional_path(rc);
     }
@@ -251,13 +251,13 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
         fill_info(p->info, meta);
         p->info.nsegments_padded = arr.nseg_padded;
         p->info.nsplit_rows = arr.nsplit;
-        rc = dev_alloc_bytes(&p->sval, (size_t)meta.nnz * elem_size(dtype));
+        rc = ctx_alloc_bytes(ctx, &p->sval, (size_t)meta.nnz * elem_size(dtype));
     }
     if (rc) {
-        if (arr.segs) (void)hipFree(arr.segs);
-        if (arr.col) (void)hipFree(arr.col);
-        if (arr.perm) (void)hipFree(arr.perm);
-        if (arr.splits) (void)hipFree(arr.splits);
+        if (arr.segs) ctx_free(ctx, arr.segs);
+        if (arr.col) ctx_free(ctx, arr.col);
+        if (arr.perm) ctx_free(ctx, arr.perm);
+        if (arr.splits) ctx_free(ctx, arr.splits);
         delete p;
         return rc;
     }
@@ -285,17 +285,17 @@ static void destroy_blocks(spc3d_plan *p)
         delete b;
     }
     p->blocks.clear();
-    if (p->c_stage) (void)hipFree(p->c_stage);
-    if (p->stage_pos) (void)hipFree(p->stage_pos);
-    if (p->stage_of) (void)hipFree(p->stage_of);
+    if (p->c_stage) ctx_free(p->ctx, p->c_stage);
+    if (p->stage_pos) ctx_free(p->ctx, p->stage_pos);
+    if (p->stage_of) ctx_free(p->ctx, p->stage_of);
     p->c_stage = nullptr;
     p->stage_pos = p->stage_of = nullptr;
-    if (p->sweep.perm) (void)hipFree(p->sweep.perm);
-    if (p->sweep.col) (void)hipFree(p->sweep.col);
-    if (p->sweep.lrow) (void)hipFree(p->sweep.lrow);
-    if (p->sweep.ptr) (void)hipFree(p->sweep.ptr);
-    if (p->sweep.tile_rows) (void)hipFree(p->sweep.tile_rows);
-    if (p->sweep_sval) (void)hipFree(p->sweep_sval);
+    if (p->sweep.perm) ctx_free(p->ctx, p->sweep.perm);
+    if (p->sweep.col) ctx_free(p->ctx, p->sweep.col);
+    if (p->sweep.lrow) ctx_free(p->ctx, p->sweep.lrow);
+    if (p->sweep.ptr) ctx_free(p->ctx, p->sweep.ptr);
+    if (p->sweep.tile_rows) ctx_free(p->ctx, p->sweep.tile_rows);
+    if (p->sweep_sval) ctx_free(p->ctx, p->sweep_sval);
     p->sweep = SweepPlan();
     p->sweep_sval = nullptr;
 }
@@ -330,7 +330,7 @@ static int choose_col_blocks(spc3d_plan *p, const spc3d_plan_opts *opts, uint32_
     const uint64_t nb = std::min<uint64_t>((panel + kBlockBytes - 1) / kBlockBytes, 256);
     uint64_t sumsq = 0;
     std::string err;
-    int rc = sum_sq_seg_len_device(p->ctx->stream, p->segs, I.nsegments_padded, &sumsq, err);
+    int rc = sum_sq_seg_len_device(dev_stream(p->ctx), p->segs, I.nsegments_padded, &sumsq, err);
     if (rc != SPC3D_OK)
         return fail(rc, err);
     const double wmean = (double)sumsq / (double)I.nnz;
@@ -350,14 +350,14 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
         return SPC3D_OK;
     std::string err;
     bool sorted = false;
-    int rc = is_nondecreasing_device(p->ctx->stream, d_jj, nnz, &sorted, err);
+    int rc = is_nondecreasing_device(dev_stream(p->ctx), d_jj, nnz, &sorted, err);
     if (rc)
         return fail(rc, err);
     if (!sorted)
         return SPC3D_OK;
     HostPlan meta;
     DevPlanArrays arr;
-    rc = build_device_plan(p->ctx->stream, ncols, nrows, nnz, d_jj, d_ii, po, meta, arr, err);
+    rc = build_device_plan(dev_stream(p->ctx), ncols, nrows, nnz, d_jj, d_ii, po, meta, arr, err);
     if (rc)
         return optional_path(fail(rc, err));
     spc3d_plan *q = nullptr;
@@ -425,7 +425,7 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
     const uint32_t per_launch = (uint32_t)std::max(1, ctx->cu_count);
     std::string err;
     SweepPlan sw;
-    int rc = build_sweep(ctx->stream, nrows, ncols, nnz, d_ii, d_jj, lanes,
+    int rc = build_sweep(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj, lanes,
                          sweep_rows_per_tile(lanes), nb, min_row, per_launch, sw, err);
     if (rc)
         return optional_path(fail(rc, err));
@@ -437,15 +437,15 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
     uint32_t *r_ii = nullptr, *r_jj = nullptr, *gperm = nullptr, *stage_pos = nullptr;
     void *c_stage = nullptr, *sval = nullptr;
     if (nrest) {
-        rc = dev_alloc(&r_ii, (size_t)nrest);
-        if (!rc) rc = dev_alloc(&r_jj, (size_t)nrest);
-        if (!rc) rc = dev_alloc(&gperm, (size_t)nrest);
+        rc = ctx_alloc(ctx, &r_ii, (size_t)nrest);
+        if (!rc) rc = ctx_alloc(ctx, &r_jj, (size_t)nrest);
+        if (!rc) rc = ctx_alloc(ctx, &gperm, (size_t)nrest);
         if (!rc) {
-            rc = gather_u32_device(ctx->stream, d_ii, sw.perm + sw.n, nrest, r_ii, err);
-            if (!rc) rc = gather_u32_device(ctx->stream, d_jj, sw.perm + sw.n, nrest, r_jj, err);
+            rc = gather_u32_device(dev_stream(ctx), d_ii, sw.perm + sw.n, nrest, r_ii, err);
+            if (!rc) rc = gather_u32_device(dev_stream(ctx), d_jj, sw.perm + sw.n, nrest, r_jj, err);
             HostPlan meta;
             DevPlanArrays arr;
-            if (!rc) rc = build_device_plan(ctx->stream, nrows, ncols, nrest, r_ii, r_jj, po, meta, arr, err);
+            if (!rc) rc = build_device_plan(dev_stream(ctx), nrows, ncols, nrest, r_ii, r_jj, po, meta, arr, err);
             if (rc)
                 fail(rc, err);
             else
@@ -453,7 +453,7 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
         }
         if (!rc) {
             // the rest's kernel order -> the caller's positions
-            rc = compose_perm_device(ctx->stream, sw.perm + sw.n, child->perm, nrest, gperm, err);
+            rc = compose_perm_device(dev_stream(ctx), sw.perm + sw.n, child->perm, nrest, gperm, err);
             if (rc)
                 fail(rc, err);
         }
@@ -463,7 +463,7 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
                 rc = fail_hip(e, "hipStreamSynchronize");
         }
         if (!rc) {
-            if (child->perm) (void)hipFree(child->perm);
+            if (child->perm) ctx_free(ctx, child->perm);
             child->perm = gperm;
             gperm = nullptr;
             child->info.order_is_identity = 0;
@@ -476,18 +476,18 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
     bool staged = (opts->flags & SPC3D_PLAN_SWEEP_STAGED) != 0;
     if (!rc && !staged) {
         uint64_t adjacent = 0;
-        rc = count_adjacent_device(ctx->stream, sw.perm, sw.n, &adjacent, err);
+        rc = count_adjacent_device(dev_stream(ctx), sw.perm, sw.n, &adjacent, err);
         if (rc)
             fail(rc, err);
         staged = adjacent * 5 < sw.n * 4;
     }
-    if (!rc && staged) rc = dev_alloc_bytes(&c_stage, (size_t)(rest_off + nrest) * w);
-    if (!rc && staged) rc = dev_alloc(&stage_pos, (size_t)nnz);
-    if (!rc) rc = dev_alloc_bytes(&sval, (size_t)sw.n * w);
+    if (!rc && staged) rc = ctx_alloc_bytes(ctx, &c_stage, (size_t)(rest_off + nrest) * w);
+    if (!rc && staged) rc = ctx_alloc(ctx, &stage_pos, (size_t)nnz);
+    if (!rc) rc = ctx_alloc_bytes(ctx, &sval, (size_t)sw.n * w);
     if (!rc && staged) {
-        rc = inverse_offsets_device(ctx->stream, sw.perm, sw.n, 0, stage_pos, err);
+        rc = inverse_offsets_device(dev_stream(ctx), sw.perm, sw.n, 0, stage_pos, err);
         if (!rc && nrest)
-            rc = inverse_offsets_device(ctx->stream, child->perm, nrest, (uint32_t)rest_off, stage_pos, err);
+            rc = inverse_offsets_device(dev_stream(ctx), child->perm, nrest, (uint32_t)rest_off, stage_pos, err);
         if (rc)
             fail(rc, err);
     }
@@ -496,9 +496,9 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
         if (e != hipSuccess)
             rc = fail_hip(e, "hipStreamSynchronize");
     }
-    if (r_ii) (void)hipFree(r_ii);
-    if (r_jj) (void)hipFree(r_jj);
-    if (gperm) (void)hipFree(gperm);
+    if (r_ii) ctx_free(ctx, r_ii);
+    if (r_jj) ctx_free(ctx, r_jj);
+    if (gperm) ctx_free(ctx, gperm);
     if (rc) {
         const std::string keep = g_err;
         if (child) {
@@ -506,11 +506,11 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
             child->magic = 0;
             delete child;
         }
-        if (c_stage) (void)hipFree(c_stage);
-        if (stage_pos) (void)hipFree(stage_pos);
-        if (sval) (void)hipFree(sval);
-        (void)hipFree(sw.perm), (void)hipFree(sw.col), (void)hipFree(sw.lrow), (void)hipFree(sw.ptr),
-            (void)hipFree(sw.tile_rows);
+        if (c_stage) ctx_free(ctx, c_stage);
+        if (stage_pos) ctx_free(ctx, stage_pos);
+        if (sval) ctx_free(ctx, sval);
+        ctx_free(ctx, sw.perm), ctx_free(ctx, sw.col), ctx_free(ctx, sw.lrow), ctx_free(ctx, sw.ptr),
+            ctx_free(ctx, sw.tile_rows);
         return optional_path(fail(rc, keep));
     }
     // the whole pattern's arrays give way
@@ -526,9 +526,9 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
             plan_free_device(child);
             child->magic = 0;
             delete child;
-            (void)hipFree(c_stage), (void)hipFree(stage_pos), (void)hipFree(sval);
-            (void)hipFree(sw.perm), (void)hipFree(sw.col), (void)hipFree(sw.lrow),
-                (void)hipFree(sw.ptr), (void)hipFree(sw.tile_rows);
+            ctx_free(ctx, c_stage), ctx_free(ctx, stage_pos), ctx_free(ctx, sval);
+            ctx_free(ctx, sw.perm), ctx_free(ctx, sw.col), ctx_free(ctx, sw.lrow),
+                ctx_free(ctx, sw.ptr), ctx_free(ctx, sw.tile_rows);
             return fail(SPC3D_ERR_ALLOC, "host allocation failed");
         }
         I.nsegments = child->info.nsegments;
@@ -563,7 +563,7 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     HostPlan meta;
     DevPlanArrays arr;
     std::string err;
-    int rc = build_device_plan(ctx->stream, nrows, ncols, nnz, d_ii, d_jj, po, meta, arr, err);
+    int rc = build_device_plan(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj, po, meta, arr, err);
     if (rc != SPC3D_OK)
         return fail(rc, err);
     spc3d_plan *p = nullptr;
@@ -616,11 +616,11 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         spc3d_plan_destroy(p);
         return fail(SPC3D_ERR_ALLOC, "host allocation failed");
     }
-    rc = dev_alloc(&b_ii, (size_t)nnz);
-    if (!rc) rc = dev_alloc(&b_jj, (size_t)nnz);
-    if (!rc) rc = dev_alloc(&order, (size_t)nnz);
+    rc = ctx_alloc(ctx, &b_ii, (size_t)nnz);
+    if (!rc) rc = ctx_alloc(ctx, &b_jj, (size_t)nnz);
+    if (!rc) rc = ctx_alloc(ctx, &order, (size_t)nnz);
     if (!rc) {
-        rc = partition_by_col_block(ctx->stream, nnz, d_ii, d_jj, ncols, nb, b_ii, b_jj, order,
+        rc = partition_by_col_block(dev_stream(ctx), nnz, d_ii, d_jj, ncols, nb, b_ii, b_jj, order,
                                     first.data(), err);
         if (rc)
             fail(rc, err);
@@ -630,7 +630,7 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     const uint32_t rows_per_tile = (uint32_t)std::max<uint64_t>(
         1, ((uint64_t)2 << 20) / (per_row * elem_size(dtype)));
     uint32_t *tile_key = nullptr;
-    if (!rc) rc = dev_alloc(&tile_key, (size_t)nnz);
+    if (!rc) rc = ctx_alloc(ctx, &tile_key, (size_t)nnz);
     spc3d_plan_info total = p->info;
     total.nsegments = total.nsegments_padded = total.nsplit_rows = total.npartial_slots = 0;
     total.nsegments_long = 0;
@@ -641,7 +641,7 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
             continue;
         HostPlan bmeta;
         DevPlanArrays barr;
-        rc = build_device_plan(ctx->stream, nrows, ncols, cnt, b_ii + first[b], b_jj + first[b], po,
+        rc = build_device_plan(dev_stream(ctx), nrows, ncols, cnt, b_ii + first[b], b_jj + first[b], po,
                                bmeta, barr, err);
         if (rc) {
             fail(rc, err);
@@ -652,30 +652,30 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         if (rc)
             break;
         p->blocks.push_back(child);
-        rc = tile_keys_device(ctx->stream, b_ii + first[b], child->perm, cnt, rows_per_tile,
+        rc = tile_keys_device(dev_stream(ctx), b_ii + first[b], child->perm, cnt, rows_per_tile,
                               tile_key + first[b], err);
         if (rc) {
             fail(rc, err);
             break;
         }
         uint32_t *gperm = nullptr;
-        rc = dev_alloc(&gperm, (size_t)cnt);
+        rc = ctx_alloc(ctx, &gperm, (size_t)cnt);
         if (!rc) {
-            rc = compose_perm_device(ctx->stream, order + first[b], child->perm, cnt, gperm, err);
+            rc = compose_perm_device(dev_stream(ctx), order + first[b], child->perm, cnt, gperm, err);
             if (rc)
                 fail(rc, err);
         }
         if (rc) {
-            if (gperm) (void)hipFree(gperm);
+            if (gperm) ctx_free(ctx, gperm);
             break;
         }
         hipError_t e = hipStreamSynchronize(ctx->stream); // child->perm is read until here
         if (e != hipSuccess) {
-            (void)hipFree(gperm);
+            ctx_free(ctx, gperm);
             rc = fail_hip(e, "hipStreamSynchronize");
             break;
         }
-        if (child->perm) (void)hipFree(child->perm);
+        if (child->perm) ctx_free(ctx, child->perm);
         child->perm = gperm;
         child->stage_off = first[b];
         child->col_base = b * ((ncols + nb - 1) / nb);
@@ -687,11 +687,11 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         total.npartial_slots = std::max(total.npartial_slots, child->info.npartial_slots);
         total.nqueues = std::max(total.nqueues, child->info.nqueues);
     }
-    if (!rc) rc = dev_alloc_bytes(&p->c_stage, (size_t)nnz * elem_size(dtype));
-    if (!rc) rc = dev_alloc(&p->stage_pos, (size_t)nnz);
-    if (!rc) rc = dev_alloc(&p->stage_of, (size_t)nnz);
+    if (!rc) rc = ctx_alloc_bytes(ctx, &p->c_stage, (size_t)nnz * elem_size(dtype));
+    if (!rc) rc = ctx_alloc(ctx, &p->stage_pos, (size_t)nnz);
+    if (!rc) rc = ctx_alloc(ctx, &p->stage_of, (size_t)nnz);
     if (!rc) {
-        rc = stable_ranks_device(ctx->stream, tile_key, nnz, (nrows - 1) / rows_per_tile,
+        rc = stable_ranks_device(dev_stream(ctx), tile_key, nnz, (nrows - 1) / rows_per_tile,
                                  p->stage_of, err);
         if (rc)
             fail(rc, err);
@@ -700,15 +700,15 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         if (rc)
             break;
         // stage_pos[caller's position of entry q] = its staging position
-        rc = scatter_device(ctx->stream, child->perm, p->stage_of + child->stage_off,
+        rc = scatter_device(dev_stream(ctx), child->perm, p->stage_of + child->stage_off,
                             child->info.nnz, p->stage_pos, err);
         if (rc)
             fail(rc, err);
     }
-    if (tile_key) (void)hipFree(tile_key);
-    if (b_ii) (void)hipFree(b_ii);
-    if (b_jj) (void)hipFree(b_jj);
-    if (order) (void)hipFree(order);
+    if (tile_key) ctx_free(ctx, tile_key);
+    if (b_ii) ctx_free(ctx, b_ii);
+    if (b_jj) ctx_free(ctx, b_jj);
+    if (order) ctx_free(ctx, order);
     if (rc) {
         std::string keep = g_err;
         spc3d_plan_destroy(p);
@@ -771,14 +771,14 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
             return rc;
         // The pattern goes up as it is; validation and everything else happens there.
         uint32_t *d_ii = nullptr, *d_jj = nullptr;
-        rc = dev_alloc(&d_ii, (size_t)nnz);
-        if (!rc) rc = dev_alloc(&d_jj, (size_t)nnz);
+        rc = ctx_alloc(ctx, &d_ii, (size_t)nnz);
+        if (!rc) rc = ctx_alloc(ctx, &d_jj, (size_t)nnz);
         if (!rc) rc = copy_h2d(ctx, d_ii, ii, (size_t)nnz * sizeof(uint32_t));
         if (!rc) rc = copy_h2d(ctx, d_jj, jj, (size_t)nnz * sizeof(uint32_t));
         if (!rc)
             rc = build_from_device(ctx, dtype, nrows, ncols, nnz, d_ii, d_jj, po, opts, &p);
-        if (d_ii) (void)hipFree(d_ii);
-        if (d_jj) (void)hipFree(d_jj);
+        if (d_ii) ctx_free(ctx, d_ii);
+        if (d_jj) ctx_free(ctx, d_jj);
         if (rc)
             return rc;
     } else {
@@ -802,11 +802,11 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
         p->dtype = dtype;
         fill_info(p->info, H);
 
-        rc = dev_alloc(&p->segs, H.segs.size());
-        if (!rc) rc = dev_alloc(&p->col, (size_t)nnz);
-        if (!rc && !H.identity) rc = dev_alloc(&p->perm, (size_t)nnz);
-        if (!rc) rc = dev_alloc_bytes(&p->sval, (size_t)nnz * elem_size(dtype));
-        if (!rc) rc = dev_alloc(&p->splits, H.splits.size());
+        rc = ctx_alloc(ctx, &p->segs, H.segs.size());
+        if (!rc) rc = ctx_alloc(ctx, &p->col, (size_t)nnz);
+        if (!rc && !H.identity) rc = ctx_alloc(ctx, &p->perm, (size_t)nnz);
+        if (!rc) rc = ctx_alloc_bytes(ctx, &p->sval, (size_t)nnz * elem_size(dtype));
+        if (!rc) rc = ctx_alloc(ctx, &p->splits, H.splits.size());
         if (!rc) rc = copy_h2d(ctx, p->segs, H.segs.data(), H.segs.size() * sizeof(Seg));
         if (!rc) rc = copy_h2d(ctx, p->col, H.col.data(), (size_t)nnz * sizeof(uint32_t));
         if (!rc && !H.identity)
@@ -850,7 +850,7 @@ int spc3d_localize_device(spc3d_ctx *ctx, uint64_t n, void *dev_idx, void *dev_l
     if (rc)
         return rc;
     std::string err;
-    rc = localize_device(ctx->stream, n, (uint32_t *)dev_idx, (uint32_t *)dev_ltg, nlocal, err);
+    rc = localize_device(dev_stream(ctx), n, (uint32_t *)dev_idx, (uint32_t *)dev_ltg, nlocal, err);
     return rc == SPC3D_OK ? rc : fail(rc, err);
 }
 
@@ -865,7 +865,7 @@ int spc3d_remap_device(spc3d_ctx *ctx, uint64_t n, void *dev_idx, const void *de
     if (rc)
         return rc;
     std::string err;
-    rc = remap_device(ctx->stream, n, (uint32_t *)dev_idx, (const uint32_t *)dev_map, map_len,
+    rc = remap_device(dev_stream(ctx), n, (uint32_t *)dev_idx, (const uint32_t *)dev_map, map_len,
                       err);
     return rc == SPC3D_OK ? rc : fail(rc, err);
 }
@@ -1008,7 +1008,7 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
         rc = copy_h2d(plan->ctx, plan->sval, vv_host, bytes);
     } else {
         void *tmp = nullptr;
-        rc = dev_alloc_bytes(&tmp, bytes);
+        rc = ctx_alloc_bytes(plan->ctx, &tmp, bytes);
         if (rc)
             return rc;
         rc = copy_h2d(plan->ctx, tmp, vv_host, bytes);
@@ -1039,7 +1039,7 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
             if (e != hipSuccess)
                 rc = fail_hip(e, "gather of sparse values");
         }
-        (void)hipFree(tmp);
+        ctx_free(plan->ctx, tmp);
     }
     if (!rc)
         plan->has_values = true;
@@ -1169,13 +1169,13 @@ static int build_other_k(spc3d_plan *S, uint32_t K)
     void *vals = nullptr;
     spc3d_plan *q = nullptr;
     std::string err;
-    rc = dev_alloc(&d_ii, (size_t)nnz);
-    if (!rc) rc = dev_alloc(&d_jj, (size_t)nnz);
+    rc = ctx_alloc(ctx, &d_ii, (size_t)nnz);
+    if (!rc) rc = ctx_alloc(ctx, &d_jj, (size_t)nnz);
     if (!rc) {
-        rc = sweep_coords_device(ctx->stream, S->sweep, d_ii, d_jj, err);
+        rc = sweep_coords_device(dev_stream(ctx), S->sweep, d_ii, d_jj, err);
         for (spc3d_plan *part : S->blocks)
             if (!rc)
-                rc = seg_coords_device(ctx->stream, part->segs, part->info.nsegments_padded,
+                rc = seg_coords_device(dev_stream(ctx), part->segs, part->info.nsegments_padded,
                                        part->col, part->perm, d_ii, d_jj, err);
         if (rc)
             fail(rc, err);
@@ -1183,7 +1183,7 @@ static int build_other_k(spc3d_plan *S, uint32_t K)
     if (!rc)
         rc = build_from_device(ctx, S->dtype, S->info.nrows, S->info.ncols, nnz, d_ii, d_jj, po, &o, &q);
     if (!rc && S->has_values) {
-        rc = dev_alloc_bytes(&vals, (size_t)nnz * w);
+        rc = ctx_alloc_bytes(ctx, &vals, (size_t)nnz * w);
         if (!rc) {
             hipError_t e = launch_scatter_vals(S->dtype, S->sweep_sval, S->sweep.perm, vals,
                                                S->sweep.n, ctx->stream);
@@ -1214,9 +1214,9 @@ static int build_other_k(spc3d_plan *S, uint32_t K)
         if (e != hipSuccess)
             rc = fail_hip(e, "hipStreamSynchronize");
     }
-    if (d_ii) (void)hipFree(d_ii);
-    if (d_jj) (void)hipFree(d_jj);
-    if (vals) (void)hipFree(vals);
+    if (d_ii) ctx_free(ctx, d_ii);
+    if (d_jj) ctx_free(ctx, d_jj);
+    if (vals) ctx_free(ctx, vals);
     if (rc) {
         const std::string keep = g_err;
         if (q)
@@ -1283,7 +1283,7 @@ int ensure_partial(spc3d_plan *p, uint32_t K)
                     "the plan's partial-sum rows are narrower than this K: create the plan with "
                     "k_hint >= K, or run the call once before recording it");
     void *grown = nullptr;
-    int rc = dev_alloc_bytes(&grown, (size_t)p->info.npartial_slots * K * elem_size(p->dtype));
+    int rc = ctx_alloc_bytes(p->ctx, &grown, (size_t)p->info.npartial_slots * K * elem_size(p->dtype));
     if (rc)
         return rc;
     if (p->partial) {
@@ -1291,7 +1291,7 @@ int ensure_partial(spc3d_plan *p, uint32_t K)
             p->retired_partial.push_back(p->partial);
             p->retired_bytes += (uint64_t)p->info.npartial_slots * p->partial_k * elem_size(p->dtype);
         } catch (const std::bad_alloc &) {
-            (void)hipFree(grown);
+            ctx_free(p->ctx, grown);
             return fail(SPC3D_ERR_ALLOC, "host allocation failed");
         }
     }

@@ -1,0 +1,144 @@
+// Device memory of the plans and of the plan builder's scratch, kept between plans.
+//
+// A program that plans a new pattern every few calls (the reference remaps its indices before
+// every group of five, miniapp/bench_both.cpp:196-205) asks for some thirty arrays of the same
+// sizes each time, and hipMalloc and hipFree of blocks this large map and unmap memory and wait
+// for the device: R-MAT 20, plan + ten calls + destruction, 182 ms with them in a process that
+// also holds other device memory, of which the kernels are 20.
+//
+// One pool per context.  Everything that touches a block runs on the context's stream (or is
+// joined back to it), so a block can be handed out again at once: what uses it next is queued
+// behind what used it last.  Panels and value vectors, whose addresses callers may hand to other
+// streams, do not come from here.
+//
+// Bounded: at most `limit` bytes are kept; beyond that the blocks unused for longest are freed.
+// Given back: by trim() (spc3d_host_cache_clear), when an allocation fails, and with the context.
+#pragma once
+#include <hip/hip_runtime_api.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <map>
+#include <mutex>
+#include <new>
+#include <unordered_map>
+
+namespace spc3d {
+
+class DevPool {
+  public:
+    DevPool() = default;
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+    ~DevPool() { trim(); }
+
+    void set_limit(size_t bytes) { limit_ = bytes; }
+
+    // A block of at least `bytes`; a kept one when its size is within a quarter of that.
+    hipError_t get(void **out, size_t bytes)
+    {
+        *out = nullptr;
+        if (bytes == 0)
+            return hipSuccess;
+        if (bytes > SIZE_MAX - kGrain)
+            return hipErrorOutOfMemory;
+        bytes = (bytes + kGrain - 1) / kGrain * kGrain;
+        std::lock_guard<std::mutex> lock(mu_);
+        try {
+            auto it = kept_.lower_bound(bytes);
+            if (it != kept_.end() && it->first <= bytes + bytes / 4) {
+                void *p = it->second.p;
+                sizes_.emplace(p, it->first);
+                kept_bytes_ -= it->first;
+                kept_.erase(it);
+                *out = p;
+                return hipSuccess;
+            }
+            void *p = nullptr;
+            hipError_t e = hipMalloc(&p, bytes);
+            if (e != hipSuccess && !kept_.empty()) {
+                (void)hipGetLastError();
+                shrink(0);
+                e = hipMalloc(&p, bytes);
+            }
+            if (e != hipSuccess)
+                return e;
+            try {
+                sizes_.emplace(p, bytes);
+            } catch (const std::bad_alloc &) {
+                (void)hipFree(p);
+                return hipErrorOutOfMemory;
+            }
+            *out = p;
+            return hipSuccess;
+        } catch (const std::bad_alloc &) {
+            return hipErrorOutOfMemory;
+        }
+    }
+
+    // Takes back a block that get() handed out.
+    void put(void *p)
+    {
+        if (!p)
+            return;
+        std::lock_guard<std::mutex> lock(mu_);
+        const auto it = sizes_.find(p);
+        const size_t bytes = it == sizes_.end() ? 0 : it->second;
+        if (it != sizes_.end())
+            sizes_.erase(it);
+        if (bytes == 0 || bytes > limit_) {
+            (void)hipFree(p);
+            return;
+        }
+        try {
+            kept_.emplace(bytes, Kept{p, ++clock_});
+        } catch (const std::bad_alloc &) {
+            (void)hipFree(p);
+            return;
+        }
+        kept_bytes_ += bytes;
+        if (kept_bytes_ > limit_)
+            shrink(limit_);
+    }
+
+    // Frees every kept block.
+    void trim()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        shrink(0);
+    }
+
+  private:
+    struct Kept {
+        void *p;
+        uint64_t since;
+    };
+    // Frees kept blocks, the ones unused for longest first, until at most `to` bytes are kept.
+    void shrink(size_t to)
+    {
+        while (kept_bytes_ > to && !kept_.empty()) {
+            auto oldest = kept_.begin();
+            for (auto it = kept_.begin(); it != kept_.end(); ++it)
+                if (it->second.since < oldest->second.since)
+                    oldest = it;
+            (void)hipFree(oldest->second.p);
+            kept_bytes_ -= oldest->first;
+            kept_.erase(oldest);
+        }
+    }
+    static constexpr size_t kGrain = 512;
+    std::mutex mu_;
+    std::multimap<size_t, Kept> kept_; // by size
+    std::unordered_map<void *, size_t> sizes_; // of the blocks handed out
+    size_t kept_bytes_ = 0, limit_ = 0;
+    uint64_t clock_ = 0;
+};
+
+// A context's stream and the pool whose blocks are used on it.
+struct DevStream {
+    hipStream_t st;
+    DevPool *pool;
+    operator hipStream_t() const { return st; }
+};
+
+} // namespace spc3d

@@ -33,7 +33,7 @@ struct Counters { // one device-resident block, zeroed (first_bad: all ones) bef
     unsigned long long pref_load[kSlices];
 };
 
-// Owning device buffer; freed on scope exit unless released.
+// Owning device buffer; back to the pool on scope exit unless released.
 template <typename T> struct DBuf {
     T *p = nullptr;
     DBuf() = default;
@@ -43,15 +43,14 @@ template <typename T> struct DBuf {
     void reset()
     {
         if (p)
-            (void)hipFree(p);
+            pool_->put(p);
         p = nullptr;
     }
-    hipError_t alloc(size_t count)
+    hipError_t alloc(const DevStream &st, size_t count)
     {
         reset();
-        if (count == 0)
-            return hipSuccess;
-        return hipMalloc((void **)&p, count * sizeof(T));
+        pool_ = st.pool;
+        return pool_->get((void **)&p, count * sizeof(T));
     }
     T *release()
     {
@@ -59,20 +58,22 @@ template <typename T> struct DBuf {
         p = nullptr;
         return r;
     }
+
+  private:
+    DevPool *pool_ = nullptr;
 };
 
-// Scratch device memory of one call: a few large blocks, handed out front to back
-// and freed together when the call returns.  (hipFree waits for the device: forty
-// hipMalloc / hipFree pairs per build cost more than all of its kernels.)
+// Scratch device memory of one call: a few large blocks of the pool, handed out front to
+// back and given back together when the call returns.
 class Arena {
   public:
-    Arena() = default;
+    explicit Arena(const DevStream &st) : pool_(*st.pool) {}
     Arena(const Arena &) = delete;
     Arena &operator=(const Arena &) = delete;
     ~Arena()
     {
         for (int i = 0; i < nblocks_; ++i)
-            (void)hipFree(blocks_[i]);
+            pool_.put(blocks_[i]);
     }
     // Makes sure that the next `bytes` come out of one block.
     hipError_t reserve(size_t bytes)
@@ -82,7 +83,7 @@ class Arena {
         if (nblocks_ == kMaxBlocks)
             return hipErrorOutOfMemory;
         void *b = nullptr;
-        const hipError_t e = hipMalloc(&b, bytes);
+        const hipError_t e = pool_.get(&b, bytes);
         if (e != hipSuccess)
             return e;
         blocks_[nblocks_++] = b;
@@ -108,6 +109,7 @@ class Arena {
   private:
     static constexpr int kMaxBlocks = 64;
     static constexpr size_t kMinBlock = (size_t)4 << 20;
+    DevPool &pool_;
     void *blocks_[kMaxBlocks] = {};
     int nblocks_ = 0;
     char *cur_ = nullptr;
@@ -710,8 +712,12 @@ __global__ void remap_check_k(const uint32_t *__restrict__ idx, uint64_t n, uint
         atomicMin(&C->first_bad, (uint32_t)e);
 }
 
-__global__ void remap_apply_k(uint32_t *idx, uint64_t n, const uint32_t *__restrict__ map)
+// Changes nothing when the check found an index outside the map.
+__global__ void remap_apply_k(uint32_t *idx, uint64_t n, const uint32_t *__restrict__ map,
+                              const Counters *__restrict__ C)
 {
+    if (C->first_bad != 0xFFFFFFFFu)
+        return;
     GRID_STRIDE(e, n) idx[e] = map[idx[e]];
 }
 
@@ -742,7 +748,7 @@ struct Temp {
 };
 
 template <typename T>
-int exclusive_sum(Temp &tmp, const T *in, T *out, size_t n, hipStream_t st, std::string &err)
+int exclusive_sum(Temp &tmp, const T *in, T *out, size_t n, const DevStream &st, std::string &err)
 {
     size_t bytes = 0;
     HIP_OK(rocprim::exclusive_scan(nullptr, bytes, in, out, T(0), n, rocprim::plus<T>(), st));
@@ -754,7 +760,7 @@ int exclusive_sum(Temp &tmp, const T *in, T *out, size_t n, hipStream_t st, std:
 // Stable ascending sort of (key, value) pairs on key bits [0, bits).
 template <typename KeyT>
 int sort_pairs(Temp &tmp, const KeyT *kin, KeyT *kout, const uint32_t *vin, uint32_t *vout,
-               uint32_t n, int bits, bool descending, hipStream_t st, std::string &err)
+               uint32_t n, int bits, bool descending, const DevStream &st, std::string &err)
 {
     size_t bytes = 0;
     if (descending) {
@@ -775,7 +781,7 @@ int sort_pairs(Temp &tmp, const KeyT *kin, KeyT *kout, const uint32_t *vin, uint
 
 // Ascending sort of keys on key bits [0, bits).
 int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bits,
-              hipStream_t st, std::string &err)
+              const DevStream &st, std::string &err)
 {
     size_t bytes = 0;
     HIP_OK(rocprim::radix_sort_keys(nullptr, bytes, kin, kout, (size_t)n, 0u, (unsigned)bits, st));
@@ -796,7 +802,7 @@ int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bi
             return rc_;                                                                           \
     } while (0)
 
-int fetch(hipStream_t st, void *host, const void *dev, size_t bytes, std::string &err)
+int fetch(const DevStream &st, void *host, const void *dev, size_t bytes, std::string &err)
 {
     HIP_OK(hipGetLastError());
     HIP_OK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
@@ -809,7 +815,7 @@ int fetch(hipStream_t st, void *host, const void *dev, size_t bytes, std::string
 // by_column: the entries are first brought into ascending column order (stable), so that
 // every row ends up ordered by column (col_bits: bits of the largest column id).
 template <typename KeyT>
-int order_entries(Arena &arena, Temp &tmp, hipStream_t st, uint64_t nnz, int key_bits, bool slices,
+int order_entries(Arena &arena, Temp &tmp, const DevStream &st, uint64_t nnz, int key_bits, bool slices,
                   bool by_column, int col_bits, const uint32_t *d_ii, const uint32_t *d_jj,
                   const uint32_t *hubflag, const uint8_t *cls, uint32_t *perm, uint32_t *col,
                   Counters *C, std::string &err)
@@ -897,7 +903,7 @@ __global__ void sum_sq_len_k(const Seg *__restrict__ segs, uint64_t n, unsigned 
 
 } // namespace
 
-int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz,
+int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                       const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &opts,
                       HostPlan &meta, DevPlanArrays &out, std::string &err)
 {
@@ -928,7 +934,7 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
     // One block for everything whose size is known now: ten arrays per row, five and
     // a class byte per column, the sorted column ids, two keys and an index per entry,
     // the primitives' scratch.
-    Arena arena;
+    Arena arena(st);
     const size_t key_bytes = bits_for(nrows ? nrows - 1 : 0) + 4 > 32 ? 8 : 4;
     HIP_OK(arena.reserve(((size_t)nrows + 1) * 40 + (size_t)ncols * 17 + (size_t)std::max(nrows, ncols) * 4 +
                          (size_t)nnz * (2 * key_bytes + 8) + (size_t)nnz / 2 + ((size_t)8 << 20)));
@@ -1036,8 +1042,8 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
 
     // ---- stable sort into kernel order ------------------------------------------------
     DBuf<uint32_t> perm, col;
-    HIP_OK(perm.alloc(nnz));
-    HIP_OK(col.alloc(nnz));
+    HIP_OK(perm.alloc(st, nnz));
+    HIP_OK(col.alloc(st, nnz));
     {
         const int row_bits = bits_for(nrows ? nrows - 1 : 0);
         const int key_bits = row_bits + (slices ? 4 : 0);
@@ -1082,7 +1088,7 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
     DBuf<SplitRow> splits;
     HIP_OK(pseg.alloc(arena, np_total));
     HIP_OK(pqueue.alloc(arena, np_total));
-    HIP_OK(splits.alloc(nsplit));
+    HIP_OK(splits.alloc(st, nsplit));
     LAUNCH(emit_pieces_k, nrows, rowptr.p, nrows, seg_max, slices, hubflag.p, hubpos.p, hubcnt.p,
            piece_off.p, split_off.p, slot_off.p, pseg.p, pqueue.p, splits.p);
 
@@ -1096,7 +1102,7 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
         HIP_OK(key_out.alloc(arena, np_total));
         HIP_OK(idx.alloc(arena, np_total));
         HIP_OK(idx_out.alloc(arena, np_total));
-        HIP_OK(segs.alloc(np_total));
+        HIP_OK(segs.alloc(st, np_total));
         LAUNCH_SMALL(len_keys_k, np_total, pseg.p, (uint64_t)np_total, seg_max, key.p, dC.p);
         LAUNCH(iota_k, np_total, idx.p, (uint64_t)np_total);
         TRY(sort_pairs<uint32_t>(tmp, key.p, key_out.p, idx.p, idx_out.p, np_total, len_bits,
@@ -1166,7 +1172,7 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
             return SPC3D_ERR_TOO_LARGE;
         }
         nseg_padded = (uint32_t)padded;
-        HIP_OK(segs.alloc(nseg_padded));
+        HIP_OK(segs.alloc(st, nseg_padded));
         LAUNCH(fill_k<Seg>, nseg_padded, segs.p, (uint64_t)nseg_padded, (Seg{0, 0, 0, kWholeRow}));
         LAUNCH(scatter_segs_k, np_total, pseg.p, comb_idx_out.p, comb_key_out.p,
                (uint64_t)np_total, seg_max, qs, segs.p);
@@ -1187,7 +1193,7 @@ int build_device_plan(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t n
     return SPC3D_OK;
 }
 
-int localize_device(hipStream_t st, uint64_t n, uint32_t *d_idx, uint32_t *d_ltg,
+int localize_device(const DevStream &st, uint64_t n, uint32_t *d_idx, uint32_t *d_ltg,
                     uint32_t *nlocal, std::string &err)
 {
     *nlocal = 0;
@@ -1197,7 +1203,7 @@ int localize_device(hipStream_t st, uint64_t n, uint32_t *d_idx, uint32_t *d_ltg
         err = "more than 2^32 - 1 indices are not supported";
         return SPC3D_ERR_TOO_LARGE;
     }
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve((size_t)n * 44 + ((size_t)8 << 20))); // ten arrays of at most n + 1, scratch
     Temp tmp(arena);
     SBuf<uint32_t> ident, key, pos, head, run_of;
@@ -1232,7 +1238,7 @@ int localize_device(hipStream_t st, uint64_t n, uint32_t *d_idx, uint32_t *d_ltg
     return SPC3D_OK;
 }
 
-int remap_device(hipStream_t st, uint64_t n, uint32_t *d_idx, const uint32_t *d_map,
+int remap_device(const DevStream &st, uint64_t n, uint32_t *d_idx, const uint32_t *d_map,
                  uint32_t map_len, std::string &err)
 {
     if (n == 0)
@@ -1243,9 +1249,11 @@ int remap_device(hipStream_t st, uint64_t n, uint32_t *d_idx, const uint32_t *d_
     }
     DBuf<Counters> dC;
     Counters hC;
-    HIP_OK(dC.alloc(1));
+    HIP_OK(dC.alloc(st, 1));
     HIP_OK(hipMemsetAsync(dC.p, 0xFF, sizeof(Counters), st));
+    // the check and the change queued together: one wait for both
     LAUNCH(remap_check_k, n, d_idx, n, map_len, dC.p);
+    LAUNCH(remap_apply_k, n, d_idx, n, d_map, dC.p);
     TRY(fetch(st, &hC, dC.p, sizeof hC, err));
     if (hC.first_bad != 0xFFFFFFFFu) {
         uint32_t v = 0;
@@ -1256,9 +1264,6 @@ int remap_device(hipStream_t st, uint64_t n, uint32_t *d_idx, const uint32_t *d_
         err = buf;
         return SPC3D_ERR_BAD_INDEX;
     }
-    LAUNCH(remap_apply_k, n, d_idx, n, d_map);
-    HIP_OK(hipGetLastError());
-    HIP_OK(hipStreamSynchronize(st));
     return SPC3D_OK;
 }
 
@@ -1266,7 +1271,7 @@ int remap_device(hipStream_t st, uint64_t n, uint32_t *d_idx, const uint32_t *d_
 
 namespace spc3d {
 
-int partition_by_col_block(hipStream_t st, uint64_t nnz, const uint32_t *d_ii, const uint32_t *d_jj,
+int partition_by_col_block(const DevStream &st, uint64_t nnz, const uint32_t *d_ii, const uint32_t *d_jj,
                            uint32_t ncols, uint32_t nblocks, uint32_t *d_ii_out, uint32_t *d_jj_out,
                            uint32_t *d_order, uint32_t *first, std::string &err)
 {
@@ -1275,7 +1280,7 @@ int partition_by_col_block(hipStream_t st, uint64_t nnz, const uint32_t *d_ii, c
     if (nnz == 0 || nblocks == 0)
         return SPC3D_OK;
     const uint32_t block_cols = (ncols + nblocks - 1) / nblocks;
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve((size_t)nnz * 12 + (size_t)nblocks * 4 + ((size_t)8 << 20)));
     Temp tmp(arena);
     SBuf<uint32_t> key, key_out, ident, dfirst;
@@ -1294,7 +1299,7 @@ int partition_by_col_block(hipStream_t st, uint64_t nnz, const uint32_t *d_ii, c
     return SPC3D_OK;
 }
 
-int compose_perm_device(hipStream_t st, const uint32_t *d_order, const uint32_t *d_perm, uint64_t n,
+int compose_perm_device(const DevStream &st, const uint32_t *d_order, const uint32_t *d_perm, uint64_t n,
                         uint32_t *d_out, std::string &err)
 {
     if (n == 0)
@@ -1304,7 +1309,7 @@ int compose_perm_device(hipStream_t st, const uint32_t *d_order, const uint32_t 
     return SPC3D_OK;
 }
 
-int scatter_device(hipStream_t st, const uint32_t *d_perm, const uint32_t *d_vals, uint64_t n,
+int scatter_device(const DevStream &st, const uint32_t *d_perm, const uint32_t *d_vals, uint64_t n,
                    uint32_t *d_out, std::string &err)
 {
     if (n == 0)
@@ -1314,7 +1319,7 @@ int scatter_device(hipStream_t st, const uint32_t *d_perm, const uint32_t *d_val
     return SPC3D_OK;
 }
 
-int tile_keys_device(hipStream_t st, const uint32_t *d_rows, const uint32_t *d_perm, uint64_t n,
+int tile_keys_device(const DevStream &st, const uint32_t *d_rows, const uint32_t *d_perm, uint64_t n,
                      uint32_t rows_per_tile, uint32_t *d_key, std::string &err)
 {
     if (n == 0)
@@ -1324,12 +1329,12 @@ int tile_keys_device(hipStream_t st, const uint32_t *d_rows, const uint32_t *d_p
     return SPC3D_OK;
 }
 
-int stable_ranks_device(hipStream_t st, const uint32_t *d_key, uint64_t n, uint32_t max_key,
+int stable_ranks_device(const DevStream &st, const uint32_t *d_key, uint64_t n, uint32_t max_key,
                         uint32_t *d_rank, std::string &err)
 {
     if (n == 0)
         return SPC3D_OK;
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve((size_t)n * 12 + ((size_t)8 << 20)));
     Temp tmp(arena);
     SBuf<uint32_t> key_out, ident, sorted;
@@ -1413,13 +1418,13 @@ __global__ void src_neighbours_k(const uint32_t *__restrict__ src, uint64_t n, u
         atomicAdd(acc, c);
 }
 
-int build_store_staging(hipStream_t st, const Seg *d_segs, uint32_t nseg, const uint32_t *d_perm,
+int build_store_staging(const DevStream &st, const Seg *d_segs, uint32_t nseg, const uint32_t *d_perm,
                         uint64_t nnz, StoreStaging &out, std::string &err)
 {
     out = StoreStaging();
     if (!d_perm || nnz == 0 || nseg == 0 || nnz >= (1ull << 31))
         return SPC3D_OK;
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve((size_t)nnz * 8 + ((size_t)8 << 20)));
     Temp tmp(arena);
     SBuf<uint32_t> flag, idx;
@@ -1440,9 +1445,9 @@ int build_store_staging(hipStream_t st, const Seg *d_segs, uint32_t nseg, const 
     if (nnz + n >= (1ull << 32))
         return SPC3D_OK;
     DBuf<uint32_t> perm2, dst, src;
-    HIP_OK(perm2.alloc(nnz));
-    HIP_OK(dst.alloc(n));
-    HIP_OK(src.alloc(n));
+    HIP_OK(perm2.alloc(st, nnz));
+    HIP_OK(dst.alloc(st, n));
+    HIP_OK(src.alloc(st, n));
     SBuf<uint32_t> key, val;
     HIP_OK(key.alloc(arena, n));
     HIP_OK(val.alloc(arena, n));
@@ -1452,7 +1457,7 @@ int build_store_staging(hipStream_t st, const Seg *d_segs, uint32_t nseg, const 
     // The final pass pays when it writes runs and reads near what its neighbours read; an
     // arbitrary order of the entries gives neither, and keeps its scattered stores.
     DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(2));
+    HIP_OK(acc.alloc(st, 2));
     HIP_OK(hipMemsetAsync(acc.p, 0, 2 * sizeof(unsigned long long), st));
     LAUNCH_SMALL(adjacent_k, n, dst.p, n, acc.p);
     LAUNCH_SMALL(src_neighbours_k, n, src.p, n, acc.p + 1);
@@ -1504,7 +1509,7 @@ __global__ void two_pass_slots_k(const uint32_t *__restrict__ sp1,
     }
 }
 
-int build_two_pass(hipStream_t st, const uint32_t *d_perm, uint64_t nnz, uint32_t T, TwoPass &out,
+int build_two_pass(const DevStream &st, const uint32_t *d_perm, uint64_t nnz, uint32_t T, TwoPass &out,
                    std::string &err)
 {
     out = TwoPass();
@@ -1514,7 +1519,7 @@ int build_two_pass(hipStream_t st, const uint32_t *d_perm, uint64_t nnz, uint32_
     if (ntiles64 * ntiles64 >= (1ull << 32))
         return SPC3D_OK;
     const uint32_t ntiles = (uint32_t)ntiles64;
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve((size_t)nnz * 24 + ((size_t)8 << 20)));
     Temp tmp(arena);
     SBuf<uint32_t> key1, key2, idx, key_out, sp1, sp2, mid_of;
@@ -1534,9 +1539,9 @@ int build_two_pass(hipStream_t st, const uint32_t *d_perm, uint64_t nnz, uint32_
     mid_of.p = key1.p; // the keys are no longer needed
     DBuf<uint16_t> l1, l2;
     DBuf<uint32_t> dst1;
-    HIP_OK(l1.alloc(nnz));
-    HIP_OK(l2.alloc(nnz));
-    HIP_OK(dst1.alloc(nnz));
+    HIP_OK(l1.alloc(st, nnz));
+    HIP_OK(l2.alloc(st, nnz));
+    HIP_OK(dst1.alloc(st, nnz));
     LAUNCH(two_pass_mid_k, nnz, sp2.p, d_perm, nnz, T, mid_of.p, l2.p);
     LAUNCH(two_pass_slots_k, nnz, sp1.p, mid_of.p, nnz, T, l1.p, dst1.p);
     HIP_OK(hipGetLastError());
@@ -1622,7 +1627,7 @@ __global__ void sweep_entries_k(const unsigned long long *__restrict__ skey,
     }
 }
 
-int build_sweep(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t *d_ii,
+int build_sweep(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t *d_ii,
                 const uint32_t *d_jj, uint32_t lanes, uint32_t R, uint32_t nb, uint32_t min_row,
                 uint32_t P, SweepPlan &out, std::string &err)
 {
@@ -1633,7 +1638,7 @@ int build_sweep(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz, co
     if (G == 0)
         return SPC3D_OK;
     const uint32_t block_cols = (ncols + nb - 1) / nb;
-    Arena arena;
+    Arena arena(st);
     HIP_OK(arena.reserve(((size_t)nrows + 1) * 40 + (size_t)nnz * 36 + ((size_t)8 << 20)));
     Temp tmp(arena);
     // ---- rows by length ----
@@ -1690,7 +1695,7 @@ int build_sweep(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz, co
                                        32 + bits_for(gens), false, st, err));
     DBuf<uint32_t> tile_rows, perm, col, ptr;
     DBuf<uint16_t> lrow;
-    HIP_OK(tile_rows.alloc((size_t)ntiles * R));
+    HIP_OK(tile_rows.alloc(st, (size_t)ntiles * R));
     HIP_OK(hipMemsetAsync(tile_rows.p, 0xFF, (size_t)ntiles * R * sizeof(uint32_t), st));
     HIP_OK(hipMemsetAsync(row_tile.p, 0xFF, (size_t)nrows * sizeof(uint32_t), st));
     LAUNCH(sweep_rows_k, nin, gkey_sorted.p, nin, P, R, (uint32_t)(gens - 1), rpt_last, row_tile.p,
@@ -1701,7 +1706,7 @@ int build_sweep(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz, co
     HIP_OK(key.alloc(arena, nnz));
     HIP_OK(skey.alloc(arena, nnz));
     HIP_OK(ident.alloc(arena, nnz));
-    HIP_OK(perm.alloc(nnz));
+    HIP_OK(perm.alloc(st, nnz));
     const unsigned long long rest_key = (unsigned long long)ntiles * nb * R;
     LAUNCH_SMALL(sweep_keys_k, nnz, d_ii, d_jj, nnz, row_tile.p, row_local.p, block_cols, nb, R,
                  rest_key, key.p, total.p);
@@ -1712,11 +1717,11 @@ int build_sweep(hipStream_t st, uint32_t nrows, uint32_t ncols, uint64_t nnz, co
     TRY(fetch(st, &n, total.p, sizeof n, err));
     if (n == 0)
         return SPC3D_OK;
-    HIP_OK(col.alloc(n));
-    HIP_OK(lrow.alloc(n));
+    HIP_OK(col.alloc(st, n));
+    HIP_OK(lrow.alloc(st, n));
     HIP_OK(bin.alloc(arena, n));
     const uint64_t nbins = (uint64_t)ntiles * nb;
-    HIP_OK(ptr.alloc(nbins + 1));
+    HIP_OK(ptr.alloc(st, nbins + 1));
     SBuf<uint32_t> bstart, bcnt;
     HIP_OK(bstart.alloc(arena, nbins));
     HIP_OK(bcnt.alloc(arena, nbins + 1));
@@ -1783,7 +1788,7 @@ __global__ void seg_coords_k(const Seg *__restrict__ segs, uint64_t nseg,
     }
 }
 
-int sweep_coords_device(hipStream_t st, const SweepPlan &sw, uint32_t *d_ii, uint32_t *d_jj,
+int sweep_coords_device(const DevStream &st, const SweepPlan &sw, uint32_t *d_ii, uint32_t *d_jj,
                         std::string &err)
 {
     if (sw.n == 0)
@@ -1794,7 +1799,7 @@ int sweep_coords_device(hipStream_t st, const SweepPlan &sw, uint32_t *d_ii, uin
     return SPC3D_OK;
 }
 
-int seg_coords_device(hipStream_t st, const Seg *d_segs, uint64_t nseg, const uint32_t *d_col,
+int seg_coords_device(const DevStream &st, const Seg *d_segs, uint64_t nseg, const uint32_t *d_col,
                       const uint32_t *d_perm, uint32_t *d_ii, uint32_t *d_jj, std::string &err)
 {
     if (nseg == 0)
@@ -1804,14 +1809,14 @@ int seg_coords_device(hipStream_t st, const Seg *d_segs, uint64_t nseg, const ui
     return SPC3D_OK;
 }
 
-int count_adjacent_device(hipStream_t st, const uint32_t *d, uint64_t n, uint64_t *out,
+int count_adjacent_device(const DevStream &st, const uint32_t *d, uint64_t n, uint64_t *out,
                           std::string &err)
 {
     *out = 0;
     if (n < 2)
         return SPC3D_OK;
     DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(1));
+    HIP_OK(acc.alloc(st, 1));
     HIP_OK(hipMemsetAsync(acc.p, 0, sizeof(unsigned long long), st));
     LAUNCH_SMALL(adjacent_k, n, d, n, acc.p);
     unsigned long long seen = 0;
@@ -1820,7 +1825,7 @@ int count_adjacent_device(hipStream_t st, const uint32_t *d, uint64_t n, uint64_
     return SPC3D_OK;
 }
 
-int inverse_offsets_device(hipStream_t st, const uint32_t *d_perm, uint64_t n, uint32_t base,
+int inverse_offsets_device(const DevStream &st, const uint32_t *d_perm, uint64_t n, uint32_t base,
                            uint32_t *d_out, std::string &err)
 {
     if (n == 0)
@@ -1830,7 +1835,7 @@ int inverse_offsets_device(hipStream_t st, const uint32_t *d_perm, uint64_t n, u
     return SPC3D_OK;
 }
 
-int gather_u32_device(hipStream_t st, const uint32_t *d_in, const uint32_t *d_idx, uint64_t n,
+int gather_u32_device(const DevStream &st, const uint32_t *d_in, const uint32_t *d_idx, uint64_t n,
                       uint32_t *d_out, std::string &err)
 {
     if (n == 0)
@@ -1851,14 +1856,14 @@ __global__ void descents_k(const uint32_t *__restrict__ d, uint64_t n, unsigned 
         atomicAdd(acc, c);
 }
 
-int is_nondecreasing_device(hipStream_t st, const uint32_t *d, uint64_t n, bool *out,
+int is_nondecreasing_device(const DevStream &st, const uint32_t *d, uint64_t n, bool *out,
                             std::string &err)
 {
     *out = true;
     if (n < 2)
         return SPC3D_OK;
     DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(1));
+    HIP_OK(acc.alloc(st, 1));
     HIP_OK(hipMemsetAsync(acc.p, 0, sizeof(unsigned long long), st));
     LAUNCH_SMALL(descents_k, n, d, n, acc.p);
     unsigned long long descents = 0;
@@ -1867,14 +1872,14 @@ int is_nondecreasing_device(hipStream_t st, const uint32_t *d, uint64_t n, bool 
     return SPC3D_OK;
 }
 
-int sum_sq_seg_len_device(hipStream_t st, const Seg *d_segs, uint64_t nseg, uint64_t *out,
+int sum_sq_seg_len_device(const DevStream &st, const Seg *d_segs, uint64_t nseg, uint64_t *out,
                           std::string &err)
 {
     *out = 0;
     if (nseg == 0)
         return SPC3D_OK;
     DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(1));
+    HIP_OK(acc.alloc(st, 1));
     HIP_OK(hipMemsetAsync(acc.p, 0, sizeof(unsigned long long), st));
     LAUNCH_SMALL(sum_sq_len_k, nseg, d_segs, nseg, acc.p);
     unsigned long long h = 0;
