@@ -1001,25 +1001,29 @@ int spc3d_rowmap_create(spc3d_ctx *ctx, uint32_t panel_rows, uint64_t n, const u
     if (!live(ctx))
         return fail(SPC3D_ERR_INVALID_ARG, "context is NULL or destroyed");
     // Group the slots by row, ascending inside a row (stable counting sort).
-    std::vector<uint32_t> cnt, urows, ptr, slots;
+    std::vector<uint32_t> at, slots;
+    std::vector<RowDest> dests;
     try {
-        cnt.assign((size_t)panel_rows + 1, 0);
+        at.assign((size_t)panel_rows, 0);
         for (uint64_t i = 0; i < n; ++i)
-            ++cnt[(size_t)rows[i] + 1];
-        std::vector<uint32_t> start((size_t)panel_rows, 0);
-        ptr.push_back(0);
-        uint32_t at = 0;
+            ++at[rows[i]];
+        dests.reserve((size_t)std::min<uint64_t>(panel_rows, n) + 1);
+        uint32_t start = 0;
         for (uint32_t r = 0; r < panel_rows; ++r) {
-            start[r] = at;
-            if (cnt[(size_t)r + 1]) {
-                urows.push_back(r);
-                at += cnt[(size_t)r + 1];
-                ptr.push_back(at);
-            }
+            const uint32_t cnt = at[r];
+            at[r] = start;
+            if (cnt)
+                dests.push_back(RowDest{r, 0, 0, start});
+            start += cnt;
         }
         slots.resize(n);
         for (uint64_t i = 0; i < n; ++i)
-            slots[start[rows[i]]++] = (uint32_t)i;
+            slots[at[rows[i]]++] = (uint32_t)i;
+        dests.push_back(RowDest{0, 0, 0, start});
+        for (size_t d = 0; d + 1 < dests.size(); ++d) {
+            dests[d].first = slots[dests[d].start];
+            dests[d].last = slots[dests[d + 1].start - 1];
+        }
     } catch (const std::bad_alloc &) {
         return fail(SPC3D_ERR_ALLOC, "host allocation failed");
     }
@@ -1032,19 +1036,16 @@ int spc3d_rowmap_create(spc3d_ctx *ctx, uint32_t panel_rows, uint64_t n, const u
     m->ctx = ctx;
     m->panel_rows = panel_rows;
     m->nslots = (uint32_t)n;
-    m->nuniq = (uint32_t)urows.size();
+    m->nuniq = (uint32_t)dests.size() - 1;
     rc = dev_alloc(ctx, &m->rows, (size_t)n);
-    if (!rc) rc = dev_alloc(ctx, &m->urows, urows.size());
-    if (!rc) rc = dev_alloc(ctx, &m->ptr, n ? ptr.size() : 0);
+    if (!rc) rc = dev_alloc(ctx, &m->dests, dests.size());
     if (!rc) rc = dev_alloc(ctx, &m->slots, (size_t)n);
     if (!rc) rc = copy_h2d(ctx, m->rows, rows, (size_t)n * 4);
-    if (!rc) rc = copy_h2d(ctx, m->urows, urows.data(), urows.size() * 4);
-    if (!rc && n) rc = copy_h2d(ctx, m->ptr, ptr.data(), ptr.size() * 4);
+    if (!rc) rc = copy_h2d(ctx, m->dests, dests.data(), dests.size() * sizeof(RowDest));
     if (!rc) rc = copy_h2d(ctx, m->slots, slots.data(), (size_t)n * 4);
     if (rc) {
         if (m->rows) (void)hipFree(m->rows);
-        if (m->urows) (void)hipFree(m->urows);
-        if (m->ptr) (void)hipFree(m->ptr);
+        if (m->dests) (void)hipFree(m->dests);
         if (m->slots) (void)hipFree(m->slots);
         delete m;
         return rc;
@@ -1063,8 +1064,7 @@ int spc3d_rowmap_destroy(spc3d_rowmap *m)
     (void)hipSetDevice(m->ctx->device);
     (void)hipStreamSynchronize(m->ctx->stream);
     if (m->rows) (void)hipFree(m->rows);
-    if (m->urows) (void)hipFree(m->urows);
-    if (m->ptr) (void)hipFree(m->ptr);
+    if (m->dests) (void)hipFree(m->dests);
     if (m->slots) (void)hipFree(m->slots);
     m->magic = 0;
     delete m;
@@ -1089,8 +1089,7 @@ static int rows_op(int op, spc3d_ctx *ctx, const spc3d_panel *P, const spc3d_row
         return rc;
     RowMapView v;
     v.rows = map->rows;
-    v.urows = map->urows;
-    v.ptr = map->ptr;
+    v.dests = map->dests;
     v.slots = map->slots;
     v.nslots = map->nslots;
     v.nuniq = map->nuniq;

@@ -115,7 +115,8 @@ struct spc3d_rowmap {
     spc3d_ctx *ctx;
     uint32_t panel_rows;
     uint32_t nslots, nuniq;
-    uint32_t *rows, *urows, *ptr, *slots; // device
+    uint32_t *rows, *slots; // device
+    RowDest *dests;         // device
 };
 
 struct spc3d_graph {

@@ -110,11 +110,16 @@ hipError_t launch_scatter_vals(int dtype, const void *in, const uint32_t *perm, 
                                uint64_t n, hipStream_t stream);
 hipError_t launch_gather_vals(int dtype, const void *in, const uint32_t *perm, void *out,
                               uint64_t n, hipStream_t stream);
+// One distinct row of a row map: its first and last buffer slot, and where its slots start in
+// RowMapView::slots (the next RowDest's `start` is where they end; one more RowDest closes the
+// list).
+struct RowDest {
+    uint32_t row, first, last, start;
+};
 // Device-side view of a row map (buffer slot i <-> dense row rows[i]).
 struct RowMapView {
     const uint32_t *rows = nullptr;  // [nslots]
-    const uint32_t *urows = nullptr; // [nuniq] distinct rows
-    const uint32_t *ptr = nullptr;   // [nuniq + 1] into slots
+    const RowDest *dests = nullptr;  // [nuniq + 1] distinct rows
     const uint32_t *slots = nullptr; // [nslots] slots grouped by row, ascending inside a row
     uint32_t nslots = 0, nuniq = 0;
 };

@@ -1381,46 +1381,176 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 // The copies either side of the reference's sparse exchanges
 // (SparseComm::copy_to_sendbuff / copy_from_recvbuff / SUM_from_recvbuff,
 // src/comm.hpp:90-103,166-189): buffer slot i holds the dense row rows[i].
-// W = what one lane moves (a 16-byte vector of reals when the row size allows,
-// else one real); upr = units of W per row.
+//
+// LPR lanes (the power of two that covers a row, at most a wavefront) move one row, a unit
+// of 16 bytes each, and several rows at a time, so that every index is asked for before the
+// first row and every row before the first store (1, 2, 4, 8 rows in flight: a sum takes 63, 63,
+// 71, 85 us at fp32 K = 50 and 102, 101, 105, 122 at fp64 K = 64, the copies are level to 4).  Bound by memory: nothing is
+// computed.  UNIT: kVec - rows of whole 16-byte vectors; kLoose - rows that end inside one
+// start at element alignment, and their last unit is the 16 bytes that END at the row's end
+// (it overlaps the unit before: a copy writes the same bytes twice, a sum stores only the
+// elements that are the unit's own); kElem - rows under 16 bytes, one real per lane.
+// 500 k random rows of a 1 M-row panel, fp32 K = 50, pack / unpack / sum-unpack: a real per lane
+// with a division per real took 45 / 85 / 130 us, this 39 / 39 / 61 (a row of 200 bytes at any
+// alignment touches 2.6 lines of 128).
+enum RowUnit { kVec, kLoose, kElem };
+constexpr int kRowsAhead = 4;    // of a copy
+constexpr int kRowsAheadSum = 2; // of a sum, which holds two units per row
+// Fewer workgroups than this (8 per CU) do not fill the chip: one row at a time then, which
+// makes more of them (50 k rows of 56 bytes: sum 6.8 against 4.8 us).
+constexpr uint64_t kRowsMinBlocks = 2048;
+constexpr uint32_t row_unit_bytes(RowUnit u, size_t elem) { return u == kElem ? (uint32_t)elem : 16u; }
+
+template <typename T, RowUnit UNIT> struct RowAccess {
+    using V = typename Vec<T>::type;
+    static __device__ __forceinline__ V load(const char *p)
+    {
+        if constexpr (UNIT == kVec)
+            return *reinterpret_cast<const V *>(p);
+        else
+            return loose_load<T>(p);
+    }
+    static __device__ __forceinline__ V load_nt(const char *p)
+    {
+        if constexpr (UNIT == kVec)
+            return nt_load(reinterpret_cast<const V *>(p));
+        else
+            return loose_load_nt<T>(p);
+    }
+    static __device__ __forceinline__ void store(V v, char *p)
+    {
+        if constexpr (UNIT == kVec)
+            *reinterpret_cast<V *>(p) = v;
+        else
+            loose_store<T>(v, p);
+    }
+    static __device__ __forceinline__ void store_nt(V v, char *p)
+    {
+        if constexpr (UNIT == kVec)
+            nt_store(v, reinterpret_cast<V *>(p));
+        else
+            loose_store_nt<T>(v, p);
+    }
+};
+template <typename T> struct RowAccess<T, kElem> {
+    using V = T;
+    static __device__ __forceinline__ V load(const char *p) { return *reinterpret_cast<const T *>(p); }
+    static __device__ __forceinline__ V load_nt(const char *p) { return nt_load(reinterpret_cast<const T *>(p)); }
+    static __device__ __forceinline__ void store(V v, char *p) { *reinterpret_cast<T *>(p) = v; }
+    static __device__ __forceinline__ void store_nt(V v, char *p) { *reinterpret_cast<T *>(p) = v; }
+};
+
+// Byte offset of unit v of a row of `bytes` bytes.
+template <typename T, RowUnit UNIT> __device__ __forceinline__ uint64_t unit_off(uint32_t v, uint64_t bytes)
+{
+    const uint64_t at = (uint64_t)v * row_unit_bytes(UNIT, sizeof(T));
+    return UNIT == kLoose && at + 16 > bytes ? bytes - 16 : at;
+}
 
 // buf[i, :] = panel[rows[i], :]
-template <typename W>
+template <typename T, RowUnit UNIT, int LPR, int U>
 __global__ void __launch_bounds__(kBlock)
-rows_pack_kernel(const W *__restrict__ panel, const uint32_t *__restrict__ rows, uint64_t total,
-                 uint32_t upr, W *__restrict__ buf)
+rows_pack_kernel(const char *__restrict__ panel, const uint32_t *__restrict__ rows, uint32_t n,
+                 uint32_t units, uint64_t bytes, char *__restrict__ buf)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x; t < total; t += stride) {
-        const uint64_t slot = t / upr;
-        const uint32_t v = (uint32_t)(t - slot * upr);
-        nt_store(panel[(uint64_t)rows[slot] * upr + v], buf + t);
+    using A = RowAccess<T, UNIT>;
+    constexpr uint32_t GPB = kBlock / LPR;
+    const uint32_t sub = threadIdx.x % LPR;
+    const uint64_t first = (uint64_t)blockIdx.x * (GPB * U) + threadIdx.x / LPR;
+    uint32_t row[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint64_t i = first + u * GPB;
+        row[u] = rows[i < n ? i : n - 1];
+    }
+    for (uint32_t v = sub; v < units; v += LPR) {
+        const uint64_t off = unit_off<T, UNIT>(v, bytes);
+        typename A::V x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            x[u] = A::load(panel + (uint64_t)row[u] * bytes + off);
+        __builtin_amdgcn_sched_barrier(0); // every row asked for before the first store
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t i = first + u * GPB;
+            if (i < n)
+                A::store_nt(x[u], buf + i * bytes + off);
+        }
     }
 }
 
-// For every distinct destination row u (urows[u], buffer slots slots[ptr[u] ..
-// ptr[u+1]) in ascending slot order): ADD = false: panel row = its last slot
-// (what the reference's sequential copy leaves); ADD = true: panel row += each
-// slot in order (the reference's sequential sum, bit for bit).
-template <typename W, bool ADD>
+// For every distinct destination row (RowDest: the row, its first and last buffer slot, and
+// where its slots start in `slots`, ascending): ADD = false: panel row = its last slot (what
+// the reference's sequential copy leaves); ADD = true: panel row += each slot in order (the
+// reference's sequential sum, bit for bit).
+template <typename T, RowUnit UNIT, int LPR, int U, bool ADD>
 __global__ void __launch_bounds__(kBlock)
-rows_unpack_kernel(W *__restrict__ panel, const uint32_t *__restrict__ urows,
-                   const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ slots,
-                   uint64_t total, uint32_t upr, const W *__restrict__ buf)
+rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
+                   const uint32_t *__restrict__ slots, uint32_t n, uint32_t units, uint64_t bytes,
+                   const char *__restrict__ buf)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x; t < total; t += stride) {
-        const uint64_t u = t / upr;
-        const uint32_t v = (uint32_t)(t - u * upr);
-        W *dst = panel + (uint64_t)urows[u] * upr + v;
-        const uint32_t lo = ptr[u], hi = ptr[u + 1];
-        if (!ADD) {
-            *dst = nt_load(buf + (uint64_t)slots[hi - 1] * upr + v);
-        } else {
-            W acc = *dst;
-            for (uint32_t s = lo; s < hi; ++s)
-                acc += nt_load(buf + (uint64_t)slots[s] * upr + v);
-            *dst = acc;
+    using A = RowAccess<T, UNIT>;
+    constexpr uint32_t GPB = kBlock / LPR;
+    const uint32_t sub = threadIdx.x % LPR;
+    const uint64_t first = (uint64_t)blockIdx.x * (GPB * U) + threadIdx.x / LPR;
+    u32x4 d[U]; // row, first slot, last slot, start in slots
+    uint32_t more = 0, left[U]; // slots of a row after its first
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint64_t i = first + u * GPB;
+        const uint64_t at = i < n ? i : n - 1;
+        d[u] = nt_load(dests + at);
+        if constexpr (ADD) {
+            left[u] = dests[at + 1][3] - d[u][3] - 1;
+            more = left[u] > more ? left[u] : more;
+        }
+    }
+    for (uint32_t v = sub; v < units; v += LPR) {
+        const uint64_t off = unit_off<T, UNIT>(v, bytes);
+        typename A::V x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            x[u] = A::load_nt(buf + (uint64_t)d[u][ADD ? 1 : 2] * bytes + off);
+            if constexpr (ADD)
+                y[u] = A::load(panel + (uint64_t)d[u][0] * bytes + off);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (ADD) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                y[u] += x[u];
+            for (uint32_t t = 1; t <= more; ++t) { // repeated rows: their t-th slots together
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (t <= left[u])
+                        x[u] = A::load_nt(buf + (uint64_t)slots[d[u][3] + t] * bytes + off);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (t <= left[u])
+                        y[u] += x[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (first + u * GPB >= n)
+                continue;
+            char *to = panel + (uint64_t)d[u][0] * bytes + off;
+            if constexpr (!ADD) {
+                A::store(x[u], to);
+            } else {
+                if constexpr (UNIT == kLoose) {
+                    const uint32_t skip = (uint32_t)((uint64_t)v * 16 - off) / (uint32_t)sizeof(T);
+                    if (skip) { // the row's last unit: its leading elements are the unit's before
+                        T *e = reinterpret_cast<T *>(to);
+#pragma unroll
+                        for (uint32_t j = 0; j < (uint32_t)Vec<T>::N; ++j)
+                            if (j >= skip)
+                                e[j] = y[u][j];
+                        continue;
+                    }
+                }
+                A::store(y[u], to);
+            }
         }
     }
 }
@@ -2230,25 +2360,71 @@ hipError_t launch_gather_vals(int dtype, const void *in, const uint32_t *perm, v
 }
 
 namespace {
-template <typename W>
-hipError_t rows_typed(int op, void *panel, const RowMapView &M, uint32_t upr, void *buf,
-                      hipStream_t st)
+template <typename T, RowUnit UNIT, int LPR, int U>
+void rows_launch_ahead(int op, char *panel, const RowMapView &M, uint32_t n, uint32_t units,
+                       uint64_t bytes, char *buf, hipStream_t st)
 {
-    if (op == 0) {
-        const uint64_t total = (uint64_t)M.nslots * upr;
-        hipLaunchKernelGGL((rows_pack_kernel<W>), dim3(stream_grid(total)), dim3(kBlock), 0, st,
-                           (const W *)panel, M.rows, total, upr, (W *)buf);
-    } else {
-        const uint64_t total = (uint64_t)M.nuniq * upr;
-        if (op == 1)
-            hipLaunchKernelGGL((rows_unpack_kernel<W, false>), dim3(stream_grid(total)),
-                               dim3(kBlock), 0, st, (W *)panel, M.urows, M.ptr, M.slots, total, upr,
-                               (const W *)buf);
-        else
-            hipLaunchKernelGGL((rows_unpack_kernel<W, true>), dim3(stream_grid(total)),
-                               dim3(kBlock), 0, st, (W *)panel, M.urows, M.ptr, M.slots, total, upr,
-                               (const W *)buf);
+    const uint32_t per = kBlock / LPR * U;
+    const dim3 grid((uint32_t)(((uint64_t)n + per - 1) / per)), block(kBlock);
+    if constexpr (U != kRowsAheadSum) {
+        if (op == 0) {
+            hipLaunchKernelGGL((rows_pack_kernel<T, UNIT, LPR, U>), grid, block, 0, st, panel, M.rows,
+                               n, units, bytes, buf);
+            return;
+        }
+        if (op == 1) {
+            hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, U, false>), grid, block, 0, st,
+                               panel, (const u32x4 *)M.dests, M.slots, n, units, bytes, buf);
+            return;
+        }
     }
+    if constexpr (U != kRowsAhead)
+        hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, U, true>), grid, block, 0, st, panel,
+                           (const u32x4 *)M.dests, M.slots, n, units, bytes, buf);
+}
+
+template <typename T, RowUnit UNIT, int LPR>
+void rows_launch(int op, char *panel, const RowMapView &M, uint32_t units, uint64_t bytes, char *buf,
+                 hipStream_t st)
+{
+    const uint32_t n = op == 0 ? M.nslots : M.nuniq;
+    const uint64_t ahead = op == 2 ? kRowsAheadSum : kRowsAhead;
+    if (n / (kBlock / LPR * ahead) < kRowsMinBlocks)
+        rows_launch_ahead<T, UNIT, LPR, 1>(op, panel, M, n, units, bytes, buf, st);
+    else if (op == 2)
+        rows_launch_ahead<T, UNIT, LPR, kRowsAheadSum>(op, panel, M, n, units, bytes, buf, st);
+    else
+        rows_launch_ahead<T, UNIT, LPR, kRowsAhead>(op, panel, M, n, units, bytes, buf, st);
+}
+
+template <typename T>
+hipError_t rows_typed(int op, void *panel, const RowMapView &M, uint32_t K, void *buf, hipStream_t st)
+{
+    const uint64_t bytes = (uint64_t)K * sizeof(T);
+    char *p = (char *)panel, *q = (char *)buf;
+    if (bytes < 16) { // at most three reals
+        rows_launch<T, kElem, 4>(op, p, M, K, bytes, q, st);
+        return hipGetLastError();
+    }
+    const uint32_t units = (uint32_t)((bytes + 15) / 16);
+#define SPC3D_ROWS(UNIT)                                                                          \
+    do {                                                                                          \
+        if (units <= 4)                                                                           \
+            rows_launch<T, UNIT, 4>(op, p, M, units, bytes, q, st);                               \
+        else if (units <= 8)                                                                      \
+            rows_launch<T, UNIT, 8>(op, p, M, units, bytes, q, st);                               \
+        else if (units <= 16)                                                                     \
+            rows_launch<T, UNIT, 16>(op, p, M, units, bytes, q, st);                              \
+        else if (units <= 32)                                                                     \
+            rows_launch<T, UNIT, 32>(op, p, M, units, bytes, q, st);                              \
+        else                                                                                      \
+            rows_launch<T, UNIT, 64>(op, p, M, units, bytes, q, st);                              \
+    } while (0)
+    if (bytes % 16 == 0)
+        SPC3D_ROWS(kVec);
+    else
+        SPC3D_ROWS(kLoose);
+#undef SPC3D_ROWS
     return hipGetLastError();
 }
 } // namespace
@@ -2258,12 +2434,6 @@ hipError_t launch_rows(int op, int dtype, void *panel, const RowMapView &M, uint
 {
     if (M.nslots == 0 || K == 0)
         return hipSuccess;
-    const size_t row_bytes = (size_t)K * (dtype == 1 ? 8 : 4);
-    if (row_bytes % 16 == 0) {
-        const uint32_t upr = (uint32_t)(row_bytes / 16);
-        return dtype == 1 ? rows_typed<Vec<double>::type>(op, panel, M, upr, buf, stream)
-                          : rows_typed<Vec<float>::type>(op, panel, M, upr, buf, stream);
-    }
     return dtype == 1 ? rows_typed<double>(op, panel, M, K, buf, stream)
                       : rows_typed<float>(op, panel, M, K, buf, stream);
 }

@@ -192,3 +192,29 @@ def test_expand_then_reduce_round_trip_at_size(ctx):
         sel = mult >= c
         want[sel] += P[sel]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("k", [2, 5, 15, 17, 50, 63, 127, 129, 255, 257, 260, 515])
+@pytest.mark.parametrize("slots", [1, 13, 1025])
+def test_rows_kernels_at_row_ends_and_partial_blocks(ctx, dtype, k, slots):
+    # rows that end inside a 16-byte unit, fill one, or take several rounds of a wavefront; row
+    # counts that end inside a workgroup's share; repeated rows
+    from spcomm3d_amd import device
+
+    P, rows, buf = case(100 + k + slots, 301, k, slots, dtype)
+    rm = device.RowMap(ctx, 301, rows)
+    dP = ctx.panel_from(P)
+    dB = ctx.vals(rows.size * k + 3, dtype)
+    dB.fill(7.0)
+    rm.pack(dP, dB)
+    got = dB.download()
+    assert np.array_equal(got[:rows.size * k].reshape(-1, k), oracle_rows(0, P, rows, buf)[1])
+    assert np.all(got[rows.size * k:] == 7.0)
+    dB.upload(np.concatenate([buf.ravel(), np.full(3, 7.0, dtype)]))
+    rm.unpack(dP, dB)
+    assert np.array_equal(dP.download(), oracle_rows(1, P, rows, buf)[0])
+    dP.upload(P)
+    rm.unpack_sum(dP, dB)
+    assert np.array_equal(dP.download(), oracle_rows(2, P, rows, buf)[0])
