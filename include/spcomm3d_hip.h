@@ -475,7 +475,7 @@ SPC3D_API int spc3d_rows_unpack_sum(spc3d_ctx *ctx, spc3d_panel *P, const spc3d_
  * what a call built for the next one, decided by CONTENT, never by address (ReMapIndices
  * rewrites ii / jj in place between groups of calls, bench_both.cpp:200-205):
  *   - up to four plans, reused when every 4 MiB block of ii and of jj has the key it had
- *     when the plan was made (four CRC-32C streams, a sum and a fold over every word),
+ *     when the plan was made (two keyed product sums, a sum and a fold over every word),
  *     nnz, sizes, type and k agree, and a sample of the indices compares equal; a new
  *     pattern is planned, and validated, as before;
  *   - up to six device panels with the keys of the host memory they equal: blocks of

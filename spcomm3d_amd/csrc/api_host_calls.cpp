@@ -193,12 +193,10 @@ void send_panel(spc3d_ctx *ctx, CachedHostPanel *slot, const void *host,
         while (e < nblocks && !(known && slot->keys[e] == keys[e]))
             ++e;
         const size_t off = b * kKeyBlockBytes, len = std::min(bytes, e * kKeyBlockBytes) - off;
-        err = hipMemcpyAsync(dst + off, src + off, len, hipMemcpyHostToDevice, ctx->stream);
+        err = ctx->stage.upload(ctx->device, dst + off, src + off, len, ctx->stream);
         mv.sent += len;
         b = e;
     }
-    if (err == hipSuccess)
-        err = hipStreamSynchronize(ctx->stream);
     if (err != hipSuccess) {
         slot->keys.clear(); // the panel's content is no longer known
         mv.rc = fail_hip(err, "upload of a dense operand");
@@ -262,81 +260,14 @@ void send_output_operand(spc3d_ctx *ctx, CachedHostPanel *slot, const void *host
     }
 }
 
-// The changed operand, after the call: fetched into the caller's memory in pieces, each
-// piece keyed by worker threads while the next one is on its way.
+// The changed operand, after the call: fetched into the caller's memory, keyed on the way.
 int fetch_output_operand(spc3d_ctx *ctx, CachedHostPanel *slot, void *host)
 {
     const spc3d_panel *P = slot->panel;
     const size_t bytes = (size_t)P->m * P->n * elem_size(P->dtype);
-    const size_t nblocks = (bytes + kKeyBlockBytes - 1) / kKeyBlockBytes;
-    std::vector<BlockKey> keys(nblocks);
-    // `ready` blocks have arrived; the workers sleep on the condition until theirs has.
-    std::mutex mu;
-    std::condition_variable cv;
-    size_t ready = 0;
-    std::atomic<size_t> next{0};
-    char *dst = static_cast<char *>(host);
-    auto publish = [&](size_t upto) {
-        {
-            std::lock_guard<std::mutex> lock(mu);
-            ready = upto;
-        }
-        cv.notify_all();
-    };
-    auto work = [&]() {
-        for (;;) {
-            const size_t b = next.fetch_add(1, std::memory_order_relaxed);
-            if (b >= nblocks)
-                return;
-            {
-                std::unique_lock<std::mutex> lock(mu);
-                cv.wait(lock, [&] { return ready > b; });
-            }
-            const size_t off = b * kKeyBlockBytes;
-            keys[b] = key_of_block(dst + off, std::min(kKeyBlockBytes, bytes - off));
-        }
-    };
-    // Workers beside the copying thread: what the context allows, at most 4 (a 16 MiB piece is
-    // keyed faster than the next one arrives).  None: this thread keys everything at the end.
-    const unsigned nthreads =
-        (unsigned)std::min<size_t>(std::min(4u, ctx->host_threads > 1 ? ctx->host_threads - 1 : 0u),
-                                   nblocks);
-    // Joined on every way out, after the workers have been let run out.
-    struct Pool {
-        std::vector<std::thread> threads;
-        std::function<void()> release;
-        ~Pool()
-        {
-            release();
-            for (std::thread &t : threads)
-                if (t.joinable())
-                    t.join();
-        }
-    } workers{{}, [&] { publish(nblocks); }};
-    std::vector<std::thread> &pool = workers.threads;
-    try {
-        pool.reserve(nthreads);
-        for (unsigned t = 0; t < nthreads; ++t)
-            pool.emplace_back(work);
-    } catch (const std::exception &) {
-        // fewer workers, or none: what is left over is keyed by this thread at the end
-    }
-    constexpr size_t kPiece = 4; // blocks per copy: 16 MiB
-    hipError_t err = hipSuccess;
-    const char *src = static_cast<const char *>(P->dev);
-    for (size_t b = 0; b < nblocks && err == hipSuccess; b += kPiece) {
-        const size_t off = b * kKeyBlockBytes;
-        const size_t len = std::min(bytes, (b + kPiece) * kKeyBlockBytes) - off;
-        err = hipMemcpyAsync(dst + off, src + off, len, hipMemcpyDeviceToHost, ctx->stream);
-        if (err == hipSuccess)
-            err = hipStreamSynchronize(ctx->stream);
-        if (err == hipSuccess)
-            publish(std::min(nblocks, b + kPiece));
-    }
-    publish(nblocks); // lets the workers run out also after a failure
-    work(); // whatever no worker has taken
-    for (std::thread &t : pool)
-        t.join();
+    std::vector<BlockKey> keys((bytes + kKeyBlockBytes - 1) / kKeyBlockBytes);
+    const hipError_t err = ctx->stage.download(ctx->device, host, P->dev, bytes, ctx->stream, keys.data(),
+                                               ctx->host_threads);
     if (err != hipSuccess) {
         slot->keys.clear();
         return fail_hip(err, "download of a dense operand");
@@ -369,6 +300,7 @@ int spc3d_host_cache_clear(spc3d_ctx *ctx)
         return fail(SPC3D_ERR_INVALID_ARG, "context is NULL or destroyed");
     std::lock_guard<std::mutex> lock(ctx->host_mutex);
     (void)hipSetDevice(ctx->device);
+    ctx->stage.release();
     HostCallCache *hc = ctx->host_cache;
     if (!hc) {
         ctx->pool.trim();

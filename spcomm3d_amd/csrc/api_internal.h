@@ -23,6 +23,7 @@
 
 #include "dev_pool.h"
 #include "host_cache.h"
+#include "host_stage.h"
 #include "kernels.h"
 #include "plan_device.h"
 #include "plan_host.h"
@@ -90,6 +91,7 @@ struct spc3d_ctx {
     unsigned host_threads;     // host threads a one-shot call may use, the caller's included
     std::mutex host_mutex;     // the one-shot calls of a context run one at a time
     DevPool pool;              // device memory of plans and of the plan builder
+    HostStage stage;           // pinned buffers of the copies from and to host memory
 };
 
 struct spc3d_panel {
@@ -303,23 +305,29 @@ template <typename T> int dev_alloc(spc3d_ctx *ctx, T **out, size_t count)
     return dev_alloc_bytes(ctx, (void **)out, count * sizeof(T));
 }
 
-// Pageable-host <-> device copy ordered after everything queued on the
-// stream; returns when the host side may be reused / read.
+// Pageable-host <-> device copies ordered after everything queued on the stream.
+// send_h2d returns when the host side may be reused, copy_h2d when the copy is done, copy_d2h
+// when the host side may be read.
+inline int send_h2d(spc3d_ctx *ctx, void *dst, const void *src, size_t bytes)
+{
+    if (bytes == 0)
+        return SPC3D_OK;
+    HIP_TRY(ctx->stage.upload(ctx->device, dst, src, bytes, ctx->stream));
+    return SPC3D_OK;
+}
+
 inline int copy_h2d(spc3d_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0)
         return SPC3D_OK;
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(ctx->stage.upload(ctx->device, dst, src, bytes, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return SPC3D_OK;
 }
 
 inline int copy_d2h(spc3d_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
-    if (bytes == 0)
-        return SPC3D_OK;
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    HIP_TRY(ctx->stage.download(ctx->device, dst, src, bytes, ctx->stream, nullptr, ctx->host_threads));
     return SPC3D_OK;
 }
 

@@ -773,8 +773,8 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
         uint32_t *d_ii = nullptr, *d_jj = nullptr;
         rc = ctx_alloc(ctx, &d_ii, (size_t)nnz);
         if (!rc) rc = ctx_alloc(ctx, &d_jj, (size_t)nnz);
-        if (!rc) rc = copy_h2d(ctx, d_ii, ii, (size_t)nnz * sizeof(uint32_t));
-        if (!rc) rc = copy_h2d(ctx, d_jj, jj, (size_t)nnz * sizeof(uint32_t));
+        if (!rc) rc = send_h2d(ctx, d_ii, ii, (size_t)nnz * sizeof(uint32_t));
+        if (!rc) rc = send_h2d(ctx, d_jj, jj, (size_t)nnz * sizeof(uint32_t));
         if (!rc)
             rc = build_from_device(ctx, dtype, nrows, ncols, nnz, d_ii, d_jj, po, opts, &p);
         if (d_ii) ctx_free(ctx, d_ii);
@@ -1005,13 +1005,13 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
         return rc;
     const size_t bytes = (size_t)nnz * elem_size(plan->dtype);
     if (plan->blocks.empty() && !plan->perm && !plan->by_col && !plan->sweep.n) {
-        rc = copy_h2d(plan->ctx, plan->sval, vv_host, bytes);
+        rc = send_h2d(plan->ctx, plan->sval, vv_host, bytes);
     } else {
         void *tmp = nullptr;
         rc = ctx_alloc_bytes(plan->ctx, &tmp, bytes);
         if (rc)
             return rc;
-        rc = copy_h2d(plan->ctx, tmp, vv_host, bytes);
+        rc = send_h2d(plan->ctx, tmp, vv_host, bytes);
         if (!rc && plan->sweep.n) {
             hipError_t e = launch_gather_vals(plan->dtype, tmp, plan->sweep.perm, plan->sweep_sval,
                                               plan->sweep.n, plan->ctx->stream);
@@ -1034,12 +1034,12 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
                 rc = fail_hip(e, "gather of sparse values");
             plan->by_col->has_values = true;
         }
-        if (!rc) {
-            hipError_t e = hipStreamSynchronize(plan->ctx->stream);
-            if (e != hipSuccess)
-                rc = fail_hip(e, "gather of sparse values");
-        }
-        ctx_free(plan->ctx, tmp);
+        ctx_free(plan->ctx, tmp); // what gets this block next is queued behind the gathers
+    }
+    if (!rc) {
+        hipError_t e = hipStreamSynchronize(plan->ctx->stream);
+        if (e != hipSuccess)
+            rc = fail_hip(e, "sparse values");
     }
     if (!rc)
         plan->has_values = true;

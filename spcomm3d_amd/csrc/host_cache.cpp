@@ -1,4 +1,4 @@
-// Content keys of host operands (see host_cache.h).  Host code only.
+// Content keys of host operands and copies of host memory (see host_cache.h).  Host code only.
 #include "host_cache.h"
 
 #include <algorithm>
@@ -8,96 +8,214 @@
 #include <thread>
 
 #if defined(__x86_64__)
-#include <nmmintrin.h>
+#include <immintrin.h>
 #endif
 
 namespace spc3d {
 
 namespace {
 
-inline uint64_t rotl(uint64_t x, int r) { return (x << r) | (x >> (64 - r)); }
+constexpr int kLanes = 8;                                   // streams of 8-byte words
+constexpr int kStripes = (int)(kKeyChunk / (8 * kLanes));   // of a chunk
 
-// Portable form: the CRC streams become multiply-xorshift chains.
-void key_plain(const unsigned char *p, size_t bytes, BlockKey &k)
+// Two constants per word of a chunk, one per NH sum.
+struct NhKeys {
+    alignas(64) uint64_t k[2][kStripes][kLanes];
+    constexpr NhKeys() : k()
+    {
+        uint64_t x = 0x243F6A8885A308D3ull; // splitmix64 from pi's fraction
+        for (auto &set : k)
+            for (auto &stripe : set)
+                for (uint64_t &v : stripe) {
+                    x += 0x9E3779B97F4A7C15ull;
+                    uint64_t z = x;
+                    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+                    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+                    v = z ^ (z >> 31);
+                }
+    }
+};
+constexpr NhKeys kNh;
+
+// Between chunks: a bijection of the chained sum (so that nothing a chunk told apart is lost)
+// that does not commute with the additions (so that the order of the chunks counts).
+constexpr uint64_t kChainXor = 0x452821E638D01377ull, kChainMul = 0x9E3779B1ull;
+inline uint64_t chain(uint64_t x) { return (x ^ (x >> 41) ^ kChainXor) * kChainMul; }
+
+inline uint64_t add_halves(uint64_t w, uint64_t k)
 {
-    uint64_t h[4] = {bytes, ~(uint64_t)bytes, 0x9E3779B97F4A7C15ull, 0xD6E8FEB86659FD93ull};
-    uint64_t sum = 0, fold = 0;
-    size_t i = 0;
-    for (; i + 32 <= bytes; i += 32) {
-        uint64_t w[4];
-        std::memcpy(w, p + i, 32);
-        for (int l = 0; l < 4; ++l) {
-            h[l] = (h[l] ^ w[l]) * 0xBF58476D1CE4E5B9ull;
-            h[l] ^= h[l] >> 29;
-            sum += w[l];
-            fold = rotl(fold, 5) ^ w[l];
-        }
+    return (uint64_t)((uint32_t)w + (uint32_t)k) | (uint64_t)((uint32_t)(w >> 32) + (uint32_t)(k >> 32)) << 32;
+}
+inline uint64_t product_of_halves(uint64_t x) { return (x & 0xFFFFFFFFu) * (x >> 32); }
+
+void chunks_plain(const unsigned char *p, size_t chunks, uint64_t *a, uint64_t *b, uint64_t *s)
+{
+    for (size_t c = 0; c < chunks; ++c, p += kKeyChunk) {
+        for (int t = 0; t < kStripes; ++t)
+            for (int l = 0; l < kLanes; ++l) {
+                uint64_t w;
+                std::memcpy(&w, p + (size_t)(t * kLanes + l) * 8, 8);
+                a[l] += product_of_halves(add_halves(w, kNh.k[0][t][l]));
+                b[l] += product_of_halves(add_halves(w, kNh.k[1][t][l]));
+                s[l] += w;
+            }
+        for (int l = 0; l < kLanes; ++l)
+            a[l] = chain(a[l]), b[l] = chain(b[l]);
     }
-    uint64_t tail[4] = {0, 0, 0, 0};
-    std::memcpy(tail, p + i, bytes - i);
-    for (int l = 0; l < 4; ++l) {
-        h[l] = (h[l] ^ tail[l]) * 0x94D049BB133111EBull;
-        sum += tail[l];
-        fold = rotl(fold, 5) ^ tail[l];
-    }
-    k.crc01 = h[0] ^ (h[1] >> 31);
-    k.crc23 = h[2] ^ (h[3] >> 31);
-    k.sum = sum;
-    k.fold = fold;
 }
 
 #if defined(__x86_64__)
-__attribute__((target("sse4.2"))) void key_crc(const unsigned char *p, size_t bytes, BlockKey &k)
+__attribute__((target("avx2"))) inline __m256i chain_avx2(__m256i x)
 {
-    uint64_t h[4] = {bytes & 0xFFFFFFFFu, 0x1F3D5B79u, 0x2E4C6A80u, 0x3D5B798Fu};
-    uint64_t sum = 0, fold = 0;
-    size_t i = 0;
-    for (; i + 32 <= bytes; i += 32) {
-        uint64_t w[4];
-        std::memcpy(w, p + i, 32);
-        h[0] = _mm_crc32_u64(h[0], w[0]);
-        h[1] = _mm_crc32_u64(h[1], w[1]);
-        h[2] = _mm_crc32_u64(h[2], w[2]);
-        h[3] = _mm_crc32_u64(h[3], w[3]);
-        sum += (w[0] + w[1]) + (w[2] + w[3]);
-        fold = rotl(fold, 5) ^ (w[0] ^ rotl(w[1], 17) ^ rotl(w[2], 31) ^ rotl(w[3], 47));
-    }
-    uint64_t tail[4] = {0, 0, 0, 0};
-    std::memcpy(tail, p + i, bytes - i);
-    for (int l = 0; l < 4; ++l) {
-        h[l] = _mm_crc32_u64(h[l], tail[l]);
-        sum += tail[l];
-    }
-    fold = rotl(fold, 5) ^ (tail[0] ^ rotl(tail[1], 17) ^ rotl(tail[2], 31) ^ rotl(tail[3], 47));
-    k.crc01 = h[0] | (h[1] << 32);
-    k.crc23 = h[2] | (h[3] << 32);
-    k.sum = sum;
-    k.fold = fold;
+    x = _mm256_xor_si256(_mm256_xor_si256(x, _mm256_srli_epi64(x, 41)), _mm256_set1_epi64x((long long)kChainXor));
+    const __m256i m = _mm256_set1_epi64x((long long)kChainMul);
+    const __m256i hi = _mm256_mul_epu32(_mm256_srli_epi64(x, 32), m);
+    return _mm256_add_epi64(_mm256_mul_epu32(x, m), _mm256_slli_epi64(hi, 32));
 }
+
+// COPY: every vector read is also stored to `to` (32-byte aligned), past the caches.
+template <bool COPY>
+__attribute__((target("avx2"))) void chunks_avx2(const unsigned char *p, unsigned char *to, size_t chunks,
+                                                 uint64_t *a, uint64_t *b, uint64_t *s)
+{
+    __m256i A[2], B[2], S[2];
+    for (int h = 0; h < 2; ++h) {
+        A[h] = _mm256_load_si256((const __m256i *)a + h);
+        B[h] = _mm256_load_si256((const __m256i *)b + h);
+        S[h] = _mm256_load_si256((const __m256i *)s + h);
+    }
+    for (size_t c = 0; c < chunks; ++c, p += kKeyChunk, to += COPY ? kKeyChunk : 0) {
+        for (int t = 0; t < kStripes; ++t)
+            for (int h = 0; h < 2; ++h) {
+                const __m256i w = _mm256_loadu_si256((const __m256i *)(p + t * 64 + h * 32));
+                const __m256i x = _mm256_add_epi32(w, _mm256_load_si256((const __m256i *)kNh.k[0][t] + h));
+                const __m256i y = _mm256_add_epi32(w, _mm256_load_si256((const __m256i *)kNh.k[1][t] + h));
+                A[h] = _mm256_add_epi64(A[h], _mm256_mul_epu32(x, _mm256_srli_epi64(x, 32)));
+                B[h] = _mm256_add_epi64(B[h], _mm256_mul_epu32(y, _mm256_srli_epi64(y, 32)));
+                S[h] = _mm256_add_epi64(S[h], w);
+                if (COPY)
+                    _mm256_stream_si256((__m256i *)(to + t * 64 + h * 32), w);
+            }
+        for (int h = 0; h < 2; ++h)
+            A[h] = chain_avx2(A[h]), B[h] = chain_avx2(B[h]);
+    }
+    for (int h = 0; h < 2; ++h) {
+        _mm256_store_si256((__m256i *)a + h, A[h]);
+        _mm256_store_si256((__m256i *)b + h, B[h]);
+        _mm256_store_si256((__m256i *)s + h, S[h]);
+    }
+    if (COPY)
+        _mm_sfence();
+}
+
+__attribute__((target("avx2"))) void stream_copy_avx2(unsigned char *to, const unsigned char *from, size_t bytes)
+{
+    const size_t head = std::min<size_t>(bytes, (32 - ((uintptr_t)to & 31)) & 31);
+    std::memcpy(to, from, head);
+    to += head, from += head, bytes -= head;
+    size_t i = 0;
+    for (; i + 128 <= bytes; i += 128) {
+        const __m256i v0 = _mm256_loadu_si256((const __m256i *)(from + i));
+        const __m256i v1 = _mm256_loadu_si256((const __m256i *)(from + i + 32));
+        const __m256i v2 = _mm256_loadu_si256((const __m256i *)(from + i + 64));
+        const __m256i v3 = _mm256_loadu_si256((const __m256i *)(from + i + 96));
+        _mm256_stream_si256((__m256i *)(to + i), v0);
+        _mm256_stream_si256((__m256i *)(to + i + 32), v1);
+        _mm256_stream_si256((__m256i *)(to + i + 64), v2);
+        _mm256_stream_si256((__m256i *)(to + i + 96), v3);
+    }
+    _mm_sfence();
+    std::memcpy(to + i, from + i, bytes - i);
+}
+
+bool have_avx2()
+{
+    static const bool yes = __builtin_cpu_supports("avx2");
+    return yes;
+}
+#else
+bool have_avx2() { return false; }
 #endif
 
 } // namespace
 
-BlockKey key_of_block_portable(const void *data, size_t bytes)
+KeyMaker::KeyMaker(bool portable) : vector_(!portable && have_avx2())
 {
+    for (int l = 0; l < kLanes; ++l) {
+        a_[l] = kNh.k[1][0][l] * 3;
+        b_[l] = kNh.k[0][1][l] * 5;
+        s_[l] = 0;
+    }
+}
+
+void KeyMaker::update(const void *data, size_t bytes)
+{
+    const unsigned char *p = static_cast<const unsigned char *>(data);
+    total_ += bytes;
+#if defined(__x86_64__)
+    if (vector_) {
+        chunks_avx2<false>(p, nullptr, bytes / kKeyChunk, a_, b_, s_);
+        return;
+    }
+#endif
+    chunks_plain(p, bytes / kKeyChunk, a_, b_, s_);
+}
+
+void KeyMaker::update_copy(void *to, const void *from, size_t bytes)
+{
+#if defined(__x86_64__)
+    if (vector_ && ((uintptr_t)to & 31) == 0) {
+        total_ += bytes;
+        chunks_avx2<true>(static_cast<const unsigned char *>(from), static_cast<unsigned char *>(to),
+                          bytes / kKeyChunk, a_, b_, s_);
+        return;
+    }
+#endif
+    // a few chunks at a time, so that the second read finds them in the first-level cache
+    const unsigned char *p = static_cast<const unsigned char *>(from);
+    unsigned char *q = static_cast<unsigned char *>(to);
+    for (size_t i = 0; i < bytes; i += 16 * kKeyChunk) {
+        const size_t n = std::min(16 * kKeyChunk, bytes - i);
+        std::memcpy(q + i, p + i, n);
+        update(p + i, n);
+    }
+}
+
+BlockKey KeyMaker::finish(const void *data, size_t bytes)
+{
+    const size_t whole = bytes / kKeyChunk * kKeyChunk;
+    if (whole)
+        update(data, whole);
+    if (bytes > whole) { // the last chunk, filled up with zeros; the length counts below
+        unsigned char last[kKeyChunk] = {0};
+        std::memcpy(last, static_cast<const unsigned char *>(data) + whole, bytes - whole);
+        update(last, kKeyChunk);
+        total_ -= kKeyChunk - (bytes - whole);
+    }
     BlockKey k;
-    key_plain(static_cast<const unsigned char *>(data), bytes, k);
+    k.nh0 = total_, k.nh1 = ~total_;
+    for (int l = 0; l < kLanes; ++l) {
+        k.nh0 = chain(k.nh0 + a_[l]);
+        k.nh1 = chain(k.nh1 + b_[l]);
+        k.sum += s_[l];
+        k.fold = chain(k.fold + s_[l]);
+    }
     return k;
 }
 
-BlockKey key_of_block(const void *data, size_t bytes)
+BlockKey key_of_block_portable(const void *data, size_t bytes) { return KeyMaker(true).finish(data, bytes); }
+
+BlockKey key_of_block(const void *data, size_t bytes) { return KeyMaker().finish(data, bytes); }
+
+void stream_copy(void *to, const void *from, size_t bytes)
 {
-    BlockKey k;
-    const unsigned char *p = static_cast<const unsigned char *>(data);
 #if defined(__x86_64__)
-    static const bool crc = __builtin_cpu_supports("sse4.2");
-    if (crc) {
-        key_crc(p, bytes, k);
-        return k;
+    if (have_avx2()) {
+        stream_copy_avx2(static_cast<unsigned char *>(to), static_cast<const unsigned char *>(from), bytes);
+        return;
     }
 #endif
-    key_plain(p, bytes, k);
-    return k;
+    std::memcpy(to, from, bytes);
 }
 
 void keys_of(const void *data, size_t bytes, std::vector<BlockKey> &out, unsigned threads)
