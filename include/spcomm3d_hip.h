@@ -126,8 +126,10 @@ typedef struct {
 /* Plan tuning; a zero field selects the default.  Only speed depends on these. */
 typedef struct {
     uint32_t seg_max;      /* longest segment in entries (default: nnz / 2048 rounded down to
-                              a power of two, within 64 .. 2048; with k_hint given, at most
-                              1024 for dense rows of 128 bytes and 512 for 64 bytes and less) */
+                              a power of two, within 64 .. 2048; with k_hint given, by what the
+                              launch gathers, nnz * bytes of a dense row / 2^21, within 16 .. 2048,
+                              at most 1024 for dense rows of 128 bytes and 512 for 64 bytes and
+                              less) */
     uint32_t k_hint;       /* K the plan will mostly run with: sizes the XCD slicing (default
                               64) and the default seg_max */
     uint32_t l2_hot_bytes; /* XCD slicing: share of one XCD's 4 MiB L2 planned for dense rows

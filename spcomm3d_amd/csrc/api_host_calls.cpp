@@ -67,6 +67,8 @@ int host_plan(spc3d_ctx *ctx, HostCallCache *hc, int dtype, uint32_t nrows, uint
     spc3d_plan_opts o = opts_from_env();
     if (!o.k_hint)
         o.k_hint = k; // the one width this plan will run with; sizes the partial-sum rows too
+    if (!o.seg_max) // rows cut as in a plan made without options: the same sums, bit for bit
+        o.seg_max = seg_max_by_entries(nnz, (uint32_t)std::min<uint64_t>(k * elem_size(dtype), 1u << 30));
     spc3d_plan *plan = nullptr;
     int rc = spc3d_plan_create_ex(ctx, dtype, nrows, ncols, nnz, ii, jj, vv, &o, &plan);
     if (rc)
@@ -342,6 +344,8 @@ static int sddmm_host_uncached(spc3d_ctx *ctx, int dtype, uint32_t m, uint32_t n
     spc3d_plan_opts o = opts_from_env();
     if (!o.k_hint)
         o.k_hint = k; // the one width this plan will ever run with
+    if (!o.seg_max)
+        o.seg_max = seg_max_by_entries(nnz, (uint32_t)std::min<uint64_t>(k * elem_size(dtype), 1u << 30));
     int rc = spc3d_plan_create_ex(ctx, dtype, m, n, nnz, ii, jj, svv, &o, &S);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, m, k, &a);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, n, k, &b);

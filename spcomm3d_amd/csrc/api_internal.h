@@ -133,6 +133,7 @@ struct spc3d_plan {
     spc3d_ctx *ctx;
     int dtype;
     spc3d_plan_info info;
+    uint64_t row_sq = 0; // HostPlan::row_sq
     bool has_values;
     // device arrays
     Seg *segs;
@@ -407,6 +408,7 @@ inline DevPlanView view_of(const spc3d_plan *p)
     v.sval = p->sval;
     v.splits = p->splits;
     v.nsplit = p->info.nsplit_rows;
+    v.nslots = p->info.npartial_slots;
     v.partial = p->partial;
     v.first_cols = p->first_cols;
     v.nnz = p->info.nnz;

@@ -249,6 +249,7 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
         p->ctx = ctx;
         p->dtype = dtype;
         fill_info(p->info, meta);
+        p->row_sq = meta.row_sq;
         p->info.nsegments_padded = arr.nseg_padded;
         p->info.nsplit_rows = arr.nsplit;
         rc = ctx_alloc_bytes(ctx, &p->sval, (size_t)meta.nnz * elem_size(dtype));
@@ -304,39 +305,38 @@ static void destroy_blocks(spc3d_plan *p)
 // Blocks pay when the dense rows the pattern gathers do not fit the L2s, the columns
 // are not skewed (then a few hot rows carry the reuse, and the plan deals them to the
 // XCDs instead), and the rows are long enough that a row's piece in one block still
-// amortises reading its A row / updating its Y row: the entry-weighted mean segment
-// length divided by the block count must stay at 16 or more.  Measured on a 2 M x 500 k
+// amortises reading its A row / updating its Y row: the entry-weighted mean row
+// length (counted to 2048) divided by the block count must stay at 16 or more.  Each L2 reads its own copy of a
+// block, so a column must also come up kBlockReuse times: 1 M entries over 290 k columns, 512-byte
+// rows, run 146 us whole and 219 in blocks, 4.2 M entries 588 and 419.  Measured on a 2 M x 500 k
 // pattern with 286 entries per row on average (capped Zipf, weighted mean 890) at 512-byte
 // dense rows: 43 -> 24 ms SDDMM, 42 -> 27 ms SpMM in 48 blocks of 5 MiB; a uniform
 // pattern of 256 entries per row gains 10 % in SDDMM and loses in SpMM, and stays whole.
-static int choose_col_blocks(spc3d_plan *p, const spc3d_plan_opts *opts, uint32_t *nblocks)
+constexpr uint32_t kBlockReuse = 5;
+static void choose_col_blocks(spc3d_plan *p, const spc3d_plan_opts *opts, uint32_t *nblocks)
 {
     *nblocks = 1;
     const uint32_t want = opts ? opts->col_blocks : 0;
     const spc3d_plan_info &I = p->info;
     if (want == 1 || I.nnz == 0 || I.ncols < 2)
-        return SPC3D_OK;
+        return;
     if (want > 1) {
         *nblocks = std::min<uint32_t>(want, I.ncols);
-        return SPC3D_OK;
+        return;
     }
     if (I.nqueues != 1)
-        return SPC3D_OK;
+        return;
     const uint64_t row_bytes = (uint64_t)planned_k(opts) * elem_size(p->dtype);
     const uint64_t panel = (uint64_t)I.cols_touched * row_bytes;
     constexpr uint64_t kBlockBytes = (uint64_t)21 << 18; // 5.25 MiB of dense rows per block
     if (panel < ((uint64_t)64 << 20))
-        return SPC3D_OK;
+        return;
     const uint64_t nb = std::min<uint64_t>((panel + kBlockBytes - 1) / kBlockBytes, 256);
-    uint64_t sumsq = 0;
-    std::string err;
-    int rc = sum_sq_seg_len_device(dev_stream(p->ctx), p->segs, I.nsegments_padded, &sumsq, err);
-    if (rc != SPC3D_OK)
-        return fail(rc, err);
-    const double wmean = (double)sumsq / (double)I.nnz;
+    if (I.nnz < (uint64_t)kBlockReuse * I.cols_touched)
+        return;
+    const double wmean = (double)p->row_sq / (double)I.nnz;
     if (wmean / (double)nb >= 16.0)
         *nblocks = (uint32_t)nb;
-    return SPC3D_OK;
 }
 
 // The companion plan for SDDMM (spc3d_plan::by_col) of a finished single plan whose results
@@ -572,8 +572,8 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         return rc;
     uint32_t nb = 1;
     const StoreOpts so = store_opts_of(opts);
-    rc = choose_col_blocks(p, opts, &nb);
-    if (!rc) {
+    choose_col_blocks(p, opts, &nb);
+    {
         uint32_t sw_lanes = 0, sw_nb = 0;
         choose_sweep(p, opts, nb, &sw_lanes, &sw_nb);
         bool taken = false;

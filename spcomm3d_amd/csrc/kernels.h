@@ -19,6 +19,7 @@ struct DevPlanView {
     const void *sval = nullptr;       // [nnz] values in kernel order
     const SplitRow *splits = nullptr;
     uint32_t nsplit = 0;
+    uint32_t nslots = 0; // partial-sum rows of all splits
     void *partial = nullptr;          // [nslots * K] partial sums of cut rows (SpMM)
     // [(nseg - nseg_long) * kFirstCols] the first column indices of every segment past
     // the long ones (launch_first_cols); read by the short-segment launch

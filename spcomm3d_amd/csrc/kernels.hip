@@ -854,7 +854,13 @@ template <int LPR> __device__ __forceinline__ uint32_t first_col(const uint32_t 
     if constexpr (LPR >= (int)kFirstCols)
         return __shfl(FC[0], j, LPR);
     else
-        return __shfl((j & LPR) ? FC[1] : FC[0], j & (LPR - 1), LPR);
+    {
+        // Values, not elements: a choice between two array elements is a choice of address, for
+        // which the compiler moves the array to LDS and reads the dispatch packet to find the
+        // thread's place in it (9 us per launch).
+        const uint32_t a = FC[0], b = FC[1];
+        return __shfl((j & LPR) ? b : a, j & (LPR - 1), LPR);
+    }
 }
 
 // PRE: the batch is entries off .. off + NB - 1 of a short segment, off + NB <=
@@ -1088,29 +1094,58 @@ spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32
     }
 }
 
-// Y[row,:] += the partial sums of a cut row, in slot order.  `lanes` (a power of
-// two, <= kBlock) threads share one cut row, kBlock / lanes rows per block.
-template <typename T>
+// Y[row,:] += the partial sums of a cut row.  A row's slots are cut into `parts` runs; `lanes`
+// threads sum a run each (four loads in flight, in slot order, one 16-byte unit of the row per
+// thread where rows are whole units, else one real), the runs are added in pairs through LDS.
+// lanes and parts are powers of two, lanes * parts <= kBlock; the other threads of the block
+// take further rows.
+// Few rows with many slots (the hubs of a small pattern) are a chain of loads each: R-MAT 13,
+// 16-entry segments, fp32 K = 16: SpMM 11.1 us with one run per row, 7.4 with runs.  Many
+// rows are bound by the slots' bytes and take one run each.
+template <typename T, typename U>
 __global__ void __launch_bounds__(kBlock)
-spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit,
-                  const T *__restrict__ partial, T *__restrict__ Y, uint32_t K, uint32_t lanes)
+spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U *__restrict__ partial,
+                  U *__restrict__ Y, uint32_t units, uint32_t lanes, uint32_t parts)
 {
-    const uint32_t idx = blockIdx.x * (kBlock / lanes) + threadIdx.x / lanes;
-    if (idx >= nsplit)
-        return;
-    const SplitRow sr = splits[idx];
-    for (uint32_t j = threadIdx.x % lanes; j < K; j += lanes) {
-        const T *p = partial + (size_t)sr.first_slot * K + j;
-        T s = (T)0;
-        uint32_t q = 0;
-        for (; q + 4 <= sr.nslots; q += 4) { // four loads in flight, added in slot order
-            const T v0 = p[(size_t)(q + 0) * K], v1 = p[(size_t)(q + 1) * K];
-            const T v2 = p[(size_t)(q + 2) * K], v3 = p[(size_t)(q + 3) * K];
-            s = (((s + v0) + v1) + v2) + v3;
+    __shared__ typename Vec<T>::type run[kBlock];
+    U *sums = reinterpret_cast<U *>(run);
+    const uint32_t per_row = lanes * parts;
+    const uint32_t idx = blockIdx.x * (kBlock / per_row) + threadIdx.x / per_row;
+    const uint32_t part = threadIdx.x % per_row / lanes;
+    SplitRow sr{};
+    if (idx < nsplit)
+        sr = splits[idx];
+    const uint32_t len = (sr.nslots + parts - 1) / parts;
+    const uint32_t q0 = part * len < sr.nslots ? part * len : sr.nslots;
+    const uint32_t q1 = q0 + len < sr.nslots ? q0 + len : sr.nslots;
+    for (uint32_t j0 = 0; j0 < units; j0 += lanes) { // the same trips for every thread
+        const uint32_t j = j0 + threadIdx.x % lanes;
+        const bool on = j < units && idx < nsplit;
+        U s{}, y{};
+        if (on) {
+            if (part == 0)
+                y = Y[(size_t)sr.row * units + j];
+            const U *p = partial + (size_t)sr.first_slot * units + j;
+            uint32_t q = q0;
+            for (; q + 4 <= q1; q += 4) {
+                const U v0 = p[(size_t)(q + 0) * units], v1 = p[(size_t)(q + 1) * units];
+                const U v2 = p[(size_t)(q + 2) * units], v3 = p[(size_t)(q + 3) * units];
+                s = (((s + v0) + v1) + v2) + v3;
+            }
+            for (; q < q1; ++q)
+                s += p[(size_t)q * units];
         }
-        for (; q < sr.nslots; ++q)
-            s += p[(size_t)q * K];
-        Y[(size_t)sr.row * K + j] += s;
+        if (parts > 1) {
+            sums[threadIdx.x] = s;
+            __syncthreads();
+            for (uint32_t step = parts / 2; step; step /= 2) { // runs i and i + step, in pairs
+                if (part < step)
+                    sums[threadIdx.x] = s += sums[threadIdx.x + step * lanes];
+                __syncthreads();
+            }
+        }
+        if (on && part == 0)
+            Y[(size_t)sr.row * units + j] = y + s;
     }
 }
 
@@ -1917,6 +1952,18 @@ inline uint32_t blocks_for_groups(uint32_t nseg, uint32_t nq, int groups_per_wav
 // 32 us at 12 k), two from 400 k on.
 constexpr uint32_t kOneLaunchSegments = 196608;
 
+// Segments for the wide launch (the first *nl) and for the short one.  Short segments that fill
+// most of a wide batch, in a pattern that has no others, go to the wide launch too: one round of
+// gathers instead of two to four.  Uniform rows of 12 to 15, fp32 K = 8: SDDMM 125 -> 116 us, SpMM 102
+// -> 99; K = 64: 404 -> 388 and 442 -> 418; rows of 11 are level or better in the short one, and so are
+// dense rows that leave lanes idle (15 entries, fp32 K = 134: 71 us together in the short one, 74).
+inline void split_launches(const DevPlanView &P, bool whole_lanes, uint32_t &nl, uint32_t &ns)
+{
+    nl = P.nseg_long, ns = P.nseg - P.nseg_long;
+    if (nl ? P.nseg <= kOneLaunchSegments : whole_lanes && P.nnz >= (uint64_t)12 * P.nseg)
+        nl = P.nseg, ns = 0;
+}
+
 // Makes the auxiliary stream wait for everything queued on the main stream so
 // far.  On failure nothing was queued on aux and the caller stays on main.
 inline bool fork_aux(const Streams &S)
@@ -1945,9 +1992,8 @@ template <typename T, int LPR, int VPL, int UB, int US, int RG, int FZ>
 hipError_t run_sddmm(const DevPlanView &P, const T *A, const T *B, T *C, T *Y, const Streams &S,
                      uint32_t nvec, uint32_t stride = 0, uint32_t accum = 0)
 {
-    uint32_t nl = P.nseg_long, ns = P.nseg - P.nseg_long;
-    if (nl && ns && P.nseg <= kOneLaunchSegments)
-        nl = P.nseg, ns = 0;
+    uint32_t nl, ns;
+    split_launches(P, RG == 0, nl, ns);
     const bool both = nl && ns && fork_aux(S);
     if (nl)
         hipLaunchKernelGGL((sddmm_seg_kernel<T, LPR, VPL, UB, RG, true, FZ>),
@@ -1972,9 +2018,8 @@ template <typename T, int LPR, int VPL, int UB, int US, int RG>
 hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, uint32_t nvec,
                     uint32_t stride = 0, size_t slice_off = 0)
 {
-    uint32_t nl = P.nseg_long, ns = P.nseg - P.nseg_long;
-    if (nl && ns && P.nseg <= kOneLaunchSegments)
-        nl = P.nseg, ns = 0;
+    uint32_t nl, ns;
+    split_launches(P, RG == 0, nl, ns);
     const bool both = nl && ns && fork_aux(S);
     if (nl)
         hipLaunchKernelGGL((spmm_seg_kernel<T, LPR, VPL, UB, RG, true>),
@@ -2012,13 +2057,26 @@ hipError_t launch_fixup(const DevPlanView &P, T *Y, uint32_t K, hipStream_t st)
 {
     if (!P.nsplit)
         return hipSuccess;
+    using V = typename Vec<T>::type;
+    const bool vec = K % Vec<T>::N == 0;
+    const uint32_t units = vec ? K / Vec<T>::N : K;
     uint32_t lanes = 4;
-    while (lanes < (uint32_t)kBlock && lanes < K)
+    while (lanes < (uint32_t)kBlock && lanes < units)
         lanes *= 2;
-    const uint32_t rows_per_block = kBlock / lanes;
-    hipLaunchKernelGGL((spmm_fixup_kernel<T>),
-                       dim3((P.nsplit + rows_per_block - 1) / rows_per_block), dim3(kBlock), 0, st,
-                       P.splits, P.nsplit, (const T *)P.partial, Y, K, lanes);
+    // Runs while the launch does not fill the chip anyway, and for rows of many slots.
+    uint32_t parts = 1;
+    while (lanes * parts < (uint32_t)kBlock &&
+           parts * P.nsplit <= 2 * (uint64_t)P.nslots &&
+           ((uint64_t)P.nsplit * lanes * parts < (1u << 18) || parts * 4 < P.nslots / P.nsplit))
+        parts *= 2;
+    const uint32_t rows = kBlock / (lanes * parts);
+    const dim3 grid((P.nsplit + rows - 1) / rows);
+    if (vec)
+        hipLaunchKernelGGL((spmm_fixup_kernel<T, V>), grid, dim3(kBlock), 0, st, P.splits, P.nsplit,
+                           (const V *)P.partial, (V *)Y, units, lanes, parts);
+    else
+        hipLaunchKernelGGL((spmm_fixup_kernel<T, T>), grid, dim3(kBlock), 0, st, P.splits, P.nsplit,
+                           (const T *)P.partial, Y, units, lanes, parts);
     return hipGetLastError();
 }
 

@@ -164,8 +164,4 @@ int build_two_pass(const DevStream &stream, const uint32_t *d_perm, uint64_t nnz
 int is_nondecreasing_device(const DevStream &stream, const uint32_t *d, uint64_t n, bool *out,
                             std::string &err);
 
-// Sum of len^2 over a plan's segments (device array); synchronous.
-int sum_sq_seg_len_device(const DevStream &stream, const Seg *d_segs, uint64_t nseg, uint64_t *out,
-                          std::string &err);
-
 } // namespace spc3d

@@ -28,6 +28,7 @@ struct Counters { // one device-resident block, zeroed (first_bad: all ones) bef
     uint32_t nlong;
     uint32_t rows_unsorted;
     unsigned long long covered;
+    unsigned long long row_sq;
     unsigned long long load[kSlices];
     unsigned long long any_load;
     unsigned long long pref_load[kSlices];
@@ -285,20 +286,26 @@ __global__ void run_lengths_k(const uint32_t *__restrict__ start, uint64_t nbins
     }
 }
 
-// Number of non-zero counts and the largest count.
+// Number of non-zero counts, the largest count and, with sq, the sum of count * min(count, 2048).
 __global__ void stats_k(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *touched,
-                        uint32_t *maxv)
+                        uint32_t *maxv, unsigned long long *sq)
 {
     uint32_t t = 0, m = 0;
+    unsigned long long s = 0;
     GRID_STRIDE(i, n)
     {
         const uint32_t v = cnt[i];
         t += v != 0;
         m = m > v ? m : v;
+        s += (unsigned long long)v * (v < 2048 ? v : 2048);
     }
     t = block_sum(t);
     m = block_max(m);
+    if (sq)
+        s = block_sum(s);
     if (threadIdx.x == 0) {
+        if (sq && s)
+            atomicAdd(sq, s);
         if (t)
             atomicAdd(touched, t);
         if (m)
@@ -888,18 +895,6 @@ __global__ void ranks_k(const uint32_t *__restrict__ sorted, uint64_t n, uint32_
 {
     GRID_STRIDE(i, n) rank[sorted[i]] = (uint32_t)i;
 }
-__global__ void sum_sq_len_k(const Seg *__restrict__ segs, uint64_t n, unsigned long long *out)
-{
-    unsigned long long s = 0;
-    GRID_STRIDE(i, n)
-    {
-        const unsigned long long l = segs[i].len;
-        s += l * l;
-    }
-    s = block_sum(s);
-    if (threadIdx.x == 0 && s)
-        atomicAdd(out, s);
-}
 
 } // namespace
 
@@ -915,8 +910,6 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         err = "ii/jj is NULL with nnz > 0";
         return SPC3D_ERR_INVALID_ARG;
     }
-    const uint32_t seg_max =
-        clamp_seg_max(opts.seg_max ? opts.seg_max : default_seg_max(nnz, opts.row_bytes), nnz);
     const uint32_t hub_min = opts.hub_min ? opts.hub_min : kDefaultHubMin;
     const bool want_slices = opts.xcd_slices == 0 || opts.xcd_slices == kSlices;
 
@@ -924,9 +917,10 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     P.nrows = nrows;
     P.ncols = ncols;
     P.nnz = nnz;
-    P.seg_max = seg_max;
     out = DevPlanArrays{};
     if (nnz == 0) {
+        P.seg_max = clamp_seg_max(
+            opts.seg_max ? opts.seg_max : default_seg_max(nnz, opts.row_bytes, nrows, 0, 0), nnz);
         meta = std::move(P);
         return SPC3D_OK;
     }
@@ -983,13 +977,20 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         LAUNCH(run_bounds_k, nnz, sorted.p, nnz, ncols, start.p, coldeg.p);
         LAUNCH(run_lengths_k, ncols, start.p, (uint64_t)ncols, coldeg.p);
     }
-    LAUNCH_SMALL(stats_k, nrows, rowcnt.p, (uint64_t)nrows, &dC.p->rows_touched, &dC.p->max_row);
-    LAUNCH_SMALL(stats_k, ncols, coldeg.p, (uint64_t)ncols, &dC.p->cols_touched, &dC.p->max_cdeg);
+    LAUNCH_SMALL(stats_k, nrows, rowcnt.p, (uint64_t)nrows, &dC.p->rows_touched, &dC.p->max_row,
+                 &dC.p->row_sq);
+    LAUNCH_SMALL(stats_k, ncols, coldeg.p, (uint64_t)ncols, &dC.p->cols_touched, &dC.p->max_cdeg,
+                 (unsigned long long *)nullptr);
     TRY(exclusive_sum(tmp, rowcnt.p, rowptr.p, (size_t)nrows + 1, st, err));
     TRY(fetch(st, &hC, dC.p, sizeof hC, err));
     P.rows_touched = hC.rows_touched;
     P.cols_touched = hC.cols_touched;
     P.max_row_nnz = hC.max_row;
+    P.row_sq = hC.row_sq;
+    const uint32_t seg_max = clamp_seg_max(
+        opts.seg_max ? opts.seg_max
+                     : default_seg_max(nnz, opts.row_bytes, nrows, hC.rows_touched, hC.max_row), nnz);
+    P.seg_max = seg_max;
     const uint32_t ctouched = hC.cols_touched, maxcdeg = hC.max_cdeg;
 
     // ---- column classes (XCD slicing only) ---------------------------------------
@@ -1869,22 +1870,6 @@ int is_nondecreasing_device(const DevStream &st, const uint32_t *d, uint64_t n, 
     unsigned long long descents = 0;
     TRY(fetch(st, &descents, acc.p, sizeof descents, err));
     *out = descents == 0;
-    return SPC3D_OK;
-}
-
-int sum_sq_seg_len_device(const DevStream &st, const Seg *d_segs, uint64_t nseg, uint64_t *out,
-                          std::string &err)
-{
-    *out = 0;
-    if (nseg == 0)
-        return SPC3D_OK;
-    DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(st, 1));
-    HIP_OK(hipMemsetAsync(acc.p, 0, sizeof(unsigned long long), st));
-    LAUNCH_SMALL(sum_sq_len_k, nseg, d_segs, nseg, acc.p);
-    unsigned long long h = 0;
-    TRY(fetch(st, &h, acc.p, sizeof h, err));
-    *out = h;
     return SPC3D_OK;
 }
 

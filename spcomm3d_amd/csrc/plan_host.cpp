@@ -68,18 +68,46 @@ void sort_longest_first(std::vector<Piece> &v, uint32_t seg_max)
 
 } // namespace
 
-// nnz / 2048 rounded down to a power of two, within 64 .. 2048; at most 1024 for dense
-// rows of 128 bytes and 512 for rows of 64 bytes and less.  One lane group walks a
-// segment batch after batch, two memory latencies per batch, and the narrower the rows
-// the more segments share a wavefront and the fewer wavefronts a launch has: the
-// longest segments then set its duration (R-MAT 20, fp32 K = 16: SDDMM 542 us at 2048,
-// 421 at 512; SpMM 322 and 244; at 256-byte rows and more 1024 and 2048 are level).
-uint32_t default_seg_max(uint64_t nnz, uint32_t row_bytes)
+static uint32_t seg_max_cap(uint32_t row_bytes)
 {
-    const uint32_t cap = row_bytes == 0 || row_bytes > 128 ? 2048u : (row_bytes > 64 ? 1024u : 512u);
+    return row_bytes == 0 || row_bytes > 128 ? 2048u : (row_bytes > 64 ? 1024u : 512u);
+}
+
+uint32_t seg_max_by_entries(uint64_t nnz, uint32_t row_bytes)
+{
+    const uint32_t cap = seg_max_cap(row_bytes);
     uint32_t s = 64;
     while (s < cap && (uint64_t)s * 2 * 2048 <= nnz)
         s *= 2;
+    return s;
+}
+
+// One lane group walks a segment batch after batch, about 0.8 us per batch of 16 entries, so
+// the longest segment should be a small part of the launch: about a fifth of what the launch's
+// gathers take at 8 TB/s, which is nnz * (bytes of a dense row) / 2^21 entries, to the nearest
+// power of two within 16 .. 2048.  (Rows of 64 bytes and less run at the rate of entries, not of
+// bytes: R-MAT 16 to 18 measured best at half the length of 64-byte rows.)  Measured, SDDMM + SpMM
+// in us, fp32 R-MAT of 14 edges per row, at nnz / 2048 and now: scale 13, 256-byte rows 15.2 -> 12.3;
+// scale 16, 64-byte rows 72 -> 29, 256-byte 60 -> 46; scale 17, 64-byte 173 -> 57, 256-byte 112
+// -> 85; scale 18, 128-byte 200 -> 101; from about 10 M entries on the lengths are those of before.
+// Even rows (the longest within 4 times the mean) of up to 128 entries or twice that length stay
+// whole: cut, each of them would cost a partial sum and the fix-up (5,000 rows of 45, 128-byte dense
+// rows: SpMM 6 us whole, 10 in pieces of 16).
+// Width not known (no k_hint), or 4 M entries and more in rows of 2048 and more: by the entries.
+uint32_t default_seg_max(uint64_t nnz, uint32_t row_bytes, uint32_t nrows, uint32_t rows_touched,
+                         uint32_t max_row)
+{
+    if (row_bytes == 0 || (nnz >= (1u << 22) && nnz / 2048 >= nrows))
+        return seg_max_by_entries(nnz, row_bytes);
+    const uint64_t bytes = row_bytes <= 64 ? 32 : std::min(row_bytes, 1024u);
+    const uint64_t want = nnz * bytes >> 21;
+    const uint32_t cap = seg_max_cap(row_bytes);
+    uint32_t s = 16;
+    while (s < cap && want * 2 >= (uint64_t)s * 3)
+        s *= 2;
+    if ((uint64_t)max_row * rows_touched <= nnz * 4 && max_row <= std::max(128u, 2 * s))
+        while (s < cap && s < max_row)
+            s *= 2;
     return s;
 }
 
@@ -89,8 +117,6 @@ int build_host_plan(uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t
     int rc = validate_coo(nrows, ncols, nnz, ii, jj, err);
     if (rc != SPC3D_OK)
         return rc;
-    const uint32_t seg_max =
-        clamp_seg_max(opts.seg_max ? opts.seg_max : default_seg_max(nnz, opts.row_bytes), nnz);
     const uint32_t hub_min = opts.hub_min ? opts.hub_min : kDefaultHubMin;
     const bool want_slices = opts.xcd_slices == 0 || opts.xcd_slices == kSlices;
 
@@ -98,7 +124,6 @@ int build_host_plan(uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t
     P.nrows = nrows;
     P.ncols = ncols;
     P.nnz = nnz;
-    P.seg_max = seg_max;
     try {
         // ---- histograms -------------------------------------------------
         std::vector<uint32_t> rowptr((size_t)nrows + 1, 0), coldeg((size_t)ncols, 0);
@@ -121,6 +146,9 @@ int build_host_plan(uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t
         P.rows_touched = touched;
         P.cols_touched = ctouched;
         P.max_row_nnz = maxlen;
+        const uint32_t seg_max = clamp_seg_max(
+            opts.seg_max ? opts.seg_max : default_seg_max(nnz, opts.row_bytes, nrows, touched, maxlen), nnz);
+        P.seg_max = seg_max;
 
         // ---- column classes (XCD slicing only) -----------------------------
         // One L2 is expected to keep hot_cols dense rows.  A sixth of that goes to

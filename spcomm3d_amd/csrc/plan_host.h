@@ -39,7 +39,7 @@ struct SplitRow {
 
 // Zero in any field selects the default.
 struct PlanOpts {
-    uint32_t seg_max = 0;    // longest segment (default: by nnz and row_bytes, 64 .. 2048)
+    uint32_t seg_max = 0;    // longest segment (default: by nnz and row_bytes, 16 .. 2048)
     uint32_t row_bytes = 0;  // bytes of the dense rows the plan will mostly run with (0: unknown)
     uint32_t xcd_slices = 0; // 8 (default): hot columns are dealt to the 8 XCD L2s; 1: off
     uint32_t hot_cols = 0;   // slicing: dense rows one L2 is expected to keep
@@ -59,6 +59,7 @@ struct HostPlan {
     uint64_t nnz = 0;
     uint32_t rows_touched = 0, cols_touched = 0;
     uint32_t max_row_nnz = 0;
+    uint64_t row_sq = 0;           // sum over rows of length * min(length, 2048) (GPU builder)
     uint32_t seg_max = 0;
     uint32_t nslots = 0;
     uint32_t nseg_real = 0;        // segments with entries (segs.size() includes padding)
@@ -215,9 +216,12 @@ SPC3D_HD inline uint32_t deal_queue_pref(uint32_t i, uint8_t pref, const DealPla
 
 // Default longest segment: long enough that few rows are cut (each cut costs a
 // partial-sum row in SpMM), short enough that the longest segments do not
-// outlast the rest of the grid: nnz / 2048 rounded down to a power of two,
-// within [64, 2048].
-uint32_t default_seg_max(uint64_t nnz, uint32_t row_bytes);
+// outlast the rest of the grid.
+uint32_t default_seg_max(uint64_t nnz, uint32_t row_bytes, uint32_t nrows, uint32_t rows_touched,
+                         uint32_t max_row);
+// nnz / 2048 rounded down to a power of two, within 64 .. 2048; at most 1024 for dense rows of
+// 128 bytes and 512 for rows of 64 bytes and less.
+uint32_t seg_max_by_entries(uint64_t nnz, uint32_t row_bytes);
 
 // A requested longest segment, brought into [1, 2^20]: the builders keep one counter
 // per segment length.
