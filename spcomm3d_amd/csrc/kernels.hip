@@ -1419,8 +1419,8 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 //
 // LPR lanes (the power of two that covers a row, at most a wavefront) move one row, a unit
 // of 16 bytes each, and several rows at a time, so that every index is asked for before the
-// first row and every row before the first store (1, 2, 4, 8 rows in flight: a sum takes 63, 63,
-// 71, 85 us at fp32 K = 50 and 102, 101, 105, 122 at fp64 K = 64, the copies are level to 4).  Bound by memory: nothing is
+// first row and every row before the first store (the copies are level from 4 rows in flight to 8; a
+// sum takes one row at a time and several of its slots).  Bound by memory: nothing is
 // computed.  UNIT: kVec - rows of whole 16-byte vectors; kLoose - rows that end inside one
 // start at element alignment, and their last unit is the 16 bytes that END at the row's end
 // (it overlaps the unit before: a copy writes the same bytes twice, a sum stores only the
@@ -1430,7 +1430,6 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 // alignment touches 2.6 lines of 128).
 enum RowUnit { kVec, kLoose, kElem };
 constexpr int kRowsAhead = 4;    // of a copy
-constexpr int kRowsAheadSum = 2; // of a sum, which holds two units per row
 // Fewer workgroups than this (8 per CU) do not fill the chip: one row at a time then, which
 // makes more of them (50 k rows of 56 bytes: sum 6.8 against 4.8 us).
 constexpr uint64_t kRowsMinBlocks = 2048;
@@ -1518,7 +1517,8 @@ rows_pack_kernel(const char *__restrict__ panel, const uint32_t *__restrict__ ro
 // where its slots start in `slots`, ascending): ADD = false: panel row = its last slot (what
 // the reference's sequential copy leaves); ADD = true: panel row += each slot in order (the
 // reference's sequential sum, bit for bit).
-template <typename T, RowUnit UNIT, int LPR, int U, bool ADD>
+// ADD: one row per lane group (U == 1), D of its slots after the first in flight.
+template <typename T, RowUnit UNIT, int LPR, int U, bool ADD, int D = 1>
 __global__ void __launch_bounds__(kBlock)
 rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
                    const uint32_t *__restrict__ slots, uint32_t n, uint32_t units, uint64_t bytes,
@@ -1526,18 +1526,18 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
 {
     using A = RowAccess<T, UNIT>;
     constexpr uint32_t GPB = kBlock / LPR;
+    static_assert(!ADD || U == 1, "sums go row by row");
     const uint32_t sub = threadIdx.x % LPR;
     const uint64_t first = (uint64_t)blockIdx.x * (GPB * U) + threadIdx.x / LPR;
     u32x4 d[U]; // row, first slot, last slot, start in slots
-    uint32_t more = 0, left[U]; // slots of a row after its first
+    uint32_t left = 0; // slots of the row after its first
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint64_t i = first + u * GPB;
         const uint64_t at = i < n ? i : n - 1;
         d[u] = nt_load(dests + at);
         if constexpr (ADD) {
-            left[u] = dests[at + 1][3] - d[u][3] - 1;
-            more = left[u] > more ? left[u] : more;
+            left = dests[at + 1][3] - d[u][3] - 1;
         }
     }
     for (uint32_t v = sub; v < units; v += LPR) {
@@ -1554,15 +1554,20 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 y[u] += x[u];
-            for (uint32_t t = 1; t <= more; ++t) { // repeated rows: their t-th slots together
+            for (uint32_t t = 1; t <= left; t += D) {
+                typename A::V z[D];
+                uint32_t slot[D];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (t <= left[u])
-                        x[u] = A::load_nt(buf + (uint64_t)slots[d[u][3] + t] * bytes + off);
+                for (int j = 0; j < D; ++j)
+                    slot[j] = slots[d[0][3] + (t + j < left ? t + j : left)];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (t <= left[u])
-                        y[u] += x[u];
+                for (int j = 0; j < D; ++j)
+                    z[j] = A::load_nt(buf + (uint64_t)slot[j] * bytes + off);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < D; ++j)
+                    if (t + j <= left)
+                        y[0] += z[j];
             }
         }
 #pragma unroll
@@ -2424,33 +2429,43 @@ void rows_launch_ahead(int op, char *panel, const RowMapView &M, uint32_t n, uin
 {
     const uint32_t per = kBlock / LPR * U;
     const dim3 grid((uint32_t)(((uint64_t)n + per - 1) / per)), block(kBlock);
-    if constexpr (U != kRowsAheadSum) {
-        if (op == 0) {
-            hipLaunchKernelGGL((rows_pack_kernel<T, UNIT, LPR, U>), grid, block, 0, st, panel, M.rows,
-                               n, units, bytes, buf);
-            return;
-        }
-        if (op == 1) {
-            hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, U, false>), grid, block, 0, st,
-                               panel, (const u32x4 *)M.dests, M.slots, n, units, bytes, buf);
-            return;
-        }
-    }
-    if constexpr (U != kRowsAhead)
-        hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, U, true>), grid, block, 0, st, panel,
+    if (op == 0)
+        hipLaunchKernelGGL((rows_pack_kernel<T, UNIT, LPR, U>), grid, block, 0, st, panel, M.rows, n,
+                           units, bytes, buf);
+    else
+        hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, U, false, 1>), grid, block, 0, st, panel,
                            (const u32x4 *)M.dests, M.slots, n, units, bytes, buf);
+}
+
+template <typename T, RowUnit UNIT, int LPR, int D>
+void rows_launch_sum(char *panel, const RowMapView &M, uint32_t units, uint64_t bytes, char *buf,
+                     hipStream_t st)
+{
+    constexpr uint32_t per = kBlock / LPR;
+    hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, 1, true, D>),
+                       dim3((M.nuniq + per - 1) / per), dim3(kBlock), 0, st, panel,
+                       (const u32x4 *)M.dests, M.slots, M.nuniq, units, bytes, buf);
 }
 
 template <typename T, RowUnit UNIT, int LPR>
 void rows_launch(int op, char *panel, const RowMapView &M, uint32_t units, uint64_t bytes, char *buf,
                  hipStream_t st)
 {
+    // The slots of a row are a chain of two loads each, so as many of them go together as rows have
+    // on average: 6,400 rows of 26 slots, fp32 K = 4, take 12 / 8.6 / 6.6 / 5.6 us by ones, twos,
+    // fours and eights; 287 k rows of 2.7, K = 8, 24 / 21 / 22.5 / 28.
+    if (op == 2) {
+        if (M.nslots >= 8 * (uint64_t)M.nuniq)
+            rows_launch_sum<T, UNIT, LPR, 8>(panel, M, units, bytes, buf, st);
+        else if (M.nslots >= 3 * (uint64_t)M.nuniq)
+            rows_launch_sum<T, UNIT, LPR, 4>(panel, M, units, bytes, buf, st);
+        else
+            rows_launch_sum<T, UNIT, LPR, 2>(panel, M, units, bytes, buf, st);
+        return;
+    }
     const uint32_t n = op == 0 ? M.nslots : M.nuniq;
-    const uint64_t ahead = op == 2 ? kRowsAheadSum : kRowsAhead;
-    if (n / (kBlock / LPR * ahead) < kRowsMinBlocks)
+    if (n / (kBlock / LPR * kRowsAhead) < kRowsMinBlocks)
         rows_launch_ahead<T, UNIT, LPR, 1>(op, panel, M, n, units, bytes, buf, st);
-    else if (op == 2)
-        rows_launch_ahead<T, UNIT, LPR, kRowsAheadSum>(op, panel, M, n, units, bytes, buf, st);
     else
         rows_launch_ahead<T, UNIT, LPR, kRowsAhead>(op, panel, M, n, units, bytes, buf, st);
 }
@@ -2467,7 +2482,11 @@ hipError_t rows_typed(int op, void *panel, const RowMapView &M, uint32_t K, void
     const uint32_t units = (uint32_t)((bytes + 15) / 16);
 #define SPC3D_ROWS(UNIT)                                                                          \
     do {                                                                                          \
-        if (units <= 4)                                                                           \
+        if (units == 1)                                                                           \
+            rows_launch<T, UNIT, 1>(op, p, M, units, bytes, q, st);                               \
+        else if (units == 2)                                                                      \
+            rows_launch<T, UNIT, 2>(op, p, M, units, bytes, q, st);                               \
+        else if (units <= 4)                                                                      \
             rows_launch<T, UNIT, 4>(op, p, M, units, bytes, q, st);                               \
         else if (units <= 8)                                                                      \
             rows_launch<T, UNIT, 8>(op, p, M, units, bytes, q, st);                               \
