@@ -173,10 +173,16 @@ typedef struct {
                               positions when four in five of them follow their predecessor
                               there (a row's entries together), else through a staging vector
                               (spc3d_plan_info.staged_entries).
+                              A plan that stays ordinary holds such tiles besides (in
+                              device_bytes, not in sweep_entries) where its columns are not
+                              skewed and calls at K = k_hint run faster over them: spc3d_sddmm,
+                              spc3d_spmm where rows are long enough; every other call and K
+                              runs the ordinary arrays.
                               0 (default): as described; 1: never; 2: whenever k_hint has such
                               a width, whatever the pattern (col_blocks, if given, is the
                               number of blocks) */
-    uint32_t sweep_min_row; /* shortest row kept in the tiles (default 64) */
+    uint32_t sweep_min_row; /* shortest row kept in the tiles (default 64; in the tiles
+                              of an ordinary plan 16 to 64, by the number of blocks) */
     uint32_t reserved[1];  /* must be 0 */
 } spc3d_plan_opts;
 /* spc3d_plan_opts.flags.  The first three keep spc3d_sddmm's plain stores where the plan

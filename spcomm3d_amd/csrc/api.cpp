@@ -779,6 +779,8 @@ int spc3d_sddmm(spc3d_ctx *ctx, spc3d_plan *S, const spc3d_panel *A, const spc3d
     rc = plan_for_k(S, K, true, &S); // a plan in row tiles at another K: its ordinary twin
     if (rc)
         return rc;
+    if (S->tiles_sddmm && K == S->tiles->sweep_k)
+        S = S->tiles;
     if (S->by_col) { // the same entries with rows and columns, and so A and B, exchanged
         const spc3d_plan *T = S->by_col;
         HIP_TRY(launch_sddmm(S->dtype, view_of(T), B->dev, A->dev, C->dev, K, streams_of(ctx)));
@@ -847,6 +849,8 @@ int spc3d_spmm(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc3d_panel
     rc = plan_for_k(Ap, K, true, &Ap);
     if (rc)
         return rc;
+    if (Ap->tiles_spmm && K == Ap->tiles->sweep_k)
+        Ap = Ap->tiles;
     std::vector<spc3d_plan *> self;
     for (spc3d_plan *part : parts_of(Ap, self)) {
         rc = ensure_partial(part, K);
@@ -870,6 +874,8 @@ int spc3d_spmm_noalloc(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc
     rc = plan_for_k(Ap, K, false, &Ap); // (this call builds nothing)
     if (rc)
         return rc;
+    if (Ap->tiles_spmm && K == Ap->tiles->sweep_k)
+        Ap = Ap->tiles;
     const uint64_t need = (uint64_t)Ap->info.npartial_slots * K * elem_size(Ap->dtype);
     if (need > kStaticScratchBytes) {
         char msg[200];

@@ -200,6 +200,10 @@ struct spc3d_plan {
     // `other_k`: an ordinary plan of the same pattern, made from this plan's own arrays by the
     // first such call (plan_for_k) and kept, with this plan's values.
     spc3d_plan *other_k = nullptr;
+    // An ordinary plan's pattern once more as row tiles, for the calls at tiles->sweep_k that run
+    // faster so (add_tiles).
+    spc3d_plan *tiles = nullptr;
+    bool tiles_sddmm = false, tiles_spmm = false; // which of them
 };
 
 inline SweepView sweep_view_of(const spc3d_plan *p)
@@ -212,6 +216,7 @@ inline SweepView sweep_view_of(const spc3d_plan *p)
     v.sval = p->sweep_sval;
     v.ntiles = p->sweep.ntiles;
     v.nblocks = p->sweep.nblocks;
+    v.K = p->sweep_k;
     v.rows_per_tile = p->sweep.rows_per_tile;
     v.lanes = p->sweep.lanes;
     v.per_launch = p->sweep.per_launch;

@@ -414,14 +414,14 @@ static void choose_sweep(const spc3d_plan *p, const spc3d_plan_opts *opts, uint3
 // or the device memory does not reach; any other failure is returned.
 static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                             const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
-                            const spc3d_plan_opts *opts, uint32_t lanes, uint32_t nb, bool *taken)
+                            const spc3d_plan_opts *opts, uint32_t lanes, uint32_t nb,
+                            uint32_t min_row, bool *taken)
 {
     *taken = false;
     if (nnz + 64 >= (1ull << 32)) // staging places are 32-bit, the rest's start rounded up to 64
         return SPC3D_OK;
     spc3d_ctx *ctx = p->ctx;
     const size_t w = elem_size(p->dtype);
-    const uint32_t min_row = opts->sweep_min_row ? opts->sweep_min_row : 64;
     const uint32_t per_launch = (uint32_t)std::max(1, ctx->cu_count);
     std::string err;
     SweepPlan sw;
@@ -553,6 +553,75 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
     return SPC3D_OK;
 }
 
+// Row tiles beside a finished single plan (spc3d_plan::tiles), for patterns that column blocks
+// would not serve.  The tiles read a block of dense rows into each L2 once per generation of
+// tiles instead of once per miss, so they pay where
+//  - the columns are not skewed and the panel is well over an L2: 4 blocks of 3.25 MiB or more
+//    (at 2 the tiles are level to 15 % slower);
+//  - every column comes up often enough for its copy in each L2: 12 entries (at 5, 1 KB rows,
+//    264 -> 317 us; at 18, 930 -> 658);
+//  - the launch is long enough for the barriers of its blocks: 512 MiB of gathers.
+// Rows shorter than the number of blocks would hold less than an entry per block and stay out,
+// as do those under 16 entries.  SpMM adds a row's sums to LDS once per block, in rows padded to the
+// lanes' width, so it takes the tiles only for rows of 24 full widths and more on average, and 1.5
+// per block (rows of 30, 512-byte rows 974 -> 831 us, 384-byte 691 -> 752).
+// SDDMM results in an arbitrary order leave the tiles through the staging vector, which costs more
+// than the ordinary plan's two passes: from 400-byte rows on the tiles make up for it (8.9 M entries:
+// 256 bytes 280 -> 318 us, 360 level, 512 582 -> 486).
+// Measured (SDDMM + SpMM): 200 k x 40 k, mean 107, 512-byte rows 2557 -> 1360 us, 1 KB 5620 -> 2620,
+// 256-byte 1095 -> 790; 70 k x 150 k, mean 44, 512-byte 456 -> 350; uniform rows of 30 over 50 k
+// columns, 512-byte 1912 -> 1384.
+// The plan itself stays: it runs every other K, the one-pass calls (which read the dense rows
+// once, as fast as either of the tiles' kernels) and what the tiles leave out.
+static int add_tiles(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz,
+                     const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
+                     const spc3d_plan_opts *opts)
+{
+    const spc3d_plan_info &I = p->info;
+    if (!opts || opts->sweep || opts->col_blocks || !opts->k_hint || opts->builder == 1 ||
+        I.nqueues != 1 || nnz == 0)
+        return SPC3D_OK;
+    const uint32_t lanes = sweep_lanes_any(p->dtype, opts->k_hint);
+    if (!lanes)
+        return SPC3D_OK;
+    constexpr uint64_t kBlockBytes = (uint64_t)13 << 18; // as in choose_sweep
+    const uint64_t row_bytes = (uint64_t)opts->k_hint * elem_size(p->dtype);
+    const uint64_t nb = ((uint64_t)I.cols_touched * row_bytes + kBlockBytes - 1) / kBlockBytes;
+    const uint32_t min_row =
+        opts->sweep_min_row ? opts->sweep_min_row : (uint32_t)std::max<uint64_t>(16, std::min<uint64_t>(nb, 64));
+    const double mean = (double)nnz / (double)I.rows_touched;
+    if (nb < 4 || nb > std::min<uint32_t>(sweep_max_blocks(lanes), ncols) ||
+        nnz < (uint64_t)12 * I.cols_touched || nnz * row_bytes < ((uint64_t)512 << 20) ||
+        (double)p->row_sq < (double)nnz * min_row ||
+        (double)I.max_row_nnz * 8 > mean * sweep_rows_per_tile(lanes)) // (a tile of one long row)
+        return SPC3D_OK;
+    spc3d_plan *q = new (std::nothrow) spc3d_plan();
+    if (!q)
+        return SPC3D_OK;
+    q->ctx = p->ctx;
+    q->dtype = p->dtype;
+    q->info = I;
+    q->info.two_pass_results = q->info.sddmm_by_column = q->info.positions_by_segment = 0;
+    bool taken = false;
+    int rc = rebuild_as_sweep(q, nrows, ncols, nnz, d_ii, d_jj, po, opts, lanes, (uint32_t)nb, min_row,
+                              &taken);
+    q->magic = kMagicPlan;
+    if (rc || !taken || q->sweep.n * 4 < nnz * 3) { // (too much left over)
+        const std::string keep = g_err;
+        (void)spc3d_plan_destroy(q);
+        return rc ? fail(rc, keep) : SPC3D_OK;
+    }
+    const double len = (double)q->sweep.n / (double)std::max(1u, q->sweep.nrows_in);
+    const bool sddmm = !I.two_pass_results || row_bytes >= 400;
+    const bool spmm = len * (double)row_bytes >= 24.0 * lanes * 16 && len >= 1.5 * (double)nb;
+    if (!sddmm && !spmm)
+        return spc3d_plan_destroy(q);
+    p->tiles = q;
+    p->tiles_sddmm = sddmm;
+    p->tiles_spmm = spmm;
+    return SPC3D_OK;
+}
+
 // Plan of a pattern that lies on the device: the single plan first (validation, the
 // whole pattern's figures), then, where choose_col_blocks says so, one plan per block
 // of columns in its place.
@@ -578,7 +647,8 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         choose_sweep(p, opts, nb, &sw_lanes, &sw_nb);
         bool taken = false;
         if (sw_lanes)
-            rc = rebuild_as_sweep(p, nrows, ncols, nnz, d_ii, d_jj, po, opts, sw_lanes, sw_nb, &taken);
+            rc = rebuild_as_sweep(p, nrows, ncols, nnz, d_ii, d_jj, po, opts, sw_lanes, sw_nb,
+                                  opts->sweep_min_row ? opts->sweep_min_row : 64, &taken);
         if (rc) {
             const std::string keep = g_err;
             spc3d_plan_destroy(p);
@@ -597,6 +667,8 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         rc = add_sddmm_companion(p, nrows, ncols, nnz, d_ii, d_jj, po, so);
     if (!rc && nb <= 1)
         rc = add_two_pass(p, so);
+    if (!rc && nb <= 1)
+        rc = add_tiles(p, nrows, ncols, nnz, d_ii, d_jj, po, opts);
     if (rc || nb <= 1) {
         if (rc) {
             const std::string keep = g_err;
@@ -979,6 +1051,10 @@ int spc3d_plan_destroy(spc3d_plan *plan)
         plan->other_k = nullptr;
         (void)spc3d_plan_destroy(o);
     }
+    if (plan->tiles) {
+        (void)spc3d_plan_destroy(plan->tiles);
+        plan->tiles = nullptr;
+    }
     if (plan->by_col) {
         plan_free_device(plan->by_col);
         plan->by_col->magic = 0;
@@ -993,6 +1069,30 @@ int spc3d_plan_destroy(spc3d_plan *plan)
 
 
 
+// The values at `vals` (device, the caller's order) into every part of the plan but other_k.
+static hipError_t gather_values(spc3d_plan *plan, const void *vals)
+{
+    hipError_t e = hipSuccess;
+    if (plan->sweep.n)
+        e = launch_gather_vals(plan->dtype, vals, plan->sweep.perm, plan->sweep_sval, plan->sweep.n,
+                               plan->ctx->stream);
+    std::vector<spc3d_plan *> self;
+    for (spc3d_plan *part : parts_of(plan, self))
+        if (e == hipSuccess)
+            e = launch_gather_vals(plan->dtype, vals, part->perm, part->sval, part->info.nnz,
+                                   plan->ctx->stream);
+    if (e == hipSuccess && plan->by_col) {
+        e = launch_gather_vals(plan->dtype, vals, plan->by_col->perm, plan->by_col->sval,
+                               plan->info.nnz, plan->ctx->stream);
+        plan->by_col->has_values = true;
+    }
+    if (e == hipSuccess && plan->tiles)
+        e = gather_values(plan->tiles, vals);
+    if (e == hipSuccess)
+        plan->has_values = true;
+    return e;
+}
+
 int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
 {
     if (!live(plan))
@@ -1004,7 +1104,7 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
     if (rc)
         return rc;
     const size_t bytes = (size_t)nnz * elem_size(plan->dtype);
-    if (plan->blocks.empty() && !plan->perm && !plan->by_col && !plan->sweep.n) {
+    if (plan->blocks.empty() && !plan->perm && !plan->by_col && !plan->sweep.n && !plan->tiles) {
         rc = send_h2d(plan->ctx, plan->sval, vv_host, bytes);
     } else {
         void *tmp = nullptr;
@@ -1012,27 +1112,10 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
         if (rc)
             return rc;
         rc = send_h2d(plan->ctx, tmp, vv_host, bytes);
-        if (!rc && plan->sweep.n) {
-            hipError_t e = launch_gather_vals(plan->dtype, tmp, plan->sweep.perm, plan->sweep_sval,
-                                              plan->sweep.n, plan->ctx->stream);
+        if (!rc) {
+            const hipError_t e = gather_values(plan, tmp);
             if (e != hipSuccess)
                 rc = fail_hip(e, "gather of sparse values");
-        }
-        std::vector<spc3d_plan *> self;
-        for (spc3d_plan *part : parts_of(plan, self)) {
-            if (rc)
-                break;
-            hipError_t e = launch_gather_vals(plan->dtype, tmp, part->perm, part->sval,
-                                              part->info.nnz, plan->ctx->stream);
-            if (e != hipSuccess)
-                rc = fail_hip(e, "gather of sparse values");
-        }
-        if (!rc && plan->by_col) {
-            hipError_t e = launch_gather_vals(plan->dtype, tmp, plan->by_col->perm,
-                                              plan->by_col->sval, nnz, plan->ctx->stream);
-            if (e != hipSuccess)
-                rc = fail_hip(e, "gather of sparse values");
-            plan->by_col->has_values = true;
         }
         ctx_free(plan->ctx, tmp); // what gets this block next is queued behind the gathers
     }
@@ -1058,19 +1141,7 @@ int spc3d_plan_set_values_device(spc3d_plan *plan, const spc3d_vals *vv)
     int rc = use_device(plan->ctx, true);
     if (rc)
         return rc;
-    if (plan->sweep.n)
-        HIP_TRY(launch_gather_vals(plan->dtype, vv->dev, plan->sweep.perm, plan->sweep_sval,
-                                   plan->sweep.n, plan->ctx->stream));
-    std::vector<spc3d_plan *> self;
-    for (spc3d_plan *part : parts_of(plan, self))
-        HIP_TRY(launch_gather_vals(plan->dtype, vv->dev, part->perm, part->sval, part->info.nnz,
-                                   plan->ctx->stream));
-    if (plan->by_col) {
-        HIP_TRY(launch_gather_vals(plan->dtype, vv->dev, plan->by_col->perm, plan->by_col->sval,
-                                   plan->info.nnz, plan->ctx->stream));
-        plan->by_col->has_values = true;
-    }
-    plan->has_values = true;
+    HIP_TRY(gather_values(plan, vv->dev));
     if (plan->other_k)
         return spc3d_plan_set_values_device(plan->other_k, vv);
     return SPC3D_OK;
@@ -1111,6 +1182,11 @@ int spc3d_plan_probe_columns(spc3d_plan *plan, int mode, uint32_t modulus)
     }
     if (plan->by_col) { // its columns are the pattern's rows
         rc = probe_columns_of(plan->by_col, mode, modulus);
+        if (rc)
+            return rc;
+    }
+    if (plan->tiles) {
+        rc = spc3d_plan_probe_columns(plan->tiles, mode, modulus);
         if (rc)
             return rc;
     }
@@ -1191,22 +1267,12 @@ static int build_other_k(spc3d_plan *S, uint32_t K)
                 if (e == hipSuccess)
                     e = launch_scatter_vals(S->dtype, part->sval, part->perm, vals, part->info.nnz,
                                             ctx->stream);
-            std::vector<spc3d_plan *> self;
-            for (spc3d_plan *part : parts_of(q, self))
-                if (e == hipSuccess)
-                    e = launch_gather_vals(S->dtype, vals, part->perm, part->sval, part->info.nnz,
-                                           ctx->stream);
-            if (e == hipSuccess && q->by_col) {
-                e = launch_gather_vals(S->dtype, vals, q->by_col->perm, q->by_col->sval, nnz,
-                                       ctx->stream);
-                q->by_col->has_values = true;
-            }
+            if (e == hipSuccess)
+                e = gather_values(q, vals);
             if (e == hipSuccess)
                 e = hipStreamSynchronize(ctx->stream);
             if (e != hipSuccess)
                 rc = fail_hip(e, "values of the plan for another K");
-            else
-                q->has_values = true;
         }
     }
     if (!rc) {
@@ -1262,10 +1328,10 @@ int spc3d_plan_get_info(const spc3d_plan *plan, spc3d_plan_info *info)
         b += own_device_bytes(blk);
     if (plan->by_col)
         b += own_device_bytes(plan->by_col);
-    if (plan->other_k) {
-        spc3d_plan_info twin;
-        if (spc3d_plan_get_info(plan->other_k, &twin) == SPC3D_OK)
-            b += twin.device_bytes;
+    for (const spc3d_plan *more : {plan->other_k, plan->tiles}) {
+        spc3d_plan_info info2;
+        if (more && spc3d_plan_get_info(more, &info2) == SPC3D_OK)
+            b += info2.device_bytes;
     }
     info->device_bytes = b;
     return SPC3D_OK;

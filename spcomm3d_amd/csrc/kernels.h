@@ -74,17 +74,20 @@ struct SweepView {
     uint32_t ntiles = 0, nblocks = 0, rows_per_tile = 0;
     uint32_t lanes = 0;                  // lanes per dense row the plan was made for: 16, 32 or 64
     uint32_t per_launch = 0;             // tiles per generation (the GPU's CU count)
+    uint32_t K = 0;                      // reals of a dense row, at most lanes * 16 bytes of them
 };
 // Lanes per dense row of K reals when the sweep kernels take that width (dense rows of 256,
 // 512 or 1024 bytes), else 0; lane groups per workgroup, rows of a tile, and the most column
 // blocks a tile's range bounds fit LDS for, for that many lanes.
 uint32_t sweep_lanes(int dtype, uint32_t K);
+// The same for dense rows that need not fill the lanes: 129 to 1024 bytes.
+uint32_t sweep_lanes_any(int dtype, uint32_t K);
 uint32_t sweep_groups(uint32_t lanes);
 uint32_t sweep_rows_per_tile(uint32_t lanes);
 uint32_t sweep_max_blocks(uint32_t lanes);
 // SDDMM over the sweep's entries: C[k] = sval[k] * <A[row of k,:], B[col[k],:]> in sweep order
-// (the caller brings them to the caller's positions); SpMM: Y[row,:] += sums.  K = lanes * 16
-// bytes / sizeof(real) exactly.  One launch per generation of per_launch tiles.
+// (the caller brings them to the caller's positions); SpMM: Y[row,:] += sums.  One launch per
+// generation of per_launch tiles.
 hipError_t launch_sweep_sddmm(int dtype, const SweepView &S, const void *A, const void *B, void *C,
                               hipStream_t stream);
 hipError_t launch_sweep_spmm(int dtype, const SweepView &S, const void *X, void *Y, hipStream_t stream);

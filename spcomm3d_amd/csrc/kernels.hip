@@ -1179,15 +1179,68 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 constexpr int kSweepBlock = 1024;
 constexpr uint32_t kSweepRowBytes = 128u << 10; // of LDS for the tile's rows
 constexpr uint32_t kSweepPtrWords = 1028;       // nb + 1 range bounds of a tile, in LDS too
-template <typename T, int LPR>
-__device__ __forceinline__ T sweep_dot(const typename Vec<T>::type &a, const typename Vec<T>::type &b)
-{
-    T d = a[0] * b[0];
+// A lane's 16 bytes of a dense row.  ANY: rows of K reals, at least 16 bytes and at most LPR * 16,
+// at element alignment; as in the "odd" variants above, the lane that holds the row's end takes
+// the 16 bytes that END there and the lanes past it the same ones, and what is not a lane's to
+// count is left out of dot products and stores.  A tile's rows stay LPR * 16 bytes apart in LDS.
+template <typename T, int LPR, bool ANY> struct SweepLane {
+    using V = typename Vec<T>::type;
+    uint32_t sub, off = 0, bytes = LPR * 16;
+    bool keep[Vec<T>::N], all = true;
+    __device__ __forceinline__ SweepLane(uint32_t lane, uint32_t K) : sub(lane)
+    {
+        if constexpr (ANY) {
+            bytes = K * (uint32_t)sizeof(T);
+            const uint32_t first = sub * 16;
+            off = first < bytes - 16 ? first : bytes - 16;
+            all = off == first;
 #pragma unroll
-    for (int i = 1; i < Vec<T>::N; ++i)
-        d += a[i] * b[i];
-    return d;
-}
+            for (int i = 0; i < Vec<T>::N; ++i)
+                keep[i] = off + (uint32_t)i * sizeof(T) >= first;
+        }
+    }
+    __device__ __forceinline__ const char *at(const T *base, uint32_t row) const
+    {
+        return reinterpret_cast<const char *>(base) + (uint64_t)row * bytes + off;
+    }
+    __device__ __forceinline__ V load(const T *base, uint32_t row) const
+    {
+        if constexpr (ANY)
+            return loose_load<T>(at(base, row));
+        else
+            return reinterpret_cast<const V *>(base)[(uint64_t)row * LPR + sub];
+    }
+    __device__ __forceinline__ V load_once(const T *base, uint32_t row) const
+    {
+        if constexpr (ANY)
+            return loose_load_nt<T>(at(base, row));
+        else
+            return nt_load(reinterpret_cast<const V *>(base) + (uint64_t)row * LPR + sub);
+    }
+    __device__ __forceinline__ void store(V v, T *base, uint32_t row) const
+    {
+        char *to = const_cast<char *>(at(base, row));
+        if (!ANY) {
+            nt_store(v, reinterpret_cast<V *>(base) + (uint64_t)row * LPR + sub);
+        } else if (all) {
+            loose_store_nt<T>(v, to);
+        } else {
+#pragma unroll
+            for (int i = 0; i < Vec<T>::N; ++i)
+                if (keep[i])
+                    reinterpret_cast<T *>(to)[i] = v[i];
+        }
+    }
+    // a . b, a with zeros where nothing is kept
+    __device__ __forceinline__ T dot(const V &a, const V &b) const
+    {
+        T d = a[0] * (ANY && !keep[0] ? (T)0 : b[0]);
+#pragma unroll
+        for (int i = 1; i < Vec<T>::N; ++i)
+            d += a[i] * (ANY && !keep[i] ? (T)0 : b[i]);
+        return d;
+    }
+};
 
 // One batch of a lane group: its entries' columns, local rows and (for the lanes that need
 // one) sparse values, asked for one batch ahead.
@@ -1196,33 +1249,38 @@ template <typename T> struct SweepIdx {
     T val = (T)0;
 };
 
-template <typename T, int LPR, int UB>
+template <typename T, int LPR, int UB, bool ANY>
 __global__ void __launch_bounds__(kSweepBlock)
 sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ tile_rows,
                    const uint32_t *__restrict__ col, const uint16_t *__restrict__ lrow,
                    const T *__restrict__ sval, const uint32_t *__restrict__ pos,
                    const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, uint32_t nb,
-                   uint32_t R, uint32_t tile0)
+                   uint32_t R, uint32_t tile0, uint32_t K)
 {
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
     __shared__ V tile_a[kSweepRowBytes / 16];
     __shared__ uint32_t lptr[kSweepPtrWords];
     const uint32_t tile = tile0 + blockIdx.x;
-    for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock) {
+    const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
+    const SweepLane<T, LPR, ANY> lane(sub, K);
+    for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock) { // i % LPR == sub
         const uint32_t g = tile_rows[(uint64_t)tile * R + i / LPR];
         V v{};
         if (g != 0xFFFFFFFFu)
-            v = nt_load(reinterpret_cast<const V *>(A) + (uint64_t)g * LPR + i % LPR);
+            v = lane.load_once(A, g);
+        if constexpr (ANY) {
+#pragma unroll
+            for (int j = 0; j < Vec<T>::N; ++j)
+                v[j] = lane.keep[j] ? v[j] : (T)0;
+        }
         tile_a[i] = v;
     }
     for (uint32_t i = threadIdx.x; i < nb + 1; i += kSweepBlock)
         lptr[i] = ptr[(uint64_t)tile * nb + i];
     __syncthreads();
-    const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
     const uint32_t uo = entry_of<LPR, UB>(sub);
     const bool wlane = is_writer<LPR, UB>(sub);
-    const V *Bv = reinterpret_cast<const V *>(B);
     auto fetch = [&](uint32_t q, uint32_t qhi) {
         SweepIdx<T> x;
         x.n = qhi - q < (uint32_t)UB ? qhi - q : (uint32_t)UB;
@@ -1260,14 +1318,14 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const uint32_t c = __shfl(cur.col, u, LPR);
-                bv[u] = Bv[(uint64_t)c * LPR + sub];
+                bv[u] = lane.load(B, c);
             }
             __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
             T part[UB];
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const uint32_t l = __shfl(cur.row, u, LPR);
-                part[u] = sweep_dot<T, LPR>(tile_a[l * LPR + sub], bv[u]);
+                part[u] = lane.dot(tile_a[l * LPR + sub], bv[u]);
             }
             group_reduce<T, LPR, UB>(part, sub);
             if (wlane && uo < cur.n) {
@@ -1288,12 +1346,13 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
     }
 }
 
-template <typename T, int LPR, int UB>
+template <typename T, int LPR, int UB, bool ANY>
 __global__ void __launch_bounds__(kSweepBlock)
 sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ tile_rows,
                   const uint32_t *__restrict__ col, const uint16_t *__restrict__ lrow,
                   const T *__restrict__ sval, const uint32_t *__restrict__ vpos,
-                  const T *__restrict__ X, T *__restrict__ Y, uint32_t nb, uint32_t R, uint32_t tile0)
+                  const T *__restrict__ X, T *__restrict__ Y, uint32_t nb, uint32_t R, uint32_t tile0,
+                  uint32_t K)
 {
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
@@ -1309,7 +1368,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         lptr[i] = ptr[(uint64_t)tile * nb + i];
     __syncthreads();
     const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
-    const V *Xv = reinterpret_cast<const V *>(X);
+    const SweepLane<T, LPR, ANY> lane(sub, K);
     auto fetch = [&](uint32_t q, uint32_t qhi) {
         SweepIdx<T> x;
         x.n = qhi - q < (uint32_t)UB ? qhi - q : (uint32_t)UB;
@@ -1365,7 +1424,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const uint32_t c = __shfl(cur.col, u, LPR);
-                xv[u] = Xv[(uint64_t)c * LPR + sub];
+                xv[u] = lane.load(X, c);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1405,10 +1464,8 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
     }
     for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock) {
         const uint32_t g = tile_rows[(uint64_t)tile * R + i / LPR];
-        if (g != 0xFFFFFFFFu) {
-            V *y = reinterpret_cast<V *>(Y) + (uint64_t)g * LPR + i % LPR;
-            nt_store(nt_load(y) + tile_y[i], y);
-        }
+        if (g != 0xFFFFFFFFu)
+            lane.store(lane.load_once(Y, g) + tile_y[i], Y, g);
     }
 }
 
@@ -2269,23 +2326,28 @@ uint32_t sweep_lanes(int dtype, uint32_t K)
     const uint64_t bytes = (uint64_t)K * (dtype == 1 ? 8 : 4);
     return bytes == 256 ? 16u : (bytes == 512 ? 32u : (bytes == 1024 ? 64u : 0u));
 }
+uint32_t sweep_lanes_any(int dtype, uint32_t K)
+{
+    const uint64_t bytes = (uint64_t)K * (dtype == 1 ? 8 : 4);
+    return bytes <= 128 || bytes > 1024 ? 0 : (bytes <= 256 ? 16u : (bytes <= 512 ? 32u : 64u));
+}
 uint32_t sweep_groups(uint32_t lanes) { return lanes ? kSweepBlock / lanes : 0; }
 uint32_t sweep_rows_per_tile(uint32_t lanes) { return lanes ? kSweepRowBytes / (lanes * 16) : 0; }
 uint32_t sweep_max_blocks(uint32_t lanes) { return lanes ? kSweepPtrWords - 1 : 0; }
 
 namespace {
-template <typename T, int LPR>
+template <typename T, int LPR, bool ANY>
 void sweep_launch(bool spmm, const SweepView &S, const T *A, const T *B, T *out, uint32_t tile0,
                   uint32_t ntiles, hipStream_t stream)
 {
     if (spmm)
-        hipLaunchKernelGGL((sweep_spmm_kernel<T, LPR, 16>), dim3(ntiles), dim3(kSweepBlock), 0,
+        hipLaunchKernelGGL((sweep_spmm_kernel<T, LPR, 16, ANY>), dim3(ntiles), dim3(kSweepBlock), 0,
                            stream, S.ptr, S.tile_rows, S.col, S.lrow, (const T *)S.sval, S.pos, B,
-                           out, S.nblocks, S.rows_per_tile, tile0);
+                           out, S.nblocks, S.rows_per_tile, tile0, S.K);
     else
-        hipLaunchKernelGGL((sweep_sddmm_kernel<T, LPR, 16>), dim3(ntiles), dim3(kSweepBlock), 0,
+        hipLaunchKernelGGL((sweep_sddmm_kernel<T, LPR, 16, ANY>), dim3(ntiles), dim3(kSweepBlock), 0,
                            stream, S.ptr, S.tile_rows, S.col, S.lrow, (const T *)S.sval, S.pos, A,
-                           B, out, S.nblocks, S.rows_per_tile, tile0);
+                           B, out, S.nblocks, S.rows_per_tile, tile0, S.K);
 }
 template <typename T>
 hipError_t sweep_run(bool spmm, const SweepView &S, const T *A, const T *B, T *out, hipStream_t stream)
@@ -2295,16 +2357,21 @@ hipError_t sweep_run(bool spmm, const SweepView &S, const T *A, const T *B, T *o
     // what the kernels assume of the plan: the tile's rows and range bounds fit their LDS
     if ((S.lanes != 16 && S.lanes != 32 && S.lanes != 64) || S.per_launch == 0 ||
         S.rows_per_tile * S.lanes * 16 > kSweepRowBytes ||
-        (uint64_t)S.nblocks + 1 > kSweepPtrWords)
+        (uint64_t)S.nblocks + 1 > kSweepPtrWords || S.K * sizeof(T) < 16 ||
+        S.K * sizeof(T) > S.lanes * 16)
         return hipErrorInvalidValue;
+    const bool any = S.K * sizeof(T) != S.lanes * 16;
     for (uint32_t t0 = 0; t0 < S.ntiles; t0 += S.per_launch) { // one generation per launch
         const uint32_t n = S.ntiles - t0 < S.per_launch ? S.ntiles - t0 : S.per_launch;
         if (S.lanes == 16)
-            sweep_launch<T, 16>(spmm, S, A, B, out, t0, n, stream);
+            any ? sweep_launch<T, 16, true>(spmm, S, A, B, out, t0, n, stream)
+                : sweep_launch<T, 16, false>(spmm, S, A, B, out, t0, n, stream);
         else if (S.lanes == 32)
-            sweep_launch<T, 32>(spmm, S, A, B, out, t0, n, stream);
+            any ? sweep_launch<T, 32, true>(spmm, S, A, B, out, t0, n, stream)
+                : sweep_launch<T, 32, false>(spmm, S, A, B, out, t0, n, stream);
         else
-            sweep_launch<T, 64>(spmm, S, A, B, out, t0, n, stream);
+            any ? sweep_launch<T, 64, true>(spmm, S, A, B, out, t0, n, stream)
+                : sweep_launch<T, 64, false>(spmm, S, A, B, out, t0, n, stream);
     }
     return hipGetLastError();
 }

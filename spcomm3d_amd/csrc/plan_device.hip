@@ -1388,14 +1388,26 @@ __global__ void staged_fill_k(const uint32_t *__restrict__ perm, const uint32_t 
     }
 }
 
+// How many neighbours follow each other.  Four loads in flight per thread: with one this small grid
+// waits, 77 us for 15 M entries.
 __global__ void adjacent_k(const uint32_t *__restrict__ sorted, uint64_t n, unsigned long long *acc)
 {
     unsigned long long c = 0;
-    GRID_STRIDE(i, n)
-    if (i + 1 < n && sorted[i + 1] == sorted[i] + 1)
-        ++c;
-    c = wave_sum(c);
-    if ((threadIdx.x & 63u) == 0 && c)
+    const uint64_t stride = (uint64_t)gridDim.x * kTB;
+    for (uint64_t i = (uint64_t)blockIdx.x * kTB + threadIdx.x; i + 1 < n; i += 4 * stride) {
+        uint32_t v[4], w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t j = i + u * stride < n - 1 ? i + u * stride : i;
+            v[u] = sorted[j];
+            w[u] = sorted[j + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            c += i + u * stride < n - 1 && w[u] == v[u] + 1;
+    }
+    c = block_sum(c);
+    if (threadIdx.x == 0 && c)
         atomicAdd(acc, c);
 }
 
@@ -1563,6 +1575,17 @@ __global__ void inverse_offsets_k(const uint32_t *__restrict__ perm, uint64_t n,
     GRID_STRIDE(q, n) out[perm[q]] = base + (uint32_t)q;
 }
 
+// Rows of at least `least` entries.
+__global__ void count_min_k(const uint32_t *__restrict__ cnt, uint64_t nrows, uint32_t least,
+                            unsigned long long *out)
+{
+    unsigned long long c = 0;
+    GRID_STRIDE(r, nrows) c += cnt[r] >= least;
+    c = block_sum(c);
+    if (threadIdx.x == 0 && c)
+        atomicAdd(out, c);
+}
+
 // key[j] = (generation of rank j) << 32 | row of rank j
 __global__ void sweep_gen_keys_k(const uint32_t *__restrict__ order, uint32_t nin, uint64_t per_gen,
                                  unsigned long long *key)
@@ -1591,11 +1614,12 @@ __global__ void sweep_rows_k(const unsigned long long *__restrict__ gen_row, uin
 
 // Sort key of entry e: (tile, block, local row); one past the largest such key for an entry
 // of a row outside the sweep (they sort last, in the caller's order).
+template <typename KeyT>
 __global__ void sweep_keys_k(const uint32_t *__restrict__ ii, const uint32_t *__restrict__ jj,
                              uint64_t nnz, const uint32_t *__restrict__ row_tile,
                              const uint32_t *__restrict__ row_local, uint32_t block_cols,
-                             uint32_t nb, uint32_t R, unsigned long long rest_key,
-                             unsigned long long *key, unsigned long long *nin)
+                             uint32_t nb, uint32_t R, KeyT rest_key, KeyT *key,
+                             unsigned long long *nin)
 {
     unsigned long long mine = 0;
     GRID_STRIDE(e, nnz)
@@ -1605,7 +1629,7 @@ __global__ void sweep_keys_k(const uint32_t *__restrict__ ii, const uint32_t *__
             key[e] = rest_key;
             continue;
         }
-        key[e] = ((unsigned long long)t * nb + jj[e] / block_cols) * R + row_local[r];
+        key[e] = ((KeyT)t * nb + jj[e] / block_cols) * R + row_local[r];
         ++mine;
     }
     mine = block_sum(mine);
@@ -1614,18 +1638,52 @@ __global__ void sweep_keys_k(const uint32_t *__restrict__ ii, const uint32_t *__
 }
 
 // Of the sorted sweep entries: column, local row, and the (tile, block) bin.
-__global__ void sweep_entries_k(const unsigned long long *__restrict__ skey,
+template <typename KeyT>
+__global__ void sweep_entries_k(const KeyT *__restrict__ skey,
                                 const uint32_t *__restrict__ perm,
                                 const uint32_t *__restrict__ jj, uint64_t n, uint32_t R,
                                 uint32_t *col, uint16_t *lrow, uint32_t *bin)
 {
     GRID_STRIDE(k, n)
     {
-        const unsigned long long key = skey[k];
+        const KeyT key = skey[k];
         bin[k] = (uint32_t)(key / R);
         lrow[k] = (uint16_t)(key % R);
         col[k] = jj[perm[k]];
     }
+}
+
+// The entries in sweep order: perm (all nnz, those outside the sweep last), and column, local row
+// and bin of the n inside.
+template <typename KeyT>
+int sweep_entries(Arena &arena, Temp &tmp, const DevStream &st, uint64_t nnz, const uint32_t *d_ii,
+                  const uint32_t *d_jj, const uint32_t *row_tile, const uint32_t *row_local,
+                  uint32_t block_cols, uint32_t nb, uint32_t R, KeyT rest_key, unsigned long long *d_n,
+                  DBuf<uint32_t> &perm, DBuf<uint32_t> &col, DBuf<uint16_t> &lrow, SBuf<uint32_t> &bin,
+                  uint64_t &n, std::string &err)
+{
+    SBuf<KeyT> key, skey;
+    SBuf<uint32_t> ident;
+    HIP_OK(key.alloc(arena, nnz));
+    HIP_OK(skey.alloc(arena, nnz));
+    HIP_OK(ident.alloc(arena, nnz));
+    HIP_OK(perm.alloc(st, nnz));
+    LAUNCH_SMALL((sweep_keys_k<KeyT>), nnz, d_ii, d_jj, nnz, row_tile, row_local, block_cols, nb, R,
+                 rest_key, key.p, d_n);
+    LAUNCH(iota_k, nnz, ident.p, nnz);
+    TRY(sort_pairs<KeyT>(tmp, key.p, skey.p, ident.p, perm.p, (uint32_t)nnz, bits_for(rest_key), false,
+                         st, err));
+    unsigned long long seen = 0;
+    TRY(fetch(st, &seen, d_n, sizeof seen, err));
+    n = seen;
+    if (n == 0)
+        return SPC3D_OK;
+    HIP_OK(col.alloc(st, n));
+    HIP_OK(lrow.alloc(st, n));
+    HIP_OK(bin.alloc(arena, n));
+    LAUNCH((sweep_entries_k<KeyT>), n, skey.p, perm.p, d_jj, n, R, col.p, lrow.p, bin.p);
+    HIP_OK(hipGetLastError());
+    return SPC3D_OK;
 }
 
 int build_sweep(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t *d_ii,
@@ -1661,17 +1719,11 @@ int build_sweep(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nn
     // entries come first and are the sweep's
     LAUNCH(iota_k, nrows, rowid.p, (uint64_t)nrows);
     TRY(sort_pairs<uint32_t>(tmp, rowcnt.p, cnt_sorted.p, rowid.p, order.p, nrows, 32, true, st, err));
-    std::vector<uint32_t> lens;
-    try {
-        lens.resize(nrows);
-    } catch (const std::bad_alloc &) {
-        err = "host allocation failed";
-        return SPC3D_ERR_ALLOC;
-    }
-    TRY(fetch(st, lens.data(), cnt_sorted.p, (size_t)nrows * sizeof(uint32_t), err));
-    uint32_t nin = 0;
-    while (nin < nrows && lens[nin] >= min_row && lens[nin] > 0)
-        ++nin;
+    LAUNCH_SMALL(count_min_k, nrows, rowcnt.p, nrows, std::max(1u, min_row), total.p);
+    unsigned long long seen = 0;
+    TRY(fetch(st, &seen, total.p, sizeof seen, err));
+    HIP_OK(hipMemsetAsync(total.p, 0, sizeof(unsigned long long), st));
+    const uint32_t nin = (uint32_t)seen;
     if (nin == 0)
         return SPC3D_OK;
     // A generation: the next P * R rows by length, which one launch of P tiles takes.  Inside
@@ -1702,32 +1754,23 @@ int build_sweep(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nn
     LAUNCH(sweep_rows_k, nin, gkey_sorted.p, nin, P, R, (uint32_t)(gens - 1), rpt_last, row_tile.p,
            row_local.p, tile_rows.p);
     // ---- entries ----
-    SBuf<unsigned long long> key, skey;
-    SBuf<uint32_t> ident, bin;
-    HIP_OK(key.alloc(arena, nnz));
-    HIP_OK(skey.alloc(arena, nnz));
-    HIP_OK(ident.alloc(arena, nnz));
-    HIP_OK(perm.alloc(st, nnz));
-    const unsigned long long rest_key = (unsigned long long)ntiles * nb * R;
-    LAUNCH_SMALL(sweep_keys_k, nnz, d_ii, d_jj, nnz, row_tile.p, row_local.p, block_cols, nb, R,
-                 rest_key, key.p, total.p);
-    LAUNCH(iota_k, nnz, ident.p, nnz);
-    TRY(sort_pairs<unsigned long long>(tmp, key.p, skey.p, ident.p, perm.p, (uint32_t)nnz,
-                                       bits_for(rest_key), false, st, err));
-    unsigned long long n = 0;
-    TRY(fetch(st, &n, total.p, sizeof n, err));
+    SBuf<uint32_t> bin;
+    const uint64_t nbins = (uint64_t)ntiles * nb;
+    const unsigned long long rest_key = (unsigned long long)nbins * R;
+    uint64_t n = 0;
+    if (rest_key >> 32)
+        TRY(sweep_entries<unsigned long long>(arena, tmp, st, nnz, d_ii, d_jj, row_tile.p, row_local.p,
+                                              block_cols, nb, R, rest_key, total.p, perm, col, lrow, bin, n, err));
+    else // half the keys' traffic in the sort
+        TRY(sweep_entries<uint32_t>(arena, tmp, st, nnz, d_ii, d_jj, row_tile.p, row_local.p, block_cols,
+                                    nb, R, (uint32_t)rest_key, total.p, perm, col, lrow, bin, n, err));
     if (n == 0)
         return SPC3D_OK;
-    HIP_OK(col.alloc(st, n));
-    HIP_OK(lrow.alloc(st, n));
-    HIP_OK(bin.alloc(arena, n));
-    const uint64_t nbins = (uint64_t)ntiles * nb;
     HIP_OK(ptr.alloc(st, nbins + 1));
     SBuf<uint32_t> bstart, bcnt;
     HIP_OK(bstart.alloc(arena, nbins));
     HIP_OK(bcnt.alloc(arena, nbins + 1));
     HIP_OK(hipMemsetAsync(bcnt.p, 0, (nbins + 1) * sizeof(uint32_t), st));
-    LAUNCH(sweep_entries_k, n, skey.p, perm.p, d_jj, n, R, col.p, lrow.p, bin.p);
     LAUNCH(run_bounds_k, n, bin.p, n, (uint32_t)nbins, bstart.p, bcnt.p);
     LAUNCH(run_lengths_k, nbins, bstart.p, nbins, bcnt.p);
     TRY(exclusive_sum(tmp, bcnt.p, ptr.p, (size_t)nbins + 1, st, err));

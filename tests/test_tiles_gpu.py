@@ -1,0 +1,83 @@
+"""Row tiles beside an ordinary plan: which calls run over them, at the edge of the rule, in both
+element types, with rows left over, in arbitrary order, and under every call a plan takes."""
+import numpy as np
+import pytest
+
+from spcomm3d_amd import device
+from tests.test_parity_gpu import check_sddmm, check_spmm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with device.Context(0) as c:
+        yield c
+
+
+def pattern(lengths, n, shuffled, seed=3):
+    rng = np.random.default_rng(seed)
+    ii = np.repeat(np.arange(len(lengths), dtype=np.uint32), lengths)
+    jj = rng.integers(0, n, ii.size).astype(np.uint32)
+    if shuffled:
+        o = rng.permutation(ii.size)
+        ii, jj = ii[o], jj[o]
+    return np.ascontiguousarray(ii), np.ascontiguousarray(jj)
+
+
+# lengths of the rows, columns; 1 KB dense rows: 4 blocks of 3.25 MiB from 9985 touched columns on
+ROWS_80 = [80] * 7000
+MIXED = [90] * 6000 + [7] * 3000 + [0] * 10 + [300] * 30
+ROWS_20 = [20] * 27000      # SDDMM only
+@pytest.mark.parametrize("dtype,k", [(np.float32, 256), (np.float64, 128)])
+@pytest.mark.parametrize("lengths,n,tiled", [(ROWS_80, 11000, True), (MIXED, 12001, True),
+                                             (ROWS_20, 12000, True), (ROWS_80, 9000, False),
+                                             ([80] * 6500, 11000, False)])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_calls_over_the_tiles(ctx, dtype, k, lengths, n, tiled, shuffled):
+    m = len(lengths)
+    ii, jj = pattern(lengths, n, shuffled)
+    rng = np.random.default_rng(k)
+    vv, v2 = (rng.uniform(0, 1, ii.size).astype(dtype) for _ in range(2))
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (m, n, m))
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k)
+    plain = ctx.plan(m, n, ii, jj, vv, k_hint=k, sweep=False)
+    assert (S.info.device_bytes > plain.info.device_bytes) == tiled
+    assert S.info.nsegments == plain.info.nsegments and S.info.sweep_entries == 0
+    dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(ii.size, dtype)
+    S.set_values(v2)
+    S.set_values(vv)
+    for again in range(2):  # eagerly, then recorded and replayed
+        dC.fill(-5.0)
+        dY.upload(Y0)
+        if again:
+            ctx.capture_begin()
+        ctx.sddmm(S, dA, dB, dC)
+        ctx.spmm(S, dB, dY)
+        if again:
+            g = ctx.capture_end()
+            g.launch()
+            ctx.sync()
+            dC.fill(-5.0)
+            dY.upload(Y0)
+            g.launch()
+        C, Y = dC.download(), dY.download()
+        if again:
+            assert np.array_equal(C, C1) and np.array_equal(Y, Y1)
+            g.close()
+        C1, Y1 = C, Y
+    check_sddmm(A, B, ii, jj, vv, C)
+    check_spmm(B, ii, jj, vv, Y0, Y)
+    dY.upload(Y0)
+    ctx.spmm_noalloc(S, dB, dY)
+    assert np.array_equal(dY.download(), Y)
+    dY.upload(Y0)
+    ctx.sddmm_spmm(S, dA, dB, dC, dY, chained=True)
+    check_sddmm(A, B, ii, jj, vv, dC.download())
+    check_spmm(B, ii, jj, dC.download(), Y0, dY.download())
+    w = 3  # another width
+    a, b = np.ascontiguousarray(A[:, :w]), np.ascontiguousarray(B[:, :w])
+    ctx.sddmm(S, ctx.panel_from(a), ctx.panel_from(b), dC)
+    check_sddmm(a, b, ii, jj, vv, dC.download())
+    S.close()
+    plain.close()
