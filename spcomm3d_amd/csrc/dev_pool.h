@@ -22,6 +22,7 @@
 #include <mutex>
 #include <new>
 #include <unordered_map>
+#include <vector>
 
 namespace spc3d {
 
@@ -30,7 +31,12 @@ class DevPool {
     DevPool() = default;
     DevPool(const DevPool &) = delete;
     DevPool &operator=(const DevPool &) = delete;
-    ~DevPool() { trim(); }
+    ~DevPool()
+    {
+        trim();
+        for (void *p : words_)
+            (void)hipHostFree(p);
+    }
 
     void set_limit(size_t bytes) { limit_ = bytes; }
 
@@ -101,6 +107,37 @@ class DevPool {
             shrink(limit_);
     }
 
+    // A few words of pinned host memory for results on their way down (kWords bytes; null when
+    // there is none).  Into pageable memory the runtime stages such a copy and waits twice.
+    static constexpr size_t kWords = 1024;
+    void *get_words()
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (!words_.empty()) {
+                void *p = words_.back();
+                words_.pop_back();
+                return p;
+            }
+        }
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kWords, hipHostMallocDefault) == hipSuccess)
+            return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void put_words(void *p)
+    {
+        if (!p)
+            return;
+        try {
+            std::lock_guard<std::mutex> lock(mu_);
+            words_.push_back(p);
+        } catch (const std::bad_alloc &) {
+            (void)hipHostFree(p);
+        }
+    }
+
     // Frees every kept block.
     void trim()
     {
@@ -128,6 +165,7 @@ class DevPool {
     }
     static constexpr size_t kGrain = 512;
     std::mutex mu_;
+    std::vector<void *> words_; // get_words() of as many threads as ever plan at once
     std::multimap<size_t, Kept> kept_; // by size
     std::unordered_map<void *, size_t> sizes_; // of the blocks handed out
     size_t kept_bytes_ = 0, limit_ = 0;

@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/spcomm3d_hip.h"
 
@@ -29,9 +30,7 @@ struct Counters { // one device-resident block, zeroed (first_bad: all ones) bef
     uint32_t rows_unsorted;
     unsigned long long covered;
     unsigned long long row_sq;
-    unsigned long long load[kSlices];
-    unsigned long long any_load;
-    unsigned long long pref_load[kSlices];
+    unsigned long long load[kSlices], any_load, pref_load[kSlices];
 };
 
 // Owning device buffer; back to the pool on scope exit unless released.
@@ -137,6 +136,14 @@ inline uint32_t small_grid_for(uint64_t n) // kernels that end in one atomic per
 {
     const uint32_t g = grid_for(n);
     return g > 1024 ? 1024 : g;
+}
+
+// Kernels that end in a dozen and more atomics per workgroup: ten nanoseconds each, one after the
+// other (17 sums over 700 k pieces: 100 us on 1,024 workgroups).
+inline uint32_t few_grid_for(uint64_t n)
+{
+    const uint32_t g = grid_for(n);
+    return g > 192 ? 192 : g;
 }
 
 inline int bits_for(uint64_t max_value) // bits needed to hold max_value (at least 1)
@@ -336,49 +343,32 @@ __global__ void hubflag_k(const uint32_t *__restrict__ rowcnt, uint32_t nrows, u
     GRID_STRIDE(r, (uint64_t)nrows + 1) flag[r] = (r < nrows && rowcnt[r] >= hub_min) ? 1u : 0u;
 }
 
-// Per hub row, the number of entries in each of the 9 groups.  Whole wavefronts
-// walk the entries together: per group, the lanes that share the row of the first
-// such lane add their count with one atomic (sorted COO puts a wavefront on one or
-// two rows), the others one each.
-__global__ void hubcount_k(const uint32_t *__restrict__ ii, const uint32_t *__restrict__ jj,
-                           uint64_t nnz, const uint32_t *__restrict__ hubflag,
-                           const uint32_t *__restrict__ hubpos, const uint8_t *__restrict__ cls,
-                           uint32_t *hubcnt)
+// Per hub row, the number of entries in each of the 9 groups, from the sorted keys (keys_k): where a
+// run of equal keys starts its position is taken off the count (zeroed before), where it ends the
+// position after it is added.  16 M entries of R-MAT 20: an atomic per group and wavefront of the
+// unsorted entries took 244 us, this 49.
+template <typename KeyT>
+__global__ void hubcount_k(const KeyT *__restrict__ key, uint64_t nnz,
+                           const uint32_t *__restrict__ hubflag,
+                           const uint32_t *__restrict__ hubpos, uint32_t *hubcnt)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t stride = (uint64_t)gridDim.x * kTB;
-    for (uint64_t base = (uint64_t)blockIdx.x * kTB + (threadIdx.x & ~63u); base < nnz;
-         base += stride) {
-        const uint64_t e = base + lane;
-        uint32_t r = 0, grp = 0;
-        bool hub = false;
-        if (e < nnz) {
-            r = ii[e];
-            hub = hubflag[r] != 0;
-            if (hub)
-                grp = hub_group(r, cls[jj[e]]);
-        }
-        if (!__any(hub))
+    GRID_STRIDE(i, nnz)
+    {
+        const KeyT k = key[i];
+        const bool first = i == 0 || key[i - 1] != k, last = i + 1 == nnz || key[i + 1] != k;
+        if (!first && !last)
             continue;
-        for (uint32_t g = 0; g < 9; ++g) {
-            const bool mine = hub && grp == g;
-            const unsigned long long m = __ballot(mine);
-            if (m == 0)
-                continue;
-            const int lead = __ffsll((long long)m) - 1;
-            const uint32_t r0 = __shfl(r, lead, 64);
-            const unsigned long long same = __ballot(mine && r == r0);
-            if ((int)lane == lead)
-                atomicAdd(hubcnt + (size_t)hubpos[r] * 9 + g, (uint32_t)__popcll(same));
-            else if (mine && r != r0)
-                atomicAdd(hubcnt + (size_t)hubpos[r] * 9 + g, 1u);
-        }
+        const uint32_t r = (uint32_t)(k >> 4);
+        if (!hubflag[r])
+            continue;
+        const uint32_t n = (last ? (uint32_t)(i + 1) : 0u) - (first ? (uint32_t)i : 0u);
+        atomicAdd(hubcnt + (size_t)hubpos[r] * 9 + (uint32_t)(k & 15), n);
     }
 }
 
 // Sort key of entry e: its row, then (hub rows of the sliced layout) its group.
 // `visit` (may be null): the keys are laid out in that order of the entries, key[v] = key of
-// entry visit[v].
+// entry visit[v]; jj is in that order already.
 template <typename KeyT>
 __global__ void keys_k(const uint32_t *__restrict__ ii, const uint32_t *__restrict__ jj,
                        uint64_t nnz, bool slices, const uint32_t *__restrict__ hubflag,
@@ -387,18 +377,18 @@ __global__ void keys_k(const uint32_t *__restrict__ ii, const uint32_t *__restri
 {
     GRID_STRIDE(v, nnz)
     {
-        const uint64_t e = visit ? visit[v] : v;
-        const uint32_t r = ii[e];
+        const uint32_t r = ii[visit ? visit[v] : v];
         if (!slices) {
             key[v] = (KeyT)r;
         } else {
-            const uint32_t g = hubflag[r] ? hub_group(r, cls[jj[e]]) : 0u;
+            const uint32_t g = hubflag[r] ? hub_group(r, cls[jj[v]]) : 0u;
             key[v] = (KeyT)(((KeyT)r << 4) | (KeyT)g);
         }
     }
 }
 
-// col[p] = jj[perm[p]]; flags an order that is not the identity.
+// col[p] = jj[perm[p]]; flags an order that is not the identity (one atomic per workgroup, and
+// none once the flag is seen to be up).
 __global__ void gather_cols_k(const uint32_t *__restrict__ jj, const uint32_t *__restrict__ perm,
                               uint64_t nnz, uint32_t *col, Counters *C)
 {
@@ -409,7 +399,8 @@ __global__ void gather_cols_k(const uint32_t *__restrict__ jj, const uint32_t *_
         col[p] = jj[e];
         moved |= e != (uint32_t)p;
     }
-    if (__any(moved) && (threadIdx.x & 63) == 0)
+    if (__syncthreads_or(moved) && threadIdx.x == 0 &&
+        !__hip_atomic_load(&C->not_identity, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicOr(&C->not_identity, 1u);
 }
 
@@ -511,52 +502,41 @@ __global__ void gather_segs_k(const Seg *__restrict__ pseg, const uint32_t *__re
     GRID_STRIDE(i, n) out[i] = pseg[idx[i]];
 }
 
-// Sliced layout, step 1: which pieces are free (any queue), the work already
-// bound to each queue, and the work that is free.
-__global__ void any_flags_k(const Seg *__restrict__ pseg, const uint8_t *__restrict__ pqueue,
-                            uint64_t n, uint32_t *anyflag, Counters *C)
-{
-    unsigned long long w[kSlices + 1] = {0}; // [8] = free work
-    GRID_STRIDE(i, (uint64_t)n + 1)
-    {
-        if (i == n) {
-            anyflag[i] = 0;
-            continue;
-        }
-        const uint8_t q = pqueue[i];
-        const unsigned long long wi = (unsigned long long)pseg[i].len + kSegCost;
-        anyflag[i] = q == kAnyQueue;
-#pragma unroll
-        for (uint32_t k = 0; k <= kSlices; ++k)
-            w[k] += (k == kSlices ? q == kAnyQueue : q == k) ? wi : 0ull;
-    }
-#pragma unroll
-    for (uint32_t k = 0; k <= kSlices; ++k) {
-        const unsigned long long t = block_sum(w[k]);
-        if (threadIdx.x == 0 && t)
-            atomicAdd(k == kSlices ? &C->any_load : &C->load[k], t);
-    }
-}
-
-// Step 1b: the slice a free piece prefers (the one most of its sliced entries belong to;
-// kNoPref without any), and the free work that prefers each slice.
+// Sliced layout, step 1: the slice a free piece (any queue) prefers, which is the one most of its
+// sliced entries belong to; kNoPref without any.  A group of 16 lanes per piece, four columns of a
+// lane in flight: a thread per piece waited for two dependent loads per entry (R-MAT 20, 700 k
+// pieces: 709 us, so 113).
+constexpr uint32_t kPrefLanes = 16;
 __global__ void pref_k(const Seg *__restrict__ pseg, const uint8_t *__restrict__ pqueue, uint64_t n,
                        const uint32_t *__restrict__ col, const uint8_t *__restrict__ cls,
-                       uint8_t *pref, Counters *C)
+                       uint8_t *pref)
 {
-    unsigned long long w[kSlices] = {0};
-    GRID_STRIDE(i, n)
+    const uint32_t sub = threadIdx.x % kPrefLanes;
+    GRID_STRIDE(t, n * kPrefLanes) // a group's lanes go round together
     {
+        const uint64_t i = t / kPrefLanes;
         uint8_t p = kNoPref;
         if (pqueue[i] == kAnyQueue) {
             const Seg g = pseg[i];
             uint32_t cnt[kSlices] = {0};
-            for (uint32_t q = g.start; q < g.start + g.len; ++q) {
-                const uint8_t c = cls[col[q]];
+            for (uint32_t q = sub; q < g.len; q += 4 * kPrefLanes) {
+                uint32_t c[4];
 #pragma unroll
-                for (uint32_t k = 0; k < kSlices; ++k)
-                    cnt[k] += c == k;
+                for (uint32_t u = 0; u < 4; ++u)
+                    c[u] = col[g.start + (q + u * kPrefLanes < g.len ? q + u * kPrefLanes : q)];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    const uint32_t s = q + u * kPrefLanes < g.len ? cls[c[u]] : 255u;
+#pragma unroll
+                    for (uint32_t k = 0; k < kSlices; ++k)
+                        cnt[k] += s == k;
+                }
             }
+#pragma unroll
+            for (uint32_t k = 0; k < kSlices; ++k)
+#pragma unroll
+                for (int s = kPrefLanes / 2; s >= 1; s >>= 1)
+                    cnt[k] += __shfl_xor(cnt[k], s, kPrefLanes);
             // ties go to the first slice from a start that the row's hash picks
             const uint32_t first = rep_slice(g.row);
             uint32_t best = first, most = 0;
@@ -576,17 +556,39 @@ __global__ void pref_k(const Seg *__restrict__ pseg, const uint8_t *__restrict__
             }
             if (most)
                 p = (uint8_t)best;
-#pragma unroll
-            for (uint32_t k = 0; k < kSlices; ++k)
-                w[k] += (most && best == k) ? (unsigned long long)g.len + kSegCost : 0ull;
         }
-        pref[i] = p;
+        if (sub == 0)
+            pref[i] = p;
+    }
+}
+
+// Step 1b: which pieces are free, the work already bound to each queue, the free work, and the free
+// work that prefers each slice.
+__global__ void any_flags_k(const Seg *__restrict__ pseg, const uint8_t *__restrict__ pqueue,
+                            const uint8_t *__restrict__ pref, uint64_t n, uint32_t *anyflag, Counters *C)
+{
+    unsigned long long w[2 * kSlices + 1] = {0}; // [8] = free work
+    GRID_STRIDE(i, (uint64_t)n + 1)
+    {
+        if (i == n) {
+            anyflag[i] = 0;
+            continue;
+        }
+        const uint8_t q = pqueue[i], p = pref[i];
+        const unsigned long long wi = (unsigned long long)pseg[i].len + kSegCost;
+        anyflag[i] = q == kAnyQueue;
+#pragma unroll
+        for (uint32_t k = 0; k < kSlices; ++k) {
+            w[k] += q == k ? wi : 0ull;
+            w[kSlices + 1 + k] += q == kAnyQueue && p == k ? wi : 0ull;
+        }
+        w[kSlices] += q == kAnyQueue ? wi : 0ull;
     }
 #pragma unroll
-    for (uint32_t k = 0; k < kSlices; ++k) {
+    for (uint32_t k = 0; k < 2 * kSlices + 1; ++k) {
         const unsigned long long t = block_sum(w[k]);
         if (threadIdx.x == 0 && t)
-            atomicAdd(&C->pref_load[k], t);
+            atomicAdd(k < kSlices ? &C->load[k] : k == kSlices ? &C->any_load : &C->pref_load[k - kSlices - 1], t);
     }
 }
 
@@ -802,6 +804,9 @@ int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bi
 #define LAUNCH_SMALL(kernel, n, ...)                                                              \
     hipLaunchKernelGGL(kernel, dim3(small_grid_for(n)), dim3(kTB), 0, st, __VA_ARGS__)
 
+#define LAUNCH_FEW(kernel, n, ...)                                                                \
+    hipLaunchKernelGGL(kernel, dim3(few_grid_for(n)), dim3(kTB), 0, st, __VA_ARGS__)
+
 #define TRY(expr)                                                                                 \
     do {                                                                                          \
         const int rc_ = (expr);                                                                   \
@@ -809,41 +814,68 @@ int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bi
             return rc_;                                                                           \
     } while (0)
 
-int fetch(const DevStream &st, void *host, const void *dev, size_t bytes, std::string &err)
+struct Fetch { // bytes from dev to host
+    void *host;
+    const void *dev;
+    size_t bytes;
+};
+// Waits for what is queued on the stream and brings the given words down, through pinned memory
+// (into pageable memory each wait takes 15 us more, and a plan has seven or more).
+int fetch_all(const DevStream &st, std::initializer_list<Fetch> list, std::string &err)
 {
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
+    size_t need = 0;
+    for (const Fetch &f : list)
+        need += (f.bytes + 15) / 16 * 16;
+    void *words = need <= DevPool::kWords ? st.pool->get_words() : nullptr;
+    hipError_t e = hipSuccess;
+    char *at = static_cast<char *>(words);
+    for (const Fetch &f : list) {
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(words ? at : f.host, f.dev, f.bytes, hipMemcpyDeviceToHost, st);
+        at += words ? (f.bytes + 15) / 16 * 16 : 0;
+    }
+    const hipError_t done = hipStreamSynchronize(st); // also before the words are given back
+    e = e == hipSuccess ? done : e;
+    at = static_cast<char *>(words);
+    if (words && e == hipSuccess)
+        for (const Fetch &f : list) {
+            std::memcpy(f.host, at, f.bytes);
+            at += (f.bytes + 15) / 16 * 16;
+        }
+    st.pool->put_words(words);
+    HIP_OK(e);
     return SPC3D_OK;
+}
+int fetch(const DevStream &st, void *host, const void *dev, size_t bytes, std::string &err)
+{
+    return fetch_all(st, {{host, dev, bytes}}, err);
 }
 
 // Sorts the entries into kernel order: perm (kernel position -> caller's
-// position) and col.  KeyT is wide enough for (row << 4 | group).
-// by_column: the entries are first brought into ascending column order (stable), so that
-// every row ends up ordered by column (col_bits: bits of the largest column id).
+// position) and col.  KeyT is wide enough for (row << 4 | group).  hubcnt (sliced layout): see
+// hubcount_k.
+// visit (may be null): the entries in ascending column order (stable), so that every row ends
+// up ordered by column; col then holds the columns in that order.
 template <typename KeyT>
 int order_entries(Arena &arena, Temp &tmp, const DevStream &st, uint64_t nnz, int key_bits, bool slices,
-                  bool by_column, int col_bits, const uint32_t *d_ii, const uint32_t *d_jj,
-                  const uint32_t *hubflag, const uint8_t *cls, uint32_t *perm, uint32_t *col,
-                  Counters *C, std::string &err)
+                  const uint32_t *visit, const uint32_t *d_ii, const uint32_t *d_jj,
+                  const uint32_t *hubflag, const uint32_t *hubpos, uint32_t *hubcnt,
+                  const uint8_t *cls, uint32_t *perm, uint32_t *col, Counters *C, std::string &err)
 {
     SBuf<KeyT> key, key_out;
     SBuf<uint32_t> ident;
     HIP_OK(key.alloc(arena, nnz));
     HIP_OK(key_out.alloc(arena, nnz));
-    HIP_OK(ident.alloc(arena, nnz));
-    LAUNCH(iota_k, nnz, ident.p, nnz);
-    const uint32_t *visit = nullptr;
-    if (by_column) {
-        // col and perm are free until the end: sorted columns (unused) and the visiting order
-        TRY(sort_pairs<uint32_t>(tmp, d_jj, col, ident.p, perm, (uint32_t)nnz, col_bits, false, st,
-                                 err));
-        HIP_OK(hipMemcpyAsync(ident.p, perm, nnz * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
-        visit = ident.p;
+    if (!visit) {
+        HIP_OK(ident.alloc(arena, nnz));
+        LAUNCH(iota_k, nnz, ident.p, nnz);
     }
-    LAUNCH((keys_k<KeyT>), nnz, d_ii, d_jj, nnz, slices, hubflag, cls, visit, key.p);
-    TRY(sort_pairs<KeyT>(tmp, key.p, key_out.p, ident.p, perm, (uint32_t)nnz, key_bits, false, st,
-                         err));
+    LAUNCH((keys_k<KeyT>), nnz, d_ii, visit ? col : d_jj, nnz, slices, hubflag, cls, visit, key.p);
+    TRY(sort_pairs<KeyT>(tmp, key.p, key_out.p, visit ? visit : ident.p, perm, (uint32_t)nnz, key_bits,
+                         false, st, err));
+    if (slices)
+        LAUNCH((hubcount_k<KeyT>), nnz, key_out.p, nnz, hubflag, hubpos, hubcnt);
     LAUNCH(gather_cols_k, nnz, d_jj, perm, nnz, col, C);
     HIP_OK(hipGetLastError());
     return SPC3D_OK;
@@ -958,13 +990,19 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         err = buf;
         return SPC3D_ERR_BAD_INDEX;
     }
-    bool rows_unsorted = false;
+    const bool rows_unsorted = hC.rows_unsorted != 0;
+    const bool by_column = rows_unsorted && !opts.keep_entry_order;
+    const int col_bits = bits_for(ncols ? ncols - 1 : 0);
+    P.by_column_in_rows = by_column;
+    DBuf<uint32_t> perm, col;
+    SBuf<uint32_t> visit;
+    HIP_OK(perm.alloc(st, nnz));
+    HIP_OK(col.alloc(st, nnz));
     {
         SBuf<uint32_t> sorted, start;
         HIP_OK(sorted.alloc(arena, nnz));
         HIP_OK(start.alloc(arena, std::max<size_t>(ncols, nrows)));
-        rows_unsorted = hC.rows_unsorted != 0;
-        if (hC.rows_unsorted) {
+        if (rows_unsorted) {
             TRY(sort_keys(tmp, d_ii, sorted.p, (uint32_t)nnz, bits_for(nrows ? nrows - 1 : 0), st,
                           err));
             LAUNCH(run_bounds_k, nnz, sorted.p, nnz, nrows, start.p, rowcnt.p);
@@ -972,9 +1010,17 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         } else {
             LAUNCH(hist_sorted_k, nnz, d_ii, nnz, rowcnt.p);
         }
-        TRY(sort_keys(tmp, d_jj, sorted.p, (uint32_t)nnz, bits_for(ncols ? ncols - 1 : 0), st,
-                      err));
-        LAUNCH(run_bounds_k, nnz, sorted.p, nnz, ncols, start.p, coldeg.p);
+        const uint32_t *by_col = sorted.p;
+        if (by_column) { // the visiting order of order_entries; its sorted columns in `col`
+            HIP_OK(visit.alloc(arena, nnz));
+            LAUNCH(iota_k, nnz, sorted.p, nnz);
+            TRY(sort_pairs<uint32_t>(tmp, d_jj, col.p, sorted.p, visit.p, (uint32_t)nnz, col_bits,
+                                     false, st, err));
+            by_col = col.p;
+        } else {
+            TRY(sort_keys(tmp, d_jj, sorted.p, (uint32_t)nnz, col_bits, st, err));
+        }
+        LAUNCH(run_bounds_k, nnz, by_col, nnz, ncols, start.p, coldeg.p);
         LAUNCH(run_lengths_k, ncols, start.p, (uint64_t)ncols, coldeg.p);
     }
     LAUNCH_SMALL(stats_k, nrows, rowcnt.p, (uint64_t)nrows, &dC.p->rows_touched, &dC.p->max_row,
@@ -1038,26 +1084,19 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         P.hub_rows = nh;
         HIP_OK(hubcnt.alloc(arena, (size_t)nh * 9 + 1));
         HIP_OK(hipMemsetAsync(hubcnt.p, 0, ((size_t)nh * 9 + 1) * sizeof(uint32_t), st));
-        LAUNCH(hubcount_k, nnz, d_ii, d_jj, nnz, hubflag.p, hubpos.p, cls.p, hubcnt.p);
     }
 
     // ---- stable sort into kernel order ------------------------------------------------
-    DBuf<uint32_t> perm, col;
-    HIP_OK(perm.alloc(st, nnz));
-    HIP_OK(col.alloc(st, nnz));
     {
-        const int row_bits = bits_for(nrows ? nrows - 1 : 0);
-        const int key_bits = row_bits + (slices ? 4 : 0);
-        const bool by_column = rows_unsorted && !opts.keep_entry_order;
-        const int col_bits = bits_for(ncols ? ncols - 1 : 0);
-        P.by_column_in_rows = by_column;
+        const int key_bits = bits_for(nrows ? nrows - 1 : 0) + (slices ? 4 : 0);
         if (key_bits <= 32)
-            TRY(order_entries<uint32_t>(arena, tmp, st, nnz, key_bits, slices, by_column, col_bits,
-                                        d_ii, d_jj, hubflag.p, cls.p, perm.p, col.p, dC.p, err));
+            TRY(order_entries<uint32_t>(arena, tmp, st, nnz, key_bits, slices, visit.p, d_ii, d_jj,
+                                        hubflag.p, hubpos.p, hubcnt.p, cls.p, perm.p, col.p, dC.p,
+                                        err));
         else
-            TRY(order_entries<unsigned long long>(arena, tmp, st, nnz, key_bits, slices, by_column,
-                                                  col_bits, d_ii, d_jj, hubflag.p, cls.p, perm.p,
-                                                  col.p, dC.p, err));
+            TRY(order_entries<unsigned long long>(arena, tmp, st, nnz, key_bits, slices, visit.p,
+                                                  d_ii, d_jj, hubflag.p, hubpos.p, hubcnt.p, cls.p,
+                                                  perm.p, col.p, dC.p, err));
     }
 
     // ---- segments --------------------------------------------------------------------
@@ -1075,9 +1114,11 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     TRY(exclusive_sum(tmp, issplit.p, split_off.p, (size_t)nrows + 1, st, err));
     TRY(exclusive_sum(tmp, nslot.p, slot_off.p, (size_t)nrows + 1, st, err));
     uint32_t totals[3] = {0, 0, 0};
-    TRY(fetch(st, &totals[0], piece_off.p + nrows, sizeof(uint32_t), err));
-    TRY(fetch(st, &totals[1], split_off.p + nrows, sizeof(uint32_t), err));
-    TRY(fetch(st, &totals[2], slot_off.p + nrows, sizeof(uint32_t), err));
+    TRY(fetch_all(st,
+                  {{&totals[0], piece_off.p + nrows, sizeof(uint32_t)},
+                   {&totals[1], split_off.p + nrows, sizeof(uint32_t)},
+                   {&totals[2], slot_off.p + nrows, sizeof(uint32_t)}},
+                  err));
     const uint32_t np_total = totals[0], nsplit = totals[1];
     P.nslots = totals[2];
     P.nseg_real = np_total;
@@ -1119,14 +1160,13 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         HIP_OK(anyflag.alloc(arena, (size_t)np_total + 1));
         HIP_OK(anypos.alloc(arena, (size_t)np_total + 1));
         HIP_OK(pref.alloc(arena, np_total));
-        LAUNCH_SMALL(any_flags_k, (uint64_t)np_total + 1, pseg.p, pqueue.p, (uint64_t)np_total,
-               anyflag.p, dC.p);
-        LAUNCH_SMALL(pref_k, np_total, pseg.p, pqueue.p, (uint64_t)np_total, col.p, cls.p, pref.p,
-                     dC.p);
+        LAUNCH(pref_k, (uint64_t)np_total * kPrefLanes, pseg.p, pqueue.p, (uint64_t)np_total, col.p,
+               cls.p, pref.p);
+        LAUNCH_FEW(any_flags_k, (uint64_t)np_total + 1, pseg.p, pqueue.p, pref.p, (uint64_t)np_total,
+                   anyflag.p, dC.p);
         TRY(exclusive_sum(tmp, anyflag.p, anypos.p, (size_t)np_total + 1, st, err));
         uint32_t nany = 0;
-        TRY(fetch(st, &nany, anypos.p + np_total, sizeof nany, err));
-        TRY(fetch(st, &hC, dC.p, sizeof hC, err));
+        TRY(fetch_all(st, {{&nany, anypos.p + np_total, sizeof nany}, {&hC, dC.p, sizeof hC}}, err));
 
         SBuf<uint32_t> any_idx, any_key, any_key_out, any_sorted;
         HIP_OK(any_idx.alloc(arena, nany));
@@ -1152,7 +1192,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         HIP_OK(comb_key.alloc(arena, np_total));
         HIP_OK(comb_idx_out.alloc(arena, np_total));
         HIP_OK(comb_key_out.alloc(arena, np_total));
-        LAUNCH_SMALL(combine_k, (uint64_t)np_total + nany, pseg.p, pqueue.p, anyflag.p, anypos.p,
+        LAUNCH_FEW(combine_k, (uint64_t)np_total + nany, pseg.p, pqueue.p, anyflag.p, anypos.p,
                any_sorted.p, pref.p, (uint64_t)np_total, (uint64_t)nany, seg_max, deal, comb_idx.p,
                comb_key.p, dC.p);
         const int comb_bits = bits_for((uint64_t)kSlices * ((uint64_t)seg_max + 1) - 1);
@@ -1448,8 +1488,7 @@ int build_store_staging(const DevStream &st, const Seg *d_segs, uint32_t nseg, c
                        nseg, d_perm, flag.p);
     TRY(exclusive_sum<uint32_t>(tmp, flag.p, idx.p, (size_t)nnz, st, err));
     uint32_t last[2] = {0, 0};
-    TRY(fetch(st, &last[0], idx.p + (nnz - 1), 4, err));
-    TRY(fetch(st, &last[1], flag.p + (nnz - 1), 4, err));
+    TRY(fetch_all(st, {{&last[0], idx.p + (nnz - 1), 4}, {&last[1], flag.p + (nnz - 1), 4}}, err));
     const uint64_t n = (uint64_t)last[0] + last[1];
     if (n == 0) {
         out.consecutive = true;
