@@ -133,7 +133,8 @@ struct spc3d_plan {
     spc3d_ctx *ctx;
     int dtype;
     spc3d_plan_info info;
-    uint64_t row_sq = 0; // HostPlan::row_sq
+    uint64_t row_sq = 0;      // HostPlan::row_sq
+    bool cols_sorted = false; // HostPlan::cols_sorted
     bool has_values;
     // device arrays
     Seg *segs;

@@ -250,6 +250,7 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
         p->dtype = dtype;
         fill_info(p->info, meta);
         p->row_sq = meta.row_sq;
+        p->cols_sorted = meta.cols_sorted;
         p->info.nsegments_padded = arr.nseg_padded;
         p->info.nsplit_rows = arr.nsplit;
         rc = ctx_alloc_bytes(ctx, &p->sval, (size_t)meta.nnz * elem_size(dtype));
@@ -346,18 +347,13 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
                                const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
                                const StoreOpts &so)
 {
-    if (!so.by_column || nnz < 2 || !p->perm || p->store.consecutive || !p->blocks.empty())
+    if (!so.by_column || nnz < 2 || !p->perm || p->store.consecutive || !p->blocks.empty() ||
+        !p->cols_sorted)
         return SPC3D_OK;
     std::string err;
-    bool sorted = false;
-    int rc = is_nondecreasing_device(dev_stream(p->ctx), d_jj, nnz, &sorted, err);
-    if (rc)
-        return fail(rc, err);
-    if (!sorted)
-        return SPC3D_OK;
     HostPlan meta;
     DevPlanArrays arr;
-    rc = build_device_plan(dev_stream(p->ctx), ncols, nrows, nnz, d_jj, d_ii, po, meta, arr, err);
+    int rc = build_device_plan(dev_stream(p->ctx), ncols, nrows, nnz, d_jj, d_ii, po, meta, arr, err);
     if (rc)
         return optional_path(fail(rc, err));
     spc3d_plan *q = nullptr;

@@ -160,8 +160,4 @@ struct TwoPass {
 int build_two_pass(const DevStream &stream, const uint32_t *d_perm, uint64_t nnz, uint32_t tile,
                    TwoPass &out, std::string &err);
 
-// *out = d[0] <= d[1] <= ... <= d[n - 1] (device array); synchronous.
-int is_nondecreasing_device(const DevStream &stream, const uint32_t *d, uint64_t n, bool *out,
-                            std::string &err);
-
 } // namespace spc3d

@@ -60,6 +60,7 @@ struct HostPlan {
     uint32_t rows_touched = 0, cols_touched = 0;
     uint32_t max_row_nnz = 0;
     uint64_t row_sq = 0;           // sum over rows of length * min(length, 2048) (GPU builder)
+    bool cols_sorted = false;      // the caller's columns never step down (GPU builder)
     uint32_t seg_max = 0;
     uint32_t nslots = 0;
     uint32_t nseg_real = 0;        // segments with entries (segs.size() includes padding)
