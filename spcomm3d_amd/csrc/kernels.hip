@@ -47,6 +47,8 @@
 // was measured to slow both kernels down by 15 to 40 %.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace spc3d {
@@ -1490,6 +1492,11 @@ constexpr int kRowsAhead = 4;    // of a copy
 // Fewer workgroups than this (8 per CU) do not fill the chip: one row at a time then, which
 // makes more of them (50 k rows of 56 bytes: sum 6.8 against 4.8 us).
 constexpr uint64_t kRowsMinBlocks = 2048;
+// More than this are not launched, a workgroup goes on with a further share of the rows: a launch
+// of 2^32 threads and more is refused, and 1.1 G rows of one real would ask for it.  (At 65,536
+// workgroups rows that a fresh one would have taken wait for a second round: 2 M rows of 520 bytes,
+// 1.5 M slots, the three copies 1097 -> 1132 us.)
+constexpr uint64_t kRowsMaxBlocks = 1 << 20;
 constexpr uint32_t row_unit_bytes(RowUnit u, size_t elem) { return u == kElem ? (uint32_t)elem : 16u; }
 
 template <typename T, RowUnit UNIT> struct RowAccess {
@@ -1547,25 +1554,28 @@ rows_pack_kernel(const char *__restrict__ panel, const uint32_t *__restrict__ ro
     using A = RowAccess<T, UNIT>;
     constexpr uint32_t GPB = kBlock / LPR;
     const uint32_t sub = threadIdx.x % LPR;
-    const uint64_t first = (uint64_t)blockIdx.x * (GPB * U) + threadIdx.x / LPR;
-    uint32_t row[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const uint64_t i = first + u * GPB;
-        row[u] = rows[i < n ? i : n - 1];
-    }
-    for (uint32_t v = sub; v < units; v += LPR) {
-        const uint64_t off = unit_off<T, UNIT>(v, bytes);
-        typename A::V x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            x[u] = A::load(panel + (uint64_t)row[u] * bytes + off);
-        __builtin_amdgcn_sched_barrier(0); // every row asked for before the first store
+    for (uint64_t share = (uint64_t)blockIdx.x * (GPB * U); share < n;
+         share += (uint64_t)gridDim.x * (GPB * U)) {
+        const uint64_t first = share + threadIdx.x / LPR;
+        uint32_t row[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint64_t i = first + u * GPB;
-            if (i < n)
-                A::store_nt(x[u], buf + i * bytes + off);
+            row[u] = rows[i < n ? i : n - 1];
+        }
+        for (uint32_t v = sub; v < units; v += LPR) {
+            const uint64_t off = unit_off<T, UNIT>(v, bytes);
+            typename A::V x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                x[u] = A::load(panel + (uint64_t)row[u] * bytes + off);
+            __builtin_amdgcn_sched_barrier(0); // every row asked for before the first store
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint64_t i = first + u * GPB;
+                if (i < n)
+                    A::store_nt(x[u], buf + i * bytes + off);
+            }
         }
     }
 }
@@ -1585,68 +1595,71 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
     constexpr uint32_t GPB = kBlock / LPR;
     static_assert(!ADD || U == 1, "sums go row by row");
     const uint32_t sub = threadIdx.x % LPR;
-    const uint64_t first = (uint64_t)blockIdx.x * (GPB * U) + threadIdx.x / LPR;
-    u32x4 d[U]; // row, first slot, last slot, start in slots
-    uint32_t left = 0; // slots of the row after its first
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const uint64_t i = first + u * GPB;
-        const uint64_t at = i < n ? i : n - 1;
-        d[u] = nt_load(dests + at);
-        if constexpr (ADD) {
-            left = dests[at + 1][3] - d[u][3] - 1;
-        }
-    }
-    for (uint32_t v = sub; v < units; v += LPR) {
-        const uint64_t off = unit_off<T, UNIT>(v, bytes);
-        typename A::V x[U], y[U];
+    for (uint64_t share = (uint64_t)blockIdx.x * (GPB * U); share < n;
+         share += (uint64_t)gridDim.x * (GPB * U)) {
+        const uint64_t first = share + threadIdx.x / LPR;
+        u32x4 d[U]; // row, first slot, last slot, start in slots
+        uint32_t left = 0; // slots of the row after its first
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            x[u] = A::load_nt(buf + (uint64_t)d[u][ADD ? 1 : 2] * bytes + off);
-            if constexpr (ADD)
-                y[u] = A::load(panel + (uint64_t)d[u][0] * bytes + off);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ADD) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                y[u] += x[u];
-            for (uint32_t t = 1; t <= left; t += D) {
-                typename A::V z[D];
-                uint32_t slot[D];
-#pragma unroll
-                for (int j = 0; j < D; ++j)
-                    slot[j] = slots[d[0][3] + (t + j < left ? t + j : left)];
-#pragma unroll
-                for (int j = 0; j < D; ++j)
-                    z[j] = A::load_nt(buf + (uint64_t)slot[j] * bytes + off);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int j = 0; j < D; ++j)
-                    if (t + j <= left)
-                        y[0] += z[j];
+            const uint64_t i = first + u * GPB;
+            const uint64_t at = i < n ? i : n - 1;
+            d[u] = nt_load(dests + at);
+            if constexpr (ADD) {
+                left = dests[at + 1][3] - d[u][3] - 1;
             }
         }
+        for (uint32_t v = sub; v < units; v += LPR) {
+            const uint64_t off = unit_off<T, UNIT>(v, bytes);
+            typename A::V x[U], y[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (first + u * GPB >= n)
-                continue;
-            char *to = panel + (uint64_t)d[u][0] * bytes + off;
-            if constexpr (!ADD) {
-                A::store(x[u], to);
-            } else {
-                if constexpr (UNIT == kLoose) {
-                    const uint32_t skip = (uint32_t)((uint64_t)v * 16 - off) / (uint32_t)sizeof(T);
-                    if (skip) { // the row's last unit: its leading elements are the unit's before
-                        T *e = reinterpret_cast<T *>(to);
+            for (int u = 0; u < U; ++u) {
+                x[u] = A::load_nt(buf + (uint64_t)d[u][ADD ? 1 : 2] * bytes + off);
+                if constexpr (ADD)
+                    y[u] = A::load(panel + (uint64_t)d[u][0] * bytes + off);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ADD) {
 #pragma unroll
-                        for (uint32_t j = 0; j < (uint32_t)Vec<T>::N; ++j)
-                            if (j >= skip)
-                                e[j] = y[u][j];
-                        continue;
-                    }
+                for (int u = 0; u < U; ++u)
+                    y[u] += x[u];
+                for (uint32_t t = 1; t <= left; t += D) {
+                    typename A::V z[D];
+                    uint32_t slot[D];
+#pragma unroll
+                    for (int j = 0; j < D; ++j)
+                        slot[j] = slots[d[0][3] + (t + j < left ? t + j : left)];
+#pragma unroll
+                    for (int j = 0; j < D; ++j)
+                        z[j] = A::load_nt(buf + (uint64_t)slot[j] * bytes + off);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < D; ++j)
+                        if (t + j <= left)
+                            y[0] += z[j];
                 }
-                A::store(y[u], to);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (first + u * GPB >= n)
+                    continue;
+                char *to = panel + (uint64_t)d[u][0] * bytes + off;
+                if constexpr (!ADD) {
+                    A::store(x[u], to);
+                } else {
+                    if constexpr (UNIT == kLoose) {
+                        const uint32_t skip = (uint32_t)((uint64_t)v * 16 - off) / (uint32_t)sizeof(T);
+                        if (skip) { // the row's last unit: its leading elements are the unit's before
+                            T *e = reinterpret_cast<T *>(to);
+#pragma unroll
+                            for (uint32_t j = 0; j < (uint32_t)Vec<T>::N; ++j)
+                                if (j >= skip)
+                                    e[j] = y[u][j];
+                            continue;
+                        }
+                    }
+                    A::store(y[u], to);
+                }
             }
         }
     }
@@ -2490,12 +2503,16 @@ hipError_t launch_gather_vals(int dtype, const void *in, const uint32_t *perm, v
 }
 
 namespace {
+inline dim3 rows_grid(uint32_t n, uint32_t per)
+{
+    return dim3((uint32_t)std::min(((uint64_t)n + per - 1) / per, kRowsMaxBlocks));
+}
+
 template <typename T, RowUnit UNIT, int LPR, int U>
 void rows_launch_ahead(int op, char *panel, const RowMapView &M, uint32_t n, uint32_t units,
                        uint64_t bytes, char *buf, hipStream_t st)
 {
-    const uint32_t per = kBlock / LPR * U;
-    const dim3 grid((uint32_t)(((uint64_t)n + per - 1) / per)), block(kBlock);
+    const dim3 grid = rows_grid(n, kBlock / LPR * U), block(kBlock);
     if (op == 0)
         hipLaunchKernelGGL((rows_pack_kernel<T, UNIT, LPR, U>), grid, block, 0, st, panel, M.rows, n,
                            units, bytes, buf);
@@ -2508,9 +2525,8 @@ template <typename T, RowUnit UNIT, int LPR, int D>
 void rows_launch_sum(char *panel, const RowMapView &M, uint32_t units, uint64_t bytes, char *buf,
                      hipStream_t st)
 {
-    constexpr uint32_t per = kBlock / LPR;
     hipLaunchKernelGGL((rows_unpack_kernel<T, UNIT, LPR, 1, true, D>),
-                       dim3((M.nuniq + per - 1) / per), dim3(kBlock), 0, st, panel,
+                       rows_grid(M.nuniq, kBlock / LPR), dim3(kBlock), 0, st, panel,
                        (const u32x4 *)M.dests, M.slots, M.nuniq, units, bytes, buf);
 }
 

@@ -218,3 +218,30 @@ def test_rows_kernels_at_row_ends_and_partial_blocks(ctx, dtype, k, slots):
     dP.upload(P)
     rm.unpack_sum(dP, dB)
     assert np.array_equal(dP.download(), oracle_rows(2, P, rows, buf)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,k,m", [(np.float32, 1, (1 << 26) + 77), (np.float64, 65, (1 << 22) + 5)])
+def test_more_rows_than_one_round_of_workgroups(ctx, dtype, k, m):
+    # sums take 64 and 4 rows per workgroup here and 2^20 workgroups at most, so some go on with a
+    # second, ragged share.  Every row is named once.
+    from spcomm3d_amd import device
+
+    rows = np.arange(m, dtype=np.uint32)[::-1].copy()
+    rm = device.RowMap(ctx, m, rows)
+    dP, dB = ctx.panel(m, k, dtype), ctx.vals(m * k, dtype)
+    if k == 1:
+        P, buf = (np.random.default_rng(s).integers(-8, 9, m, dtype=np.int8).astype(dtype) for s in (1, 2))
+        dP.upload(P.reshape(m, 1))
+        dB.upload(buf)
+        rm.unpack_sum(dP, dB)
+        assert np.array_equal(dP.download().reshape(-1), P + buf[::-1])
+        rm.pack(dP, dB)
+        assert np.array_equal(dB.download(), P[::-1] + buf)
+    else:
+        dP.fill(1.0)
+        dB.fill(2.0)
+        rm.unpack_sum(dP, dB)
+        assert np.all(dP.download() == 3.0)
+    for h in (dP, dB, rm):
+        h.close()
