@@ -4,34 +4,50 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <new>
-#include <system_error>
 #include <thread>
 
 namespace spc3d {
 
-hipError_t HostStage::lane(unsigned i, Lane **out)
+HostStage::Lane *HostStage::lane(unsigned i, size_t piece)
 {
-    *out = nullptr;
+    piece = piece > kMinPiece ? kMaxPiece : kMinPiece;
     try {
+        lanes_.reserve(kMaxLanes);
         while (lanes_.size() <= i) {
             std::unique_ptr<Lane> l(new Lane());
-            hipError_t e = hipHostMalloc((void **)&l->buf, kMaxPiece * kBufs, hipHostMallocDefault);
+            hipError_t e = hipSuccess;
             for (unsigned b = 0; b < kBufs && e == hipSuccess; ++b)
                 e = hipEventCreateWithFlags(&l->ev[b], hipEventDisableTiming);
             if (e != hipSuccess) {
+                (void)hipGetLastError();
                 for (hipEvent_t ev : l->ev)
                     if (ev) (void)hipEventDestroy(ev);
-                if (l->buf) (void)hipHostFree(l->buf);
-                return e;
+                return nullptr;
             }
             lanes_.push_back(std::move(l));
         }
     } catch (const std::bad_alloc &) {
-        return hipErrorOutOfMemory;
+        return nullptr;
     }
-    *out = lanes_[i].get();
-    return hipSuccess;
+    Lane &l = *lanes_[i];
+    for (; l.piece < piece; piece = kMinPiece) {
+        char *buf = nullptr;
+        if (hipHostMalloc((void **)&buf, piece * kBufs, hipHostMallocDefault) == hipSuccess) {
+            for (unsigned b = 0; b < kBufs; ++b)
+                (void)wait(l, b);
+            if (l.buf)
+                (void)hipHostFree(l.buf);
+            l.buf = buf;
+            l.piece = piece;
+            break;
+        }
+        (void)hipGetLastError();
+        if (piece == kMinPiece)
+            break;
+    }
+    return l.buf ? &l : nullptr;
 }
 
 void HostStage::release()
@@ -42,7 +58,8 @@ void HostStage::release()
             (void)wait(*l, b);
             (void)hipEventDestroy(l->ev[b]);
         }
-        (void)hipHostFree(l->buf);
+        if (l->buf)
+            (void)hipHostFree(l->buf);
     }
     lanes_.clear();
 }
@@ -71,27 +88,25 @@ hipError_t HostStage::upload(int device, void *dev, const void *host, size_t byt
     hipError_t e = hipSetDevice(device);
     if (e != hipSuccess)
         return e;
-    if (bytes > kMaxUpload || !unpinned(host)) {
-        e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
-        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    if (bytes <= kMaxUpload && unpinned(host)) {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (Lane *l = lane(0, kMinPiece)) {
+            const unsigned b = l->next++ % kBufs;
+            e = wait(*l, b);
+            if (e != hipSuccess)
+                return e;
+            char *buf = l->buf + b * l->piece;
+            std::memcpy(buf, host, bytes);
+            e = hipMemcpyAsync(dev, buf, bytes, hipMemcpyHostToDevice, st);
+            if (e == hipSuccess) {
+                l->busy[b] = true;
+                e = hipEventRecord(l->ev[b], st);
+            }
+            return e;
+        }
     }
-    std::lock_guard<std::mutex> lock(mu_);
-    Lane *l = nullptr;
-    e = lane(0, &l);
-    if (e != hipSuccess)
-        return e;
-    const unsigned b = l->next++ % kBufs;
-    e = wait(*l, b);
-    if (e != hipSuccess)
-        return e;
-    char *buf = l->buf + b * kMaxPiece;
-    std::memcpy(buf, host, bytes);
-    e = hipMemcpyAsync(dev, buf, bytes, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) {
-        l->busy[b] = true;
-        e = hipEventRecord(l->ev[b], st);
-    }
-    return e;
+    e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
 }
 
 struct HostStage::Fetch {
@@ -136,7 +151,7 @@ hipError_t HostStage::fetch(Lane &l, Fetch &f)
             p.last = at == end;
             e = wait(l, b);
             if (e == hipSuccess)
-                e = hipMemcpyAsync(f.direct ? f.host + p.off : l.buf + b * kMaxPiece, f.dev + p.off, p.len,
+                e = hipMemcpyAsync(f.direct ? f.host + p.off : l.buf + b * l.piece, f.dev + p.off, p.len,
                                    hipMemcpyDeviceToHost, f.st);
             if (e == hipSuccess) {
                 l.busy[b] = true;
@@ -152,7 +167,7 @@ hipError_t HostStage::fetch(Lane &l, Fetch &f)
         if (e != hipSuccess)
             return e;
         char *to = f.host + p.off;
-        const char *from = l.buf + b * kMaxPiece;
+        const char *from = l.buf + b * l.piece;
         if (f.keys) {
             const size_t whole = p.len / kKeyChunk * kKeyChunk;
             if (f.direct) {
@@ -170,6 +185,20 @@ hipError_t HostStage::fetch(Lane &l, Fetch &f)
         }
         ++taken;
     }
+}
+
+// A whole download by the runtime's own copy, keyed where it arrived.
+hipError_t HostStage::fetch_unstaged(Fetch &f)
+{
+    hipError_t e = hipSetDevice(f.device);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(f.host, f.dev, f.bytes, hipMemcpyDeviceToHost, f.st);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(f.st);
+    for (size_t b = 0; e == hipSuccess && f.keys && b < f.nblocks; ++b)
+        f.keys[b] = key_of_block(f.host + b * kKeyBlockBytes,
+                                 std::min(kKeyBlockBytes, f.bytes - b * kKeyBlockBytes));
+    return e;
 }
 
 hipError_t HostStage::download(int device, void *host, const void *dev, size_t bytes, hipStream_t st,
@@ -191,20 +220,20 @@ hipError_t HostStage::download(int device, void *host, const void *dev, size_t b
     f.keys = keys;
     f.direct = !unpinned(host);
     threads = (unsigned)std::min<size_t>(std::min(std::max(1u, threads), kMaxLanes), f.nblocks);
-    std::vector<Lane *> lanes(threads);
-    for (unsigned t = 0; t < threads; ++t) {
-        const hipError_t e = lane(t, &lanes[t]);
-        if (e != hipSuccess && t == 0)
-            return e;
-        if (e != hipSuccess) { // fewer threads then
-            (void)hipGetLastError();
-            lanes.resize(t);
+    Lane *lanes[kMaxLanes] = {};
+    unsigned n = 0;
+    for (; n < threads; ++n) { // fewer threads when there is no memory for more
+        lanes[n] = lane(n, f.piece);
+        if (!lanes[n])
             break;
-        }
+        f.piece = std::min(f.piece, lanes[n]->piece);
     }
-    std::vector<hipError_t> rc(lanes.size(), hipSuccess);
+    if (n == 0)
+        return fetch_unstaged(f);
+    hipError_t rc[kMaxLanes];
+    std::fill(rc, rc + kMaxLanes, hipSuccess);
     struct Pool {
-        std::vector<std::thread> threads;
+        std::thread threads[kMaxLanes];
         ~Pool()
         {
             for (std::thread &t : threads)
@@ -215,10 +244,9 @@ hipError_t HostStage::download(int device, void *host, const void *dev, size_t b
     {
         Pool pool;
         try {
-            pool.threads.reserve(lanes.size());
-            for (size_t t = 1; t < lanes.size(); ++t)
-                pool.threads.emplace_back([&, t] { rc[t] = fetch(*lanes[t], f); });
-        } catch (const std::system_error &) {
+            for (unsigned t = 1; t < n; ++t)
+                pool.threads[t] = std::thread([&, t] { rc[t] = fetch(*lanes[t], f); });
+        } catch (const std::exception &) {
             // no more threads to be had: those that started and this one share the blocks
         }
         rc[0] = fetch(*lanes[0], f);

@@ -8,8 +8,9 @@
 // An upload has nothing to overlap with but the copy itself: above 512 KiB the runtime, which
 // pins the caller's pages, is as fast, and only smaller ones take a buffer (0.25 MiB: 25 us).
 //
-// The pinned memory (12 MiB per host thread that takes part) is allocated by the first transfer
-// and freed with the context or its host-call cache.
+// The pinned memory is allocated by the first transfer that uses it (1.5 MiB for small ones, 12 MiB
+// per host thread that takes part in a large one) and freed with the context or its host-call cache.
+// Without it (the host's pinned memory is used up) transfers go the runtime's own way, slower.
 #pragma once
 #include <hip/hip_runtime_api.h>
 
@@ -47,14 +48,18 @@ class HostStage {
     static constexpr size_t kMaxUpload = (size_t)1 << 19; // through a buffer
     struct Lane { // the buffers of one thread
         char *buf = nullptr;
+        size_t piece = 0; // bytes of one of them: kMinPiece or kMaxPiece
         hipEvent_t ev[kBufs] = {};
         bool busy[kBufs] = {}; // a copy out of (into) the buffer may be under way
         unsigned next = 0;
     };
-    hipError_t lane(unsigned i, Lane **out);
+    // Thread i's buffers, for pieces of `piece` bytes (or less, when there is only memory for
+    // kMinPiece).  Null: there is none.
+    Lane *lane(unsigned i, size_t piece);
     static hipError_t wait(Lane &l, unsigned b);
     struct Fetch;
     static hipError_t fetch(Lane &l, Fetch &f);
+    static hipError_t fetch_unstaged(Fetch &f);
     std::mutex mu_;
     std::vector<std::unique_ptr<Lane>> lanes_;
 };

@@ -1,0 +1,127 @@
+// Host-only test of the copies between host memory and the device (spcomm3d_amd/csrc/host_stage.cpp)
+// where pinned memory runs out: over a stand-in for the few HIP calls they make, in which
+// "device" memory is host memory and the pinned memory that can be had is set by the test.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <random>
+#include <vector>
+
+#include "../../spcomm3d_amd/csrc/host_stage.h"
+
+using namespace spc3d;
+
+static int g_fail = 0;
+#define CHECK(cond)                                                                               \
+    do {                                                                                          \
+        if (!(cond)) {                                                                            \
+            std::printf("FAIL %s:%d: %s\n", __FILE__, __LINE__, #cond);                           \
+            ++g_fail;                                                                             \
+        }                                                                                         \
+    } while (0)
+
+// ---- the stand-in ------------------------------------------------------------------------
+static std::mutex g_mu;
+static size_t g_pinned_room;            // bytes of pinned memory that can still be had
+static std::map<void *, size_t> g_pinned;
+static size_t pinned_now()
+{
+    size_t n = 0;
+    for (auto &p : g_pinned)
+        n += p.second;
+    return n;
+}
+
+extern "C" {
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    std::lock_guard<std::mutex> lock(g_mu);
+    *p = nullptr;
+    if (n > g_pinned_room)
+        return hipErrorOutOfMemory;
+    *p = std::malloc(n);
+    g_pinned[*p] = n;
+    g_pinned_room -= n;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    std::lock_guard<std::mutex> lock(g_mu);
+    CHECK(g_pinned.count(p) == 1);
+    g_pinned_room += g_pinned[p];
+    g_pinned.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::memcpy(to, from, n);
+    return hipSuccess;
+}
+}
+
+// ---- copies with none, some and all of the pinned memory they would use -------------------
+static void copies(size_t room, unsigned threads)
+{
+    g_pinned_room = room;
+    std::mt19937_64 g(7);
+    HostStage stage;
+    for (size_t bytes : {(size_t)4, (size_t)4096, (size_t)1 << 19, ((size_t)1 << 19) + 4, (size_t)9 << 20,
+                         ((size_t)21 << 20) + 12}) {
+        std::vector<char> src(bytes), dev(bytes, 1), back(bytes, 2);
+        for (auto &c : src)
+            c = (char)g();
+        CHECK(stage.upload(0, dev.data(), src.data(), bytes, nullptr) == hipSuccess);
+        CHECK(dev == src);
+        CHECK(stage.download(0, back.data(), dev.data(), bytes, nullptr, nullptr, threads) == hipSuccess);
+        CHECK(back == src);
+        std::vector<BlockKey> want, keys((bytes + kKeyBlockBytes - 1) / kKeyBlockBytes);
+        keys_of(src.data(), bytes, want, 1);
+        std::fill(back.begin(), back.end(), 3);
+        CHECK(stage.download(0, back.data(), dev.data(), bytes, nullptr, keys.data(), threads) == hipSuccess);
+        CHECK(back == src);
+        CHECK(keys == want);
+        CHECK(pinned_now() <= room);
+    }
+    stage.release();
+    CHECK(g_pinned.empty());
+}
+
+// A small transfer holds little pinned memory.
+static void small_transfers_pin_little()
+{
+    g_pinned_room = (size_t)1 << 30;
+    HostStage stage;
+    char host[64] = {}, dev[64] = {};
+    CHECK(stage.download(0, host, dev, sizeof host, nullptr, nullptr, 8) == hipSuccess);
+    CHECK(stage.upload(0, dev, host, sizeof host, nullptr) == hipSuccess);
+    CHECK(pinned_now() > 0 && pinned_now() <= (size_t)2 << 20);
+}
+
+int main()
+{
+    for (unsigned threads : {1u, 3u})
+        for (size_t room : {(size_t)0, (size_t)1 << 20, (size_t)2 << 20, (size_t)13 << 20, (size_t)30 << 20,
+                            (size_t)1 << 30})
+            copies(room, threads);
+    small_transfers_pin_little();
+    CHECK(g_pinned.empty());
+    std::printf(g_fail ? "FAILED (%d)\n" : "PASSED\n", g_fail);
+    return g_fail != 0;
+}

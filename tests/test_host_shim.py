@@ -132,6 +132,11 @@ def test_content_keys_of_the_one_shot_host_calls():
     _run("test_keys")
 
 
+def test_copies_between_host_and_device_without_pinned_memory():
+    # the library's transfers where pinned memory cannot be had, or only some of it
+    _run("test_host_memory")
+
+
 @pytest.mark.gpu
 def test_shim_without_the_cache_of_the_one_shot_calls():
     # SPC3D_HOST_CACHE=0: plan, upload, run, download, free on every call; same results
