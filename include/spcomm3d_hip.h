@@ -112,15 +112,19 @@ typedef struct {
                                   bytes per entry in fp64, 16 in fp32) */
     uint32_t entries_by_column; /* 1: the rows arrived unsorted, and the plan orders the entries
                                   of every row by column (spc3d_spmm then adds a row's entries
-                                  in that order); 0: the caller's order inside every row */
+                                  in that order); 0: the caller's order inside every row.  Column
+                                  blocks and row tiles (below) add block after block, each in
+                                  this order */
     uint64_t device_bytes;     /* device memory the plan holds: its arrays, values, partial-sum
                                   rows, result staging, a companion plan, every column block */
     uint64_t sweep_entries;    /* entries kept as row tiles x column blocks (spc3d_plan_opts.sweep);
                                   0: none.  The segment counts above are then those of the plan
                                   of the other entries */
-    uint32_t sweep_tiles;      /* tiles of rows of that layout */
-    uint32_t sweep_k;          /* the K it is laid out for (k_hint); calls at another K run an
-                                  ordinary plan of the same pattern, made on first use */
+    uint32_t sweep_tiles;      /* tiles of rows of that layout; with sweep_entries == 0: of the
+                                  tiles that a plan of ordinary arrays holds besides */
+    uint32_t sweep_k;          /* the K it is laid out for (k_hint); calls at another K run the
+                                  plan's ordinary arrays, or an ordinary plan of the same
+                                  pattern, made on first use */
 } spc3d_plan_info;
 
 /* Plan tuning; a zero field selects the default.  Only speed depends on these. */
@@ -174,10 +178,11 @@ typedef struct {
                               there (a row's entries together), else through a staging vector
                               (spc3d_plan_info.staged_entries).
                               A plan that stays ordinary holds such tiles besides (in
-                              device_bytes, not in sweep_entries) where its columns are not
-                              skewed and calls at K = k_hint run faster over them: spc3d_sddmm,
-                              spc3d_spmm where rows are long enough; every other call and K
-                              runs the ordinary arrays.
+                              device_bytes and sweep_tiles, not in sweep_entries) where its
+                              columns are not skewed and calls at K = k_hint run faster over
+                              them: spc3d_sddmm, spc3d_spmm where rows are long enough; every
+                              other call and K runs the ordinary arrays.  Not with
+                              SPC3D_PLAN_KEEP_ENTRY_ORDER: they add block after block.
                               0 (default): as described; 1: never; 2: whenever k_hint has such
                               a width, whatever the pattern (col_blocks, if given, is the
                               number of blocks) */

@@ -569,13 +569,15 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
 // columns, 512-byte 1912 -> 1384.
 // The plan itself stays: it runs every other K, the one-pass calls (which read the dense rows
 // once, as fast as either of the tiles' kernels) and what the tiles leave out.
+// The tiles add a row's entries block after block, so a caller that asked for the order of its own
+// gets none.
 static int add_tiles(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                      const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
                      const spc3d_plan_opts *opts)
 {
     const spc3d_plan_info &I = p->info;
     if (!opts || opts->sweep || opts->col_blocks || !opts->k_hint || opts->builder == 1 ||
-        I.nqueues != 1 || nnz == 0)
+        po.keep_entry_order || I.nqueues != 1 || nnz == 0)
         return SPC3D_OK;
     const uint32_t lanes = sweep_lanes_any(p->dtype, opts->k_hint);
     if (!lanes)
@@ -615,6 +617,8 @@ static int add_tiles(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz
     p->tiles = q;
     p->tiles_sddmm = sddmm;
     p->tiles_spmm = spmm;
+    p->info.sweep_tiles = q->info.sweep_tiles;
+    p->info.sweep_k = q->info.sweep_k;
     return SPC3D_OK;
 }
 

@@ -81,3 +81,23 @@ def test_calls_over_the_tiles(ctx, dtype, k, lengths, n, tiled, shuffled):
     check_sddmm(a, b, ii, jj, vv, dC.download())
     S.close()
     plain.close()
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_the_callers_order_is_kept_where_it_is_asked_for(ctx, shuffled):
+    # SPC3D_PLAN_KEEP_ENTRY_ORDER: no tiles, which add block after block; and tiles show in the info
+    k, n, m = 128, 11000, len(ROWS_80)
+    ii, jj = pattern(ROWS_80, n, shuffled)
+    rng = np.random.default_rng(1)
+    vv = rng.uniform(0, 1, ii.size)
+    B, Y0 = rng.uniform(-1, 1, (n, k)), rng.uniform(-1, 1, (m, k))
+    dB, got = ctx.panel_from(B), []
+    for opts in ({"keep_entry_order": True}, {"keep_entry_order": True, "sweep": False}, {}):
+        S, dY = ctx.plan(m, n, ii, jj, vv, k_hint=k, **opts), ctx.panel_from(Y0)
+        ctx.spmm(S, dB, dY)
+        got.append((S.info, dY.download()))
+        S.close()
+    (kept, Y), (plain, Y_plain), (tiled, _) = got
+    assert np.array_equal(Y, Y_plain) and kept.device_bytes == plain.device_bytes
+    assert kept.sweep_tiles == kept.sweep_k == 0
+    assert tiled.sweep_tiles > 0 and tiled.sweep_k == k and tiled.sweep_entries == 0
