@@ -101,3 +101,52 @@ def test_the_callers_order_is_kept_where_it_is_asked_for(ctx, shuffled):
     assert np.array_equal(Y, Y_plain) and kept.device_bytes == plain.device_bytes
     assert kept.sweep_tiles == kept.sweep_k == 0
     assert tiled.sweep_tiles > 0 and tiled.sweep_k == k and tiled.sweep_entries == 0
+
+
+# widths that leave lanes of the tiles idle or end inside a 16-byte unit, at the edges of each lane
+# count (16 lanes to 256 bytes, 32 to 512, 64 to 1024), and widths that fill them
+@pytest.mark.parametrize("dtype,k", [(np.float32, k) for k in (33, 36, 50, 63, 64, 65, 67, 96, 127, 128, 129,
+                                                               131, 175, 252, 255)] +
+                                    [(np.float64, k) for k in (17, 31, 33, 50, 63, 65, 100, 127)])
+@pytest.mark.parametrize("by_column", [False, True])  # results staged, or straight to their places
+def test_tiles_of_any_width(ctx, dtype, k, by_column):
+    row_bytes = k * np.dtype(dtype).itemsize
+    n = 11 * (13 << 18) // (3 * row_bytes)              # 4 blocks of 3.25 MiB
+    nnz = max(13 * n, (545 << 20) // row_bytes)
+    lengths = [80] * (nnz // 80) + [7] * 500 + [0] * 9 + [211] * 40
+    lengths = np.random.default_rng(5).permutation(lengths)
+    m = len(lengths)
+    ii, jj = pattern(lengths, n, False)
+    if by_column:
+        o = np.lexsort((jj, ii))
+        ii, jj = ii[o], jj[o]
+    rng = np.random.default_rng(k)
+    vv = rng.uniform(0, 1, ii.size).astype(dtype)
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (m, n, m))
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k)
+    assert S.info.sweep_tiles > 0 and S.info.sweep_entries == 0
+    dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(ii.size, dtype)
+    dC.fill(-5.0)
+    ctx.sddmm(S, dA, dB, dC)
+    ctx.spmm(S, dB, dY)
+    C, Y = dC.download(), dY.download()
+    check_sddmm(A, B, ii, jj, vv, C)
+    check_spmm(B, ii, jj, vv, Y0, Y)
+    dY.upload(Y0)
+    ctx.spmm(S, dB, dY)
+    assert np.array_equal(dY.download(), Y)
+    # an infinity in the part of a row that two lanes load and one counts goes where it belongs only
+    at, c = k - 2, int(jj[0])
+    B[c, at] = np.inf
+    dB.upload(B)
+    dY.upload(Y0)
+    ctx.sddmm(S, dA, dB, dC)
+    ctx.spmm(S, dB, dY)
+    C, Y = dC.download(), dY.download()
+    assert not np.isnan(C).any() and np.array_equal(np.isinf(C), (jj == c) & (vv != 0))
+    assert not np.isnan(Y).any()
+    want = np.zeros((m, k), dtype=bool)
+    want[ii[(jj == c) & (vv != 0)], at] = True
+    assert np.array_equal(np.isinf(Y), want)
+    for h in (S, dA, dB, dY, dC):
+        h.close()
