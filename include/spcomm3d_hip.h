@@ -431,7 +431,9 @@ SPC3D_API int spc3d_spmm(spc3d_ctx *ctx, spc3d_plan *A, const spc3d_panel *X, sp
  * library is used on holds it until the process ends) instead of to memory owned by
  * the plan, and the call performs no allocation and frees nothing.  A plan whose
  * partial sums need more (npartial_slots * K * sizeof(real) bytes) is refused with
- * SPC3D_ERR_TOO_LARGE and nothing is queued.  All calls on one GPU share the array:
+ * SPC3D_ERR_TOO_LARGE and nothing is queued, unless its segments are shorter than nnz / 2048
+ * for its k_hint (spc3d_plan_opts.seg_max): it then runs as many columns at a time as the
+ * array holds.  All calls on one GPU share the array:
  * two such calls must not overlap in time (calls on one context never do; contexts
  * on the same GPU must not run it concurrently).  Asynchronous on the context's
  * stream; may be recorded between spc3d_capture_begin and spc3d_capture_end. */

@@ -876,8 +876,17 @@ int spc3d_spmm_noalloc(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc
         return rc;
     if (Ap->tiles_spmm && K == Ap->tiles->sweep_k)
         Ap = Ap->tiles;
-    const uint64_t need = (uint64_t)Ap->info.npartial_slots * K * elem_size(Ap->dtype);
-    if (need > kStaticScratchBytes) {
+    const size_t nparts = Ap->blocks.empty() ? (Ap->sweep.n ? 0 : 1) : Ap->blocks.size();
+    const uint64_t per_col = (uint64_t)Ap->info.npartial_slots * elem_size(Ap->dtype);
+    const uint64_t need = per_col * K;
+    // A plan whose segments were made shorter for the narrow rows of its k_hint has more partial
+    // sums than a call at wider ones need be refused for: it runs so many columns at a time.
+    uint32_t cols = 0;
+    if (need > kStaticScratchBytes && per_col <= kStaticScratchBytes)
+        for (size_t i = 0; i < nparts; ++i)
+            if ((Ap->blocks.empty() ? Ap : Ap->blocks[i])->seg_shortened)
+                cols = (uint32_t)(kStaticScratchBytes / per_col);
+    if (need > kStaticScratchBytes && cols == 0) {
         char msg[200];
         std::snprintf(msg, sizeof msg,
                       "the partial sums of this plan's cut rows take %llu bytes at K = %u; "
@@ -893,10 +902,10 @@ int spc3d_spmm_noalloc(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc
     // blocks of a plan kept in column blocks use the array one after the other;
     // npartial_slots is the largest block's.)
     // no container: no host heap either
-    const size_t nparts = Ap->blocks.empty() ? (Ap->sweep.n ? 0 : 1) : Ap->blocks.size();
     for (size_t i = 0; i < nparts; ++i) {
         DevPlanView view = view_of(Ap->blocks.empty() ? Ap : Ap->blocks[i]);
         view.partial = ctx->scratch;
+        view.partial_cols = cols;
         HIP_TRY(launch_spmm(Ap->dtype, view, X->dev, Y->dev, K, streams_of(ctx)));
     }
     if (Ap->sweep.n) // the tiles' sums live in LDS: nothing to allocate either

@@ -135,6 +135,7 @@ struct spc3d_plan {
     spc3d_plan_info info;
     uint64_t row_sq = 0;      // HostPlan::row_sq
     bool cols_sorted = false; // HostPlan::cols_sorted
+    bool seg_shortened = false; // HostPlan::seg_shortened
     bool has_values;
     // device arrays
     Seg *segs;

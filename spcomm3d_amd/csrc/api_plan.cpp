@@ -251,6 +251,7 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
         fill_info(p->info, meta);
         p->row_sq = meta.row_sq;
         p->cols_sorted = meta.cols_sorted;
+        p->seg_shortened = meta.seg_shortened;
         p->info.nsegments_padded = arr.nseg_padded;
         p->info.nsplit_rows = arr.nsplit;
         rc = ctx_alloc_bytes(ctx, &p->sval, (size_t)meta.nnz * elem_size(dtype));
@@ -873,6 +874,7 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
         p->ctx = ctx;
         p->dtype = dtype;
         fill_info(p->info, H);
+        p->seg_shortened = H.seg_shortened;
 
         rc = ctx_alloc(ctx, &p->segs, H.segs.size());
         if (!rc) rc = ctx_alloc(ctx, &p->col, (size_t)nnz);

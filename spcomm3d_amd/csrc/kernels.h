@@ -21,6 +21,8 @@ struct DevPlanView {
     uint32_t nsplit = 0;
     uint32_t nslots = 0; // partial-sum rows of all splits
     void *partial = nullptr;          // [nslots * K] partial sums of cut rows (SpMM)
+    // launch_spmm: columns that `partial` holds of each (0: all K); it then runs so many at a time
+    uint32_t partial_cols = 0;
     // [(nseg - nseg_long) * kFirstCols] the first column indices of every segment past
     // the long ones (launch_first_cols); read by the short-segment launch
     const uint32_t *first_cols = nullptr;

@@ -1043,7 +1043,8 @@ __global__ void __launch_bounds__(kBlock)
 spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32_t rot,
                 const uint32_t *__restrict__ col, const T *__restrict__ sval,
                 const T *__restrict__ X, T *__restrict__ Y, T *__restrict__ partial,
-                uint32_t nvec, uint32_t stride, const uint32_t *__restrict__ first_cols)
+                uint32_t nvec, uint32_t stride, uint32_t pstride,
+                const uint32_t *__restrict__ first_cols)
 {
     static_assert(UB <= 16 && LPR <= 64, "at most 16 entries in flight per lane");
     using V = typename Vec<T>::type;
@@ -1066,7 +1067,7 @@ spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32
     }
     if constexpr (RG >= 2) {
         char *drow = const_cast<char *>(whole ? odd_row<T, RG>(Y, sg[0], stride)
-                                              : odd_row<T, RG>(partial, sg[3], stride));
+                                              : odd_row<T, RG>(partial, sg[3], pstride));
         if (whole) {
 #pragma unroll
             for (int v = 0; v < VPL; ++v)
@@ -1100,14 +1101,14 @@ spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32
 // threads sum a run each (four loads in flight, in slot order, one 16-byte unit of the row per
 // thread where rows are whole units, else one real), the runs are added in pairs through LDS.
 // lanes and parts are powers of two, lanes * parts <= kBlock; the other threads of the block
-// take further rows.
+// take further rows.  A row of Y is yunits units, of which `units` are summed from Y on.
 // Few rows with many slots (the hubs of a small pattern) are a chain of loads each: R-MAT 13,
 // 16-entry segments, fp32 K = 16: SpMM 11.1 us with one run per row, 7.4 with runs.  Many
 // rows are bound by the slots' bytes and take one run each.
 template <typename T, typename U>
 __global__ void __launch_bounds__(kBlock)
 spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U *__restrict__ partial,
-                  U *__restrict__ Y, uint32_t units, uint32_t lanes, uint32_t parts)
+                  U *__restrict__ Y, uint32_t units, uint32_t yunits, uint32_t lanes, uint32_t parts)
 {
     __shared__ typename Vec<T>::type run[kBlock];
     U *sums = reinterpret_cast<U *>(run);
@@ -1126,7 +1127,7 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
         U s{}, y{};
         if (on) {
             if (part == 0)
-                y = Y[(size_t)sr.row * units + j];
+                y = Y[(size_t)sr.row * yunits + j];
             const U *p = partial + (size_t)sr.first_slot * units + j;
             uint32_t q = q0;
             for (; q + 4 <= q1; q += 4) {
@@ -1147,7 +1148,7 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
             }
         }
         if (on && part == 0)
-            Y[(size_t)sr.row * units + j] = y + s;
+            Y[(size_t)sr.row * yunits + j] = y + s;
     }
 }
 
@@ -2091,7 +2092,7 @@ hipError_t run_sddmm(const DevPlanView &P, const T *A, const T *B, T *C, T *Y, c
 
 template <typename T, int LPR, int VPL, int UB, int US, int RG>
 hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, uint32_t nvec,
-                    uint32_t stride = 0, size_t slice_off = 0)
+                    uint32_t stride = 0, size_t slice_off = 0, uint32_t pstride = 0)
 {
     uint32_t nl, ns;
     split_launches(P, RG == 0, nl, ns);
@@ -2100,14 +2101,15 @@ hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, ui
         hipLaunchKernelGGL((spmm_seg_kernel<T, LPR, VPL, UB, RG, true>),
                            dim3(blocks_for_groups(nl, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
                            S.main, P.segs, nl, P.nqueues, 0u, P.col, (const T *)P.sval, X, Y,
-                           (T *)P.partial + slice_off, nvec, stride ? stride : nvec,
+                           (T *)P.partial + slice_off, nvec, stride ? stride : nvec, pstride,
                            (const uint32_t *)nullptr);
     if (ns)
         hipLaunchKernelGGL((spmm_seg_kernel<T, LPR, VPL, US, RG, false>),
                            dim3(blocks_for_groups(ns, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
                            both ? S.aux : S.main, P.segs + nl, ns, P.nqueues,
                            both ? S.aux_rot : 0u, P.col, (const T *)P.sval, X, Y,
-                           (T *)P.partial + slice_off, nvec, stride ? stride : nvec, P.first_cols);
+                           (T *)P.partial + slice_off, nvec, stride ? stride : nvec, pstride,
+                           P.first_cols);
     const hipError_t launched = hipGetLastError();
     const hipError_t joined = both ? join_aux(S) : hipSuccess;
     return launched != hipSuccess ? launched : joined;
@@ -2127,8 +2129,10 @@ hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, ui
     X(64, 2, 8, 4, 2) X(64, 4, 4, 2, 1)
 #define SPC3D_FOR_RAGGED_SHAPES(X) X(32, 1, 16, 8, 4) X(64, 1, 16, 8, 4) X(64, 2, 8, 4, 2) X(64, 4, 4, 2, 1)
 
+// Columns [at, at + w) of K (w == 0: all of them); the runs are those of the whole row either way.
 template <typename T>
-hipError_t launch_fixup(const DevPlanView &P, T *Y, uint32_t K, hipStream_t st)
+hipError_t launch_fixup(const DevPlanView &P, T *Y, uint32_t K, hipStream_t st, uint32_t at = 0,
+                        uint32_t w = 0)
 {
     if (!P.nsplit)
         return hipSuccess;
@@ -2146,12 +2150,12 @@ hipError_t launch_fixup(const DevPlanView &P, T *Y, uint32_t K, hipStream_t st)
         parts *= 2;
     const uint32_t rows = kBlock / (lanes * parts);
     const dim3 grid((P.nsplit + rows - 1) / rows);
-    if (vec)
+    if (vec && w == 0)
         hipLaunchKernelGGL((spmm_fixup_kernel<T, V>), grid, dim3(kBlock), 0, st, P.splits, P.nsplit,
-                           (const V *)P.partial, (V *)Y, units, lanes, parts);
+                           (const V *)P.partial, (V *)Y, units, units, lanes, parts);
     else
         hipLaunchKernelGGL((spmm_fixup_kernel<T, T>), grid, dim3(kBlock), 0, st, P.splits, P.nsplit,
-                           (const T *)P.partial, Y, units, lanes, parts);
+                           (const T *)P.partial, Y + at, w ? w : K, K, lanes, parts);
     return hipGetLastError();
 }
 
@@ -2244,16 +2248,36 @@ hipError_t sddmm_typed(const DevPlanView &P, const void *A, const void *B, void 
 
 template <typename T>
 hipError_t run_spmm_odd(const Shape &sh, const DevPlanView &P, const T *X, T *Y,
-                        const Streams &SS, uint32_t stride, size_t slice_off)
+                        const Streams &SS, uint32_t stride, size_t slice_off, uint32_t pstride)
 {
 #define X(L, V, U, S, S2)                                                                         \
     if (sh.mode == 2 && sh.lpr == L && sh.vpl == V)                                               \
-        return run_spmm<T, L, V, U, S2, 2>(P, X, Y, SS, sh.nvec, stride, slice_off);
+        return run_spmm<T, L, V, U, S2, 2>(P, X, Y, SS, sh.nvec, stride, slice_off, pstride);
     SPC3D_FOR_ODD_SHAPES(X)
 #undef X
     if (sh.mode == 3)
-        return run_spmm<T, 4, 1, 16, 4, 3>(P, X, Y, SS, sh.nvec, stride, slice_off);
+        return run_spmm<T, 4, 1, 16, 4, 3>(P, X, Y, SS, sh.nvec, stride, slice_off, pstride);
     return hipErrorInvalidValue;
+}
+
+// The SpMM of a plan whose partial-sum rows hold fewer than K columns: so many columns at a time,
+// each time the segments and the fix-up, which leaves the partial-sum rows to the next.  Every
+// column is summed as in the whole call: the same bits.
+template <typename T>
+hipError_t spmm_by_columns(const DevPlanView &P, const T *X, T *Y, uint32_t K, const Streams &SS)
+{
+    const uint32_t per = std::min(P.partial_cols, kSliceBytes / (uint32_t)sizeof(T));
+    for (uint32_t at = 0; at < K; at += per) {
+        const uint32_t w = std::min(K - at, per);
+        hipError_t e = run_spmm_odd<T>(odd_shape(sizeof(T), w), P, X + at, Y + at, SS, K, 0, w);
+        if (e == hipSuccess)
+            e = hipGetLastError();
+        if (e == hipSuccess)
+            e = launch_fixup<T>(P, Y, K, SS.main, at, w);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
 }
 
 template <typename T>
@@ -2263,6 +2287,8 @@ hipError_t spmm_typed(const DevPlanView &P, const void *X_, void *Y, uint32_t K,
     const hipStream_t st = SS.main;
     if (P.nseg == 0)
         return hipSuccess;
+    if (P.partial_cols && P.partial_cols < K && P.nsplit)
+        return spmm_by_columns<T>(P, (const T *)X_, (T *)Y, K, SS);
     const Shape sh = pick_shape(sizeof(T), K);
     bool done = false;
     hipError_t e = hipSuccess;
@@ -2281,7 +2307,7 @@ hipError_t spmm_typed(const DevPlanView &P, const void *X_, void *Y, uint32_t K,
     SPC3D_FOR_RAGGED_SHAPES(X)
 #undef X
     if (!done && sh.mode >= 2) {
-        e = run_spmm_odd<T>(sh, P, (const T *)X_, (T *)Y, SS, K, 0);
+        e = run_spmm_odd<T>(sh, P, (const T *)X_, (T *)Y, SS, K, 0, K);
         done = true;
     }
     if (!done) {
@@ -2291,7 +2317,7 @@ hipError_t spmm_typed(const DevPlanView &P, const void *X_, void *Y, uint32_t K,
         for (uint32_t at = 0; at < K && e == hipSuccess; at += per) {
             const uint32_t w = K - at < per ? K - at : per;
             e = run_spmm_odd<T>(odd_shape(sizeof(T), w), P, (const T *)X_ + at, (T *)Y + at, SS, K,
-                                at);
+                                at, K);
         }
     }
     if (e == hipSuccess)

@@ -1076,6 +1076,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         opts.seg_max ? opts.seg_max
                      : default_seg_max(nnz, opts.row_bytes, nrows, hC.rows_touched, hC.max_row), nnz);
     P.seg_max = seg_max;
+    P.seg_shortened = !opts.seg_max && seg_max < seg_max_by_entries(nnz, opts.row_bytes);
     const uint32_t ctouched = hC.cols_touched, maxcdeg = hC.max_cdeg;
 
     // ---- column classes (XCD slicing only) ---------------------------------------

@@ -149,6 +149,7 @@ int build_host_plan(uint32_t nrows, uint32_t ncols, uint64_t nnz, const uint32_t
         const uint32_t seg_max = clamp_seg_max(
             opts.seg_max ? opts.seg_max : default_seg_max(nnz, opts.row_bytes, nrows, touched, maxlen), nnz);
         P.seg_max = seg_max;
+        P.seg_shortened = !opts.seg_max && seg_max < seg_max_by_entries(nnz, opts.row_bytes);
 
         // ---- column classes (XCD slicing only) -----------------------------
         // One L2 is expected to keep hot_cols dense rows.  A sixth of that goes to

@@ -62,6 +62,7 @@ struct HostPlan {
     uint64_t row_sq = 0;           // sum over rows of length * min(length, 2048) (GPU builder)
     bool cols_sorted = false;      // the caller's columns never step down (GPU builder)
     uint32_t seg_max = 0;
+    bool seg_shortened = false;    // by default, and for the width: under seg_max_by_entries
     uint32_t nslots = 0;
     uint32_t nseg_real = 0;        // segments with entries (segs.size() includes padding)
     uint32_t nseg_long = 0;        // leading stored segments, a whole number of chunk rounds, all

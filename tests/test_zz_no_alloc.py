@@ -68,3 +68,28 @@ def test_a_plan_beyond_the_array_is_refused_and_nothing_runs(ctx):
     assert np.array_equal(dY.download(), Y0)
     for h in (S, dX, dY):
         h.close()
+
+
+@pytest.mark.parametrize("dtype,k", [(np.float32, 128), (np.float32, 201), (np.float64, 64), (np.float64, 515)])
+@pytest.mark.parametrize("opts", [{}, {"col_blocks": 2}, {"builder": "host"}])
+def test_segments_shortened_for_narrow_rows_do_not_refuse_wide_calls(ctx, dtype, k, opts):
+    # planned for 32 and 64 bytes, 1,000 entries a row are cut into 32 pieces where 2 would be made
+    # for wide rows; the partial sums are then over the array at these widths, and the call runs a
+    # part of the columns at a time
+    rng = np.random.default_rng(k)
+    m, n, per = 2700, 3000, 1000
+    ii = np.repeat(np.arange(m, dtype=np.uint32), per)
+    jj = rng.integers(0, n, ii.size).astype(np.uint32)
+    vv = rng.uniform(0, 1, ii.size).astype(dtype)
+    X, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (n, m))
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=8, **opts)
+    w = np.dtype(dtype).itemsize
+    assert S.info.npartial_slots * k * w > 32 << 20 and 2 * m * k * w <= 32 << 20
+    dX, dY1, dY2 = ctx.panel_from(X), ctx.panel_from(Y0), ctx.panel_from(Y0)
+    ctx.spmm(S, dX, dY1)
+    ctx.spmm_noalloc(S, dX, dY2)
+    Y = dY1.download()
+    assert np.array_equal(dY2.download(), Y)
+    assert oracle.spmm_rel_err(X, ii, jj, vv, Y0, Y) <= (1e-12 if w == 8 else 1e-5)
+    for h in (S, dX, dY1, dY2):
+        h.close()
