@@ -159,7 +159,7 @@ int spc3d_ctx_create_ex(int device, const spc3d_ctx_opts *opts, spc3d_ctx **out)
         (void)hipGetLastError();
         mem_total = 0;
     }
-    c->pool.set_limit(mem_total / 64);
+    c->pool.open(device, mem_total / 64);
     if (!(o.flags & SPC3D_CTX_NO_AUX_STREAM)) {
         e = hipStreamCreateWithFlags(&c->aux_stream, hipStreamNonBlocking);
         if (e == hipSuccess)

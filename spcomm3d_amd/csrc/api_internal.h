@@ -288,19 +288,14 @@ inline int use_device(const spc3d_ctx *ctx, bool capturable = false)
     return SPC3D_OK;
 }
 
-// Device memory that callers may see (panels, value vectors, row maps); kept blocks of the
-// context's pool give way to it.
+// Device memory that callers may see (panels, value vectors, row maps); blocks that the pools of
+// contexts on this device keep give way to it.
 inline int dev_alloc_bytes(spc3d_ctx *ctx, void **out, size_t bytes)
 {
     *out = nullptr;
     if (bytes == 0)
         return SPC3D_OK;
-    hipError_t e = hipMalloc(out, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        ctx->pool.trim();
-        e = hipMalloc(out, bytes);
-    }
+    const hipError_t e = DevPool::device_alloc(ctx->device, out, bytes);
     if (e != hipSuccess)
         return fail_hip(e, "hipMalloc");
     return SPC3D_OK;

@@ -12,7 +12,8 @@
 // streams, do not come from here.
 //
 // Bounded: at most `limit` bytes are kept; beyond that the blocks unused for longest are freed.
-// Given back: by trim() (spc3d_host_cache_clear), when an allocation fails, and with the context.
+// Given back: by trim() (spc3d_host_cache_clear), with the context, and when an allocation of any
+// context of the process on the same device fails (trim_all).
 #pragma once
 #include <hip/hip_runtime_api.h>
 
@@ -33,12 +34,28 @@ class DevPool {
     DevPool &operator=(const DevPool &) = delete;
     ~DevPool()
     {
+        {
+            std::lock_guard<std::mutex> lock(registry_mutex());
+            for (DevPool **at = &registry(); *at; at = &(*at)->next_)
+                if (*at == this) {
+                    *at = next_;
+                    break;
+                }
+        }
         trim();
         for (void *p : words_)
             (void)hipHostFree(p);
     }
 
-    void set_limit(size_t bytes) { limit_ = bytes; }
+    // Keeps up to `limit` bytes of `device`'s memory.  Once, before the first block.
+    void open(int device, size_t limit)
+    {
+        device_ = device;
+        limit_ = limit;
+        std::lock_guard<std::mutex> lock(registry_mutex());
+        next_ = registry();
+        registry() = this;
+    }
 
     // A block of at least `bytes`; a kept one when its size is within a quarter of that.
     hipError_t get(void **out, size_t bytes)
@@ -49,8 +66,8 @@ class DevPool {
         if (bytes > SIZE_MAX - kGrain)
             return hipErrorOutOfMemory;
         bytes = (bytes + kGrain - 1) / kGrain * kGrain;
-        std::lock_guard<std::mutex> lock(mu_);
         try {
+            std::lock_guard<std::mutex> lock(mu_);
             auto it = kept_.lower_bound(bytes);
             if (it != kept_.end() && it->first <= bytes + bytes / 4) {
                 void *p = it->second.p;
@@ -60,26 +77,34 @@ class DevPool {
                 *out = p;
                 return hipSuccess;
             }
-            void *p = nullptr;
-            hipError_t e = hipMalloc(&p, bytes);
-            if (e != hipSuccess && !kept_.empty()) {
-                (void)hipGetLastError();
-                shrink(0);
-                e = hipMalloc(&p, bytes);
-            }
-            if (e != hipSuccess)
-                return e;
-            try {
-                sizes_.emplace(p, bytes);
-            } catch (const std::bad_alloc &) {
-                (void)hipFree(p);
-                return hipErrorOutOfMemory;
-            }
-            *out = p;
-            return hipSuccess;
         } catch (const std::bad_alloc &) {
             return hipErrorOutOfMemory;
         }
+        void *p = nullptr;
+        const hipError_t e = device_alloc(device_, &p, bytes); // (no lock held: it may trim this pool)
+        if (e != hipSuccess)
+            return e;
+        try {
+            std::lock_guard<std::mutex> lock(mu_);
+            sizes_.emplace(p, bytes);
+        } catch (const std::bad_alloc &) {
+            (void)hipFree(p);
+            return hipErrorOutOfMemory;
+        }
+        *out = p;
+        return hipSuccess;
+    }
+
+    // hipMalloc on `device` (which is current), to which every pool's kept blocks there give way.
+    static hipError_t device_alloc(int device, void **out, size_t bytes)
+    {
+        hipError_t e = hipMalloc(out, bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            trim_all(device);
+            e = hipMalloc(out, bytes);
+        }
+        return e;
     }
 
     // Takes back a block that get() handed out.
@@ -144,6 +169,14 @@ class DevPool {
         std::lock_guard<std::mutex> lock(mu_);
         shrink(0);
     }
+    // Frees every block that a pool of this process keeps on `device`.
+    static void trim_all(int device)
+    {
+        std::lock_guard<std::mutex> lock(registry_mutex());
+        for (DevPool *p = registry(); p; p = p->next_)
+            if (p->device_ == device)
+                p->trim();
+    }
 
   private:
     struct Kept {
@@ -163,6 +196,20 @@ class DevPool {
             kept_.erase(oldest);
         }
     }
+    // The open pools of the process, one after the other.  registry_mutex() is taken before a
+    // pool's own and never while one is held.
+    static std::mutex &registry_mutex()
+    {
+        static std::mutex *m = new std::mutex(); // outlives every context, static ones too
+        return *m;
+    }
+    static DevPool *&registry()
+    {
+        static DevPool *first = nullptr;
+        return first;
+    }
+    DevPool *next_ = nullptr;
+    int device_ = 0;
     static constexpr size_t kGrain = 512;
     std::mutex mu_;
     std::vector<void *> words_; // get_words() of as many threads as ever plan at once

@@ -1,6 +1,7 @@
 // Host-only test of the copies between host memory and the device (spcomm3d_amd/csrc/host_stage.cpp)
-// where pinned memory runs out: over a stand-in for the few HIP calls they make, in which
-// "device" memory is host memory and the pinned memory that can be had is set by the test.
+// where pinned memory runs out, and of the contexts' pools of device memory (dev_pool.h) where
+// device memory does: over a stand-in for the few HIP calls they make, in which "device" memory is
+// host memory and what can be had of either is set by the test.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -9,8 +10,10 @@
 #include <map>
 #include <mutex>
 #include <random>
+#include <thread>
 #include <vector>
 
+#include "../../spcomm3d_amd/csrc/dev_pool.h"
 #include "../../spcomm3d_amd/csrc/host_stage.h"
 
 using namespace spc3d;
@@ -36,7 +39,29 @@ static size_t pinned_now()
     return n;
 }
 
+static size_t g_device_room;
+static std::map<void *, size_t> g_device;
+
 extern "C" {
+hipError_t hipMalloc(void **p, size_t n)
+{
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (n > g_device_room)
+        return hipErrorOutOfMemory;
+    *p = std::malloc(1);
+    g_device[*p] = n;
+    g_device_room -= n;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    std::lock_guard<std::mutex> lock(g_mu);
+    CHECK(g_device.count(p) == 1);
+    g_device_room += g_device[p];
+    g_device.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
     std::lock_guard<std::mutex> lock(g_mu);
@@ -114,8 +139,61 @@ static void small_transfers_pin_little()
     CHECK(pinned_now() > 0 && pinned_now() <= (size_t)2 << 20);
 }
 
+// What one context's pool keeps gives way to another context that runs out; other devices' pools
+// and blocks in use do not.
+static void pools_give_way()
+{
+    g_device_room = 100 << 10;
+    {
+        DevPool a, b, other;
+        a.open(0, 90 << 10);
+        b.open(0, 90 << 10);
+        other.open(1, 90 << 10);
+        void *p = nullptr, *q = nullptr, *r = nullptr, *s = nullptr;
+        CHECK(a.get(&p, 40 << 10) == hipSuccess && a.get(&q, 20 << 10) == hipSuccess);
+        CHECK(other.get(&r, 20 << 10) == hipSuccess);
+        a.put(p);
+        other.put(r);
+        CHECK(g_device.size() == 3);
+        CHECK(b.get(&s, 50 << 10) == hipSuccess && s); // fits once a's 40 KiB are free
+        CHECK(g_device.size() == 3 && g_device.count(q) && g_device.count(r));
+        b.put(s);
+        CHECK(DevPool::device_alloc(0, &p, 60 << 10) == hipSuccess); // a panel's: b's 50 KiB give way
+        CHECK(b.get(&s, 30 << 10) == hipErrorOutOfMemory && s == nullptr);
+        CHECK(hipFree(p) == hipSuccess);
+        a.put(q);
+    }
+    CHECK(g_device.empty());
+    std::vector<std::thread> threads; // pools made, run dry and dropped side by side
+    g_device_room = 400 << 10;
+    for (int t = 0; t < 4; ++t)
+        threads.emplace_back([t] {
+            std::mt19937 g(t);
+            for (int round = 0; round < 200; ++round) {
+                DevPool pool;
+                pool.open(t % 2, 200 << 10);
+                std::vector<void *> held;
+                for (int i = 0; i < 12; ++i) {
+                    void *p = nullptr;
+                    if (pool.get(&p, (g() % 64 + 1) << 10) == hipSuccess)
+                        held.push_back(p);
+                    if (!held.empty() && g() % 2) {
+                        pool.put(held.back());
+                        held.pop_back();
+                    }
+                }
+                for (void *p : held)
+                    pool.put(p);
+            }
+        });
+    for (auto &t : threads)
+        t.join();
+    CHECK(g_device.empty());
+}
+
 int main()
 {
+    pools_give_way();
     for (unsigned threads : {1u, 3u})
         for (size_t room : {(size_t)0, (size_t)1 << 20, (size_t)2 << 20, (size_t)13 << 20, (size_t)30 << 20,
                             (size_t)1 << 30})

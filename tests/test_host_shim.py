@@ -132,8 +132,9 @@ def test_content_keys_of_the_one_shot_host_calls():
     _run("test_keys")
 
 
-def test_copies_between_host_and_device_without_pinned_memory():
-    # the library's transfers where pinned memory cannot be had, or only some of it
+def test_copies_and_pools_where_memory_runs_out():
+    # the library's transfers where pinned memory cannot be had, or only some of it; and what one
+    # context's pool keeps of device memory gives way to another context
     _run("test_host_memory")
 
 
