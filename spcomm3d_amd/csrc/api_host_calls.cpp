@@ -67,7 +67,7 @@ int host_plan(spc3d_ctx *ctx, HostCallCache *hc, int dtype, uint32_t nrows, uint
     spc3d_plan_opts o = opts_from_env();
     if (!o.k_hint)
         o.k_hint = k; // the one width this plan will run with; sizes the partial-sum rows too
-    if (!o.seg_max) // rows cut as in a plan made without options: the same sums, bit for bit
+    if (!o.seg_max) // rows cut as in a plan made without options
         o.seg_max = seg_max_by_entries(nnz, (uint32_t)std::min<uint64_t>(k * elem_size(dtype), 1u << 30));
     spc3d_plan *plan = nullptr;
     int rc = spc3d_plan_create_ex(ctx, dtype, nrows, ncols, nnz, ii, jj, vv, &o, &plan);
@@ -346,7 +346,7 @@ static int sddmm_host_uncached(spc3d_ctx *ctx, int dtype, uint32_t m, uint32_t n
         o.k_hint = k; // the one width this plan will ever run with
     if (!o.seg_max)
         o.seg_max = seg_max_by_entries(nnz, (uint32_t)std::min<uint64_t>(k * elem_size(dtype), 1u << 30));
-    int rc = spc3d_plan_create_ex(ctx, dtype, m, n, nnz, ii, jj, svv, &o, &S);
+    int rc = create_plan(ctx, dtype, m, n, nnz, ii, jj, svv, &o, true, &S);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, m, k, &a);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, n, k, &b);
     if (!rc) rc = spc3d_vals_create(ctx, dtype, nnz, &c);
@@ -420,7 +420,7 @@ static int spmm_host_uncached(spc3d_ctx *ctx, int dtype, uint32_t ncols, uint32_
     spc3d_plan_opts o = opts_from_env();
     if (!o.k_hint)
         o.k_hint = k;
-    int rc = spc3d_plan_create_ex(ctx, dtype, nrows, ncols, nnz, ii, jj, avv, &o, &S);
+    int rc = create_plan(ctx, dtype, nrows, ncols, nnz, ii, jj, avv, &o, true, &S);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, ncols, k, &x);
     if (!rc) rc = spc3d_panel_create(ctx, dtype, nrows, k, &y);
     if (!rc) rc = spc3d_panel_upload(x, X);

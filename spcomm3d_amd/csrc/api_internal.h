@@ -482,6 +482,10 @@ extern "C" int ensure_partial(spc3d_plan *p, uint32_t K);
 // than it was laid out for, its ordinary twin (built on first use unless may_build is false;
 // never while the context records).
 extern "C" int plan_for_k(spc3d_plan *plan, uint32_t K, bool may_build, spc3d_plan **out);
+// spc3d_plan_create_ex; one_call: PlanOpts::one_call.
+extern "C" int create_plan(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t ncols, uint64_t nnz,
+                           const uint32_t *ii, const uint32_t *jj, const void *vv,
+                           const spc3d_plan_opts *opts, bool one_call, spc3d_plan **out);
 // The defaults of spc3d_plan_create and of the one-shot host calls: the library's, each
 // overridable from the environment.
 extern "C" spc3d_plan_opts opts_from_env();

@@ -571,14 +571,14 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
 // The plan itself stays: it runs every other K, the one-pass calls (which read the dense rows
 // once, as fast as either of the tiles' kernels) and what the tiles leave out.
 // The tiles add a row's entries block after block, so a caller that asked for the order of its own
-// gets none.
+// gets none; nor does a plan that serves one call.
 static int add_tiles(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                      const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
                      const spc3d_plan_opts *opts)
 {
     const spc3d_plan_info &I = p->info;
     if (!opts || opts->sweep || opts->col_blocks || !opts->k_hint || opts->builder == 1 ||
-        po.keep_entry_order || I.nqueues != 1 || nnz == 0)
+        po.keep_entry_order || po.one_call || I.nqueues != 1 || nnz == 0)
         return SPC3D_OK;
     const uint32_t lanes = sweep_lanes_any(p->dtype, opts->k_hint);
     if (!lanes)
@@ -823,6 +823,13 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
                          const uint32_t *ii, const uint32_t *jj, const void *vv,
                          const spc3d_plan_opts *opts, spc3d_plan **out)
 {
+    return create_plan(ctx, dtype, nrows, ncols, nnz, ii, jj, vv, opts, false, out);
+}
+
+int create_plan(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t ncols, uint64_t nnz,
+                const uint32_t *ii, const uint32_t *jj, const void *vv, const spc3d_plan_opts *opts,
+                bool one_call, spc3d_plan **out)
+{
     if (!out)
         return fail(SPC3D_ERR_INVALID_ARG, "out is NULL");
     *out = nullptr;
@@ -832,6 +839,7 @@ int spc3d_plan_create_ex(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t nco
     int rc = resolve_opts(dtype, opts, po);
     if (rc)
         return rc;
+    po.one_call = one_call;
     const bool on_host = opts && opts->builder == 1;
     spc3d_plan *p = nullptr;
     if (!on_host && live(ctx)) {

@@ -52,6 +52,8 @@ struct PlanOpts {
     // slicing: false keeps the free segments dealt by rank alone (no affinity to the slice of
     // their entries, see deal_plan)
     bool slice_affinity = true;
+    // the plan serves one call: no row tiles beside it, which take several to repay their making
+    bool one_call = false;
 };
 
 struct HostPlan {

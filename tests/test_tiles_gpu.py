@@ -103,6 +103,22 @@ def test_the_callers_order_is_kept_where_it_is_asked_for(ctx, shuffled):
     assert tiled.sweep_tiles > 0 and tiled.sweep_k == k and tiled.sweep_entries == 0
 
 
+def test_a_plan_for_one_call_has_no_tiles(ctx):
+    # one-shot calls that keep nothing: SpMM adds in the order of the ordinary plan, not by blocks
+    k, n, m = 128, 11000, len(ROWS_80)
+    ii, jj = pattern(ROWS_80, n, False)
+    rng = np.random.default_rng(2)
+    vv = rng.uniform(0, 1, ii.size)
+    B, Y0 = rng.uniform(-1, 1, (n, k)), rng.uniform(-1, 1, (m, k))
+    S, dY = ctx.plan(m, n, ii, jj, vv, k_hint=k, sweep=False), ctx.panel_from(Y0)
+    ctx.spmm(S, ctx.panel_from(B), dY)
+    S.close()
+    with device.Context(0, host_cache=False) as c:
+        Y = Y0.copy()
+        c.spmm_host(B, ii, jj, vv, Y)
+    assert np.array_equal(Y, dY.download())
+
+
 # widths that leave lanes of the tiles idle or end inside a 16-byte unit, at the edges of each lane
 # count (16 lanes to 256 bytes, 32 to 512, 64 to 1024), and widths that fill them
 @pytest.mark.parametrize("dtype,k", [(np.float32, k) for k in (33, 36, 50, 63, 64, 65, 67, 96, 127, 128, 129,
