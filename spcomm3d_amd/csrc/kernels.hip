@@ -1103,8 +1103,10 @@ spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32
 // lanes and parts are powers of two, lanes * parts <= kBlock; the other threads of the block
 // take further rows.  A row of Y is yunits units, of which `units` are summed from Y on.
 // Few rows with many slots (the hubs of a small pattern) are a chain of loads each: R-MAT 13,
-// 16-entry segments, fp32 K = 16: SpMM 11.1 us with one run per row, 7.4 with runs.  Many
-// rows are bound by the slots' bytes and take one run each.
+// 16-entry segments, fp32 K = 16: SpMM 11.1 us with one run per row, 7.4 with runs.  Rows that fill
+// the chip are bound by the slots' bytes and take one run each, also where they have many: SpMM of
+// 30,000 rows of 125 slots, fp32 K = 20, 431 us in runs and 422 without, 20,000 of 100, fp64 K = 100,
+// 1941 and 1944, 4,500 of 250, fp32 K = 256, 2320 and 2340; R-MAT 18 and 20 are 0.2 % faster without.
 template <typename T, typename U>
 __global__ void __launch_bounds__(kBlock)
 spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U *__restrict__ partial,
@@ -2142,11 +2144,10 @@ hipError_t launch_fixup(const DevPlanView &P, T *Y, uint32_t K, hipStream_t st, 
     uint32_t lanes = 4;
     while (lanes < (uint32_t)kBlock && lanes < units)
         lanes *= 2;
-    // Runs while the launch does not fill the chip anyway, and for rows of many slots.
+    // Runs while the launch does not fill the chip anyway.
     uint32_t parts = 1;
-    while (lanes * parts < (uint32_t)kBlock &&
-           parts * P.nsplit <= 2 * (uint64_t)P.nslots &&
-           ((uint64_t)P.nsplit * lanes * parts < (1u << 18) || parts * 4 < P.nslots / P.nsplit))
+    while (lanes * parts < (uint32_t)kBlock && parts * P.nsplit <= 2 * (uint64_t)P.nslots &&
+           (uint64_t)P.nsplit * lanes * parts < (1u << 18))
         parts *= 2;
     const uint32_t rows = kBlock / (lanes * parts);
     const dim3 grid((P.nsplit + rows - 1) / rows);
