@@ -552,16 +552,26 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
 
 // Row tiles beside a finished single plan (spc3d_plan::tiles), for patterns that column blocks
 // would not serve.  The tiles read a block of dense rows into each L2 once per generation of
-// tiles instead of once per miss, so they pay where
+// tiles instead of once per miss.  Making them costs the plan 0.76 to 1.05 ms for 6 to 10 M entries,
+// which three to five steps repay, so they are made where a step gains a good part of that.  The
+// lines below, with SDDMM + SpMM in us without and with tiles (fp32 K = 128, uniform rows of 60
+// entries, unless said otherwise):
 //  - the columns are not skewed and the panel is well over an L2: 4 blocks of 3.25 MiB or more
-//    (at 2 the tiles are level to 15 % slower);
-//  - every column comes up often enough for its copy in each L2: 12 entries (at 5, 1 KB rows,
-//    264 -> 317 us; at 18, 930 -> 658);
-//  - the launch is long enough for the barriers of its blocks: 512 MiB of gathers.
+//    (3 M entries: 2 blocks 210 -> 198, 3: 279 -> 201, 4: 317 -> 203, 6: 363 -> 216);
+//  - every column comes up often enough for its copy in each L2: 12 entries (16 blocks: 6 entries
+//    88 -> 115, 9: 132 -> 133, 12: 172 -> 159, 18: 255 -> 195);
+//  - the launch is long enough for the barriers of its blocks: 512 MiB of gathers (4 blocks: 161 MiB
+//    43 -> 51, 317: 79 -> 70, 488: 114 -> 90, 732: 165 -> 118);
+//  - no row is as long as a good part of a tile, whose workgroup would outlast the others: an eighth
+//    of the mean tile (15,360 entries here; a row of 1,920: 364 -> 228, 3,840: 373 -> 254, 7,680:
+//    368 -> 304, 20,000: 369 -> 481);
+//  - what is left over is little: a quarter of the entries (6 M; a tenth 724 -> 484, a quarter
+//    763 -> 544, half 788 -> 612, three quarters 809 -> 725).
 // Rows shorter than the number of blocks would hold less than an entry per block and stay out,
-// as do those under 16 entries.  SpMM adds a row's sums to LDS once per block, in rows padded to the
-// lanes' width, so it takes the tiles only for rows of 24 full widths and more on average, and 1.5
-// per block (rows of 30, 512-byte rows 974 -> 831 us, 384-byte 691 -> 752).
+// as do those under 16 entries (10 blocks, SDDMM: rows of 20 406 -> 300, of 30 394 -> 260).  SpMM adds
+// a row's sums to LDS once per block, in rows padded to the lanes' width, so it takes the tiles only
+// for rows of 24 full widths and more on average, and 1.5 per block (10 blocks, SpMM: rows of 20
+// 426 -> 440, of 30 408 -> 370, of 45 400 -> 306; 384-byte rows of 30 691 -> 752).
 // SDDMM results in an arbitrary order leave the tiles through the staging vector, which costs more
 // than the ordinary plan's two passes: from 400-byte rows on the tiles make up for it (8.9 M entries:
 // 256 bytes 280 -> 318 us, 360 level, 512 582 -> 486).

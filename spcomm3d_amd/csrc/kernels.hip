@@ -1487,9 +1487,11 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 // start at element alignment, and their last unit is the 16 bytes that END at the row's end
 // (it overlaps the unit before: a copy writes the same bytes twice, a sum stores only the
 // elements that are the unit's own); kElem - rows under 16 bytes, one real per lane.
-// 500 k random rows of a 1 M-row panel, fp32 K = 50, pack / unpack / sum-unpack: a real per lane
-// with a division per real took 45 / 85 / 130 us, this 39 / 39 / 61 (a row of 200 bytes at any
-// alignment touches 2.6 lines of 128).
+// 500 k random rows of a 1 M-row panel, fp32 K = 50, pack / unpack / sum-unpack one after the other,
+// each over its own panel: a real per lane with a division per real took 76 / 89 / 135 us, this
+// 50 / 50 / 69 (a row of 200 bytes at any alignment touches 2.6 lines of 128; repeated alone, on a
+// panel of which much stays in the Infinity Cache, 45 / 85 / 129 and 39 / 40 / 62).  Over panels that
+// change from pass to pass the three take 298 and 202 us together.
 enum RowUnit { kVec, kLoose, kElem };
 constexpr int kRowsAhead = 4;    // of a copy
 // Fewer workgroups than this (8 per CU) do not fill the chip: one row at a time then, which
