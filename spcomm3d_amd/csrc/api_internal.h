@@ -144,6 +144,12 @@ struct spc3d_plan {
     void *sval;     // values in kernel order
     SplitRow *splits;
     uint32_t *first_cols; // [(nsegments_padded - nsegments_long) * kFirstCols], see kernels.h
+    // Hot rows that crowd (DevPlanView): nhot columns; the other three are made by add_hot_rows and
+    // null without it.
+    uint32_t *hot_cols = nullptr;
+    uint32_t nhot = 0, hot_row_bytes = 0;
+    uint32_t *hot_col = nullptr, *hot_first_cols = nullptr;
+    void *hot_rows = nullptr;
     void *partial; // [npartial_slots * partial_k] reals
     uint32_t partial_k;
     // Partial-sum blocks that a call at a larger K has replaced.  They stay allocated
@@ -353,6 +359,17 @@ inline void ctx_free(spc3d_ctx *ctx, void *p) { ctx->pool.put(p); }
 
 inline DevStream dev_stream(spc3d_ctx *ctx) { return DevStream{ctx->stream, &ctx->pool}; }
 
+inline void drop_hot_rows(spc3d_plan *p)
+{
+    if (p->hot_cols) ctx_free(p->ctx, p->hot_cols);
+    if (p->hot_col) ctx_free(p->ctx, p->hot_col);
+    if (p->hot_first_cols) ctx_free(p->ctx, p->hot_first_cols);
+    if (p->hot_rows) ctx_free(p->ctx, p->hot_rows);
+    p->hot_cols = p->hot_col = p->hot_first_cols = nullptr;
+    p->hot_rows = nullptr;
+    p->nhot = p->hot_row_bytes = 0;
+}
+
 inline void plan_free_device(spc3d_plan *p)
 {
     if (p->segs) ctx_free(p->ctx, p->segs);
@@ -361,6 +378,7 @@ inline void plan_free_device(spc3d_plan *p)
     if (p->sval) ctx_free(p->ctx, p->sval);
     if (p->splits) ctx_free(p->ctx, p->splits);
     if (p->first_cols) ctx_free(p->ctx, p->first_cols);
+    drop_hot_rows(p);
     if (p->store.perm2) ctx_free(p->ctx, p->store.perm2);
     if (p->store.dst) ctx_free(p->ctx, p->store.dst);
     if (p->store.src) ctx_free(p->ctx, p->store.src);
@@ -415,6 +433,15 @@ inline DevPlanView view_of(const spc3d_plan *p)
     v.first_cols = p->first_cols;
     v.nnz = p->info.nnz;
     v.seg_base = p->store.consecutive;
+    if (p->hot_rows) {
+        v.hot_cols = p->hot_cols;
+        v.nhot = p->nhot;
+        v.ncols = p->info.ncols;
+        v.hot_row_bytes = p->hot_row_bytes;
+        v.hot_rows = p->hot_rows;
+        v.hot_col = p->hot_col;
+        v.hot_first_cols = p->hot_first_cols;
+    }
     if (p->two.n)
         v.perm = nullptr; // results in kernel order (into c_stage, see sddmm_out)
     if (p->store.n) {

@@ -261,6 +261,7 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
         if (arr.col) ctx_free(ctx, arr.col);
         if (arr.perm) ctx_free(ctx, arr.perm);
         if (arr.splits) ctx_free(ctx, arr.splits);
+        if (arr.hot_cols) ctx_free(ctx, arr.hot_cols);
         delete p;
         return rc;
     }
@@ -268,6 +269,8 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
     p->col = arr.col;
     p->perm = arr.perm;
     p->splits = arr.splits;
+    p->hot_cols = arr.hot_cols;
+    p->nhot = arr.nhot;
     arr = DevPlanArrays{};
     rc = finish_plan(p, k0);
     if (rc) {
@@ -277,6 +280,35 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
     }
     p->magic = kMagicPlan;
     *out = p;
+    return SPC3D_OK;
+}
+
+// What the calls of a finished single plan whose hot rows crowd (p->nhot, set by the builder) need
+// beside its arrays: the column indices with those columns named by rank, and room for their dense
+// rows at the planned width.
+static int add_hot_rows(spc3d_plan *p, uint32_t k0)
+{
+    if (!p->nhot)
+        return SPC3D_OK;
+    const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
+    const uint64_t row_bytes = (uint64_t)k0 * elem_size(p->dtype);
+    int rc = ctx_alloc(p->ctx, &p->hot_col, (size_t)p->info.nnz);
+    if (!rc) rc = ctx_alloc(p->ctx, &p->hot_first_cols, (size_t)nshort * kFirstCols);
+    if (!rc) rc = ctx_alloc_bytes(p->ctx, &p->hot_rows, (size_t)p->nhot * row_bytes + kHotUnit);
+    std::string err;
+    if (!rc) {
+        rc = encode_hot_device(dev_stream(p->ctx), p->col, p->info.nnz, p->hot_cols, p->nhot,
+                               p->info.ncols, p->hot_col, err);
+        if (rc)
+            fail(rc, err);
+    }
+    if (rc) {
+        drop_hot_rows(p);
+        return optional_path(rc);
+    }
+    p->hot_row_bytes = (uint32_t)row_bytes;
+    HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->hot_col, p->hot_first_cols,
+                              p->ctx->stream));
     return SPC3D_OK;
 }
 
@@ -361,6 +393,8 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
     rc = adopt_device_plan(p->ctx, p->dtype, meta, arr, 0 /* never runs SpMM */, &q);
     if (!rc)
         rc = add_store_staging(q, so);
+    if (!rc)
+        rc = add_hot_rows(q, po.row_bytes / (uint32_t)elem_size(p->dtype));
     if (rc || (q->perm && !q->store.consecutive)) { // no better than what there is
         if (q) {
             const std::string keep = g_err;
@@ -672,6 +706,8 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
         if (sw_lanes && opts->sweep == 2 && opts->col_blocks <= 1)
             nb = 1; // asked for tiles, not for blocks
     }
+    if (!rc && nb <= 1)
+        rc = add_hot_rows(p, planned_k(opts));
     if (!rc && nb <= 1)
         rc = add_store_staging(p, so);
     if (!rc && nb <= 1)
@@ -1170,6 +1206,7 @@ int spc3d_plan_set_values_device(spc3d_plan *plan, const spc3d_vals *vv)
 // One plan's columns rewritten in place, and its table of first columns with them.
 static int probe_columns_of(spc3d_plan *p, int mode, uint32_t modulus)
 {
+    p->hot_row_bytes = 0; // the probe's columns are gathered where they lie
     HIP_TRY(launch_probe_cols(p->col, p->info.nnz, (uint32_t)mode, p->col_base, modulus,
                               p->info.ncols, p->ctx->stream));
     const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
@@ -1226,6 +1263,10 @@ static uint64_t own_device_bytes(const spc3d_plan *p)
     if (p->splits) b += (uint64_t)p->info.nsplit_rows * sizeof(SplitRow);
     if (p->first_cols)
         b += (uint64_t)(p->info.nsegments_padded - p->info.nsegments_long) * kFirstCols * 4;
+    if (p->hot_rows) {
+        b += (uint64_t)p->nhot * (4 + p->hot_row_bytes) + nnz * 4;
+        b += (uint64_t)(p->info.nsegments_padded - p->info.nsegments_long) * kFirstCols * 4;
+    }
     if (p->partial) b += (uint64_t)p->info.npartial_slots * p->partial_k * w;
     b += p->retired_bytes;
     if (p->store.perm2) b += nnz * 4;

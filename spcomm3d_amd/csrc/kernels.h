@@ -36,6 +36,14 @@ struct DevPlanView {
     // every segment's positions in `perm` are perm[start], perm[start] + 1, ...: SDDMM
     // reads one position per segment
     bool seg_base = false;
+    // Hot rows that crowd (kHotRow in plan_host.h): the columns, the buffer their dense rows are
+    // copied to (hot_row_bytes each), and `col` and `first_cols` with those columns named by rank;
+    // null: none
+    const uint32_t *hot_cols = nullptr;
+    uint32_t nhot = 0, hot_row_bytes = 0, ncols = 0;
+    void *hot_rows = nullptr;
+    const uint32_t *hot_col = nullptr, *hot_first_cols = nullptr;
+    uint32_t ref_at = 0, hot_at = 0; // set for a launch that gathers from there
 };
 
 // The context's stream, plus an auxiliary stream of the same (default) priority

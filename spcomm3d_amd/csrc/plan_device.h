@@ -20,6 +20,8 @@ struct DevPlanArrays {
     uint32_t *perm = nullptr;   // [nnz]; null when the caller's order is the kernel order
     SplitRow *splits = nullptr; // [nsplit]
     uint32_t nsplit = 0;
+    uint32_t *hot_cols = nullptr; // [nhot] the hottest columns where their rows crowd (hot_rows_crowd)
+    uint32_t nhot = 0;
 };
 
 // d_ii, d_jj: device arrays of nnz entries.  On success fills `meta` (every
@@ -30,6 +32,11 @@ struct DevPlanArrays {
 int build_device_plan(const DevStream &stream, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                       const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &opts,
                       HostPlan &meta, DevPlanArrays &out, std::string &err);
+
+// d_out[q] = kHotRow | i where d_col[q] == d_hot[i], else d_col[q]; q < n, d_col[q] < ncols <= kHotRow.
+// Asynchronous on `stream`.
+int encode_hot_device(const DevStream &stream, const uint32_t *d_col, uint64_t n, const uint32_t *d_hot,
+                      uint32_t nhot, uint32_t ncols, uint32_t *d_out, std::string &err);
 
 // COOMatrix::localizeIndices (src/SparseMatrix.hpp:69-99) on one device array of n
 // indices: every distinct value gets the next local id the first time it

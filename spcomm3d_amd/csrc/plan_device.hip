@@ -32,6 +32,7 @@ struct Counters { // one device-resident block, zeroed (first_bad: all ones) bef
     unsigned long long covered;
     unsigned long long row_sq;
     unsigned long long load[kSlices], any_load, pref_load[kSlices];
+    unsigned long long hot_weight[kHotClasses];
 };
 
 // Owning device buffer; back to the pool on scope exit unless released.
@@ -357,6 +358,37 @@ __global__ void sum_first_k(const uint32_t *__restrict__ v, uint64_t n, unsigned
     s = block_sum(s);
     if (threadIdx.x == 0 && s)
         atomicAdd(out, s);
+}
+
+// Entries of the n hottest columns by the low bits of the column (hot_rows_crowd); one workgroup.
+__global__ void __launch_bounds__(kTB)
+hot_weight_k(const uint32_t *__restrict__ order, const uint32_t *__restrict__ deg, uint32_t n,
+             unsigned long long *__restrict__ weight)
+{
+    __shared__ unsigned long long sum[kHotClasses];
+    if (threadIdx.x < kHotClasses)
+        sum[threadIdx.x] = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += kTB)
+        atomicAdd(&sum[order[i] % kHotClasses], (unsigned long long)deg[i]);
+    __syncthreads();
+    if (threadIdx.x < kHotClasses)
+        weight[threadIdx.x] = sum[threadIdx.x];
+}
+
+// rank[hot[i]] = i (rank: all ones before)
+__global__ void hot_ranks_k(const uint32_t *__restrict__ hot, uint64_t n, uint16_t *__restrict__ rank)
+{
+    GRID_STRIDE(i, n) rank[hot[i]] = (uint16_t)i;
+}
+__global__ void encode_hot_k(const uint32_t *__restrict__ col, uint64_t n,
+                             const uint16_t *__restrict__ rank, uint32_t *__restrict__ out)
+{
+    GRID_STRIDE(q, n)
+    {
+        const uint32_t c = col[q], r = rank[c];
+        out[q] = r == 0xFFFFu ? c : kHotRow | r;
+    }
 }
 
 // Classes of the htot hottest columns (order[] = columns by degree, highest first).
@@ -1081,6 +1113,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
 
     // ---- column classes (XCD slicing only) ---------------------------------------
     SBuf<uint8_t> cls;
+    DBuf<uint32_t> hot;
     bool slices = false;
     if (want_slices && opts.hot_cols > 0 && ctouched > opts.hot_cols) {
         const uint32_t h1 = opts.hot_cols;
@@ -1097,6 +1130,11 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         TRY(sort_pairs<uint32_t>(tmp, coldeg.p, deg_sorted.p, colid.p, order.p, ncols,
                                  bits_for(maxcdeg), true, st, err));
         LAUNCH_SMALL(sum_first_k, htot, deg_sorted.p, htot, &dC.p->covered);
+        const bool hot_form = !opts.one_call && ncols <= kHotRow && hot_rows_pay(nnz, opts.row_bytes);
+        const uint32_t nhot = (uint32_t)std::min<uint64_t>(kHotRows, htot);
+        if (hot_form)
+            hipLaunchKernelGGL(hot_weight_k, dim3(1), dim3(kTB), 0, st, order.p, deg_sorted.p, nhot,
+                               dC.p->hot_weight);
         TRY(fetch(st, &hC, dC.p, sizeof hC, err));
         const uint64_t covered = hC.covered;
         const double coverage = (double)covered / (double)nnz;
@@ -1108,6 +1146,14 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
             LAUNCH(classify_k, htot, order.p, htot, hrep, cls.p);
             P.hot_cols = (uint32_t)htot;
             P.hot_entries = covered;
+            uint64_t weight[kHotClasses];
+            for (uint32_t i = 0; i < kHotClasses; ++i)
+                weight[i] = hC.hot_weight[i];
+            if (hot_form && hot_rows_crowd(weight)) {
+                HIP_OK(hot.alloc(st, nhot));
+                HIP_OK(hipMemcpyAsync(hot.p, order.p, nhot * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
+                out.nhot = nhot;
+            }
         }
         HIP_OK(hipGetLastError());
     }
@@ -1271,7 +1317,20 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     out.perm = P.identity ? nullptr : perm.release();
     out.splits = splits.release();
     out.nsplit = nsplit;
+    out.hot_cols = hot.release();
     meta = std::move(P);
+    return SPC3D_OK;
+}
+
+int encode_hot_device(const DevStream &st, const uint32_t *d_col, uint64_t n, const uint32_t *d_hot,
+                      uint32_t nhot, uint32_t ncols, uint32_t *d_out, std::string &err)
+{
+    DBuf<uint16_t> rank;
+    HIP_OK(rank.alloc(st, ncols));
+    LAUNCH(fill_k<uint16_t>, ncols, rank.p, (uint64_t)ncols, (uint16_t)0xFFFFu);
+    LAUNCH(hot_ranks_k, nhot, d_hot, (uint64_t)nhot, rank.p);
+    LAUNCH(encode_hot_k, n, d_col, n, rank.p, d_out);
+    HIP_OK(hipGetLastError());
     return SPC3D_OK;
 }
 

@@ -37,6 +37,47 @@ struct SplitRow {
     uint32_t pad;
 };
 
+// ---- hot rows that crowd ---------------------------------------------------------
+// Dense rows a power of two apart whose numbers share their low bits (the hubs of an R-MAT graph,
+// whose numbers have few one-bits) share channels and sets of every L2, and the hottest of them carry
+// most of the gathers.  A plan whose hottest columns crowd so keeps a second list of its column indices
+// in which they are named by rank (kHotRow | rank), and a call copies their dense rows side by side
+// (4 MB at 512-byte rows, 4 us with its launch) and gathers them from there.
+constexpr uint32_t kHotRow = 0x80000000u;
+// At most this many columns.  R-MAT 20, fp64 K = 64, SDDMM / SpMM in us: none 907 / 876, 1024 885 / 848,
+// 4096 859 / 829, 8192 847 / 817, 16384 845 / 817; fp32: 457 / 420, 439 / 401, 433 / 394, 427 / 389,
+// 427 / 388 (column numbers scrambled, where nothing crowds: 837 / 806 and 417 / 379).
+constexpr uint32_t kHotRows = 8192;
+constexpr uint32_t kHotUnit = 128;   // bytes, see the kernels' RG == -1
+constexpr uint32_t kHotClasses = 32; // of column numbers, by their low bits
+// Dense rows for which the kernels have such a form: powers of two, 256 to 4096 bytes.  (Rows that are
+// none spread by themselves: R-MAT 18 to 20, 320, 384, 768, 800, 1280 and 1536 bytes within 1 % either
+// way; rows of 128 bytes run at the rate of entries: 288 / 230 -> 299 / 229.)
+SPC3D_HD inline bool hot_row_width(uint64_t bytes)
+{
+    return bytes >= 256 && bytes <= 4096 && (bytes & (bytes - 1)) == 0;
+}
+// A launch must be long enough to repay the copy: 3 GiB of gathers in rows of 256 bytes, half of that in
+// wider ones.  SDDMM + SpMM in us without and with, 256 bytes: 1.0 GB 199 -> 202, 2.0 411 -> 409, 4.1
+// 877 -> 816; 512 bytes: 1.0 GB 195 -> 198, 2.0 407 -> 382; 1 KB: 2.0 GB 392 -> 368; 4 KB: 16 GB 4050 ->
+// 3376.
+inline bool hot_rows_pay(uint64_t nnz, uint64_t row_bytes)
+{
+    return hot_row_width(row_bytes) && nnz * row_bytes >= ((uint64_t)(row_bytes == 256 ? 6 : 3) << 29);
+}
+// weight[c]: entries in the hottest columns whose number is c mod kHotClasses.  They crowd when one of
+// the classes holds four times its share (natural R-MAT numbers: ten times; scrambled ones, which gain
+// nothing and would pay 5 us: up to twice).
+inline bool hot_rows_crowd(const uint64_t (&weight)[kHotClasses])
+{
+    uint64_t most = 0, total = 0;
+    for (uint64_t w : weight) {
+        most = w > most ? w : most;
+        total += w;
+    }
+    return total && most * kHotClasses >= 4 * total;
+}
+
 // Zero in any field selects the default.
 struct PlanOpts {
     uint32_t seg_max = 0;    // longest segment (default: by nnz and row_bytes, 16 .. 2048)

@@ -1,0 +1,124 @@
+"""Hot dense rows whose numbers crowd (a power of two apart, few low bits): calls that gather them
+from a copy side by side give the bits of calls that gather them where they lie."""
+import numpy as np
+import pytest
+
+from spcomm3d_amd import device
+from tests.test_parity_gpu import check_sddmm, check_spmm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with device.Context(0) as c:
+        yield c
+
+
+def pattern(m, n, nnz, order, crowded=True, seed=5):
+    """Half of the entries in every 32nd row and column (or in as many that do not crowd), skewed."""
+    rng = np.random.default_rng(seed)
+
+    def ids(size):
+        hot = (size // 32 * rng.random(nnz) ** 2).astype(np.uint32)
+        hot = hot * 32 if crowded else hot * 31 % np.uint32(size)
+        return np.where(rng.random(nnz) < 0.6, hot, rng.integers(0, size, nnz)).astype(np.uint32)
+
+    ii, jj = ids(m), ids(n)
+    o = np.lexsort((jj, ii)) if order == "sorted" else (
+        np.lexsort((ii, jj)) if order == "column" else rng.permutation(nnz))
+    return np.ascontiguousarray(ii[o]), np.ascontiguousarray(jj[o])
+
+
+# 256-byte rows need 12.6 M entries, wider ones 1.5 GiB of gathers
+CASES = [(np.float32, 64, 4000, 240000, 12700000, "sorted"), (np.float64, 64, 9000, 130000, 3200000, "sorted"),
+         (np.float64, 64, 100000, 130000, 3200000, "shuffled"), (np.float64, 64, 120000, 130000, 3200000, "column"),
+         (np.float32, 256, 3000, 70000, 1600000, "sorted"), (np.float64, 256, 3000, 36000, 800000, "sorted"),
+         (np.float64, 512, 2500, 18000, 400000, "sorted")]
+
+
+@pytest.mark.parametrize("dtype,k,m,n,nnz,order", CASES)
+def test_copied_rows_give_the_bits_of_rows_in_place(ctx, dtype, k, m, n, nnz, order):
+    ii, jj = pattern(m, n, nnz, order)
+    rng = np.random.default_rng(k)
+    w = np.dtype(dtype).itemsize
+    vv = rng.uniform(0, 1, nnz).astype(dtype)
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (m, n, m))
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k, seg_max=512)
+    # the same layout, planned for rows that are no power of two
+    plain = ctx.plan(m, n, ii, jj, vv, k_hint=k * 3 // 2, l2_hot_bytes=3 << 20, seg_max=512)
+    sums = plain.info.npartial_slots * (k // 2) * w
+    assert S.info.nsegments == plain.info.nsegments and S.info.hot_cols == plain.info.hot_cols > 0
+    assert S.info.device_bytes + sums >= plain.info.device_bytes + 4 * nnz
+    dA, dY, dC = ctx.panel_from(A), ctx.panel_from(Y0), ctx.vals(nnz, dtype)
+    raw = ctx.panel_from(np.vstack([np.full((1, k), np.nan, dtype), B, np.full((1, k), np.nan, dtype)]))
+    for off in (0, 16):  # the operand on whole lines, and 16 bytes past one
+        dB = device.Panel(ctx, n, k, dtype, dev=raw.device_ptr() + k * w - off)
+        if off:
+            dB.upload(B)
+        out = []
+        for plan in (plain, S):
+            dC.fill(-5.0)
+            dY.upload(Y0)
+            ctx.sddmm(plan, dA, dB, dC)
+            C = dC.download()
+            ctx.spmm(plan, dB, dY)
+            Y = dY.download()
+            ctx.sddmm_spmm(plan, dA, dB, dC, dY, chained=True)
+            out.append((C, Y, dC.download(), dY.download()))
+        for want, got in zip(*out):
+            assert np.array_equal(want, got)
+    check_sddmm(A, B, ii, jj, vv, out[1][0])
+    check_spmm(B, ii, jj, vv, Y0, out[1][1])
+
+
+def test_other_widths_recordings_and_the_call_without_allocations(ctx):
+    dtype, k, m, n, nnz, order = np.float64, 64, 3000, 130000, 3200000, "sorted"
+    ii, jj = pattern(m, n, nnz, order)
+    rng = np.random.default_rng(1)
+    vv = rng.uniform(0, 1, nnz).astype(dtype)
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k)
+    for kk in (32, 60, 128):  # narrower rows out of the same buffer, a width without, wider ones
+        A, B, Y0 = (rng.uniform(-1, 1, (r, kk)).astype(dtype) for r in (m, n, m))
+        dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(nnz, dtype)
+        ctx.sddmm(S, dA, dB, dC)
+        ctx.spmm(S, dB, dY)
+        C, Y = dC.download(), dY.download()
+        check_sddmm(A, B, ii, jj, vv, C)
+        check_spmm(B, ii, jj, vv, Y0, Y)
+        dC.fill(-5.0)
+        dY.upload(Y0)
+        ctx.capture_begin()
+        ctx.sddmm(S, dA, dB, dC)
+        ctx.spmm(S, dB, dY)
+        g = ctx.capture_end()
+        for _ in range(2):
+            dB.upload(B)
+            dY.upload(Y0)
+            g.launch()
+            ctx.sync()
+            assert np.array_equal(dC.download(), C) and np.array_equal(dY.download(), Y)
+        # what a replay gathers is the operand as it is then
+        dB.upload(B * 2)
+        dY.upload(Y0)
+        g.launch()
+        assert np.array_equal(dC.download(), C * 2)
+        check_spmm(B * 2, ii, jj, vv, Y0, dY.download())
+        g.close()
+        dB.upload(B)
+        dY.upload(Y0)
+        ctx.spmm_noalloc(S, dB, dY)
+        assert np.array_equal(dY.download(), Y)
+
+
+@pytest.mark.parametrize("k,nnz,crowded,taken", [(64, 3200000, True, True), (64, 3000000, True, False),
+                                                 (64, 3200000, False, False), (62, 3400000, True, False)])
+def test_where_the_line_lies(ctx, k, nnz, crowded, taken):
+    m, n = 9000, 130000
+    ii, jj = pattern(m, n, nnz, "sorted", crowded)
+    opts = dict(seg_max=512, dtype=np.float64)
+    S = ctx.plan(m, n, ii, jj, k_hint=k, l2_hot_bytes=k * 8 * 4096, **opts)
+    plain = ctx.plan(m, n, ii, jj, k_hint=96, l2_hot_bytes=96 * 8 * 4096, **opts)
+    assert S.info.hot_cols == plain.info.hot_cols > 0
+    more = S.info.device_bytes - (plain.info.device_bytes - plain.info.npartial_slots * (96 - k) * 8)
+    assert (more >= 4 * nnz) == taken
