@@ -8,7 +8,7 @@
 // row.  A dense row of K reals is nvec 16-byte vectors, covered by LPR lanes
 // holding VPL vectors each (nvec = LPR * VPL with the row stride a compile-time
 // constant, or nvec < LPR * VPL given at run time in the "ragged" variants, whose
-// spare lanes idle, or a row that ends inside its last vector in the "odd"
+// spare lanes load a vector and count nothing, or a row that ends inside its last vector in the "odd"
 // variants, or one shorter than a vector in the "thin" variant; rows over 4 KiB
 // run as 4 KiB column slices, one launch each); one wavefront works on 64 / LPR
 // segments at once and every global load instruction moves 64 x 16 B.  Segments
@@ -220,6 +220,47 @@ template <int LPR, int NB> __device__ __forceinline__ constexpr int writer_lane(
     return lane;
 }
 
+// bcast(v, lane): v of lane `lane` of the group.  A group of 64 is the wavefront: the value goes to a
+// scalar register, which spares the LDS permute, the address arithmetic of a gather (scalar base, the
+// lane's offset) and the registers that hold a batch's weights (R-MAT 18, fp64 K = 128, on top of the copied
+// hot rows: SDDMM 370 -> 357 us, SpMM 410 -> 369).  Smaller groups permute through LDS, the
+// lane in the instruction's offset: `first` (the byte address of the group's first lane) is made per
+// batch, or the compiler would add the lane to it outside the loop and keep all 16 sums in registers.
+template <int LPR> struct Bcast {
+    int first;
+    __device__ __forceinline__ Bcast() : first(0)
+    {
+        if constexpr (LPR < 64) {
+            first = (int)(threadIdx.x & 63u & ~(uint32_t)(LPR - 1)) * 4;
+            asm volatile("" : "+v"(first));
+        }
+    }
+    __device__ __forceinline__ uint32_t operator()(uint32_t v, int lane) const
+    {
+        if constexpr (LPR == 64)
+            return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+        else
+            return (uint32_t)__builtin_amdgcn_ds_bpermute(first + 4 * lane, (int)v);
+    }
+    __device__ __forceinline__ float operator()(float v, int lane) const
+    {
+        return __uint_as_float((*this)(__float_as_uint(v), lane));
+    }
+    __device__ __forceinline__ double operator()(double v, int lane) const
+    {
+        return __hiloint2double((int)(*this)((uint32_t)__double2hiint(v), lane),
+                                (int)(*this)((uint32_t)__double2loint(v), lane));
+    }
+};
+
+// A segment of the whole wavefront.
+__device__ __forceinline__ void uniform(u32x4 &sg)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        sg[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)sg[i]);
+}
+
 // Segment this lane group works on.  Segments are stored in chunks of kChunk;
 // with nq == 8, chunk v belongs to queue v % 8.  The hardware deals the
 // workgroups of a dispatch to the 8 XCDs round-robin by workgroup id, starting
@@ -308,7 +349,7 @@ first_cols_kernel(const Seg *__restrict__ segs, uint32_t n, const uint32_t *__re
 }
 
 // RG == 1 ("ragged"): a dense row is nvec 16-byte vectors with nvec < LPR * VPL,
-// given at run time; lanes whose vector index is >= nvec idle.  RG == 0: nvec ==
+// given at run time; lanes whose vector index is >= nvec load the last one and count nothing.  RG == 0: nvec ==
 // LPR * VPL exactly and the row stride is a compile-time constant.  RG == 2, 3: below.
 template <typename T, int LPR, int VPL, int RG>
 __device__ __forceinline__ const typename Vec<T>::type *row_ptr(const T *base, uint32_t row,
@@ -331,6 +372,19 @@ __device__ __forceinline__ bool lane_on(uint32_t sub, int v, uint32_t nvec)
 template <typename T> __device__ __forceinline__ typename Vec<T>::type loose_load(const char *p)
 {
     return *reinterpret_cast<const typename Vec<T>::loose *>(p);
+}
+// The vector `off` bytes past `at`, the same in every lane of the wavefront.  (Left to itself the compiler
+// adds the lane's offset to the loop-invariant base and does the rest in vector registers.)
+template <typename T, bool LOOSE>
+__device__ __forceinline__ typename Vec<T>::type load_beside(const char *at, uint32_t off)
+{
+    typedef __attribute__((address_space(1))) const char *Global;
+    Global p = (Global)at;
+    asm("" : "+s"(p));
+    if constexpr (LOOSE)
+        return *reinterpret_cast<__attribute__((address_space(1))) const typename Vec<T>::loose *>(p + off);
+    else
+        return *reinterpret_cast<__attribute__((address_space(1))) const typename Vec<T>::type *>(p + off);
 }
 template <typename T> __device__ __forceinline__ typename Vec<T>::type loose_load_nt(const char *p)
 {
@@ -379,6 +433,15 @@ template <typename T, int VPL, int RG> struct Odd {};
 template <typename T, int VPL> struct Odd<T, VPL, -1> {
     uint32_t at, hot_at; // of row 0 of the operand; of "row kHotRow", the buffer's first
 };
+// RG == 1: where this lane's vectors lie in a row, and which of them are its own; a lane past the row's
+// end loads the row's last vector and counts nothing: one select per dot product.  (Lanes switched off
+// around each load were a branch and four moves per row: R-MAT 18, fp64 K = 100, SDDMM / SpMM 315 / 338
+// -> 304 / 305 us with the scalar base of a 64-lane group; fp32 K = 96 150 / 141 -> 146 / 130; switched
+// off once for a whole batch: level, rows of 75 vectors 4 % slower.)
+template <typename T, int VPL> struct Odd<T, VPL, 1> {
+    uint32_t off[VPL];
+    bool on[VPL];
+};
 template <typename T, int VPL> struct Odd<T, VPL, 2> : OddLanes<T, VPL> {};
 template <typename T, int VPL> struct Odd<T, VPL, 3> : OddLanes<T, VPL> {};
 
@@ -390,6 +453,14 @@ __device__ __forceinline__ Odd<T, VPL, RG> odd_lanes(uint32_t sub, uint32_t K, u
     if constexpr (RG >= 2) {
         o.stride = stride;
         o.accum = accum != 0;
+    }
+    if constexpr (RG == 1) { // `K` carries nvec
+#pragma unroll
+        for (int v = 0; v < VPL; ++v) {
+            const uint32_t i = sub + (uint32_t)v * LPR;
+            o.on[v] = i < K;
+            o.off[v] = (i < K ? i : K - 1) * 16;
+        }
     }
     if constexpr (RG == 2) {
         const uint32_t bytes = K * (uint32_t)sizeof(T); // >= 16: see pick_shape
@@ -462,20 +533,47 @@ __device__ __forceinline__ void gather_row(typename Vec<T>::type (&out)[VPL], co
                                            const Odd<T, VPL, RG> &odd)
 {
     using V = typename Vec<T>::type;
-    if constexpr (RG >= 2) {
-        const char *r = odd_row<T, RG>(base, row, odd.stride);
+    // where the row starts, and the lane's vector v in it
+    const char *r = reinterpret_cast<const char *>(base);
+    if constexpr (RG >= 2)
+        r = odd_row<T, RG>(base, row, odd.stride);
+    else if constexpr (RG == 1)
+        r += (uint64_t)row * (nvec * 16);
+    else
+        r += (uint64_t)row * (RG == -1 ? kHotUnit : (uint32_t)(LPR * VPL * 16));
 #pragma unroll
-        for (int v = 0; v < VPL; ++v)
+    for (int v = 0; v < VPL; ++v) {
+        if constexpr (RG == 3) {
             out[v] = odd_load<T, RG, VPL>(r, v, nvec, odd);
-    } else {
-        const V *r;
-        if constexpr (RG == -1)
-            r = reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + (uint64_t)row * kHotUnit) + sub;
-        else
-            r = row_ptr<T, LPR, VPL, RG>(base, row, sub, nvec);
+        } else {
+            uint32_t off;
+            if constexpr (RG >= 1)
+                off = odd.off[v];
+            else
+                off = (sub + (uint32_t)v * LPR) * 16;
+            if constexpr (LPR == 64) // row is uniform: a scalar base, the lane's offset beside it
+                out[v] = load_beside<T, RG == 2>(r, off);
+            else if constexpr (RG == 2)
+                out[v] = loose_load<T>(r + off);
+            else
+                out[v] = *reinterpret_cast<const V *>(r + off);
+        }
+    }
+}
+
+// The lane's offsets in a row, made here and not outside the loop over batches, where the compiler would
+// widen them to 64 bits and not find a gather's scalar base with a 32-bit offset any more.
+template <typename T, int LPR, int VPL, int RG>
+__device__ __forceinline__ void pin_offsets(uint32_t &sub, Odd<T, VPL, RG> &odd)
+{
+    if constexpr (LPR == 64) {
+        if constexpr (RG == 1 || RG == 2) {
 #pragma unroll
-        for (int v = 0; v < VPL; ++v)
-            out[v] = lane_on<LPR, RG>(sub, v, nvec) ? r[v * LPR] : V{};
+            for (int v = 0; v < VPL; ++v)
+                asm volatile("" : "+v"(odd.off[v]));
+        } else {
+            asm volatile("" : "+v"(sub));
+        }
     }
 }
 
@@ -487,7 +585,8 @@ __device__ __forceinline__ T lane_dot(const typename Vec<T>::type (&a)[VPL],
 {
     T dot = (T)0;
 #pragma unroll
-    for (int v = 0; v < VPL; ++v)
+    for (int v = 0; v < VPL; ++v) {
+        const T before = dot;
 #pragma unroll
         for (int i = 0; i < Vec<T>::N; ++i) {
             if constexpr (RG >= 2)
@@ -495,6 +594,10 @@ __device__ __forceinline__ T lane_dot(const typename Vec<T>::type (&a)[VPL],
             else
                 dot += a[v][i] * b[v][i];
         }
+        if constexpr (RG == 1)
+            if (VPL == 1 || v > 0) // (rows of more than LPR vectors: every lane has its first)
+                dot = odd.on[v] ? dot : before;
+    }
     return dot;
 }
 
@@ -573,10 +676,22 @@ sddmm_batch_one(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type (&a
 
     static_assert(NG >= 1 && NG <= NB && (MK || NG == NB), "NG < NB only in a masked batch");
     V b[NG][VPL];
+    uint32_t at = sub;
+    Odd<T, VPL, RG> row = odd;
+    pin_offsets<T, LPR, VPL, RG>(at, row);
+    const Bcast<LPR> bcast;
+    // The second half of a wide batch makes its addresses when the first half's loads are under way:
+    // half the address registers (with the lane in the permutes' offset 100 -> 94 of them in SDDMM and
+    // 138 -> 122 in the one-pass kernel at fp64 K = 64: a wavefront more per SIMD).
+    uint32_t c[NG];
+#pragma unroll
+    for (int u = 0; u < NG; ++u)
+        c[u] = bcast(cme, u);
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
-        const uint32_t c = __shfl(cme, u, LPR);
-        gather_row<T, LPR, VPL, RG>(b[u], B, c, sub, nvec, odd);
+        gather_row<T, LPR, VPL, RG>(b[u], B, c[u], at, nvec, row);
+        if (LPR < 64 && NB >= 8 && u + 1 == NG / 2)
+            __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
 
@@ -610,7 +725,7 @@ sddmm_batch_one(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type (&a
 #pragma unroll
         for (int u = 0; u < NG; ++u) {
             const bool on = !MK || (uint32_t)u < n;
-            const T w = on ? __shfl(mine, writer_lane<LPR, NB>(u), LPR) : (T)0;
+            const T w = on ? bcast(mine, writer_lane<LPR, NB>(u)) : (T)0;
 #pragma unroll
             for (int v = 0; v < VPL; ++v)
                 acc[v] += (on ? b[u][v] : V{}) * w;
@@ -660,9 +775,10 @@ sddmm_batch_rounds(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type 
     }
 
     V b[NB][VPL];
+    const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = __shfl(cme[j / G], j % G, LPR);
+        const uint32_t c = bcast(cme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(b[j], B, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -696,7 +812,7 @@ sddmm_batch_rounds(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type 
 #pragma unroll
             for (int u = 0; u < G; ++u) {
                 const bool on = !MK || (uint32_t)(r * G + u) < n;
-                const T w = on ? __shfl(mine, writer_lane<LPR, G>(u), LPR) : (T)0;
+                const T w = on ? bcast(mine, writer_lane<LPR, G>(u)) : (T)0;
 #pragma unroll
                 for (int v = 0; v < VPL; ++v)
                     acc[v] += (on ? b[r * G + u][v] : V{}) * w;
@@ -794,7 +910,7 @@ sddmm_walk(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type (&acc)[V
 // FZ != 0: also Y[row,:] += sum of the segment's w_u * B[c_u,:] (partial-sum slot for
 // a cut row, as in spmm_seg_kernel); Y and partial are unused otherwise.
 template <typename T, int LPR, int VPL, int UB, int RG, bool WIDE, int FZ>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock, 1)
 sddmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32_t rot,
                  const uint32_t *__restrict__ col, const uint32_t *__restrict__ perm,
                  const T *__restrict__ sval, const T *__restrict__ A, const T *__restrict__ B,
@@ -812,9 +928,11 @@ sddmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint3
     ex.stream_c = (flags & kStoreStream) != 0;
     ex.stage = stage;
     ex.stage_from = stage_from;
-    const u32x4 sg = nt_load(reinterpret_cast<const u32x4 *>(segs) + sid); // row, start, len, slot
+    u32x4 sg = nt_load(reinterpret_cast<const u32x4 *>(segs) + sid); // row, start, len, slot
     if (sg[2] == 0)
         return;
+    if constexpr (LPR == 64)
+        uniform(sg);
     if (flags & kStoreSegBase) { // one position per segment instead of one per entry
         ex.shift = nt_load(perm + sg[1]) - sg[1];
         perm = nullptr;
@@ -875,17 +993,18 @@ sddmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint3
 // Column of entry j < kFirstCols of a short segment out of the indices loaded ahead:
 // lane u of the group holds that of entry u in FC[0] (groups of 4 lanes: of entries u
 // and 4 + u in FC[0] and FC[1]).
-template <int LPR> __device__ __forceinline__ uint32_t first_col(const uint32_t (&FC)[2], uint32_t j)
+template <int LPR>
+__device__ __forceinline__ uint32_t first_col(const Bcast<LPR> &bcast, const uint32_t (&FC)[2], uint32_t j)
 {
     if constexpr (LPR >= (int)kFirstCols)
-        return __shfl(FC[0], j, LPR);
+        return bcast(FC[0], (int)j);
     else
     {
         // Values, not elements: a choice between two array elements is a choice of address, for
         // which the compiler moves the array to LDS and reads the dispatch packet to find the
         // thread's place in it (9 us per launch).
         const uint32_t a = FC[0], b = FC[1];
-        return __shfl((j & LPR) ? b : a, j & (LPR - 1), LPR);
+        return bcast((j & LPR) ? b : a, (int)(j & (LPR - 1)));
     }
 }
 
@@ -910,16 +1029,31 @@ spmm_batch_one(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict__ c
 
     V x[NB][VPL];
     T av[NB];
+    uint32_t at = sub;
+    Odd<T, VPL, RG> row = odd;
+    pin_offsets<T, LPR, VPL, RG>(at, row);
+    const Bcast<LPR> bcast;
+    uint32_t c[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+        c[u] = PRE ? first_col<LPR>(bcast, ex.first, off + u) : bcast(cme, u);
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
-        const uint32_t c = PRE ? first_col<LPR>(ex.first, off + u) : __shfl(cme, u, LPR);
-        av[u] = __shfl(vme, u, LPR);
-        gather_row<T, LPR, VPL, RG>(x[u], X, c, sub, nvec, odd);
+        gather_row<T, LPR, VPL, RG>(x[u], X, c[u], at, nvec, row);
+        if (LPR < 64 && NB >= 8 && u + 1 == NB / 2)
+            __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
     // Entries are added in kernel order.
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
+        // The weights four entries ahead of their use, four at a time: all of them at once held 32
+        // registers beside the gathers at fp64 (136 -> 98 with the rest: 4 wavefronts per SIMD, not 3;
+        // R-MAT 18, K = 64: 188 -> 174 us).
+        if (u % 4 == 0)
+#pragma unroll
+            for (int w = u ? u + 4 : 0; w < u + 8 && w < NB; ++w)
+                av[w] = bcast(vme, w);
         const bool on = !MK || (uint32_t)u < n;
         const T a = on ? av[u] : (T)0;
 #pragma unroll
@@ -954,10 +1088,11 @@ spmm_batch_rounds(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict_
 
     V x[NB][VPL];
     T av[NB];
+    const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = __shfl(cme[j / G], j % G, LPR);
-        av[j] = __shfl(vme[j / G], j % G, LPR);
+        const uint32_t c = bcast(cme[j / G], j % G);
+        av[j] = bcast(vme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(x[j], X, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -1077,9 +1212,11 @@ spmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint32
     if (sid >= nseg)
         return;
     Ahead ex = load_first_cols<LPR, WIDE>(first_cols, sid, sub);
-    const u32x4 sg = nt_load(reinterpret_cast<const u32x4 *>(segs) + sid); // row, start, len, slot
+    u32x4 sg = nt_load(reinterpret_cast<const u32x4 *>(segs) + sid); // row, start, len, slot
     if (sg[2] == 0)
         return;
+    if constexpr (LPR == 64)
+        uniform(sg);
     const bool whole = sg[3] == kWholeRow;
     Odd<T, VPL, RG> odd = odd_lanes<T, LPR, VPL, RG>(sub, nvec, stride, 0u);
     if constexpr (RG == -1)
@@ -2018,11 +2155,9 @@ Shape pick_shape(size_t elem, uint32_t K)
             return {lpr, (int)vpl, 0, nvec};
         break;
     }
-    // Narrow rows that leave lanes idle also run the odd variant: its idle lanes load a
-    // vector of the row and count nothing, where the ragged variant's skip the load
-    // under a branch (measured on R-MAT 20, fp32 K = 4: SDDMM 644 -> 557 us, SpMM
-    // 467 -> 339 us; K = 20: 510 -> 446 and 404 -> 324; level at 9 to 16 vectors, and
-    // from 17 vectors on the selects in the dot product cost SDDMM 2 to 4 %).
+    // Narrow rows that leave lanes idle also run the odd variant, which loads whole vectors at
+    // element alignment; from 17 vectors on its selects per element would cost SDDMM 2 to 4 %
+    // over the ragged variant's one per dot product.
     const int mode = (odd || nvec <= 16) ? 2 : 1;
     const uint32_t arg = mode == 2 ? K : nvec;
     if (nvec > 128)
