@@ -432,6 +432,7 @@ inline DevPlanView view_of(const spc3d_plan *p)
     v.partial = p->partial;
     v.first_cols = p->first_cols;
     v.nnz = p->info.nnz;
+    v.cols_touched = p->info.cols_touched;
     v.seg_base = p->store.consecutive;
     if (p->hot_rows) {
         v.hot_cols = p->hot_cols;

@@ -27,6 +27,7 @@ struct DevPlanView {
     // the long ones (launch_first_cols); read by the short-segment launch
     const uint32_t *first_cols = nullptr;
     uint64_t nnz = 0;
+    uint32_t cols_touched = 0;        // columns with entries
     bool stream_c = false;            // SDDMM: streaming stores also at permuted positions
     // SDDMM results whose position in `perm` is stage_from or more go to place (position -
     // stage_from) of `stage` (see build_store_staging in plan_device.h); launch_unstage_pairs

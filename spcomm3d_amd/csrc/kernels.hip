@@ -2202,10 +2202,12 @@ constexpr uint32_t kOneLaunchSegments = 196608;
 // gathers instead of two to four.  Uniform rows of 12 to 15, fp32 K = 8: SDDMM 125 -> 116 us, SpMM 102
 // -> 99; K = 64: 404 -> 388 and 442 -> 418; rows of 11 are level or better in the short one, and so are
 // dense rows that leave lanes idle (15 entries, fp32 K = 134: 71 us together in the short one, 74).
+// A few short ones left over from whole chunks of long ones go with those (500 k rows of 16, fp64 K = 64:
+// the second launch and its fork cost 12 us of 608).
 inline void split_launches(const DevPlanView &P, bool whole_lanes, uint32_t &nl, uint32_t &ns)
 {
     nl = P.nseg_long, ns = P.nseg - P.nseg_long;
-    if (nl ? P.nseg <= kOneLaunchSegments : whole_lanes && P.nnz >= (uint64_t)12 * P.nseg)
+    if (nl ? P.nseg <= kOneLaunchSegments || ns <= nl / 64 : whole_lanes && P.nnz >= (uint64_t)12 * P.nseg)
         nl = P.nseg, ns = 0;
 }
 
@@ -2228,6 +2230,49 @@ inline hipError_t join_aux(const Streams &S)
     return hipStreamSynchronize(S.aux);
 }
 
+enum LaunchOf { kSddmm, kOnePass, kSpmm };
+
+// Dynamic LDS that keeps the workgroups of a segment launch down to fewer per CU than its registers
+// allow (4 to 8), or 0.  Where nearly every gather misses the L2s and a launch has more than enough of
+// them in flight, fewer at once are served faster: unskewed columns (no slices), a panel over the L2s (64
+// MiB) that the Infinity Cache mostly holds (320), segments of one kind, four rounds of wavefronts and
+// more, at least three lanes in four busy.  Uniform rows of 4 to 48 entries over 60 k to 3 M columns,
+// speed of SDDMM / SpMM / one-pass against all wavefronts:
+//  - the wide launch at 3 workgroups, from 16 entries on 1.00 .. 1.07 / 1.01 .. 1.05, one-pass from 32 on 1.00
+//    .. 1.06 (12 entries: 0.88 / 0.90 / 0.82; one-pass at 20: 0.97); rows that leave lanes idle from 32 on (20
+//    entries: 0.94 / 0.99 / 0.92);
+//  - the short one from 6 entries on: SpMM at 5 1.01 .. 1.07 (5 entries: 0.93); SDDMM at 5 1.00 .. 1.07, with idle
+//    lanes 6, 0.99 .. 1.02; one-pass at 6 0.99 .. 1.05, a row to a wavefront 5, 1.02 .. 1.06;
+//  - the short one at 4 and 5 entries, SpMM over dense rows of 512 bytes and more, whatever the panel: 7, 1.01
+//    .. 1.04 from 65,536 wavefronts on (half of them: 0.99).
+// Panels in the caches or far beyond them want every wavefront (30 k rows of 40 over 30 k columns 0.89 /
+// 0.90 / 0.86 at 3; 300 k of 20 over 1 M columns, 512-byte rows, 0.92 / 0.97 / 0.87), and so do half-empty groups
+// (1 M rows of 8, fp32 K = 135, at 5: 0.91 / 0.84).
+template <typename T, int LPR, int VPL, int RG>
+inline uint32_t crowding_lds(const DevPlanView &P, bool wide, uint32_t nseg, LaunchOf what, uint32_t nvec)
+{
+    constexpr uint64_t kFull = (uint64_t)LPR * VPL * 16;
+    const uint64_t bytes = RG <= 0 ? kFull : (uint64_t)nvec * (RG == 1 ? 16 : sizeof(T));
+    const uint64_t waves = (uint64_t)nseg * LPR / 64, panel = P.cols_touched * bytes;
+    if (P.nqueues != 1 || nseg != P.nseg || waves < 16384 || panel < ((uint64_t)64 << 20) ||
+        bytes * 4 < kFull * 3)
+        return 0;
+    const bool cached = panel <= ((uint64_t)320 << 20);
+    uint32_t blocks = 0; // per CU
+    if (wide) {
+        if (cached && nseg - P.nseg_long <= nseg / 64 &&
+            P.nnz >= (uint64_t)(RG == 1 || what == kOnePass ? 32 : 16) * nseg)
+            blocks = 3;
+    } else if (P.nnz >= (uint64_t)6 * nseg) {
+        if (cached)
+            blocks = what == kSpmm ? 5 : (RG <= 0 && (what == kSddmm || LPR == 64) ? 5 : 6);
+    } else if (what == kSpmm && RG <= 0 && kFull >= 512 && P.nnz >= (uint64_t)4 * nseg && waves >= 65536) {
+        blocks = 7;
+    }
+    constexpr uint32_t kLds = 160u << 10; // of a CU
+    return blocks ? kLds / blocks & ~1023u : 0;
+}
+
 inline uint32_t store_flags(const DevPlanView &P)
 {
     return (P.stream_c ? kStoreStream : 0u) | (P.perm && P.seg_base ? kStoreSegBase : 0u);
@@ -2240,16 +2285,19 @@ hipError_t run_sddmm(const DevPlanView &P, const T *A, const T *B, T *C, T *Y, c
     uint32_t nl, ns;
     split_launches(P, RG <= 0, nl, ns);
     const bool both = nl && ns && fork_aux(S);
+    constexpr LaunchOf kind = FZ ? kOnePass : kSddmm;
     if (nl)
         hipLaunchKernelGGL((sddmm_seg_kernel<T, LPR, VPL, UB, RG, true, FZ>),
-                           dim3(blocks_for_groups(nl, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
+                           dim3(blocks_for_groups(nl, P.nqueues, 64 / LPR)), dim3(kBlock),
+                           (crowding_lds<T, LPR, VPL, RG>(P, true, nl, kind, nvec)),
                            S.main, P.segs, nl, P.nqueues, 0u, P.col, P.perm, (const T *)P.sval,
                            A, B, C, Y, (T *)P.partial, nvec, stride ? stride : nvec, accum,
                            (const uint32_t *)nullptr, store_flags(P), (T *)P.stage,
                            P.stage_from, P.ref_at, P.hot_at);
     if (ns)
         hipLaunchKernelGGL((sddmm_seg_kernel<T, LPR, VPL, US, RG, false, FZ>),
-                           dim3(blocks_for_groups(ns, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
+                           dim3(blocks_for_groups(ns, P.nqueues, 64 / LPR)), dim3(kBlock),
+                           (crowding_lds<T, LPR, VPL, RG>(P, false, ns, kind, nvec)),
                            both ? S.aux : S.main, P.segs + nl, ns, P.nqueues,
                            both ? S.aux_rot : 0u, P.col, P.perm, (const T *)P.sval, A, B, C, Y,
                            (T *)P.partial, nvec, stride ? stride : nvec, accum, P.first_cols,
@@ -2268,13 +2316,15 @@ hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, ui
     const bool both = nl && ns && fork_aux(S);
     if (nl)
         hipLaunchKernelGGL((spmm_seg_kernel<T, LPR, VPL, UB, RG, true>),
-                           dim3(blocks_for_groups(nl, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
+                           dim3(blocks_for_groups(nl, P.nqueues, 64 / LPR)), dim3(kBlock),
+                           (crowding_lds<T, LPR, VPL, RG>(P, true, nl, kSpmm, nvec)),
                            S.main, P.segs, nl, P.nqueues, 0u, P.col, (const T *)P.sval, X, Y,
                            (T *)P.partial + slice_off, nvec, stride ? stride : nvec, pstride,
                            (const uint32_t *)nullptr, P.ref_at, P.hot_at);
     if (ns)
         hipLaunchKernelGGL((spmm_seg_kernel<T, LPR, VPL, US, RG, false>),
-                           dim3(blocks_for_groups(ns, P.nqueues, 64 / LPR)), dim3(kBlock), 0,
+                           dim3(blocks_for_groups(ns, P.nqueues, 64 / LPR)), dim3(kBlock),
+                           (crowding_lds<T, LPR, VPL, RG>(P, false, ns, kSpmm, nvec)),
                            both ? S.aux : S.main, P.segs + nl, ns, P.nqueues,
                            both ? S.aux_rot : 0u, P.col, (const T *)P.sval, X, Y,
                            (T *)P.partial + slice_off, nvec, stride ? stride : nvec, pstride,

@@ -50,3 +50,18 @@ def test_uniform_short_rows(ctx, dtype, k, length):
     A, B, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (m, n, m))
     check_sddmm(A, B, ii, jj, vv, gpu_sddmm(ctx, m, n, ii, jj, vv, A, B))
     check_spmm(B, ii, jj, vv, Y0, gpu_spmm(ctx, m, n, ii, jj, vv, B, Y0))
+
+
+# even rows over a panel of 64 MiB, a workgroup either side of the launch that is kept to fewer
+# workgroups per CU, and with a chunk of segments left over
+@pytest.mark.parametrize("dtype,k", [(np.float64, 64), (np.float32, 127)])
+@pytest.mark.parametrize("m,length", [(32767, 16), (32768, 16), (32771, 17), (32768, 6), (200001, 16)])
+def test_even_rows_over_a_large_panel(ctx, dtype, k, m, length):
+    n = 132000
+    ii, jj = rows_of([length] * m, n, length)
+    jj[:n] = np.arange(n)  # every column is touched
+    rng = np.random.default_rng(m)
+    vv = rng.uniform(0, 1, ii.size).astype(dtype)
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)).astype(dtype) for r in (m, n, m))
+    check_sddmm(A, B, ii, jj, vv, gpu_sddmm(ctx, m, n, ii, jj, vv, A, B))
+    check_spmm(B, ii, jj, vv, Y0, gpu_spmm(ctx, m, n, ii, jj, vv, B, Y0))
