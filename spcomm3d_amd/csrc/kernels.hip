@@ -2254,14 +2254,14 @@ inline uint32_t crowding_lds(const DevPlanView &P, bool wide, uint32_t nseg, Lau
     constexpr uint64_t kFull = (uint64_t)LPR * VPL * 16;
     const uint64_t bytes = RG <= 0 ? kFull : (uint64_t)nvec * (RG == 1 ? 16 : sizeof(T));
     const uint64_t waves = (uint64_t)nseg * LPR / 64, panel = P.cols_touched * bytes;
-    if (P.nqueues != 1 || nseg != P.nseg || waves < 16384 || panel < ((uint64_t)64 << 20) ||
-        bytes * 4 < kFull * 3)
+    const uint64_t least = (uint64_t)(wide ? 24 : 64) << 20;
+    if (P.nqueues != 1 || nseg != P.nseg || waves < 16384 || panel < least || bytes * 4 < kFull * 3)
         return 0;
     const bool cached = panel <= ((uint64_t)320 << 20);
     uint32_t blocks = 0; // per CU
     if (wide) {
         if (cached && nseg - P.nseg_long <= nseg / 64 &&
-            P.nnz >= (uint64_t)(RG == 1 || what == kOnePass ? 32 : 16) * nseg)
+            P.nnz >= (uint64_t)(RG == 1 && LPR < 64 ? 32 : (RG == 1 || what == kOnePass ? 24 : 16)) * nseg)
             blocks = 3;
     } else if (P.nnz >= (uint64_t)6 * nseg) {
         if (cached)
