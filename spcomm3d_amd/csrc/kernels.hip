@@ -1335,11 +1335,15 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // what an L2 sees, and the gathers hit.
 //
 // The plan (build_sweep in plan_device.h) orders a tile's entries by block, inside a block by
-// row; ptr[tile * nb + b] .. [.. + 1) is the range of block b.  Both kernels cut that range
-// into batches of UB entries and deal them to the G lane groups of the workgroup, which
-// leaves the lane groups within one batch of each other in every block.
-// SDDMM, where any lane group can take any entry: batch i to lane group i % G.
-// SpMM: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum of
+// row; ptr[tile * nb + b] .. [.. + 1) is the range of block b.
+// SDDMM, where any lane group can take any entry, takes the tile's entries as one stream: batch i of UB
+// entries goes to lane group i % G, across the blocks' boundaries, with a barrier per round of G batches.
+// (Dealt block by block a round was filled to 6.7 batches of 7 at best, 2.3 of 3 for shorter rows; and with a
+// barrier per block instead of per round the wavefronts drift and gathers miss: 2 M rows over 500 k columns, 560 M
+// entries, fp32 K = 128: block by block 19.7 ms for the call, as a stream with a barrier per block 19.2,
+// per half block 18.3, per round 17.3.  Gathers as byte offsets in 32 bits, three instructions fewer each:
+// between 6 % faster, 256- and 1024-byte rows, and 5 % slower here; not kept.)
+// SpMM cuts every block's range into batches of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum of
 // a row's run of entries is kept in registers and added to the row's accumulator in LDS when
 // the run ends.  A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
@@ -1432,7 +1436,6 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
     __shared__ V tile_a[kSweepRowBytes / 16];
-    __shared__ uint32_t lptr[kSweepPtrWords];
     const uint32_t tile = tile0 + blockIdx.x;
     const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
     const SweepLane<T, LPR, ANY> lane(sub, K);
@@ -1448,14 +1451,16 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
         }
         tile_a[i] = v;
     }
-    for (uint32_t i = threadIdx.x; i < nb + 1; i += kSweepBlock)
-        lptr[i] = ptr[(uint64_t)tile * nb + i];
+    const uint32_t lo = ptr[(uint64_t)tile * nb], hi = ptr[(uint64_t)tile * nb + nb];
+    const uint32_t rounds = (hi - lo + G * UB - 1) / (G * UB); // of a batch per lane group
     __syncthreads();
     const uint32_t uo = entry_of<LPR, UB>(sub);
     const bool wlane = is_writer<LPR, UB>(sub);
-    auto fetch = [&](uint32_t q, uint32_t qhi) {
+    auto fetch = [&](uint32_t q) {
         SweepIdx<T> x;
-        x.n = qhi - q < (uint32_t)UB ? qhi - q : (uint32_t)UB;
+        if (q >= hi)
+            return x;
+        x.n = hi - q < (uint32_t)UB ? hi - q : (uint32_t)UB;
         uint32_t e = sub & (UB - 1);
         e = e < x.n ? e : x.n - 1;
         x.col = nt_load(col + q + e);
@@ -1465,56 +1470,33 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
             x.pos = (wlane && uo < x.n) ? nt_load(pos + q + uo) : 0u;
         return x;
     };
-    // batch i of a block's range belongs to lane group i % G
-    uint32_t p = lptr[0] + grp * UB, hi = lptr[1];
-    SweepIdx<T> cur;
-    if (p < hi)
-        cur = fetch(p, hi);
-    for (uint32_t b = 0; b < nb; ++b) {
-        uint32_t p_nb = 0, hi_nb = 0; // the next block's range
-        if (b + 1 < nb) {
-            p_nb = lptr[b + 1] + grp * UB;
-            hi_nb = lptr[b + 2];
-        }
-        const bool had = p < hi;
-        while (p < hi) {
-            // the next batch's indices (this block's, or the first of the next block) before
-            // this batch's gathers
-            const uint32_t np = p + G * UB;
-            SweepIdx<T> nxt;
-            if (np < hi)
-                nxt = fetch(np, hi);
-            else if (p_nb < hi_nb)
-                nxt = fetch(p_nb, hi_nb);
-            V bv[UB];
+    uint32_t p = lo + grp * UB;
+    SweepIdx<T> cur = fetch(p);
+    for (uint32_t r = 0; r < rounds; ++r, p += G * UB) {
+        if (r)
+            __syncthreads();
+        if (p >= hi) // (the last round)
+            continue;
+        const SweepIdx<T> nxt = fetch(p + G * UB); // the next batch's indices before this one's gathers
+        const Bcast<LPR> bcast;
+        V bv[UB];
 #pragma unroll
-            for (int u = 0; u < UB; ++u) {
-                const uint32_t c = __shfl(cur.col, u, LPR);
-                bv[u] = lane.load(B, c);
-            }
-            __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
-            T part[UB];
+        for (int u = 0; u < UB; ++u)
+            bv[u] = lane.load(B, bcast(cur.col, u));
+        __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
+        T part[UB];
 #pragma unroll
-            for (int u = 0; u < UB; ++u) {
-                const uint32_t l = __shfl(cur.row, u, LPR);
-                part[u] = lane.dot(tile_a[l * LPR + sub], bv[u]);
-            }
-            group_reduce<T, LPR, UB>(part, sub);
-            if (wlane && uo < cur.n) {
-                if (pos) // the caller's positions: pieces of lines that this workgroup's next
-                         // blocks complete, so plain stores, which the L2 merges
-                    C[cur.pos] = part[0] * cur.val;
-                else
-                    nt_store(part[0] * cur.val, C + p + uo); // kernel order: whole lines, streaming
-            }
-            p = np;
-            cur = nxt;
+        for (int u = 0; u < UB; ++u)
+            part[u] = lane.dot(tile_a[bcast(cur.row, u) * LPR + sub], bv[u]);
+        group_reduce<T, LPR, UB>(part, sub);
+        if (wlane && uo < cur.n) {
+            if (pos) // the caller's positions: pieces of lines that this workgroup's next
+                     // blocks complete, so plain stores, which the L2 merges
+                C[cur.pos] = part[0] * cur.val;
+            else
+                nt_store(part[0] * cur.val, C + p + uo); // kernel order: whole lines, streaming
         }
-        p = p_nb;
-        hi = hi_nb;
-        if (!had && p < hi) // nothing of this group in block b: the next batch was not asked for
-            cur = fetch(p, hi);
-        __syncthreads(); // every lane group leaves block b before any enters block b + 1
+        cur = nxt;
     }
 }
 
@@ -1549,6 +1531,8 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         x.col = nt_load(col + q + e);
         x.row = nt_load(lrow + q + e);
         x.val = vpos ? sval[nt_load(vpos + q + e)] : nt_load(sval + q + e);
+        if ((sub & (UB - 1)) >= x.n)
+            x.val = (T)0;
         return x;
     };
     // this lane group's chunk of block b: ceil(nbat / G) batches each, from lane group 0 on, so
@@ -1592,26 +1576,50 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
                 nxt = fetch(np, hi);
             else if (p_nb < hi_nb)
                 nxt = fetch(p_nb, hi_nb);
+            const Bcast<LPR> bcast;
             V xv[UB];
 #pragma unroll
-            for (int u = 0; u < UB; ++u) {
-                const uint32_t c = __shfl(cur.col, u, LPR);
-                xv[u] = lane.load(X, c);
-            }
+            for (int u = 0; u < UB; ++u)
+                xv[u] = lane.load(X, bcast(cur.col, u));
             __builtin_amdgcn_sched_barrier(0);
+            // where a row begins: lane u of a group holds entry u and sees entry u - 1 (lane 0 the row
+            // that is being summed); the wavefront steps aside only where one of its groups needs it.
+            // (A broadcast of the row and a comparison per entry instead: 128 registers and spills of 20
+            // bytes against 112 and none; 300 k x 100 k, fp64 K = 128 SpMM 2432 -> 2284 us, 512-byte rows
+            // level.  A barrier per batch, as in SDDMM, cost 12 %: the groups' runs differ.)
+            const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(
+                (int)row, (int)cur.row, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
+            const uint64_t begins = __ballot(cur.row != before);
+            const uint64_t past = __ballot((sub & (UB - 1)) >= cur.n); // the batch has ended
+            const uint32_t mine = (uint32_t)(begins >> (threadIdx.x & 63u & ~(uint32_t)(LPR - 1)));
+            uint32_t any = 0, any_past = 0;
+#pragma unroll
+            for (int g = 0; g < 64 / LPR; ++g) {
+                any |= (uint32_t)(begins >> (g * LPR));
+                any_past |= (uint32_t)(past >> (g * LPR));
+            }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
-                const uint32_t l = __shfl(cur.row, u, LPR);
-                const T a = (uint32_t)u < cur.n ? __shfl(cur.val, u, LPR) : (T)0;
-                if (l != row) {
-                    if (row != kNone) {
-                        flush();
-                        first = false;
+                if (any >> u & 1) {
+                    const uint32_t l = bcast(cur.row, u);
+                    bool here = true; // the lanes of the groups in which entry u begins a row
+                    if constexpr (LPR == 32)
+                        here = __builtin_amdgcn_inverse_ballot_w64((begins >> u & 1 ? 0xFFFFFFFFull : 0) |
+                                                                   (begins >> (32 + u) & 1 ? ~0ull << 32 : 0));
+                    else if constexpr (LPR < 32)
+                        here = mine >> u & 1;
+                    if (here) {
+                        if (row != kNone) {
+                            flush();
+                            first = false;
+                        }
+                        acc = V{};
+                        row = l;
                     }
-                    acc = V{};
-                    row = l;
                 }
-                acc += xv[u] * a;
+                if (any_past >> u & 1)
+                    xv[u] = (uint32_t)u < cur.n ? xv[u] : V{};
+                acc += xv[u] * bcast(cur.val, u);
             }
             p = np;
             cur = nxt;
@@ -2235,12 +2243,12 @@ enum LaunchOf { kSddmm, kOnePass, kSpmm };
 // Dynamic LDS that keeps the workgroups of a segment launch down to fewer per CU than its registers
 // allow (4 to 8), or 0.  Where nearly every gather misses the L2s and a launch has more than enough of
 // them in flight, fewer at once are served faster: unskewed columns (no slices), a panel over the L2s (64
-// MiB) that the Infinity Cache mostly holds (320), segments of one kind, four rounds of wavefronts and
+// MiB; 24 for the wide launch) that the Infinity Cache mostly holds (320), segments of one kind, four rounds of wavefronts and
 // more, at least three lanes in four busy.  Uniform rows of 4 to 48 entries over 60 k to 3 M columns,
 // speed of SDDMM / SpMM / one-pass against all wavefronts:
-//  - the wide launch at 3 workgroups, from 16 entries on 1.00 .. 1.07 / 1.01 .. 1.05, one-pass from 32 on 1.00
-//    .. 1.06 (12 entries: 0.88 / 0.90 / 0.82; one-pass at 20: 0.97); rows that leave lanes idle from 32 on (20
-//    entries: 0.94 / 0.99 / 0.92);
+//  - the wide launch at 3 workgroups, from 16 entries on 1.00 .. 1.07 / 1.01 .. 1.05, one-pass from 24 on 1.00
+//    .. 1.06 (12 entries: 0.88 / 0.90 / 0.82; one-pass at 20: 0.97); rows that leave lanes idle from 24 on, in
+//    groups of 32 lanes from 32 on (20 entries: 0.94 / 0.99 / 0.92);
 //  - the short one from 6 entries on: SpMM at 5 1.01 .. 1.07 (5 entries: 0.93); SDDMM at 5 1.00 .. 1.07, with idle
 //    lanes 6, 0.99 .. 1.02; one-pass at 6 0.99 .. 1.05, a row to a wavefront 5, 1.02 .. 1.06;
 //  - the short one at 4 and 5 entries, SpMM over dense rows of 512 bytes and more, whatever the panel: 7, 1.01
