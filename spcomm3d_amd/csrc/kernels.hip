@@ -1330,9 +1330,9 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // of A rows (SDDMM, read-only) or of Y accumulators (SpMM), one workgroup per CU, one launch
 // per "generation" of as many tiles as the GPU has CUs.  The workgroups of a generation start
 // together and meet the same amount of work in every block, so they walk the blocks in step,
-// and a barrier per block keeps the wavefronts of one workgroup in step too (without it the
-// oldest wavefronts run ahead by tens of blocks): at any time one block of dense rows is
-// what an L2 sees, and the gathers hit.
+// and barriers keep the wavefronts of one workgroup in step too (without them the oldest
+// wavefronts run ahead by tens of blocks): at any time one block of dense rows is what an L2
+// sees, and the gathers hit.
 //
 // The plan (build_sweep in plan_device.h) orders a tile's entries by block, inside a block by
 // row; ptr[tile * nb + b] .. [.. + 1) is the range of block b.
@@ -1343,9 +1343,9 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // entries, fp32 K = 128: block by block 19.7 ms for the call, as a stream with a barrier per block 19.2,
 // per half block 18.3, per round 17.3.  Gathers as byte offsets in 32 bits, three instructions fewer each:
 // between 6 % faster, 256- and 1024-byte rows, and 5 % slower here; not kept.)
-// SpMM cuts every block's range into batches of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum of
-// a row's run of entries is kept in registers and added to the row's accumulator in LDS when
-// the run ends.  A row's entries are contiguous, so a row is shared between lane groups only
+// SpMM, with a barrier per block (one per batch measured 12 % slower), cuts every block's range into batches
+// of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum
+// of a row's run of entries is kept in registers and added to the row's accumulator in LDS when the run ends.  A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
 // is added to the accumulator by that lane group), the later parts each BEGIN a chunk.  The
 // first run of every chunk therefore goes to an edge slot of its lane group instead, and
