@@ -79,6 +79,7 @@ static int resolve_opts(int dtype, const spc3d_plan_opts *o, PlanOpts &out)
     const uint64_t bytes = z.l2_hot_bytes ? z.l2_hot_bytes : 2u << 20;
     out.hot_cols = (uint32_t)(bytes / (k * elem_size(dtype)));
     out.row_bytes = (uint32_t)std::min<uint64_t>((uint64_t)z.k_hint * elem_size(dtype), 1u << 30);
+    out.hot_row_bytes = (uint32_t)std::min<uint64_t>(k * elem_size(dtype), 1u << 30);
     return SPC3D_OK;
 }
 
@@ -394,7 +395,7 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
     if (!rc)
         rc = add_store_staging(q, so);
     if (!rc)
-        rc = add_hot_rows(q, po.row_bytes / (uint32_t)elem_size(p->dtype));
+        rc = add_hot_rows(q, po.hot_row_bytes / (uint32_t)elem_size(p->dtype));
     if (rc || (q->perm && !q->store.consecutive)) { // no better than what there is
         if (q) {
             const std::string keep = g_err;

@@ -1130,7 +1130,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         TRY(sort_pairs<uint32_t>(tmp, coldeg.p, deg_sorted.p, colid.p, order.p, ncols,
                                  bits_for(maxcdeg), true, st, err));
         LAUNCH_SMALL(sum_first_k, htot, deg_sorted.p, htot, &dC.p->covered);
-        const bool hot_form = !opts.one_call && ncols <= kHotRow && hot_rows_pay(nnz, opts.row_bytes);
+        const bool hot_form = !opts.one_call && ncols <= kHotRow && hot_rows_pay(nnz, opts.hot_row_bytes);
         const uint32_t nhot = (uint32_t)std::min<uint64_t>(kHotRows, htot);
         if (hot_form)
             hipLaunchKernelGGL(hot_weight_k, dim3(1), dim3(kTB), 0, st, order.p, deg_sorted.p, nhot,

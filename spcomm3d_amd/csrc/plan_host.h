@@ -82,6 +82,7 @@ inline bool hot_rows_crowd(const uint64_t (&weight)[kHotClasses])
 struct PlanOpts {
     uint32_t seg_max = 0;    // longest segment (default: by nnz and row_bytes, 16 .. 2048)
     uint32_t row_bytes = 0;  // bytes of the dense rows the plan will mostly run with (0: unknown)
+    uint32_t hot_row_bytes = 0; // the same for hot rows that crowd (64 columns where the caller names no width)
     uint32_t xcd_slices = 0; // 8 (default): hot columns are dealt to the 8 XCD L2s; 1: off
     uint32_t hot_cols = 0;   // slicing: dense rows one L2 is expected to keep
     uint32_t hub_min = 0;    // slicing: rows with at least this many entries are cut by slice (default 128)

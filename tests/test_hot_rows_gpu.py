@@ -122,3 +122,20 @@ def test_where_the_line_lies(ctx, k, nnz, crowded, taken):
     assert S.info.hot_cols == plain.info.hot_cols > 0
     more = S.info.device_bytes - (plain.info.device_bytes - plain.info.npartial_slots * (96 - k) * 8)
     assert (more >= 4 * nnz) == taken
+
+
+def test_a_plan_without_a_width_is_for_64_columns(ctx):
+    k, m, n, nnz = 64, 9000, 130000, 3200000
+    ii, jj = pattern(m, n, nnz, "sorted")
+    vv = np.random.default_rng(3).uniform(0, 1, nnz)
+    opts = dict(seg_max=512, dtype=np.float64)
+    S, hinted = ctx.plan(m, n, ii, jj, vv, **opts), ctx.plan(m, n, ii, jj, vv, k_hint=k, **opts)
+    assert S.info.device_bytes == hinted.info.device_bytes > ctx.plan(m, n, ii, jj, vv, k_hint=60, l2_hot_bytes=15 << 17,
+                                                                      **opts).info.device_bytes + 4 * nnz
+    rng = np.random.default_rng(4)
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)) for r in (m, n, m))
+    dA, dB, dC, dY = ctx.panel_from(A), ctx.panel_from(B), ctx.vals(nnz, np.float64), ctx.panel_from(Y0)
+    ctx.sddmm(S, dA, dB, dC)
+    check_sddmm(A, B, ii, jj, vv, dC.download())
+    ctx.spmm(S, dB, dY)
+    check_spmm(B, ii, jj, vv, Y0, dY.download())
