@@ -134,8 +134,8 @@ typedef struct {
                               launch gathers, nnz * bytes of a dense row / 2^21, within 16 .. 2048,
                               at most 1024 for dense rows of 128 bytes and 512 for 64 bytes and
                               less) */
-    uint32_t k_hint;       /* K the plan will mostly run with: sizes the XCD slicing (default
-                              64) and the default seg_max */
+    uint32_t k_hint;       /* K the plan will mostly run with: sizes the XCD slicing and the
+                              copy of hot dense rows (default 64), and the default seg_max */
     uint32_t l2_hot_bytes; /* XCD slicing: share of one XCD's 4 MiB L2 planned for dense rows
                               (default 2 MiB) */
     uint32_t hub_min;      /* XCD slicing: rows with at least this many entries are cut by
