@@ -450,7 +450,7 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
                             uint32_t min_row, bool *taken)
 {
     *taken = false;
-    if (nnz + 64 >= (1ull << 32)) // staging places are 32-bit, the rest's start rounded up to 64
+    if (!sweep_fits(nnz)) // (staging places are 32-bit too, the rest's start rounded up to 64)
         return SPC3D_OK;
     spc3d_ctx *ctx = p->ctx;
     const size_t w = elem_size(p->dtype);

@@ -1435,6 +1435,7 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
 {
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
+    static_assert(G * UB <= kSweepRound, "positions may pass the last entry by a round");
     __shared__ V tile_a[kSweepRowBytes / 16];
     const uint32_t tile = tile0 + blockIdx.x;
     const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;

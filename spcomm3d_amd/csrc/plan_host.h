@@ -37,6 +37,14 @@ struct SplitRow {
     uint32_t pad;
 };
 
+// ---- row tiles -------------------------------------------------------------------
+// SDDMM over a tile's entries runs in rounds of at most kSweepRound of them, and asks for a round's
+// indices one round ahead: its 32-bit positions go up to a round past the last entry.  Patterns that
+// come nearer than that to 2^32 entries get no tiles: the positions would begin again at 0, inside
+// another tile's range.
+constexpr uint32_t kSweepRound = 1024;
+inline bool sweep_fits(uint64_t nnz) { return nnz + kSweepRound <= (1ull << 32); }
+
 // ---- hot rows that crowd ---------------------------------------------------------
 // Dense rows a power of two apart whose numbers share their low bits (the hubs of an R-MAT graph,
 // whose numbers have few one-bits) share channels and sets of every L2, and the hottest of them carry

@@ -138,6 +138,10 @@ def test_copies_and_pools_where_memory_runs_out():
     _run("test_host_memory")
 
 
+def test_rules_of_the_plans_that_decide_by_size():
+    _run("test_plan_rules")
+
+
 @pytest.mark.gpu
 def test_shim_without_the_cache_of_the_one_shot_calls():
     # SPC3D_HOST_CACHE=0: plan, upload, run, download, free on every call; same results
