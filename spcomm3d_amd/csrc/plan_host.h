@@ -67,8 +67,9 @@ SPC3D_HD inline bool hot_row_width(uint64_t bytes)
 }
 // A launch must be long enough to repay the copy: 3 GiB of gathers in rows of 256 bytes, half of that in
 // wider ones.  SDDMM + SpMM in us without and with, 256 bytes: 1.0 GB 199 -> 202, 2.0 411 -> 409, 4.1
-// 877 -> 816; 512 bytes: 1.0 GB 195 -> 198, 2.0 407 -> 382; 1 KB: 2.0 GB 392 -> 368; 4 KB: 16 GB 4050 ->
-// 3376.
+// 877 -> 816; 512 bytes: 1.0 GB 195 -> 198, 2.0 407 -> 382; 1 KB: 2.0 GB 392 -> 368; 2 KB: 1.7 GB 355 -> 300;
+// 4 KB: 1.7 GB 347 -> 296, 16 GB 4050 -> 3376.  Asked for the planned width when the plan is made, and for
+// the width of a call by every call.
 inline bool hot_rows_pay(uint64_t nnz, uint64_t row_bytes)
 {
     return hot_row_width(row_bytes) && nnz * row_bytes >= ((uint64_t)(row_bytes == 256 ? 6 : 3) << 29);

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from spcomm3d_amd import device
+from tests._launches import launches
 from tests.test_parity_gpu import check_sddmm, check_spmm
 
 pytestmark = pytest.mark.gpu
@@ -72,13 +73,15 @@ def test_copied_rows_give_the_bits_of_rows_in_place(ctx, dtype, k, m, n, nnz, or
     check_spmm(B, ii, jj, vv, Y0, out[1][1])
 
 
-def test_other_widths_recordings_and_the_call_without_allocations(ctx):
-    dtype, k, m, n, nnz, order = np.float64, 64, 3000, 130000, 3200000, "sorted"
+# (planned for 64 columns no other width repays the copy; for 128 columns 64 do, out of the same buffer)
+@pytest.mark.parametrize("k,widths", [(64, (32, 60, 128)), (128, (64, 128))])
+def test_other_widths_recordings_and_the_call_without_allocations(ctx, k, widths):
+    dtype, m, n, nnz, order = np.float64, 3000, 130000, 3200000, "sorted"
     ii, jj = pattern(m, n, nnz, order)
     rng = np.random.default_rng(1)
     vv = rng.uniform(0, 1, nnz).astype(dtype)
     S = ctx.plan(m, n, ii, jj, vv, k_hint=k)
-    for kk in (32, 60, 128):  # narrower rows out of the same buffer, a width without, wider ones
+    for kk in widths:
         A, B, Y0 = (rng.uniform(-1, 1, (r, kk)).astype(dtype) for r in (m, n, m))
         dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(nnz, dtype)
         ctx.sddmm(S, dA, dB, dC)
@@ -122,6 +125,26 @@ def test_where_the_line_lies(ctx, k, nnz, crowded, taken):
     assert S.info.hot_cols == plain.info.hot_cols > 0
     more = S.info.device_bytes - (plain.info.device_bytes - plain.info.npartial_slots * (96 - k) * 8)
     assert (more >= 4 * nnz) == taken
+
+
+@pytest.mark.parametrize("hint,nnz,widths", [(512, 400000, {32: 0, 64: 0, 256: 0, 512: 1}),
+                                             (128, 3200000, {32: 0, 64: 1, 128: 1, 256: 0})])
+def test_the_copy_is_made_where_the_call_repays_it(ctx, hint, nnz, widths):
+    """widths: columns of a call and how many kernels more than without hot rows it launches."""
+    m, n = 2500, 130000 if hint == 128 else 18000
+    ii, jj = pattern(m, n, nnz, "sorted")
+    vv = np.ones(nnz)
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=hint, seg_max=512)
+    plain = ctx.plan(m, n, ii, jj, vv, k_hint=hint * 3 // 2, l2_hot_bytes=3 << 20, seg_max=512)
+    assert S.info.nsegments == plain.info.nsegments and S.info.hot_cols == plain.info.hot_cols > 0
+    for k, more in widths.items():
+        dA, dB, dY = (ctx.panel(r, k, np.float64) for r in (m, n, m))
+        dC = ctx.vals(nnz, np.float64)
+        for call in (lambda P: ctx.sddmm(P, dA, dB, dC), lambda P: ctx.spmm(P, dB, dY),
+                     lambda P: ctx.sddmm_spmm(P, dA, dB, dC, dY)):
+            call(S), call(plain)
+            with_copy, without = (launches(ctx, lambda: call(P)) for P in (S, plain))
+            assert len(with_copy) == len(without) + more, (k, with_copy, without)
 
 
 def test_a_plan_without_a_width_is_for_64_columns(ctx):
