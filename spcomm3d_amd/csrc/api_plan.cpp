@@ -284,6 +284,21 @@ static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, De
     return SPC3D_OK;
 }
 
+// The plan's column indices, and the first ones of its short segments, with its hot columns named by
+// rank (asynchronous).
+static int name_hot_columns(spc3d_plan *p)
+{
+    std::string err;
+    const int rc = encode_hot_device(dev_stream(p->ctx), p->col, p->info.nnz, p->hot_cols, p->nhot,
+                                     p->info.ncols, p->hot_col, err);
+    if (rc)
+        return fail(rc, err);
+    const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
+    HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->hot_col, p->hot_first_cols,
+                              p->ctx->stream));
+    return SPC3D_OK;
+}
+
 // What the calls of a finished single plan whose hot rows crowd (p->nhot, set by the builder) need
 // beside its arrays: the column indices with those columns named by rank, and room for their dense
 // rows at the planned width.
@@ -296,20 +311,12 @@ static int add_hot_rows(spc3d_plan *p, uint32_t k0)
     int rc = ctx_alloc(p->ctx, &p->hot_col, (size_t)p->info.nnz);
     if (!rc) rc = ctx_alloc(p->ctx, &p->hot_first_cols, (size_t)nshort * kFirstCols);
     if (!rc) rc = ctx_alloc_bytes(p->ctx, &p->hot_rows, (size_t)p->nhot * row_bytes + kHotUnit);
-    std::string err;
-    if (!rc) {
-        rc = encode_hot_device(dev_stream(p->ctx), p->col, p->info.nnz, p->hot_cols, p->nhot,
-                               p->info.ncols, p->hot_col, err);
-        if (rc)
-            fail(rc, err);
-    }
+    if (!rc) rc = name_hot_columns(p);
     if (rc) {
         drop_hot_rows(p);
         return optional_path(rc);
     }
     p->hot_row_bytes = (uint32_t)row_bytes;
-    HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->hot_col, p->hot_first_cols,
-                              p->ctx->stream));
     return SPC3D_OK;
 }
 
@@ -1207,12 +1214,18 @@ int spc3d_plan_set_values_device(spc3d_plan *plan, const spc3d_vals *vv)
 // One plan's columns rewritten in place, and its table of first columns with them.
 static int probe_columns_of(spc3d_plan *p, int mode, uint32_t modulus)
 {
-    p->hot_row_bytes = 0; // the probe's columns are gathered where they lie
     HIP_TRY(launch_probe_cols(p->col, p->info.nnz, (uint32_t)mode, p->col_base, modulus,
                               p->info.ncols, p->ctx->stream));
     const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
     HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->col, p->first_cols,
                               p->ctx->stream));
+    if (p->hot_rows) { // the copy and the kernels that gather from it stay part of the calls
+        const int rc = name_hot_columns(p);
+        if (rc) {
+            drop_hot_rows(p);
+            return rc;
+        }
+    }
     return SPC3D_OK;
 }
 

@@ -147,6 +147,36 @@ def test_the_copy_is_made_where_the_call_repays_it(ctx, hint, nnz, widths):
             assert len(with_copy) == len(without) + more, (k, with_copy, without)
 
 
+@pytest.mark.parametrize("mode,order", [("all_hit", "sorted"), ("all_miss", "sorted"), ("all_hit", "column")])
+def test_probed_columns_keep_the_copy(ctx, mode, order):
+    """spc3d_plan_probe_columns on a plan with copied hot rows: its calls launch what they launched, hold
+    the memory they held and give the bits of a plan without, probed the same way."""
+    k, m, n, nnz = 64, 120000, 130000, 3200000
+    ii, jj = pattern(m, n, nnz, order)
+    rng = np.random.default_rng(7)
+    vv = rng.uniform(0, 1, nnz)
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k, seg_max=512)
+    plain = ctx.plan(m, n, ii, jj, vv, k_hint=k * 3 // 2, l2_hot_bytes=3 << 20, seg_max=512)
+    A, B, Y0 = (rng.uniform(-1, 1, (r, k)) for r in (m, n, m))
+    dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(nnz, np.float64)
+    calls = (lambda P: ctx.sddmm(P, dA, dB, dC), lambda P: ctx.spmm(P, dB, dY))
+    for call in calls:
+        call(S), call(plain)
+    before = [launches(ctx, lambda: call(S)) for call in calls]
+    assert [len(b) for b in before] == [len(launches(ctx, lambda: call(plain))) + 1 for call in calls]
+    held = S.info.device_bytes
+    out = []
+    for plan in (plain, S):
+        plan.probe_columns(mode, 2048)
+        dY.upload(Y0)
+        for call in calls:
+            call(plan)
+        out.append((dC.download(), dY.download()))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert [launches(ctx, lambda: call(S)) for call in calls] == before
+    assert S.info.device_bytes == held
+
+
 def test_a_plan_without_a_width_is_for_64_columns(ctx):
     k, m, n, nnz = 64, 9000, 130000, 3200000
     ii, jj = pattern(m, n, nnz, "sorted")
