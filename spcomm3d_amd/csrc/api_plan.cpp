@@ -238,6 +238,13 @@ static int add_two_pass(spc3d_plan *p, const StoreOpts &so)
 // Row width a plan is created for: sizes the partial-sum rows of its cut rows.
 static uint32_t planned_k(const spc3d_plan_opts *o) { return o && o->k_hint ? o->k_hint : 64u; }
 
+// Options for the arrays of plans on which add_hot_rows is not called: no list of hot columns is made.
+static PlanOpts without_hot_rows(PlanOpts po)
+{
+    po.hot_row_bytes = 0;
+    return po;
+}
+
 // Plan over arrays that build_device_plan left on the device.
 static int adopt_device_plan(spc3d_ctx *ctx, int dtype, const HostPlan &meta, DevPlanArrays &arr,
                              uint32_t k0, spc3d_plan **out)
@@ -484,7 +491,9 @@ static int rebuild_as_sweep(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint6
             if (!rc) rc = gather_u32_device(dev_stream(ctx), d_jj, sw.perm + sw.n, nrest, r_jj, err);
             HostPlan meta;
             DevPlanArrays arr;
-            if (!rc) rc = build_device_plan(dev_stream(ctx), nrows, ncols, nrest, r_ii, r_jj, po, meta, arr, err);
+            if (!rc)
+                rc = build_device_plan(dev_stream(ctx), nrows, ncols, nrest, r_ii, r_jj, without_hot_rows(po),
+                                       meta, arr, err);
             if (rc)
                 fail(rc, err);
             else
@@ -685,7 +694,9 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     HostPlan meta;
     DevPlanArrays arr;
     std::string err;
-    int rc = build_device_plan(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj, po, meta, arr, err);
+    const bool blocks = opts && opts->col_blocks > 1; // (for certain: choose_col_blocks follows the caller)
+    int rc = build_device_plan(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj,
+                               blocks ? without_hot_rows(po) : po, meta, arr, err);
     if (rc != SPC3D_OK)
         return fail(rc, err);
     spc3d_plan *p = nullptr;
@@ -768,8 +779,8 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
             continue;
         HostPlan bmeta;
         DevPlanArrays barr;
-        rc = build_device_plan(dev_stream(ctx), nrows, ncols, cnt, b_ii + first[b], b_jj + first[b], po,
-                               bmeta, barr, err);
+        rc = build_device_plan(dev_stream(ctx), nrows, ncols, cnt, b_ii + first[b], b_jj + first[b],
+                               without_hot_rows(po), bmeta, barr, err);
         if (rc) {
             fail(rc, err);
             break;
@@ -1277,8 +1288,9 @@ static uint64_t own_device_bytes(const spc3d_plan *p)
     if (p->splits) b += (uint64_t)p->info.nsplit_rows * sizeof(SplitRow);
     if (p->first_cols)
         b += (uint64_t)(p->info.nsegments_padded - p->info.nsegments_long) * kFirstCols * 4;
+    if (p->hot_cols) b += (uint64_t)p->nhot * 4;
     if (p->hot_rows) {
-        b += (uint64_t)p->nhot * (4 + p->hot_row_bytes) + nnz * 4;
+        b += (uint64_t)p->nhot * p->hot_row_bytes + kHotUnit + nnz * 4;
         b += (uint64_t)(p->info.nsegments_padded - p->info.nsegments_long) * kFirstCols * 4;
     }
     if (p->partial) b += (uint64_t)p->info.npartial_slots * p->partial_k * w;

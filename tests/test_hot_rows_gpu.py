@@ -177,6 +177,20 @@ def test_probed_columns_keep_the_copy(ctx, mode, order):
     assert S.info.device_bytes == held
 
 
+def test_plans_that_never_copy_hot_rows_hold_no_list_of_them(ctx):
+    """Column blocks whose hot rows crowd: the memory of the same blocks planned for a width without."""
+    m, n, nnz = 9000, 130000, 5500000
+    ii, jj = pattern(m, n, nnz, "sorted")
+    # no row is cut: the only memory that depends on the width would be the hot rows'
+    opts = dict(seg_max=1 << 20, hub_min=1 << 20, dtype=np.float64)
+    S, plain = (ctx.plan(m, n, ii, jj, k_hint=k, l2_hot_bytes=k * 8 * 1024, col_blocks=2, **opts) for k in (64, 96))
+    assert S.info.ncol_blocks == plain.info.ncol_blocks == 2 and S.info.nqueues == plain.info.nqueues == 8
+    assert S.info.npartial_slots == plain.info.npartial_slots == 0
+    assert S.info.device_bytes == plain.info.device_bytes
+    whole, plain = (ctx.plan(m, n, ii, jj, k_hint=k, l2_hot_bytes=k * 8 * 1024, **opts) for k in (64, 96))
+    assert whole.info.device_bytes > plain.info.device_bytes + 4 * nnz  # (they do crowd)
+
+
 def test_a_plan_without_a_width_is_for_64_columns(ctx):
     k, m, n, nnz = 64, 9000, 130000, 3200000
     ii, jj = pattern(m, n, nnz, "sorted")
