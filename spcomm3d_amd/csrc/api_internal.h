@@ -150,6 +150,7 @@ struct spc3d_plan {
     uint32_t nhot = 0, hot_row_bytes = 0;
     uint32_t *hot_col = nullptr, *hot_first_cols = nullptr;
     void *hot_rows = nullptr;
+    bool hot_stale = false; // hot_col is not of `col`: calls gather the rows where they lie
     void *partial; // [npartial_slots * partial_k] reals
     uint32_t partial_k;
     // Partial-sum blocks that a call at a larger K has replaced.  They stay allocated
@@ -434,7 +435,7 @@ inline DevPlanView view_of(const spc3d_plan *p)
     v.nnz = p->info.nnz;
     v.cols_touched = p->info.cols_touched;
     v.seg_base = p->store.consecutive;
-    if (p->hot_rows) {
+    if (p->hot_rows && !p->hot_stale) {
         v.hot_cols = p->hot_cols;
         v.nhot = p->nhot;
         v.ncols = p->info.ncols;

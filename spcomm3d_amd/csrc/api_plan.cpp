@@ -1230,14 +1230,11 @@ static int probe_columns_of(spc3d_plan *p, int mode, uint32_t modulus)
     const uint32_t nshort = p->info.nsegments_padded - p->info.nsegments_long;
     HIP_TRY(launch_first_cols(p->segs + p->info.nsegments_long, nshort, p->col, p->first_cols,
                               p->ctx->stream));
-    if (p->hot_rows) { // the copy and the kernels that gather from it stay part of the calls
-        const int rc = name_hot_columns(p);
-        if (rc) {
-            drop_hot_rows(p);
-            return rc;
-        }
-    }
-    return SPC3D_OK;
+    // The copy and the kernels that gather from it stay part of the calls; where there is no memory to name
+    // the columns, the calls do without.  (Nothing is freed: recordings of the plan's calls may use it.)
+    const int rc = p->hot_rows ? name_hot_columns(p) : SPC3D_OK;
+    p->hot_stale = rc != SPC3D_OK;
+    return rc;
 }
 
 int spc3d_plan_probe_columns(spc3d_plan *plan, int mode, uint32_t modulus)
