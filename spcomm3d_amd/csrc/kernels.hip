@@ -2241,45 +2241,95 @@ inline hipError_t join_aux(const Streams &S)
 
 enum LaunchOf { kSddmm, kOnePass, kSpmm };
 
-// Dynamic LDS that keeps the workgroups of a segment launch down to fewer per CU than its registers
-// allow (4 to 8), or 0.  Where nearly every gather misses the L2s and a launch has more than enough of
-// them in flight, fewer at once are served faster: unskewed columns (no slices), a panel over the L2s (64
-// MiB; 24 for the wide launch) that the Infinity Cache mostly holds (320), segments of one kind, four rounds of wavefronts and
-// more, at least three lanes in four busy.  Uniform rows of 4 to 48 entries over 60 k to 3 M columns,
-// speed of SDDMM / SpMM / one-pass against all wavefronts:
-//  - the wide launch at 3 workgroups, from 16 entries on 1.00 .. 1.07 / 1.01 .. 1.05, one-pass from 24 on 1.00
-//    .. 1.06 (12 entries: 0.88 / 0.90 / 0.82; one-pass at 20: 0.97); rows that leave lanes idle from 24 on, in
-//    groups of 32 lanes from 32 on (20 entries: 0.94 / 0.99 / 0.92);
-//  - the short one from 6 entries on: SpMM at 5 1.01 .. 1.07 (5 entries: 0.93); SDDMM at 5 1.00 .. 1.07, with idle
-//    lanes 6, 0.99 .. 1.02; one-pass at 6 0.99 .. 1.05, a row to a wavefront 5, 1.02 .. 1.06;
-//  - the short one at 4 and 5 entries, SpMM over dense rows of 512 bytes and more, whatever the panel: 7, 1.01
+// Workgroups of a segment launch per CU, or 0: as many as its registers allow (4 to 8).  Where nearly every
+// gather misses the L2s and a launch has more than enough of them in flight, fewer at once are served
+// faster: unskewed columns (no slices), four rounds of wavefronts and more, at least three lanes in four busy.
+// `cached`: panels (of touched rows) that the Infinity Cache mostly holds.  Speed against as many as fit, median and
+// range over uniform rows of 3 to 32 entries, 64 to 4096 bytes wide, over 2 k to 1 M columns:
+//  - the wide launch, cached panels: 2 from 24 MiB and 16 entries on (rows that leave lanes of 64 idle from 24, of fewer
+//    from 32; one-pass from 24 in groups of 64 without idle lanes, else from 32) 1.03 (0.99 .. 1.11); 3 from 16 MiB and 12
+//    entries on (SpMM over mixed lengths from 8) 1.02 (0.97 .. 1.07).  Beyond 320 MiB SpMM over even rows alone: 3, 1.02
+//    (0.99 .. 1.04); SDDMM and one-pass would lose up to 5 %;
+//  - the short launch, cached panels of 64 MiB and more, from 6 entries on: 4, SDDMM 1.03 (1.00 .. 1.11), SpMM 1.02 (1.00 ..
+//    1.09; idle lanes of 64 and longer rows or 8 entries 1.04, 1.02 .. 1.07; idle lanes of 32 1.04, under 25 busy 5,
+//    1.02); SDDMM with idle lanes 6, 1.01 (0.99 .. 1.05; under 25 of 32 busy 0.97, so none);
+//  - SpMM whose rows leave lanes of 64 idle, otherwise: 6 from 32 MiB and 5 entries on, 1.01 (0.98 .. 1.05);
+//  - one-pass in groups of 64 lanes, whose short launch holds up to 8 rows per wavefront: one vector per lane 4 (cached, 64
+//    MiB, 6 entries) 1.05 (1.02 .. 1.08), else 5 (8 MiB, where they end inside a
+//    vector 16, 5 entries) 1.02 (0.98 .. 1.07); with idle lanes 6 (cached, 32 MiB, 6
+//    entries) 1.01 (0.98 .. 1.03), from 12 entries and 24 MiB on 5, 1.03; longer rows 4 (8 MiB, 3 entries) 1.03 (0.97 .. 1.08), where they
+//    end inside a vector 5 (32 MiB), where lanes idle 5 (cached, 7 entries), 1.03 (1.00 .. 1.06);
+//  - one-pass otherwise as the short launch, but 6: 1.00 (0.97 .. 1.01); from 12 entries over rows that end inside a vector
+//    4, 1.04;
+//  - SpMM's short launch at 4 and 5 entries, dense rows of 512 bytes and more, whatever the panel: 7, 1.01
 //    .. 1.04 from 65,536 wavefronts on (half of them: 0.99).
-// Panels in the caches or far beyond them want every wavefront (30 k rows of 40 over 30 k columns 0.89 /
-// 0.90 / 0.86 at 3; 300 k of 20 over 1 M columns, 512-byte rows, 0.92 / 0.97 / 0.87), and so do half-empty groups
-// (1 M rows of 8, fp32 K = 135, at 5: 0.91 / 0.84).
+// Rows of mixed lengths (Poisson), whose two launches are asked one by one: SpMM 0.99 .. 1.04, the others level.  Panels in
+// the L2s want every wavefront (100 k rows of 20 over 2 k columns, fp64 K = 128: 0.87 / 0.92 / 0.91 at 3), and so do
+// half-empty groups (400 k rows of 8, fp64 K = 65: 0.89 / 0.83 / 0.85 at 4).
+template <int LPR, int VPL, int RG>
+inline uint32_t workgroups_per_cu(const DevPlanView &P, bool wide, uint32_t nseg, LaunchOf what, uint64_t row_bytes)
+{
+    constexpr uint64_t kFull = (uint64_t)LPR * VPL * 16;
+    const uint64_t panel = P.cols_touched * row_bytes, waves = (uint64_t)nseg * LPR / 64;
+    if (P.nqueues != 1 || waves < 16384)
+        return 0;
+    const auto from = [&](uint64_t entries) { return P.nnz >= entries * P.nseg; }; // per segment, on average
+    const auto holds = [&](uint64_t mib) { return panel >= mib << 20; };
+    const bool cached = panel <= (uint64_t)320 << 20;
+    const bool filled = row_bytes * 4 >= kFull * 3;
+    if (wide) {
+        const uint64_t least = what == kOnePass ? (LPR == 64 && RG != 1 ? 24 : 32)
+                                                : (RG == 1 ? (LPR == 64 ? 24 : 32) : 16);
+        const bool even = nseg == P.nseg && (nseg - P.nseg_long <= nseg / 64 || !P.nseg_long);
+        if (!filled)
+            return 0;
+        if (cached && holds(24) && even && from(least))
+            return 2;
+        if (LPR < 16 || !holds(16))
+            return 0;
+        if (what == kSpmm)
+            return cached ? (from(8) ? 3 : 0) : (even && from(12) ? 3 : 0);
+        return cached && from(12) ? 3 : 0;
+    }
+    const bool near = cached && holds(64) && from(6);
+    if (what == kOnePass && LPR == 64 && VPL > 1) {
+        if (RG <= 0)
+            return holds(8) && from(3) ? 4 : 0;
+        if (RG == 2 && filled)
+            return holds(32) && from(3) ? 5 : 0;
+        return cached && holds(32) && from(7) ? 5 : 0;
+    }
+    if (!filled)
+        return 0;
+    if (what == kOnePass && LPR == 64) {
+        if (RG == 1)
+            return holds(24) && from(12) ? 5 : (cached && holds(32) && from(6) ? 6 : 0);
+        return near ? 4 : (holds(RG == 2 ? 16 : 8) && from(5) ? 5 : 0);
+    }
+    if (what == kOnePass)
+        return near ? (RG == 2 && from(12) ? 4 : 6) : 0;
+    const bool idle = RG == 1 && LPR < 64 && row_bytes * 32 < kFull * 25; // fewer than 25 of 32 lanes busy
+    if (what == kSddmm)
+        return near && !idle ? (RG == 1 ? 6 : 4) : 0;
+    if (RG == 1 && LPR < 64)
+        return near ? (idle ? 5 : 4) : 0;
+    if (RG == 1)
+        return near && (VPL > 1 || from(8)) ? 4 : (holds(32) && from(5) ? 6 : 0);
+    if (near)
+        return 4;
+    const bool few = RG <= 0 && kFull >= 512 && nseg == P.nseg && holds(64) && from(4) && !from(6);
+    return few && waves >= 65536 ? 7 : 0;
+}
+
+// The least dynamic LDS with which no more of them fit a CU, whose 160 KiB are handed out in pieces of 1280
+// bytes.
 template <typename T, int LPR, int VPL, int RG>
 inline uint32_t crowding_lds(const DevPlanView &P, bool wide, uint32_t nseg, LaunchOf what, uint32_t nvec)
 {
-    constexpr uint64_t kFull = (uint64_t)LPR * VPL * 16;
-    const uint64_t bytes = RG <= 0 ? kFull : (uint64_t)nvec * (RG == 1 ? 16 : sizeof(T));
-    const uint64_t waves = (uint64_t)nseg * LPR / 64, panel = P.cols_touched * bytes;
-    const uint64_t least = (uint64_t)(wide ? 24 : 64) << 20;
-    if (P.nqueues != 1 || nseg != P.nseg || waves < 16384 || panel < least || bytes * 4 < kFull * 3)
-        return 0;
-    const bool cached = panel <= ((uint64_t)320 << 20);
-    uint32_t blocks = 0; // per CU
-    if (wide) {
-        if (cached && nseg - P.nseg_long <= nseg / 64 &&
-            P.nnz >= (uint64_t)(RG == 1 && LPR < 64 ? 32 : (RG == 1 || what == kOnePass ? 24 : 16)) * nseg)
-            blocks = 3;
-    } else if (P.nnz >= (uint64_t)6 * nseg) {
-        if (cached)
-            blocks = what == kSpmm ? 5 : (RG <= 0 && (what == kSddmm || LPR == 64) ? 5 : 6);
-    } else if (what == kSpmm && RG <= 0 && kFull >= 512 && P.nnz >= (uint64_t)4 * nseg && waves >= 65536) {
-        blocks = 7;
-    }
-    constexpr uint32_t kLds = 160u << 10; // of a CU
-    return blocks ? kLds / blocks & ~1023u : 0;
+    constexpr uint32_t kPiece = 1280, kPieces = (160u << 10) / kPiece;
+    const uint64_t row_bytes = RG <= 0 ? (uint64_t)LPR * VPL * 16 : (uint64_t)nvec * (RG == 1 ? 16 : sizeof(T));
+    const uint32_t n = workgroups_per_cu<LPR, VPL, RG>(P, wide, nseg, what, row_bytes);
+    return n ? (kPieces / (n + 1) + 1) * kPiece : 0;
 }
 
 inline uint32_t store_flags(const DevPlanView &P)

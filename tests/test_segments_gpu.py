@@ -78,45 +78,78 @@ def test_even_rows_over_a_large_panel(ctx, dtype, k, n, m, length):
         h.close()
 
 
-# rows of `length`, `m` of them, over `n` columns: workgroups per CU of SDDMM, SpMM and the one-pass
-# call, 0 where nothing limits them; on both sides of every line of the rule
-F64_512, F64_1K, F32_ODD, F64_RAG32, F64_RAG64 = (np.float64, 64), (np.float64, 128), (np.float32, 127), \
-    (np.float64, 54), (np.float64, 100)
+# rows of (how many, how long) over `n` columns: workgroups per CU of every launch of SDDMM, SpMM and the
+# one-pass call, 0 where nothing limits them; on both sides of every line of the rule
+F64_512, F64_1K, F64_2K, F32_ODD, F64_ODD1K, F64_ODD2K = (np.float64, 64), (np.float64, 128), \
+    (np.float64, 256), (np.float32, 127), (np.float64, 127), (np.float64, 255)
+# rows that leave lanes idle: 24 and 27 of 32 busy, 47, 48 and 50 of 64, 65 and 100 of 128
+IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100 = ((np.float64, 2 * n) for n in (24, 27, 47, 48, 50, 65, 100))
 
 
-@pytest.mark.parametrize("dtype_k,m,n,length,want", [
-    # the wide launch, by length, panel and wavefronts
-    (F64_512, 40000, 133000, 16, (3, 3, 0)), (F64_512, 40000, 133000, 15, (0, 0, 0)),
-    (F64_512, 40000, 133000, 23, (3, 3, 0)), (F64_512, 40000, 133000, 24, (3, 3, 3)),
-    (F64_512, 40000, 49152, 24, (3, 3, 3)), (F64_512, 40000, 49151, 24, (0, 0, 0)),
-    (F64_512, 32768, 133000, 24, (3, 3, 3)), (F64_512, 32766, 133000, 24, (0, 0, 0)),
-    (F64_1K, 40000, 327680, 16, (3, 3, 0)), (F64_1K, 40000, 327681, 16, (0, 0, 0)),
-    # rows that end inside a vector; that leave lanes of 32 and of 64 idle; too many of them
-    (F32_ODD, 40000, 133000, 16, (3, 3, 0)), (F32_ODD, 40000, 133000, 24, (3, 3, 3)),
-    (F64_RAG32, 40000, 133000, 31, (0, 0, 0)), (F64_RAG32, 40000, 133000, 32, (3, 3, 3)),
-    (F64_RAG64, 40000, 133000, 23, (0, 0, 0)), (F64_RAG64, 40000, 133000, 24, (3, 3, 3)),
-    ((np.float64, 94), 40000, 133000, 32, (0, 0, 0)), ((np.float64, 96), 40000, 133000, 32, (3, 3, 3)),
-    # the short launch
-    (F64_512, 40000, 133000, 6, (5, 5, 6)), (F64_512, 40000, 133000, 5, (0, 0, 0)),
-    (F64_512, 40000, 131072, 6, (5, 5, 6)), (F64_512, 40000, 131071, 6, (0, 0, 0)),
-    (F64_1K, 40000, 133000, 6, (5, 5, 5)), (F64_1K, 55000, 327680, 6, (5, 5, 5)),
-    (F64_1K, 55000, 327681, 6, (0, 0, 0)), (F32_ODD, 40000, 133000, 6, (6, 5, 6)),
-    (F64_RAG64, 40000, 133000, 6, (6, 5, 6)),
-    (F64_512, 131072, 133000, 5, (0, 7, 0)), (F64_512, 131070, 133000, 5, (0, 0, 0)),
-    (F64_512, 131072, 133000, 4, (0, 7, 0)), (F64_512, 131072, 133000, 3, (0, 0, 0)),
-    (F64_1K, 90000, 327681, 5, (0, 7, 0)), (F32_ODD, 140000, 133000, 5, (0, 0, 0))])
-def test_launches_kept_to_fewer_workgroups_per_cu(ctx, dtype_k, m, n, length, want):
+@pytest.mark.parametrize("dtype_k,n,rows,want", [
+    # the wide launch, by length, panel, wavefronts and lanes
+    (F64_512, 133000, [(40000, 12)], (3, 3, 3)), (F64_512, 133000, [(40000, 15)], (3, 3, 3)),
+    (F64_512, 133000, [(40000, 16)], (2, 2, 3)), (F64_512, 133000, [(40000, 23)], (2, 2, 3)),
+    (F64_512, 133000, [(40000, 31)], (2, 2, 3)), (F64_512, 133000, [(40000, 32)], (2, 2, 2)),
+    (F64_512, 49152, [(40000, 32)], (2, 2, 2)), (F64_512, 49151, [(40000, 32)], (3, 3, 3)),
+    (F64_512, 32768, [(40000, 32)], (3, 3, 3)), (F64_512, 32767, [(40000, 32)], (0, 0, 0)),
+    (F64_512, 133000, [(32768, 32)], (2, 2, 2)), (F64_512, 133000, [(32766, 32)], (0, 0, 0)),
+    (F64_1K, 133000, [(40000, 23)], (2, 2, 3)), (F64_1K, 133000, [(40000, 24)], (2, 2, 2)),
+    (F64_1K, 327680, [(40000, 16)], (2, 2, 3)),
+    (F64_1K, 327681, [(40000, 16)], (0, 3, 0)), (F64_1K, 327681, [(20032, 8), (20032, 24)], (0, 0, 0)),
+    (F32_ODD, 133000, [(40000, 16)], (2, 2, 3)), (F32_ODD, 133000, [(40000, 32)], (2, 2, 2)),
+    (IDLE27, 133000, [(40000, 31)], (3, 3, 3)), (IDLE27, 133000, [(40000, 32)], (2, 2, 2)),
+    (IDLE50, 133000, [(40000, 23)], (3, 3, 3)), (IDLE50, 133000, [(40000, 24)], (2, 2, 3)),
+    (IDLE50, 133000, [(40000, 32)], (2, 2, 2)), (IDLE47, 133000, [(40000, 32)], (0, 0, 0)),
+    (IDLE48, 133000, [(40000, 32)], (2, 2, 2)), ((np.float64, 16), 200000, [(140032, 16)], (2, 2, 0)),
+    ((np.float64, 16), 200000, [(140032, 12)], (0, 0, 0)),
+    # rows of mixed lengths, all of them in one launch and in two
+    (F64_512, 133000, [(20032, 8), (20032, 24)], (3, 3, 3)), (F64_512, 133000, [(36032, 8), (4032, 24)], (0, 3, 0)),
+    (F64_512, 133000, [(36032, 7), (4032, 16)], (0, 0, 0)),
+    (F64_512, 133000, [(200000, 8), (200000, 24)], ((3, 4), (3, 4), (3, 6))),
+    # the short launch, one vector per lane
+    (F64_512, 133000, [(40000, 11)], (4, 4, 6)), (F64_512, 133000, [(40000, 6)], (4, 4, 6)),
+    (F64_512, 133000, [(40000, 5)], (0, 0, 0)), (F64_512, 131072, [(40000, 6)], (4, 4, 6)),
+    (F64_512, 131071, [(40000, 6)], (0, 0, 0)), (F64_1K, 133000, [(40000, 6)], (4, 4, 4)),
+    (F64_1K, 327680, [(60000, 6)], (4, 4, 4)), (F64_1K, 327681, [(60000, 6)], (0, 0, 5)),
+    (F64_1K, 133000, [(40000, 5)], (0, 0, 5)), (F64_1K, 133000, [(40000, 4)], (0, 0, 0)),
+    (F64_1K, 8192, [(40000, 5)], (0, 0, 5)), (F64_1K, 8191, [(40000, 5)], (0, 0, 0)),
+    (F64_ODD1K, 16514, [(40000, 5)], (0, 0, 5)), (F64_ODD1K, 16513, [(40000, 5)], (0, 0, 0)),
+    (F32_ODD, 133000, [(40000, 6)], (4, 4, 6)), (F32_ODD, 133000, [(40000, 12)], (4, 4, 4)),
+    (IDLE27, 156000, [(40000, 6)], (6, 4, 6)), (IDLE24, 180000, [(40000, 6)], (0, 5, 6)),
+    (IDLE50, 133000, [(40000, 5)], (0, 6, 0)), (IDLE50, 133000, [(40000, 6)], (6, 6, 6)),
+    (IDLE50, 133000, [(40000, 8)], (6, 4, 6)), (IDLE50, 133000, [(40000, 12)], (6, 4, 5)),
+    (IDLE50, 41944, [(40000, 6)], (0, 6, 6)), (IDLE50, 41943, [(40000, 6)], (0, 0, 0)),
+    (IDLE50, 31458, [(40000, 12)], (0, 0, 5)), (IDLE50, 31457, [(40000, 12)], (0, 0, 0)),
+    (IDLE50, 419431, [(80000, 6)], (0, 6, 0)), (IDLE50, 419431, [(80000, 12)], (0, 6, 5)),
+    (F64_512, 133000, [(131072, 5)], (0, 7, 0)), (F64_512, 133000, [(131070, 5)], (0, 0, 0)),
+    (F64_512, 133000, [(131072, 4)], (0, 7, 0)), (F64_512, 133000, [(131072, 3)], (0, 0, 0)),
+    (F64_1K, 327681, [(90000, 5)], (0, 7, 5)), (F32_ODD, 133000, [(140000, 5)], (0, 0, 0)),
+    # the short launch, longer rows
+    (F64_2K, 4096, [(20000, 3)], (0, 0, 4)), (F64_2K, 4095, [(20000, 3)], (0, 0, 0)),
+    (F64_2K, 4096, [(20000, 2)], (0, 0, 0)), (F64_2K, 40000, [(20000, 6)], (4, 4, 4)),
+    (F64_ODD2K, 16449, [(20000, 3)], (0, 0, 5)), (F64_ODD2K, 16448, [(20000, 3)], (0, 0, 0)),
+    (F64_ODD2K, 40000, [(20000, 6)], (4, 4, 5)), (IDLE100, 20972, [(20000, 7)], (0, 6, 5)),
+    (IDLE100, 20971, [(20000, 7)], (0, 0, 0)), (IDLE100, 20972, [(20000, 6)], (0, 6, 0)),
+    (IDLE100, 50000, [(20000, 7)], (6, 4, 5)), (IDLE65, 40000, [(20000, 7)], (0, 0, 5))])
+def test_launches_kept_to_fewer_workgroups_per_cu(ctx, dtype_k, n, rows, want):
     dtype, k = dtype_k
-    ii, jj = rows_of([length] * m, n, length)
-    touched = min(n, jj.size)
-    jj[:touched] = np.arange(touched)
-    want_lds = [(160 * 1024 // w) // 1024 * 1024 if w else 0 for w in want]
+    lengths = np.repeat([length for _, length in rows], [count for count, _ in rows])
+    m = lengths.size
+    ii, jj = rows_of(lengths, n, m)
+    jj[:n] = np.arange(n)  # every column is touched
     S, dC = ctx.plan(m, n, ii, jj, np.ones(jj.size, dtype)), ctx.vals(jj.size, dtype)
     dA, dB, dY = (ctx.panel(r, k, dtype) for r in (m, n, m))
-    assert S.info.nqueues == 1 and S.info.cols_touched == n
-    for call, lds in zip((lambda: ctx.sddmm(S, dA, dB, dC), lambda: ctx.spmm(S, dB, dY),
-                          lambda: ctx.sddmm_spmm(S, dA, dB, dC, dY)), want_lds):
+    assert S.info.nqueues == 1 and S.info.cols_touched == n and S.info.nsegments == m
+    for call, limits in zip((lambda: ctx.sddmm(S, dA, dB, dC), lambda: ctx.spmm(S, dB, dY),
+                             lambda: ctx.sddmm_spmm(S, dA, dB, dC, dY)), want):
         call()
-        assert [b for _, b in launches(ctx, call)] == [lds]
+        got = [lds for _, lds in launches(ctx, call)]
+        limits = limits if isinstance(limits, tuple) else (limits,)
+        assert len(got) == len(limits)
+        for lds, limit in zip(sorted(got, reverse=True), limits):
+            # a CU's 160 KiB in pieces of 1280 bytes: as many fit as said, and one more does not
+            pieces = -(-lds // 1280)
+            assert (128 // pieces if pieces else 0) == limit, (got, limits)
     for h in (S, dA, dB, dY, dC):
         h.close()
