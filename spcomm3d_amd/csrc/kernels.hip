@@ -988,8 +988,6 @@ sddmm_seg_kernel(const Seg *__restrict__ segs, uint32_t nseg, uint32_t nq, uint3
 }
 
 // ----------------------------------------------------------------- SpMM ----
-// MK: only the first n of the NB entries exist; the others repeat the loads of
-// entry n - 1 and add zero times zero.
 // Column of entry j < kFirstCols of a short segment out of the indices loaded ahead:
 // lane u of the group holds that of entry u in FC[0] (groups of 4 lanes: of entries u
 // and 4 + u in FC[0] and FC[1]).
@@ -1008,6 +1006,8 @@ __device__ __forceinline__ uint32_t first_col(const Bcast<LPR> &bcast, const uin
     }
 }
 
+// MK: only the first n of the NB entries exist; the others repeat the loads of
+// entry n - 1 and add zero times zero.
 // PRE: the batch is entries off .. off + NB - 1 of a short segment, off + NB <=
 // kFirstCols, and takes its column indices from `ex.first` (first_col).
 template <typename T, int LPR, int VPL, int NB, int RG, bool MK, bool PRE>
