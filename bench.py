@@ -242,8 +242,8 @@ def run_floors(w, dtype, steps, warmup, seg_max=None):
     """The two floors of the same launches: the plan of `w` as the timed runs build it, with
     its columns rewritten on the device (spc3d_plan_probe_columns) so that every gathered
     dense row is found in the L2 (a table of 1 MiB per L2), then so that nearly none is
-    (uniform random columns).  Segments, queues, streams and instruction stream are those
-    of the real plan; only the gather addresses differ."""
+    (uniform random columns).  Segments, queues, streams, the copy of hot dense rows and the
+    instruction stream are those of the real plan; only the gather addresses differ."""
     from spcomm3d_amd import device
     from spcomm3d_amd import workloads as W
 
