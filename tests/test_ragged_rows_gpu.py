@@ -17,7 +17,7 @@ def ctx():
 
 # vectors per row: 32, 64, 64 x 2 and 64 x 4 lanes, from the first of each range to the last
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("nvec", [17, 24, 31, 33, 50, 63, 65, 96, 127, 129, 191, 193, 255])
+@pytest.mark.parametrize("nvec", [17, 24, 31, 33, 50, 63, 65, 96, 127, 129, 191, 192, 193, 255])
 def test_widths_of_every_lane_count(ctx, dtype, nvec):
     k = nvec * 16 // np.dtype(dtype).itemsize
     rng = np.random.default_rng(nvec)
