@@ -2249,13 +2249,14 @@ enum LaunchOf { kSddmm, kOnePass, kSpmm };
 
 // Workgroups of a segment launch per CU, or 0: as many as its registers allow (4 to 8).  Where nearly every
 // gather misses the L2s and a launch has more than enough of them in flight, fewer at once are served
-// faster: unskewed columns (no slices), four rounds of wavefronts and more, at least three lanes in four busy.
+// faster: unskewed columns (no slices), four rounds of wavefronts and more, mostly at least three lanes in four busy.
 // `cached`: panels (of touched rows) that the Infinity Cache mostly holds.  Speed against as many as fit, median and
 // range over uniform rows of 3 to 32 entries, 64 to 4096 bytes wide, over 2 k to 1 M columns:
 //  - the wide launch, cached panels: 2 from 24 MiB and 16 entries on (rows that leave lanes of 64 idle from 24, of fewer
-//    from 32; one-pass from 24 in groups of 64 without idle lanes, else from 32) 1.03 (0.99 .. 1.11); 3 from 16 MiB and 12
+//    from 32; one-pass from 24 in groups of 64 without idle lanes or with longer rows, else from 32) 1.03 (0.99 .. 1.11); 3 from 16 MiB and 12
 //    entries on (SpMM over mixed lengths from 8) 1.02 (0.97 .. 1.07).  Beyond 320 MiB SpMM over even rows alone: 3, 1.02
-//    (0.99 .. 1.04); SDDMM and one-pass would lose up to 5 %;
+//    (0.99 .. 1.04); SDDMM and one-pass would lose up to 5 %.  Fewer than three lanes in four busy, cached panels, 16
+//    entries on: 3, SpMM from 32 MiB 1.02 (0.98 .. 1.07), one-pass over longer rows from 16 MiB 1.02 (0.98 .. 1.04);
 //  - the short launch, cached panels of 64 MiB and more, from 6 entries on: 4, SDDMM 1.03 (1.00 .. 1.11), SpMM 1.02 (1.00 ..
 //    1.09; idle lanes of 64 and longer rows or 8 entries 1.04, 1.02 .. 1.07; idle lanes of 32 1.04, under 25 busy 5,
 //    1.02); SDDMM with idle lanes 6, 1.01 (0.99 .. 1.05; under 25 of 32 busy 0.97, so none);
@@ -2264,7 +2265,8 @@ enum LaunchOf { kSddmm, kOnePass, kSpmm };
 //    MiB, 6 entries) 1.05 (1.02 .. 1.08), else 5 (8 MiB, where they end inside a
 //    vector 16, 5 entries) 1.02 (0.98 .. 1.07); with idle lanes 6 (cached, 32 MiB, 6
 //    entries) 1.01 (0.98 .. 1.03), from 12 entries and 24 MiB on 5, 1.03; longer rows 4 (8 MiB, 3 entries) 1.03 (0.97 .. 1.08), where they
-//    end inside a vector 5 (32 MiB), where lanes idle 5 (cached, 7 entries), 1.03 (1.00 .. 1.06);
+//    end inside a vector or lanes idle 5 (32 MiB, 3 entries; fewer than three lanes in four busy: cached, 7 entries) 1.03
+//    (1.00 .. 1.06), over 2 KiB 4 (16 MiB and the same) 1.02 (0.99 .. 1.04);
 //  - one-pass otherwise as the short launch, but 6: 1.00 (0.97 .. 1.01); from 12 entries over rows that end inside a vector
 //    4, 1.04;
 //  - SpMM's short launch at 4 and 5 entries, dense rows of 512 bytes and more, whatever the panel: 7, 1.01
@@ -2284,11 +2286,11 @@ inline uint32_t workgroups_per_cu(const DevPlanView &P, bool wide, uint32_t nseg
     const bool cached = panel <= (uint64_t)320 << 20;
     const bool filled = row_bytes * 4 >= kFull * 3;
     if (wide) {
-        const uint64_t least = what == kOnePass ? (LPR == 64 && RG != 1 ? 24 : 32)
+        const uint64_t least = what == kOnePass ? (LPR == 64 && (RG != 1 || VPL > 1) ? 24 : 32)
                                                 : (RG == 1 ? (LPR == 64 ? 24 : 32) : 16);
         const bool even = nseg == P.nseg && (nseg - P.nseg_long <= nseg / 64 || !P.nseg_long);
         if (!filled)
-            return 0;
+            return cached && from(16) && (what == kSpmm ? holds(32) : what == kOnePass && VPL > 1 && holds(16)) ? 3 : 0;
         if (cached && holds(24) && even && from(least))
             return 2;
         if (LPR < 16 || !holds(16))
@@ -2301,7 +2303,9 @@ inline uint32_t workgroups_per_cu(const DevPlanView &P, bool wide, uint32_t nseg
     if (what == kOnePass && LPR == 64 && VPL > 1) {
         if (RG <= 0)
             return holds(8) && from(3) ? 4 : 0;
-        if (RG == 2 && filled)
+        if (VPL == 4)
+            return holds(16) && (filled ? from(3) : cached && from(7)) ? 4 : 0;
+        if (filled)
             return holds(32) && from(3) ? 5 : 0;
         return cached && holds(32) && from(7) ? 5 : 0;
     }

@@ -82,8 +82,9 @@ def test_even_rows_over_a_large_panel(ctx, dtype, k, n, m, length):
 # one-pass call, 0 where nothing limits them; on both sides of every line of the rule
 F64_512, F64_1K, F64_2K, F32_ODD, F64_ODD1K, F64_ODD2K = (np.float64, 64), (np.float64, 128), \
     (np.float64, 256), (np.float32, 127), (np.float64, 127), (np.float64, 255)
-# rows that leave lanes idle: 24 and 27 of 32 busy, 47, 48 and 50 of 64, 65 and 100 of 128
-IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100 = ((np.float64, 2 * n) for n in (24, 27, 47, 48, 50, 65, 100))
+# rows that leave lanes idle: 24 and 27 of 32 busy, 47, 48 and 50 of 64, 65 and 100 of 128, 130 and 200 of 256
+IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100, IDLE130, IDLE200 = (
+    (np.float64, 2 * n) for n in (24, 27, 47, 48, 50, 65, 100, 130, 200))
 
 
 @pytest.mark.parametrize("dtype_k,n,rows,want", [
@@ -100,7 +101,11 @@ IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100 = ((np.float64, 2 * n) f
     (F32_ODD, 133000, [(40000, 16)], (2, 2, 3)), (F32_ODD, 133000, [(40000, 32)], (2, 2, 2)),
     (IDLE27, 133000, [(40000, 31)], (3, 3, 3)), (IDLE27, 133000, [(40000, 32)], (2, 2, 2)),
     (IDLE50, 133000, [(40000, 23)], (3, 3, 3)), (IDLE50, 133000, [(40000, 24)], (2, 2, 3)),
-    (IDLE50, 133000, [(40000, 32)], (2, 2, 2)), (IDLE47, 133000, [(40000, 32)], (0, 0, 0)),
+    (IDLE50, 133000, [(40000, 32)], (2, 2, 2)), (IDLE100, 50000, [(20032, 23)], (3, 3, 3)),
+    (IDLE100, 50000, [(20032, 24)], (2, 2, 2)), (IDLE47, 133000, [(40000, 15)], (0, 0, 0)),
+    (IDLE47, 44621, [(40000, 16)], (0, 3, 0)), (IDLE47, 44620, [(40000, 16)], (0, 0, 0)),
+    (IDLE65, 40000, [(20032, 16)], (0, 3, 3)), (IDLE65, 16132, [(20032, 16)], (0, 0, 3)),
+    (IDLE65, 16131, [(20032, 16)], (0, 0, 0)),
     (IDLE48, 133000, [(40000, 32)], (2, 2, 2)), ((np.float64, 16), 200000, [(140032, 16)], (2, 2, 0)),
     ((np.float64, 16), 200000, [(140032, 12)], (0, 0, 0)),
     # rows of mixed lengths, all of them in one launch and in two
@@ -130,8 +135,12 @@ IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100 = ((np.float64, 2 * n) f
     (F64_2K, 4096, [(20000, 2)], (0, 0, 0)), (F64_2K, 40000, [(20000, 6)], (4, 4, 4)),
     (F64_ODD2K, 16449, [(20000, 3)], (0, 0, 5)), (F64_ODD2K, 16448, [(20000, 3)], (0, 0, 0)),
     (F64_ODD2K, 40000, [(20000, 6)], (4, 4, 5)), (IDLE100, 20972, [(20000, 7)], (0, 6, 5)),
-    (IDLE100, 20971, [(20000, 7)], (0, 0, 0)), (IDLE100, 20972, [(20000, 6)], (0, 6, 0)),
-    (IDLE100, 50000, [(20000, 7)], (6, 4, 5)), (IDLE65, 40000, [(20000, 7)], (0, 0, 5))])
+    (IDLE100, 20971, [(20000, 7)], (0, 0, 0)), (IDLE100, 20972, [(20000, 3)], (0, 0, 5)),
+    (IDLE100, 20972, [(20000, 2)], (0, 0, 0)), (IDLE65, 40000, [(20000, 6)], (0, 0, 0)),
+    (IDLE100, 50000, [(20000, 7)], (6, 4, 5)), (IDLE65, 40000, [(20000, 7)], (0, 0, 5)),
+    (IDLE200, 5243, [(20000, 3)], (0, 0, 4)), (IDLE200, 5242, [(20000, 3)], (0, 0, 0)),
+    ((np.float64, 401), 5230, [(20000, 3)], (0, 0, 4)), (IDLE130, 8066, [(20000, 7)], (0, 0, 4)),
+    (IDLE130, 8066, [(20000, 6)], (0, 0, 0)), (IDLE130, 8065, [(20000, 7)], (0, 0, 0))])
 def test_launches_kept_to_fewer_workgroups_per_cu(ctx, dtype_k, n, rows, want):
     dtype, k = dtype_k
     lengths = np.repeat([length for _, length in rows], [count for count, _ in rows])
