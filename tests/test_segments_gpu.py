@@ -112,6 +112,8 @@ IDLE24, IDLE27, IDLE47, IDLE48, IDLE50, IDLE65, IDLE100, IDLE130, IDLE200 = (
     (F64_512, 133000, [(20032, 8), (20032, 24)], (3, 3, 3)), (F64_512, 133000, [(36032, 8), (4032, 24)], (0, 3, 0)),
     (F64_512, 133000, [(36032, 7), (4032, 16)], (0, 0, 0)),
     (F64_512, 133000, [(200000, 8), (200000, 24)], ((3, 4), (3, 4), (3, 6))),
+    (F64_512, 133000, [(180032, 7), (40000, 20)], ((0, 0), (3, 0), (0, 0))),
+    (F64_512, 133000, [(180032, 7), (23040, 20)], ((4, 0), (4, 0), (6, 0))),
     # the short launch, one vector per lane
     (F64_512, 133000, [(40000, 11)], (4, 4, 6)), (F64_512, 133000, [(40000, 6)], (4, 4, 6)),
     (F64_512, 133000, [(40000, 5)], (0, 0, 0)), (F64_512, 131072, [(40000, 6)], (4, 4, 6)),
