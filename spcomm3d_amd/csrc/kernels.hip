@@ -91,6 +91,38 @@ template <int CTRL> __device__ __forceinline__ int dpp_mov(int v)
     // no invalid source lane): no previous value to set up
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false);
 }
+// Lane u of every 16-lane row (of every quad) to the whole row (quad); u is a constant once the loop
+// around it is unrolled.
+__device__ __forceinline__ int row_bcast(int v, int u)
+{
+    switch (u) { // row_newbcast:u
+    case 0: return dpp_mov<0x150>(v);
+    case 1: return dpp_mov<0x151>(v);
+    case 2: return dpp_mov<0x152>(v);
+    case 3: return dpp_mov<0x153>(v);
+    case 4: return dpp_mov<0x154>(v);
+    case 5: return dpp_mov<0x155>(v);
+    case 6: return dpp_mov<0x156>(v);
+    case 7: return dpp_mov<0x157>(v);
+    case 8: return dpp_mov<0x158>(v);
+    case 9: return dpp_mov<0x159>(v);
+    case 10: return dpp_mov<0x15A>(v);
+    case 11: return dpp_mov<0x15B>(v);
+    case 12: return dpp_mov<0x15C>(v);
+    case 13: return dpp_mov<0x15D>(v);
+    case 14: return dpp_mov<0x15E>(v);
+    default: return dpp_mov<0x15F>(v);
+    }
+}
+__device__ __forceinline__ int quad_bcast(int v, int u)
+{
+    switch (u) {
+    case 0: return dpp_mov<0x00>(v);
+    case 1: return dpp_mov<0x55>(v);
+    case 2: return dpp_mov<0xAA>(v);
+    default: return dpp_mov<0xFF>(v);
+    }
+}
 template <int S> __device__ __forceinline__ int xchg_i32(int v)
 {
     if constexpr (S == 1)
@@ -226,6 +258,12 @@ template <int LPR, int NB> __device__ __forceinline__ constexpr int writer_lane(
 // hot rows: SDDMM 370 -> 357 us, SpMM 410 -> 369).  Smaller groups permute through LDS, the
 // lane in the instruction's offset: `first` (the byte address of the group's first lane) is made per
 // batch, or the compiler would add the lane to it outside the loop and keep all 16 sums in registers.
+//
+// entry(v, u): where every lane holds what its entry (lane % NB, NB a power of two up to 16) has, a
+// 16-lane DPP row holds the whole batch, and one move takes lane u of each row to all of the row: no LDS
+// instruction, no wait, 1 to 5 registers fewer (row tiles, 560 M entries, fp32 K = 128, SDDMM + SpMM 36.77 ->
+// 36.47 ms; the segment kernels, whose LDS is idle, 0 to 0.2 % faster).  Groups of 8 share a DPP row with
+// another and permute.
 template <int LPR> struct Bcast {
     int first;
     __device__ __forceinline__ Bcast() : first(0)
@@ -241,6 +279,24 @@ template <int LPR> struct Bcast {
             return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
         else
             return (uint32_t)__builtin_amdgcn_ds_bpermute(first + 4 * lane, (int)v);
+    }
+    __device__ __forceinline__ uint32_t entry(uint32_t v, int u) const
+    {
+        if constexpr (LPR == 4)
+            return (uint32_t)quad_bcast((int)v, u);
+        else if constexpr (LPR == 16 || LPR == 32)
+            return (uint32_t)row_bcast((int)v, u);
+        else
+            return (*this)(v, u);
+    }
+    __device__ __forceinline__ float entry(float v, int u) const
+    {
+        return __uint_as_float(entry(__float_as_uint(v), u));
+    }
+    __device__ __forceinline__ double entry(double v, int u) const
+    {
+        return __hiloint2double((int)entry((uint32_t)__double2hiint(v), u),
+                                (int)entry((uint32_t)__double2loint(v), u));
     }
     __device__ __forceinline__ float operator()(float v, int lane) const
     {
@@ -692,7 +748,7 @@ sddmm_batch_one(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type (&a
     uint32_t c[NG];
 #pragma unroll
     for (int u = 0; u < NG; ++u)
-        c[u] = bcast(cme, u);
+        c[u] = bcast.entry(cme, u);
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
         gather_row<T, LPR, VPL, RG>(b[u], B, c[u], at, nvec, row);
@@ -784,7 +840,7 @@ sddmm_batch_rounds(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type 
     const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = bcast(cme[j / G], j % G);
+        const uint32_t c = bcast.entry(cme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(b[j], B, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -1042,7 +1098,7 @@ spmm_batch_one(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict__ c
     uint32_t c[NB];
 #pragma unroll
     for (int u = 0; u < NB; ++u)
-        c[u] = PRE ? first_col<LPR>(bcast, ex.first, off + u) : bcast(cme, u);
+        c[u] = PRE ? first_col<LPR>(bcast, ex.first, off + u) : bcast.entry(cme, u);
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
         gather_row<T, LPR, VPL, RG>(x[u], X, c[u], at, nvec, row);
@@ -1059,7 +1115,7 @@ spmm_batch_one(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict__ c
         if (u % 4 == 0)
 #pragma unroll
             for (int w = u ? u + 4 : 0; w < u + 8 && w < NB; ++w)
-                av[w] = bcast(vme, w);
+                av[w] = bcast.entry(vme, w);
         const bool on = !MK || (uint32_t)u < n;
         const T a = on ? av[u] : (T)0;
 #pragma unroll
@@ -1097,8 +1153,8 @@ spmm_batch_rounds(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict_
     const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = bcast(cme[j / G], j % G);
-        av[j] = bcast(vme[j / G], j % G);
+        const uint32_t c = bcast.entry(cme[j / G], j % G);
+        av[j] = bcast.entry(vme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(x[j], X, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -1489,12 +1545,12 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
         V bv[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u)
-            bv[u] = lane.load(B, bcast(cur.col, u));
+            bv[u] = lane.load(B, bcast.entry(cur.col, u));
         __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
         T part[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u)
-            part[u] = lane.dot(tile_a[bcast(cur.row, u) * LPR + sub], bv[u]);
+            part[u] = lane.dot(tile_a[bcast.entry(cur.row, u) * LPR + sub], bv[u]);
         group_reduce<T, LPR, UB>(part, sub);
         if (wlane && uo < cur.n) {
             if (pos) // the caller's positions: pieces of lines that this workgroup's next
@@ -1587,7 +1643,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
             V xv[UB];
 #pragma unroll
             for (int u = 0; u < UB; ++u)
-                xv[u] = lane.load(X, bcast(cur.col, u));
+                xv[u] = lane.load(X, bcast.entry(cur.col, u));
             __builtin_amdgcn_sched_barrier(0);
             // where a row begins: lane u of a group holds entry u and sees entry u - 1 (lane 0 the row
             // that is being summed); the wavefront steps aside only where one of its groups needs it.
@@ -1608,7 +1664,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 if (any >> u & 1) {
-                    const uint32_t l = bcast(cur.row, u);
+                    const uint32_t l = bcast.entry(cur.row, u);
                     bool here = true; // the lanes of the groups in which entry u begins a row
                     if constexpr (LPR == 32)
                         here = __builtin_amdgcn_inverse_ballot_w64((begins >> u & 1 ? 0xFFFFFFFFull : 0) |
@@ -1626,7 +1682,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
                 }
                 if (any_past >> u & 1)
                     xv[u] = (uint32_t)u < cur.n ? xv[u] : V{};
-                acc += xv[u] * bcast(cur.val, u);
+                acc += xv[u] * bcast.entry(cur.val, u);
             }
             p = np;
             cur = nxt;
