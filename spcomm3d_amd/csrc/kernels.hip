@@ -91,8 +91,7 @@ template <int CTRL> __device__ __forceinline__ int dpp_mov(int v)
     // no invalid source lane): no previous value to set up
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false);
 }
-// Lane u of every 16-lane row (of every quad) to the whole row (quad); u is a constant once the loop
-// around it is unrolled.
+// Lane u of every 16-lane row to the whole row; u is a constant once the loop around it is unrolled.
 __device__ __forceinline__ int row_bcast(int v, int u)
 {
     switch (u) { // row_newbcast:u
@@ -112,15 +111,6 @@ __device__ __forceinline__ int row_bcast(int v, int u)
     case 13: return dpp_mov<0x15D>(v);
     case 14: return dpp_mov<0x15E>(v);
     default: return dpp_mov<0x15F>(v);
-    }
-}
-__device__ __forceinline__ int quad_bcast(int v, int u)
-{
-    switch (u) {
-    case 0: return dpp_mov<0x00>(v);
-    case 1: return dpp_mov<0x55>(v);
-    case 2: return dpp_mov<0xAA>(v);
-    default: return dpp_mov<0xFF>(v);
     }
 }
 template <int S> __device__ __forceinline__ int xchg_i32(int v)
@@ -259,11 +249,10 @@ template <int LPR, int NB> __device__ __forceinline__ constexpr int writer_lane(
 // lane in the instruction's offset: `first` (the byte address of the group's first lane) is made per
 // batch, or the compiler would add the lane to it outside the loop and keep all 16 sums in registers.
 //
-// entry(v, u): where every lane holds what its entry (lane % NB, NB a power of two up to 16) has, a
-// 16-lane DPP row holds the whole batch, and one move takes lane u of each row to all of the row: no LDS
-// instruction, no wait, 1 to 5 registers fewer (row tiles, 560 M entries, fp32 K = 128, SDDMM + SpMM 36.77 ->
-// 36.47 ms; the segment kernels, whose LDS is idle, 0 to 0.2 % faster).  Groups of 8 share a DPP row with
-// another and permute.
+// entry(v, u): where every lane holds what its entry (lane % 16) of a batch of 16 has, a 16-lane DPP row
+// holds the whole batch, and one move takes lane u of each row to all of the row: no LDS instruction, no
+// wait (SpMM over row tiles, 560 M entries, fp32 K = 128, 19.25 -> 18.83 ms; SDDMM, which has vector
+// instructions enough, 17.45 -> 17.75, and the segment kernels, level to 1 % slower, permute).
 template <int LPR> struct Bcast {
     int first;
     __device__ __forceinline__ Bcast() : first(0)
@@ -282,9 +271,7 @@ template <int LPR> struct Bcast {
     }
     __device__ __forceinline__ uint32_t entry(uint32_t v, int u) const
     {
-        if constexpr (LPR == 4)
-            return (uint32_t)quad_bcast((int)v, u);
-        else if constexpr (LPR == 16 || LPR == 32)
+        if constexpr (LPR == 16 || LPR == 32)
             return (uint32_t)row_bcast((int)v, u);
         else
             return (*this)(v, u);
@@ -748,7 +735,7 @@ sddmm_batch_one(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type (&a
     uint32_t c[NG];
 #pragma unroll
     for (int u = 0; u < NG; ++u)
-        c[u] = bcast.entry(cme, u);
+        c[u] = bcast(cme, u);
 #pragma unroll
     for (int u = 0; u < NG; ++u) {
         gather_row<T, LPR, VPL, RG>(b[u], B, c[u], at, nvec, row);
@@ -840,7 +827,7 @@ sddmm_batch_rounds(const typename Vec<T>::type (&a)[VPL], typename Vec<T>::type 
     const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = bcast.entry(cme[j / G], j % G);
+        const uint32_t c = bcast(cme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(b[j], B, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -1098,7 +1085,7 @@ spmm_batch_one(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict__ c
     uint32_t c[NB];
 #pragma unroll
     for (int u = 0; u < NB; ++u)
-        c[u] = PRE ? first_col<LPR>(bcast, ex.first, off + u) : bcast.entry(cme, u);
+        c[u] = PRE ? first_col<LPR>(bcast, ex.first, off + u) : bcast(cme, u);
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
         gather_row<T, LPR, VPL, RG>(x[u], X, c[u], at, nvec, row);
@@ -1115,7 +1102,7 @@ spmm_batch_one(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict__ c
         if (u % 4 == 0)
 #pragma unroll
             for (int w = u ? u + 4 : 0; w < u + 8 && w < NB; ++w)
-                av[w] = bcast.entry(vme, w);
+                av[w] = bcast(vme, w);
         const bool on = !MK || (uint32_t)u < n;
         const T a = on ? av[u] : (T)0;
 #pragma unroll
@@ -1153,8 +1140,8 @@ spmm_batch_rounds(typename Vec<T>::type (&acc)[VPL], const uint32_t *__restrict_
     const Bcast<LPR> bcast;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        const uint32_t c = bcast.entry(cme[j / G], j % G);
-        av[j] = bcast.entry(vme[j / G], j % G);
+        const uint32_t c = bcast(cme[j / G], j % G);
+        av[j] = bcast(vme[j / G], j % G);
         gather_row<T, LPR, VPL, RG>(x[j], X, c, sub, nvec, odd);
     }
     __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
@@ -1407,13 +1394,23 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // between 6 % faster, 256- and 1024-byte rows, and 5 % slower here; not kept.)
 // SpMM, with a barrier per block (one per batch measured 12 % slower), cuts every block's range into batches
 // of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum
-// of a row's run of entries is kept in registers and added to the row's accumulator in LDS when the run ends.  A row's entries are contiguous, so a row is shared between lane groups only
+// of a row's run of entries is kept in registers, from the row's sum in LDS on, and stored there when the run
+// ends.  A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
-// is added to the accumulator by that lane group), the later parts each BEGIN a chunk.  The
+// goes to the row's sum by that lane group), the later parts each BEGIN a chunk.  The
 // first run of every chunk therefore goes to an edge slot of its lane group instead, and
 // after the block's barrier the edge slots are added to their rows in lane-group order, one
 // lane group per row (the first of those that hold it); a second barrier ends the block.
 // No atomics, one fixed order of additions: the same bits run to run.
+// SpMM's loop is bound by the instructions of an entry (with every gather a hit it took 31 ps per entry where
+// SDDMM took 23), so whatever an entry does not need is out of it: the edge slots lie behind the sums, where a
+// run goes is one index, and entries past a chunk's end are cleared for the whole batch.  (Branches on
+// "first run" and "no run yet" and four selects per entry before: 19.25 -> 17.75 ms for those 560 M entries;
+// 200 k rows of 30 over 50 k columns 332 -> 274 us, fp64 107 over 40 k 1354 -> 1264.  Rows' sums asked for two
+// entries ahead of a run: 17.95, 285 and 1315; a batch's gathers issued before the barriers of its block:
+// rows of 30 7 % faster, longer ones 6 to 8 % slower, as are SDDMM's before its own, 2 %: the wavefronts drift.
+// Every lane group with rows of its own, without edges or a barrier per block: a tenth faster with every
+// gather a hit, and 9 % slower, at 65 % hits and not 88: chance makes the groups drift by half a block.)
 constexpr int kSweepBlock = 1024;
 constexpr uint32_t kSweepRowBytes = 128u << 10; // of LDS for the tile's rows
 constexpr uint32_t kSweepPtrWords = 1028;       // nb + 1 range bounds of a tile, in LDS too
@@ -1545,12 +1542,12 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
         V bv[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u)
-            bv[u] = lane.load(B, bcast.entry(cur.col, u));
+            bv[u] = lane.load(B, bcast(cur.col, u));
         __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
         T part[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u)
-            part[u] = lane.dot(tile_a[bcast.entry(cur.row, u) * LPR + sub], bv[u]);
+            part[u] = lane.dot(tile_a[bcast(cur.row, u) * LPR + sub], bv[u]);
         group_reduce<T, LPR, UB>(part, sub);
         if (wlane && uo < cur.n) {
             if (pos) // the caller's positions: pieces of lines that this workgroup's next
@@ -1574,10 +1571,11 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
     constexpr uint32_t kNone = 0xFFFFFFFFu;
-    __shared__ V tile_y[kSweepRowBytes / 16];
-    __shared__ V edge[kSweepBlock];   // the sum of the first run of every lane group's chunk
+    // the tile's sums, and behind them an edge slot per lane group: the sum of its chunk's first run
+    __shared__ V tile_y[kSweepRowBytes / 16 + kSweepBlock];
     __shared__ uint32_t edge_row[G];  // and its row (kNone: the chunk is empty)
     __shared__ uint32_t lptr[kSweepPtrWords];
+    constexpr uint32_t kEdge = kSweepRowBytes / 16;
     const uint32_t tile = tile0 + blockIdx.x;
     for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock)
         tile_y[i] = V{};
@@ -1619,19 +1617,13 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         if (b + 1 < nb)
             chunk(b + 1, p_nb, hi_nb);
         const bool had = p < hi;
-        uint32_t row = kNone;
-        bool first = true; // the run in `acc` is the chunk's first
-        V acc{};
-        // (The accumulator is read, added to and written back: LDS additions that return
-        // nothing, which need no wait, were measured 2.6 times slower for the whole call.)
-        auto flush = [&]() {
-            if (first)
-                edge[threadIdx.x] = acc;
-            else
-                tile_y[row * LPR + sub] += acc;
-        };
+        const Bcast<LPR> head;
+        uint32_t row = had ? head.entry(cur.row, 0) : kNone;
         if (sub == 0)
-            edge_row[grp] = had ? cur.row : kNone; // lane 0 holds the chunk's first entry
+            edge_row[grp] = row;
+        // the run that is being summed, and where its sum goes: the chunk's first to the edge slot
+        V acc{};
+        uint32_t to = kEdge + threadIdx.x;
         while (p < hi) {
             const uint32_t np = p + UB;
             SweepIdx<T> nxt;
@@ -1653,42 +1645,34 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
             const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(
                 (int)row, (int)cur.row, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
             const uint64_t begins = __ballot(cur.row != before);
-            const uint64_t past = __ballot((sub & (UB - 1)) >= cur.n); // the batch has ended
             const uint32_t mine = (uint32_t)(begins >> (threadIdx.x & 63u & ~(uint32_t)(LPR - 1)));
-            uint32_t any = 0, any_past = 0;
+            uint32_t any = 0;
 #pragma unroll
-            for (int g = 0; g < 64 / LPR; ++g) {
+            for (int g = 0; g < 64 / LPR; ++g)
                 any |= (uint32_t)(begins >> (g * LPR));
-                any_past |= (uint32_t)(past >> (g * LPR));
+            if (__ballot(cur.n < (uint32_t)UB)) { // a chunk's last batch
+#pragma unroll
+                for (int u = 0; u < UB; ++u)
+                    xv[u] = (uint32_t)u < cur.n ? xv[u] : V{};
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 if (any >> u & 1) {
-                    const uint32_t l = bcast.entry(cur.row, u);
-                    bool here = true; // the lanes of the groups in which entry u begins a row
-                    if constexpr (LPR == 32)
-                        here = __builtin_amdgcn_inverse_ballot_w64((begins >> u & 1 ? 0xFFFFFFFFull : 0) |
-                                                                   (begins >> (32 + u) & 1 ? ~0ull << 32 : 0));
-                    else if constexpr (LPR < 32)
-                        here = mine >> u & 1;
-                    if (here) {
-                        if (row != kNone) {
-                            flush();
-                            first = false;
-                        }
-                        acc = V{};
-                        row = l;
+                    const uint32_t l = bcast.entry(cur.row, u) * LPR + sub;
+                    if (mine >> u & 1) {
+                        tile_y[to] = acc;
+                        acc = tile_y[l];
+                        to = l;
                     }
                 }
-                if (any_past >> u & 1)
-                    xv[u] = (uint32_t)u < cur.n ? xv[u] : V{};
                 acc += xv[u] * bcast.entry(cur.val, u);
             }
+            row = bcast.entry(cur.row, UB - 1);
             p = np;
             cur = nxt;
         }
-        if (row != kNone)
-            flush();
+        if (had)
+            tile_y[to] = acc;
         p = p_nb;
         hi = hi_nb;
         if (!had && p < hi)
@@ -1700,7 +1684,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         if (er != kNone && (grp == 0 || edge_row[grp - 1] != er)) {
             V sum = tile_y[er * LPR + sub];
             for (uint32_t h = grp; h < G && edge_row[h] == er; ++h)
-                sum += edge[h * LPR + sub];
+                sum += tile_y[kEdge + h * LPR + sub];
             tile_y[er * LPR + sub] = sum;
         }
         __syncthreads(); // before block b + 1 writes edge slots and accumulators again
