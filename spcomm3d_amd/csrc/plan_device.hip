@@ -288,12 +288,9 @@ __global__ void hist_sorted_k(const uint32_t *__restrict__ ii, uint64_t nnz, uin
     }
 }
 
-// Histogram from sorted ids: the columns', and the rows' of a pattern that is not
-// sorted by row (a device-wide atomic per entry is served at the memory side, 1.5 ms
-// for 16 M entries; the radix sort and these two passes take a third of that).
-// Where a run of equal ids starts, its position goes to start[id]; where it ends,
-// the position after it goes to deg[id] (zeroed before); deg[id] -= start[id] then
-// leaves the run's length.  The ids were checked against nbins before.
+// Histogram from sorted ids, where there are any: where a run of equal ids starts, its position goes to
+// start[id]; where it ends, the position after it goes to deg[id] (zeroed before); deg[id] -= start[id]
+// then leaves the run's length.  The ids were checked against nbins before.
 __global__ void run_bounds_k(const uint32_t *__restrict__ sorted, uint64_t n, uint32_t nbins,
                              uint32_t *start, uint32_t *deg)
 {
@@ -315,6 +312,90 @@ __global__ void run_lengths_k(const uint32_t *__restrict__ start, uint64_t nbins
         const uint32_t end = deg[c];
         if (end)
             deg[c] = end - start[c];
+    }
+}
+
+// How often every id comes (count_ids): the ids lie in buckets of 1 << low by their upper bits, which are cut
+// into parts of at most `part` entries; a workgroup counts a part in LDS.
+constexpr uint32_t kCountBits = 14; // 64 KiB of counters, two workgroups to a CU
+constexpr int kCountTB = 1024;
+
+// The first of n keys, ascending in key >> low, that is `bucket` or above there.  By a wavefront, 64 probes at a time.
+__device__ __forceinline__ uint32_t bucket_start(const uint32_t *__restrict__ key, uint32_t n, uint32_t low,
+                                                 uint32_t bucket)
+{
+    uint32_t lo = 0, len = n; // the answer is in [lo, lo + len]
+    while (len) {
+        const uint32_t step = len / 64 + 1, lane = threadIdx.x & 63u;
+        const bool in = (uint64_t)lane * step < len;
+        const unsigned long long below = __ballot(in && key[lo + (in ? lane * step : 0u)] >> low < bucket);
+        const uint32_t k = (uint32_t)__popcll(below); // probes 0 .. k - 1 are below, the others are not
+        if (k == 0)
+            return lo;
+        const uint32_t past = (k - 1) * step + 1; // of lo: at least so much further, and less than a step more
+        lo += past;
+        len = len - past < step - 1 ? len - past : step - 1;
+    }
+    return lo;
+}
+__global__ void bucket_parts_k(const uint32_t *__restrict__ key, uint32_t n, uint32_t low, uint32_t nbuckets,
+                               uint32_t part, uint32_t *start, uint32_t *parts)
+{
+    const uint32_t b = blockIdx.x * (kTB / 64) + threadIdx.x / 64;
+    if (b > nbuckets)
+        return;
+    const uint32_t lo = b < nbuckets ? bucket_start(key, n, low, b) : n;
+    const uint32_t hi = b < nbuckets ? bucket_start(key, n, low, b + 1) : n;
+    if ((threadIdx.x & 63u) == 0) {
+        start[b] = lo;
+        parts[b] = (hi - lo + part - 1) / part;
+    }
+}
+__global__ void __launch_bounds__(kCountTB)
+bucket_count_k(const uint32_t *__restrict__ key, const uint32_t *__restrict__ start,
+               const uint32_t *__restrict__ first_part, uint32_t low, uint32_t nbuckets, uint32_t part, uint32_t *counts)
+{
+    __shared__ uint32_t count[1u << kCountBits];
+    const uint32_t g = blockIdx.x, mask = (1u << low) - 1;
+    if (g >= first_part[nbuckets])
+        return;
+    uint32_t b = 0, up = nbuckets; // first_part[b] <= g < first_part[up]
+    while (up - b > 1) {
+        const uint32_t mid = b + (up - b) / 2;
+        if (first_part[mid] <= g)
+            b = mid;
+        else
+            up = mid;
+    }
+    const uint32_t from = start[b] + (g - first_part[b]) * part, left = start[b + 1] - from;
+    const uint32_t n = left < part ? left : part;
+    for (uint32_t i = threadIdx.x; i <= mask; i += kCountTB)
+        count[i] = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += 4 * kCountTB) {
+        uint32_t v[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            v[u] = key[from + (i + u * kCountTB < n ? i + u * kCountTB : i)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (i + u * kCountTB < n)
+                atomicAdd(&count[v[u] & mask], 1u);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i <= mask; i += kCountTB)
+        counts[((uint64_t)g << low) + i] = count[i];
+}
+__global__ void bucket_sum_k(const uint32_t *__restrict__ counts, const uint32_t *__restrict__ first_part,
+                             uint32_t low, uint64_t nbins, uint32_t *cnt)
+{
+    GRID_STRIDE(c, nbins)
+    {
+        const uint32_t b = (uint32_t)(c >> low), at = (uint32_t)c & ((1u << low) - 1);
+        uint32_t sum = 0;
+        for (uint32_t g = first_part[b]; g < first_part[b + 1]; ++g)
+            sum += counts[((uint64_t)g << low) + at];
+        cnt[c] = sum;
     }
 }
 
@@ -856,17 +937,6 @@ int sort_pairs(Temp &tmp, const KeyT *kin, KeyT *kout, const uint32_t *vin, uint
     return SPC3D_OK;
 }
 
-// Ascending sort of keys on key bits [0, bits).
-int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bits,
-              const DevStream &st, std::string &err)
-{
-    size_t bytes = 0;
-    HIP_OK(rocprim::radix_sort_keys<SortConfig>(nullptr, bytes, kin, kout, (size_t)n, 0u, (unsigned)bits, st));
-    HIP_OK(tmp.need(bytes));
-    HIP_OK(rocprim::radix_sort_keys<SortConfig>(tmp.p, bytes, kin, kout, (size_t)n, 0u, (unsigned)bits, st));
-    return SPC3D_OK;
-}
-
 #define LAUNCH(kernel, n, ...)                                                                    \
     hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kTB), 0, st, __VA_ARGS__)
 #define LAUNCH_SMALL(kernel, n, ...)                                                              \
@@ -881,6 +951,38 @@ int sort_keys(Temp &tmp, const uint32_t *kin, uint32_t *kout, uint32_t n, int bi
         if (rc_ != SPC3D_OK)                                                                      \
             return rc_;                                                                           \
     } while (0)
+
+// cnt[id] = how often id < nbins comes among n ids of an arbitrary order.  A device-wide atomic per entry is
+// served at the memory side, 1.5 ms for 16.8 M; sorting the ids and finding the runs takes 320 us; what is done, one
+// digit of that sort at most (to 4 M bins) and counters in LDS, 190.  `scratch` is for n ids.
+int count_ids(Temp &tmp, Arena &arena, const uint32_t *ids, uint32_t n, uint32_t nbins, uint32_t *scratch,
+              uint32_t *cnt, const DevStream &st, std::string &err)
+{
+    const uint32_t bits = (uint32_t)bits_for(nbins ? nbins - 1 : 0);
+    const uint32_t low = bits <= kCountBits ? bits : std::min(kCountBits, bits - 8); // (a digit has 8 bits)
+    const uint32_t nbuckets = ((nbins ? nbins - 1 : 0) >> low) + 1;
+    const uint32_t part = std::max(n / 64, 1u << 16);
+    const uint32_t most = n / part + nbuckets; // parts
+    if (low < bits) {
+        size_t bytes = 0;
+        HIP_OK(rocprim::radix_sort_keys<SortConfig>(nullptr, bytes, ids, scratch, (size_t)n, low, bits, st));
+        HIP_OK(tmp.need(bytes));
+        HIP_OK(rocprim::radix_sort_keys<SortConfig>(tmp.p, bytes, ids, scratch, (size_t)n, low, bits, st));
+        ids = scratch;
+    }
+    SBuf<uint32_t> start, parts, first_part, counts;
+    HIP_OK(start.alloc(arena, (size_t)nbuckets + 1));
+    HIP_OK(parts.alloc(arena, (size_t)nbuckets + 1));
+    HIP_OK(first_part.alloc(arena, (size_t)nbuckets + 1));
+    HIP_OK(counts.alloc(arena, (size_t)most << low));
+    hipLaunchKernelGGL(bucket_parts_k, dim3(nbuckets / (kTB / 64) + 1), dim3(kTB), 0, st, ids, n, low, nbuckets, part,
+                       start.p, parts.p);
+    TRY(exclusive_sum(tmp, parts.p, first_part.p, (size_t)nbuckets + 1, st, err));
+    hipLaunchKernelGGL(bucket_count_k, dim3(most), dim3(kCountTB), 0, st, ids, start.p, first_part.p, low, nbuckets,
+                       part, counts.p);
+    LAUNCH(bucket_sum_k, nbins, counts.p, first_part.p, low, (uint64_t)nbins, cnt);
+    return SPC3D_OK;
+}
 
 struct Fetch { // bytes from dev to host
     void *host;
@@ -1070,29 +1172,23 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     {
         SBuf<uint32_t> sorted, start;
         HIP_OK(sorted.alloc(arena, nnz));
-        HIP_OK(start.alloc(arena, std::max<size_t>(ncols, nrows)));
-        // Rows that come in runs are counted run by run (hist_sorted_k); an arbitrary order would be an
-        // atomic per entry, 1.5 ms for 16 M, and is sorted, 0.33 ms, which eight per run still beat.
+        HIP_OK(start.alloc(arena, ncols));
+        // Rows that come in runs are counted run by run (hist_sorted_k), which eight per run already pay for.
         if (rows_unsorted && (uint64_t)hC.row_changes * 8 > nnz) {
-            TRY(sort_keys(tmp, d_ii, sorted.p, (uint32_t)nnz, bits_for(nrows ? nrows - 1 : 0), st,
-                          err));
-            LAUNCH(run_bounds_k, nnz, sorted.p, nnz, nrows, start.p, rowcnt.p);
-            LAUNCH(run_lengths_k, nrows, start.p, (uint64_t)nrows, rowcnt.p);
+            TRY(count_ids(tmp, arena, d_ii, (uint32_t)nnz, nrows, sorted.p, rowcnt.p, st, err));
         } else {
             LAUNCH(hist_sorted_k, nnz, d_ii, nnz, rowcnt.p);
         }
-        const uint32_t *by_col = sorted.p;
         if (by_column) { // the visiting order of order_entries; its sorted columns in `col`
             HIP_OK(visit.alloc(arena, nnz));
             LAUNCH(iota_k, nnz, sorted.p, nnz);
             TRY(sort_pairs<uint32_t>(tmp, d_jj, col.p, sorted.p, visit.p, (uint32_t)nnz, col_bits,
                                      false, st, err));
-            by_col = col.p;
+            LAUNCH(run_bounds_k, nnz, col.p, nnz, ncols, start.p, coldeg.p);
+            LAUNCH(run_lengths_k, ncols, start.p, (uint64_t)ncols, coldeg.p);
         } else {
-            TRY(sort_keys(tmp, d_jj, sorted.p, (uint32_t)nnz, col_bits, st, err));
+            TRY(count_ids(tmp, arena, d_jj, (uint32_t)nnz, ncols, sorted.p, coldeg.p, st, err));
         }
-        LAUNCH(run_bounds_k, nnz, by_col, nnz, ncols, start.p, coldeg.p);
-        LAUNCH(run_lengths_k, ncols, start.p, (uint64_t)ncols, coldeg.p);
     }
     LAUNCH_FEW(stats_k, nrows, rowcnt.p, (uint64_t)nrows, &dC.p->rows_touched, &dC.p->max_row,
                  &dC.p->row_sq);
@@ -1495,7 +1591,7 @@ int stable_ranks_device(const DevStream &st, const uint32_t *d_key, uint64_t n, 
 // whose caller's positions are not perm[start], perm[start] + 1, ...
 constexpr uint32_t kFlagLanes = 16;
 __global__ void staged_flags_k(const Seg *__restrict__ segs, uint32_t nseg,
-                               const uint32_t *__restrict__ perm, uint32_t *__restrict__ flag)
+                               const uint32_t *__restrict__ perm, uint8_t *__restrict__ flag)
 {
     const uint32_t sub = threadIdx.x % kFlagLanes;
     GRID_STRIDE(t, (uint64_t)nseg * kFlagLanes) // a group's lanes go round together
@@ -1513,27 +1609,107 @@ __global__ void staged_flags_k(const Seg *__restrict__ segs, uint32_t nseg,
             for (uint32_t v = 0; v < 4; ++v)
                 bad |= p[v] != base + u + v * kFlagLanes;
         }
-        const uint32_t any =
-            (__ballot(bad) >> (threadIdx.x & 63u & ~(kFlagLanes - 1))) & ((1ull << kFlagLanes) - 1) ? 1u : 0u;
+        const uint8_t any =
+            (__ballot(bad) >> (threadIdx.x & 63u & ~(kFlagLanes - 1))) & ((1ull << kFlagLanes) - 1) ? 1 : 0;
         for (uint32_t u = sub; u < sg.len; u += kFlagLanes)
             flag[sg.start + u] = any;
     }
 }
 
-__global__ void staged_fill_k(const uint32_t *__restrict__ perm, const uint32_t *__restrict__ flag,
-                              const uint32_t *__restrict__ idx, uint64_t nnz, uint32_t *perm2,
-                              uint32_t *key, uint32_t *val)
+// Numbers for what is marked of n items, in their order: every tile of kMarkTile items counted (count_marks_k),
+// a sum over the counts, then a tile's own (mark_ranks).
+constexpr int kMarkRounds = 16;
+constexpr uint32_t kMarkTile = kTB * kMarkRounds;
+constexpr uint32_t kNoHome = 0xFFFFFFFFu;
+__device__ __forceinline__ bool marked(uint8_t v) { return v != 0; }
+__device__ __forceinline__ bool marked(uint32_t v) { return v != kNoHome; }
+
+template <typename T> __global__ void count_marks_k(const T *__restrict__ v, uint64_t n, uint32_t *cnt)
 {
-    GRID_STRIDE(p, nnz)
-    {
-        if (flag[p]) {
-            perm2[p] = (uint32_t)nnz + idx[p];
-            key[idx[p]] = perm[p];
-            val[idx[p]] = idx[p];
-        } else {
-            perm2[p] = perm[p];
-        }
+    const uint64_t base = (uint64_t)blockIdx.x * kMarkTile + threadIdx.x;
+    uint32_t c = 0;
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u)
+        c += base + u * kTB < n && marked(v[base + u * kTB]);
+    c = block_sum(c);
+    if (threadIdx.x == 0) {
+        cnt[blockIdx.x] = c;
+        if (blockIdx.x == 0)
+            cnt[gridDim.x] = 0; // the sum's last word is the total
     }
+}
+// rank[u]: how many are marked before item u * kTB + threadIdx.x of the tile, from `before` on.
+__device__ __forceinline__ void mark_ranks(const bool (&on)[kMarkRounds], uint32_t before, uint32_t (&rank)[kMarkRounds])
+{
+    constexpr int kWaves = kTB / 64;
+    static_assert(kMarkRounds * kWaves == 64, "one count for every lane");
+    __shared__ uint32_t part[64];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u) {
+        const unsigned long long m = __ballot(on[u]);
+        rank[u] = (uint32_t)__popcll(m & ((1ull << lane) - 1));
+        if (lane == 0)
+            part[u * kWaves + w] = (uint32_t)__popcll(m);
+    }
+    __syncthreads();
+    if (w == 0) {
+        const uint32_t mine = part[lane];
+        uint32_t upto = mine;
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(upto, d, 64);
+            upto += lane >= d ? o : 0u;
+        }
+        part[lane] = before + upto - mine;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u)
+        rank[u] += part[u * kWaves + w];
+}
+
+// A staged entry's slot is its number among them; home: of every caller's position the slot, or kNoHome.
+__global__ void staged_fill_k(const uint32_t *__restrict__ perm, const uint8_t *__restrict__ flag,
+                              const uint32_t *__restrict__ before, uint64_t nnz, uint32_t *perm2,
+                              uint32_t *home)
+{
+    const uint64_t base = (uint64_t)blockIdx.x * kMarkTile + threadIdx.x;
+    bool on[kMarkRounds];
+    uint32_t at[kMarkRounds], slot[kMarkRounds];
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u) {
+        const uint64_t p = base + u * kTB < nnz ? base + u * kTB : nnz - 1;
+        on[u] = base + u * kTB < nnz && flag[p];
+        at[u] = perm[p];
+    }
+    mark_ranks(on, before[blockIdx.x], slot);
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u)
+        if (base + u * kTB < nnz) {
+            perm2[base + u * kTB] = on[u] ? (uint32_t)nnz + slot[u] : at[u];
+            home[at[u]] = on[u] ? slot[u] : kNoHome;
+        }
+}
+// The staged results in the caller's order.  This is a sort of (position, slot) pairs whose keys are all
+// different: 10.5 M of 16.8 M positions, rows sorted, 310 us by digits and 60 with home written, counted and packed.
+__global__ void staged_order_k(const uint32_t *__restrict__ home, const uint32_t *__restrict__ before, uint64_t nnz,
+                               uint32_t *dst, uint32_t *src)
+{
+    const uint64_t base = (uint64_t)blockIdx.x * kMarkTile + threadIdx.x;
+    bool on[kMarkRounds];
+    uint32_t slot[kMarkRounds], h[kMarkRounds];
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u) {
+        slot[u] = home[base + u * kTB < nnz ? base + u * kTB : nnz - 1];
+        on[u] = base + u * kTB < nnz && marked(slot[u]);
+    }
+    mark_ranks(on, before[blockIdx.x], h);
+#pragma unroll
+    for (int u = 0; u < kMarkRounds; ++u)
+        if (on[u]) {
+            dst[h[u]] = (uint32_t)(base + u * kTB);
+            src[h[u]] = slot[u];
+        }
 }
 
 // How many neighbours follow each other.  Four loads in flight per thread: with one this small grid
@@ -1583,24 +1759,31 @@ __global__ void near_k(const uint32_t *__restrict__ v, uint64_t n, unsigned long
         atomicAdd(acc, c);
 }
 
-// How many of the n staged results are read next to another one of the same wavefront of
-// the final pass (64 consecutive h): src[h] - 1 is the src of another lane.
-__global__ void src_neighbours_k(const uint32_t *__restrict__ src, uint64_t n, unsigned long long *acc)
+// How many of the staged results are read next to another one of the same wavefront of
+// the final pass (64 consecutive h): src[h] - 1 is the src of another lane.  Of every `every`-th wavefront's
+// (a share is asked for, and 10 M results took 135 us; acc[1]: how many were looked at).
+__global__ void src_neighbours_k(const uint32_t *__restrict__ src, uint64_t n, uint32_t every,
+                                 unsigned long long *acc)
 {
-    unsigned long long c = 0;
-    const uint64_t nround = (n + 63) / 64 * 64;
-    GRID_STRIDE(h, nround)
+    unsigned long long c = 0, looked = 0;
+    const uint64_t nround = (n + (uint64_t)64 * every - 1) / ((uint64_t)64 * every) * 64;
+    GRID_STRIDE(i, nround)
     {
+        const uint64_t h = i / 64 * 64 * every + i % 64;
         const uint32_t mine = h < n ? src[h] : 0xFFFFFFFFu;
         bool near = false;
         for (int j = 0; j < 64; ++j)
             near |= __shfl(mine, j) + 1 == mine;
+        looked += h < n;
         if (h < n && near)
             ++c;
     }
-    c = wave_sum(c);
-    if ((threadIdx.x & 63u) == 0 && c)
+    c = block_sum(c);
+    looked = block_sum(looked);
+    if (threadIdx.x == 0 && looked) {
         atomicAdd(acc, c);
+        atomicAdd(acc + 1, looked);
+    }
 }
 
 int build_store_staging(const DevStream &st, const Seg *d_segs, uint32_t nseg, const uint32_t *d_perm,
@@ -1610,51 +1793,52 @@ int build_store_staging(const DevStream &st, const Seg *d_segs, uint32_t nseg, c
     if (!d_perm || nnz == 0 || nseg == 0 || nnz >= (1ull << 31))
         return SPC3D_OK;
     Arena arena(st);
-    HIP_OK(arena.reserve((size_t)nnz * 8 + ((size_t)8 << 20)));
+    HIP_OK(arena.reserve((size_t)nnz * 6 + ((size_t)8 << 20)));
     Temp tmp(arena);
-    SBuf<uint32_t> flag, idx;
+    const uint32_t ntiles = (uint32_t)((nnz + kMarkTile - 1) / kMarkTile);
+    SBuf<uint8_t> flag;
+    SBuf<uint32_t> cnt, before, home;
     HIP_OK(flag.alloc(arena, nnz));
-    HIP_OK(idx.alloc(arena, nnz));
-    HIP_OK(hipMemsetAsync(flag.p, 0, (size_t)nnz * 4, st));
+    HIP_OK(cnt.alloc(arena, (size_t)ntiles + 1));
+    HIP_OK(before.alloc(arena, (size_t)ntiles + 1));
+    HIP_OK(hipMemsetAsync(flag.p, 0, (size_t)nnz, st));
     LAUNCH(staged_flags_k, (uint64_t)nseg * kFlagLanes, d_segs, nseg, d_perm, flag.p);
-    TRY(exclusive_sum<uint32_t>(tmp, flag.p, idx.p, (size_t)nnz, st, err));
-    uint32_t last[2] = {0, 0};
+    hipLaunchKernelGGL(count_marks_k<uint8_t>, dim3(ntiles), dim3(kTB), 0, st, flag.p, nnz, cnt.p);
+    TRY(exclusive_sum(tmp, cnt.p, before.p, (size_t)ntiles + 1, st, err));
+    uint32_t n = 0;
     DBuf<unsigned long long> acc;
-    HIP_OK(acc.alloc(st, 3));
-    HIP_OK(hipMemsetAsync(acc.p, 0, 3 * sizeof(unsigned long long), st));
-    LAUNCH_SMALL(near_k, nnz, d_perm, nnz, acc.p + 2);
+    HIP_OK(acc.alloc(st, 4));
+    HIP_OK(hipMemsetAsync(acc.p, 0, 4 * sizeof(unsigned long long), st));
+    LAUNCH_SMALL(near_k, nnz, d_perm, nnz, acc.p + 3);
     unsigned long long near = 0;
-    TRY(fetch_all(st, {{&last[0], idx.p + (nnz - 1), 4},
-                       {&last[1], flag.p + (nnz - 1), 4},
-                       {&near, acc.p + 2, sizeof near}}, err));
-    const uint64_t n = (uint64_t)last[0] + last[1];
+    TRY(fetch_all(st, {{&n, before.p + ntiles, sizeof n}, {&near, acc.p + 3, sizeof near}}, err));
     if (n == 0) {
         out.consecutive = true;
         return SPC3D_OK;
     }
     if (nnz + n >= (1ull << 32))
         return SPC3D_OK;
-    // What the last check below would turn down, before the sort for it (R-MAT 20 with its rows and
-    // columns renumbered: 0.55 ms)
-    if (n * 4 >= nnz * 3 && near / 32 < n)
+    // What the last check below would turn down, before the work for it (R-MAT 20 with its rows and
+    // columns renumbered)
+    if ((uint64_t)n * 4 >= nnz * 3 && near / 32 < n)
         return SPC3D_OK;
     DBuf<uint32_t> perm2, dst, src;
     HIP_OK(perm2.alloc(st, nnz));
     HIP_OK(dst.alloc(st, n));
     HIP_OK(src.alloc(st, n));
-    SBuf<uint32_t> key, val;
-    HIP_OK(key.alloc(arena, n));
-    HIP_OK(val.alloc(arena, n));
-    LAUNCH(staged_fill_k, nnz, d_perm, flag.p, idx.p, nnz, perm2.p, key.p, val.p);
-    TRY(sort_pairs<uint32_t>(tmp, key.p, dst.p, val.p, src.p, (uint32_t)n, bits_for(nnz - 1), false,
-                             st, err));
+    HIP_OK(home.alloc(arena, nnz));
+    hipLaunchKernelGGL(staged_fill_k, dim3(ntiles), dim3(kTB), 0, st, d_perm, flag.p, before.p, nnz, perm2.p, home.p);
+    hipLaunchKernelGGL(count_marks_k<uint32_t>, dim3(ntiles), dim3(kTB), 0, st, home.p, nnz, cnt.p);
+    TRY(exclusive_sum(tmp, cnt.p, before.p, (size_t)ntiles + 1, st, err));
+    hipLaunchKernelGGL(staged_order_k, dim3(ntiles), dim3(kTB), 0, st, home.p, before.p, nnz, dst.p, src.p);
     // The final pass pays when it writes runs and reads near what its neighbours read; an
     // arbitrary order of the entries gives neither, and keeps its scattered stores.
-    LAUNCH_SMALL(adjacent_k, n, dst.p, n, acc.p);
-    LAUNCH_SMALL(src_neighbours_k, n, src.p, n, acc.p + 1);
-    unsigned long long seen[2] = {0, 0};
+    LAUNCH_SMALL(adjacent_k, n, dst.p, (uint64_t)n, acc.p);
+    const uint32_t every = n >= (1u << 20) ? 16 : 1;
+    LAUNCH_SMALL(src_neighbours_k, n / every + 1, src.p, (uint64_t)n, every, acc.p + 1);
+    unsigned long long seen[3] = {0, 0, 0};
     TRY(fetch(st, seen, acc.p, sizeof seen, err));
-    if (seen[0] * 2 < n || seen[1] * 2 < n)
+    if (seen[0] * 2 < n || seen[1] * 2 < seen[2])
         return SPC3D_OK; // (the DBufs free themselves)
     out.perm2 = perm2.release();
     out.dst = dst.release();
