@@ -57,3 +57,19 @@ def test_staged_results_come_home(ctx, nnz):
         got.append(dC.download())
         S.close()
     assert np.array_equal(got[0], got[1]) and not np.isnan(got[0]).any()
+
+
+# entries that come in the order of their rows, 1024 of them to a wavefront, 64 at a time: rows that end where
+# those do or next to it, go over several, and the whole pattern; hub rows from 1 entry on and from 64
+@pytest.mark.parametrize("lengths", [[1024] * 5, [1023, 1, 1024, 1025, 1], [64] * 40, [63, 65, 2, 0, 300] * 30,
+                                     [5000, 3, 9000, 1, 1], [20000], [1] * 500 + [2048, 7, 4096] + [2] * 300,
+                                     [1, 70000, 1], [130] * 600])
+@pytest.mark.parametrize("hub_min", [1, 64])
+def test_rows_in_order(ctx, lengths, hub_min):
+    rng = np.random.default_rng(len(lengths))
+    ii = np.repeat(np.arange(len(lengths), dtype=np.uint32), lengths)
+    n = 4000
+    jj = np.minimum(rng.pareto(0.6, ii.size) * 4, n - 1).astype(np.uint32)
+    P = both(ctx, len(lengths), n, ii, jj, xcd_slices=8, l2_hot_bytes=256, hub_min=hub_min, k_hint=4, seg_max=500)
+    assert P["info"].nqueues == 8 and P["info"].hub_rows == sum(v >= hub_min for v in lengths)
+    both(ctx, len(lengths), n, ii, jj, xcd_slices=1)
