@@ -185,6 +185,13 @@ typedef struct {
                               SPC3D_PLAN_KEEP_ENTRY_ORDER: they add block after block.  They
                               make the plan 0.76 to 1.05 ms slower at 6 to 10 M entries, which
                               three to five steps repay: for a plan of fewer calls, sweep = 1.
+                              Where its columns are skewed (XCD slices) and a call gathers
+                              2.5 GiB and more, it holds tiles of its longest rows, one to a
+                              CU (device_bytes only; none where seg_max is given): spc3d_sddmm, spc3d_spmm and
+                              spc3d_spmm_noalloc at K = k_hint run over them and the segments
+                              of the other rows.  They make the plan 0.4 to 0.5 ms slower at
+                              16 M entries (one step of fp64, K = 64, repays that; of fp32,
+                              ten).
                               0 (default): as described; 1: never; 2: whenever k_hint has such
                               a width, whatever the pattern (col_blocks, if given, is the
                               number of blocks) */

@@ -745,6 +745,40 @@ static void *staged_out(const spc3d_plan *parent, const spc3d_plan *)
     return static_cast<char *>(parent->c_stage) + parent->rest_off * elem_size(parent->dtype);
 }
 
+// One plan's SDDMM and SpMM at K columns: over its tiles and the segments of the other rows where it has
+// tiles for that width, else over its segments.
+static hipError_t single_sddmm(const spc3d_plan *S, const void *A, const void *B, void *C, uint32_t K)
+{
+    const Streams st = streams_of(S->ctx);
+    if (S->hub.n && K == S->hub_k && (S->hub.direct || S->hub_stage)) {
+        SweepView v = hub_view_of(S);
+        if (S->hub.direct)
+            v.pos = S->hub.perm;
+        void *out = S->hub_by_pos ? C : sddmm_out(S, C);
+        const hipError_t e = launch_hub_sddmm(S->dtype, rest_view_of(S), v, A, B, out, S->hub_stage, st);
+        if (e != hipErrorNotSupported)
+            return e == hipSuccess && !S->hub_by_pos ? finish_sddmm(S, C) : e;
+    }
+    const hipError_t e = launch_sddmm(S->dtype, view_of(S), A, B, sddmm_out(S, C), K, st);
+    return e != hipSuccess ? e : finish_sddmm(S, C);
+}
+static hipError_t single_spmm(const spc3d_plan *S, const DevPlanView &view, const void *X, void *Y, uint32_t K)
+{
+    const Streams st = streams_of(S->ctx);
+    if (S->hub.n && K == S->hub_k) {
+        DevPlanView v = rest_view_of(S);
+        const hipError_t e = launch_hub_spmm(S->dtype, v, hub_view_of(S), X, Y, st);
+        if (e != hipErrorNotSupported) {
+            v.splits = S->hub.splits;
+            v.nsplit = S->hub.nsplit;
+            v.nslots = S->hub.nslots;
+            v.partial = S->hub_partial;
+            return e != hipSuccess ? e : launch_split_sums(S->dtype, v, Y, K, st.main);
+        }
+    }
+    return launch_spmm(S->dtype, view, X, Y, K, st);
+}
+
 /* ---- hot path ------------------------------------------------------------ */
 int spc3d_sddmm(spc3d_ctx *ctx, spc3d_plan *S, const spc3d_panel *A, const spc3d_panel *B,
                 spc3d_vals *C)
@@ -782,15 +816,11 @@ int spc3d_sddmm(spc3d_ctx *ctx, spc3d_plan *S, const spc3d_panel *A, const spc3d
     if (S->tiles_sddmm && K == S->tiles->sweep_k)
         S = S->tiles;
     if (S->by_col) { // the same entries with rows and columns, and so A and B, exchanged
-        const spc3d_plan *T = S->by_col;
-        HIP_TRY(launch_sddmm(S->dtype, view_of(T), B->dev, A->dev, C->dev, K, streams_of(ctx)));
-        HIP_TRY(unstage_stores(T, C->dev));
+        HIP_TRY(single_sddmm(S->by_col, B->dev, A->dev, C->dev, K));
         return SPC3D_OK;
     }
     if (S->blocks.empty() && !S->sweep.n) {
-        HIP_TRY(launch_sddmm(S->dtype, view_of(S), A->dev, B->dev, sddmm_out(S, C->dev), K,
-                             streams_of(ctx)));
-        HIP_TRY(finish_sddmm(S, C->dev));
+        HIP_TRY(single_sddmm(S, A->dev, B->dev, C->dev, K));
         return SPC3D_OK;
     }
     if (S->sweep.n && !S->c_stage) { // the tiles and the rest store at the caller's positions
@@ -859,7 +889,7 @@ int spc3d_spmm(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc3d_panel
     }
     // The blocks add into Y one after the other on the stream: a fixed order.
     for (spc3d_plan *part : parts_of(Ap, self))
-        HIP_TRY(launch_spmm(Ap->dtype, view_of(part), X->dev, Y->dev, K, streams_of(ctx)));
+        HIP_TRY(single_spmm(part, view_of(part), X->dev, Y->dev, K));
     if (Ap->sweep.n) // rows of their own: none of them is in the plan of the rest
         HIP_TRY(launch_sweep_spmm(Ap->dtype, sweep_view_of(Ap), X->dev, Y->dev, ctx->stream));
     return SPC3D_OK;
@@ -903,10 +933,11 @@ int spc3d_spmm_noalloc(spc3d_ctx *ctx, spc3d_plan *Ap, const spc3d_panel *X, spc
     // npartial_slots is the largest block's.)
     // no container: no host heap either
     for (size_t i = 0; i < nparts; ++i) {
-        DevPlanView view = view_of(Ap->blocks.empty() ? Ap : Ap->blocks[i]);
+        const spc3d_plan *part = Ap->blocks.empty() ? Ap : Ap->blocks[i];
+        DevPlanView view = view_of(part);
         view.partial = ctx->scratch;
         view.partial_cols = cols;
-        HIP_TRY(launch_spmm(Ap->dtype, view, X->dev, Y->dev, K, streams_of(ctx)));
+        HIP_TRY(single_spmm(part, view, X->dev, Y->dev, K)); // (the tiles' partial sums are the plan's)
     }
     if (Ap->sweep.n) // the tiles' sums live in LDS: nothing to allocate either
         HIP_TRY(launch_sweep_spmm(Ap->dtype, sweep_view_of(Ap), X->dev, Y->dev, ctx->stream));

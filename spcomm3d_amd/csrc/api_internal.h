@@ -213,6 +213,15 @@ struct spc3d_plan {
     // faster so (add_tiles).
     spc3d_plan *tiles = nullptr;
     bool tiles_sddmm = false, tiles_spmm = false; // which of them
+    // A sliced plan's longest rows once more as tiles (HubTiles in plan_device.h), for the calls at hub_k
+    // columns; the other rows' segments in hub.rest, with their table of first columns (like hub.col in the hot
+    // form where the plan has one).
+    HubTiles hub;
+    uint32_t hub_k = 0, hub_lanes = 0;
+    bool hub_by_pos = true; // SDDMM's results go to the caller's positions, else to the kernel's (two)
+    bool hub_by_kernel = false; // hub.perm counts in kernel order, else in the caller's
+    uint32_t *hub_first_cols = nullptr;
+    void *hub_sval = nullptr, *hub_stage = nullptr, *hub_partial = nullptr; // values, results, partial sums
 };
 
 inline SweepView sweep_view_of(const spc3d_plan *p)
@@ -229,6 +238,28 @@ inline SweepView sweep_view_of(const spc3d_plan *p)
     v.rows_per_tile = p->sweep.rows_per_tile;
     v.lanes = p->sweep.lanes;
     v.per_launch = p->sweep.per_launch;
+    return v;
+}
+
+inline SweepView hub_view_of(const spc3d_plan *p)
+{
+    SweepView v;
+    v.ptr = p->hub.ptr;
+    v.tile_rows = p->hub.tile_rows;
+    v.col = p->hub.col;
+    v.lrow = p->hub.lrow;
+    v.sval = p->hub_sval;
+    v.slot = p->hub.nsplit ? p->hub.slot : nullptr;
+    v.partial = p->hub_partial;
+    v.src = p->hub.src;
+    v.dst = p->hub.dst;
+    v.rest_entries = p->info.nnz - p->hub.n;
+    v.ntiles = p->hub.ntiles;
+    v.nblocks = p->hub.nblocks;
+    v.K = p->hub_k;
+    v.lanes = p->hub_lanes;
+    v.rows_per_tile = sweep_rows_per_tile(p->hub_lanes);
+    v.per_launch = (uint32_t)std::max(1, p->ctx->cu_count);
     return v;
 }
 
@@ -451,6 +482,19 @@ inline DevPlanView view_of(const spc3d_plan *p)
         v.stage = p->c_stage;
         v.stage_from = (uint32_t)p->info.nnz;
     }
+    return v;
+}
+// The rows beside the tiles of a sliced plan.
+inline DevPlanView rest_view_of(const spc3d_plan *p)
+{
+    DevPlanView v = view_of(p);
+    v.segs = p->hub.rest;
+    v.nseg = p->hub.nrest;
+    v.nseg_long = 0;
+    v.first_cols = v.hot_first_cols = p->hub_first_cols;
+    if (p->two.n && p->hub_by_pos)
+        v.perm = p->perm;
+    v.nsplit = v.nslots = 0;
     return v;
 }
 

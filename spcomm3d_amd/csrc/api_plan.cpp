@@ -327,6 +327,27 @@ static int add_hot_rows(spc3d_plan *p, uint32_t k0)
     return SPC3D_OK;
 }
 
+static void free_hub_tiles(spc3d_ctx *ctx, HubTiles &t)
+{
+    for (uint32_t *a : {t.col, t.perm, t.ptr, t.tile_rows, t.slot, t.src, t.dst})
+        if (a) ctx_free(ctx, a);
+    if (t.lrow) ctx_free(ctx, t.lrow);
+    if (t.splits) ctx_free(ctx, t.splits);
+    if (t.rest) ctx_free(ctx, t.rest);
+    t = HubTiles();
+}
+static void drop_hub_tiles(spc3d_plan *p)
+{
+    free_hub_tiles(p->ctx, p->hub);
+    if (p->hub_first_cols) ctx_free(p->ctx, p->hub_first_cols);
+    p->hub_first_cols = nullptr;
+    for (void **a : {&p->hub_sval, &p->hub_stage, &p->hub_partial}) {
+        if (*a) ctx_free(p->ctx, *a);
+        *a = nullptr;
+    }
+    p->hub_k = p->hub_lanes = 0;
+}
+
 static void destroy_blocks(spc3d_plan *p)
 {
     for (spc3d_plan *b : p->blocks) {
@@ -388,12 +409,120 @@ static void choose_col_blocks(spc3d_plan *p, const spc3d_plan_opts *opts, uint32
         *nblocks = (uint32_t)nb;
 }
 
+// Row tiles beside a sliced plan (spc3d_plan::hub), from so many bytes of gathered rows on.  The calls are then
+// bound by what misses the L2s no longer, but a call pays for the start of 256 tiles, the barriers between their
+// blocks and the pass that brings SDDMM's results home, so it has to gather much.
+// R-MAT patterns of 2^17 to 2^20 rows, 4 to 32 entries per row, time over the segments / over the tiles and the
+// segments of the other rows: gathers of 0.5 - 1 GiB 1 / 1 - 1.4, to 1.9 GiB 1 / 0.95 - 1.1, from 2.5 GiB on SDDMM
+// 1 / 0.77 - 0.98, SpMM 1 / 0.77 - 1.02 (16.8 M entries, fp64: K = 64 872 / 685 us and 778 / 698; K = 17 level).
+// Fewer and longer rows gain more: 12.7 M entries in 1000 to 128000 rows, 3 GiB, 1 / 0.67 - 0.77 and 1 / 0.77 - 0.92.
+constexpr uint64_t kHubGather = (uint64_t)5 << 29;
+// Of an L2's 4 MiB; the tiles of an XCD are not in the same block at the same moment, so more of it is too much and
+// less only adds barriers (R-MAT 20, fp64: 3.5 - 7 MiB level within 1 %, 10 MiB 4 % slower).
+constexpr uint64_t kHubBlock = (uint64_t)5 << 20;
+// With fewer the panel nearly fits the L2s.
+constexpr uint32_t kHubMinBlocks = 4;
+// Rows of fewer entries gain nothing from a place in a tile (8 and 12 level, 16 up to 3 % slower, 4 fills more tiles).
+constexpr uint32_t kHubMinRow = 8;
+static bool wants_hub_tiles(int dtype, uint64_t nnz, const spc3d_plan_opts *opts, const PlanOpts &po)
+{
+    // (a caller who sets seg_max says how rows are cut, and with it the order of their sums)
+    return opts && !opts->sweep && !opts->col_blocks && !opts->seg_max && !po.keep_entry_order && !po.one_call &&
+           nnz * opts->k_hint * elem_size(dtype) >= kHubGather;
+}
+
+// What build_device_plan kept for row tiles (DevPlanArrays::rowptr, coldeg), until the plan is made.
+struct KeptCounts {
+    spc3d_ctx *ctx;
+    uint32_t *rowptr, *coldeg;
+    KeptCounts(spc3d_ctx *c, const DevPlanArrays &arr) : ctx(c), rowptr(arr.rowptr), coldeg(arr.coldeg) {}
+    KeptCounts(const KeptCounts &) = delete;
+    KeptCounts &operator=(const KeptCounts &) = delete;
+    ~KeptCounts()
+    {
+        if (rowptr) ctx_free(ctx, rowptr);
+        if (coldeg) ctx_free(ctx, coldeg);
+    }
+    // The pattern by row: the caller's own arrays where they are in that order, else the plan's kernel order.
+    // Results go to the caller's positions where a row's lie together, whatever their order; elsewhere to the
+    // kernel's, from which two passes bring them home.
+    HubSource source(const spc3d_plan *p, const HostPlan &meta, const uint32_t *d_jj) const
+    {
+        HubSource s;
+        s.nrows = p->info.nrows;
+        s.ncols = p->info.ncols;
+        s.nnz = p->info.nnz;
+        s.rowptr = rowptr;
+        s.coldeg = coldeg;
+        s.by_pos = !p->two.n || meta.row_runs == meta.rows_touched;
+        const bool callers = meta.rows_sorted && s.by_pos;
+        s.col = callers ? d_jj : p->col;
+        s.pos = callers ? nullptr : p->perm;
+        return s;
+    }
+};
+
+// Row tiles beside a finished sliced plan `p` (spc3d_plan::hub) of the pattern that `in` gives by row, for its
+// longest rows.
+static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const spc3d_plan_opts *opts)
+{
+    const spc3d_plan_info &I = p->info;
+    if (!wants_hub_tiles(p->dtype, I.nnz, opts, po) || I.nqueues != kSlices || !in.rowptr || (p->store.n && in.pos))
+        return SPC3D_OK; // (staged results of rows beside the tiles would need the pass that brings them home)
+    const uint32_t lanes = sweep_lanes_any(p->dtype, opts->k_hint);
+    const uint64_t w = elem_size(p->dtype), row_bytes = (uint64_t)opts->k_hint * w;
+    if (!lanes)
+        return SPC3D_OK;
+    spc3d_ctx *ctx = p->ctx;
+    in.segs = p->segs;
+    in.nseg = I.nsegments_padded;
+    if (p->hot_rows) {
+        in.hot_cols = p->hot_cols;
+        in.nhot = p->nhot;
+    }
+    in.rows_per_tile = sweep_rows_per_tile(lanes);
+    in.per_launch = (uint32_t)std::max(1, ctx->cu_count);
+    in.results = !p->by_col;
+    in.min_row = opts->sweep_min_row ? opts->sweep_min_row : kHubMinRow;
+    in.must = std::min(po.hub_min ? po.hub_min : kDefaultHubMin, I.seg_max + 1);
+    in.row_bytes = row_bytes;
+    in.block_bytes = kHubBlock;
+    in.min_blocks = kHubMinBlocks;
+    in.max_blocks = sweep_max_blocks(lanes);
+    std::string err;
+    int rc = build_hub_tiles(dev_stream(ctx), in, p->hub, err);
+    if (rc)
+        return optional_path(fail(rc, err));
+    const HubTiles &t = p->hub;
+    if (t.n == 0)
+        return SPC3D_OK;
+    p->hub_k = opts->k_hint;
+    p->hub_lanes = lanes;
+    p->hub_by_pos = in.by_pos;
+    p->hub_by_kernel = in.col == p->col;
+    rc = ctx_alloc_bytes(ctx, &p->hub_sval, (size_t)t.n * w);
+    if (!rc && t.src) rc = ctx_alloc_bytes(ctx, &p->hub_stage, (size_t)t.n * w);
+    if (!rc) rc = ctx_alloc_bytes(ctx, &p->hub_partial, (size_t)t.nslots * row_bytes);
+    if (!rc) rc = ctx_alloc(ctx, &p->hub_first_cols, (size_t)t.nrest * kFirstCols);
+    if (!rc) {
+        const hipError_t e = launch_first_cols(t.rest, t.nrest, p->hot_rows ? p->hot_col : p->col, p->hub_first_cols,
+                                               ctx->stream);
+        if (e != hipSuccess)
+            rc = fail_hip(e, "first columns");
+    }
+    if (rc) {
+        drop_hub_tiles(p);
+        return optional_path(rc);
+    }
+    return SPC3D_OK;
+}
+
 // The companion plan for SDDMM (spc3d_plan::by_col) of a finished single plan whose results
 // would be stored one by one, when the pattern is sorted by column and the exchanged plan
 // does store in runs.  SPC3D_PLAN_NO_SDDMM_BY_COLUMN switches it off.
 static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, uint64_t nnz,
                                const uint32_t *d_ii, const uint32_t *d_jj, const PlanOpts &po,
-                               const StoreOpts &so)
+                               const StoreOpts &so, const spc3d_plan_opts *opts)
 {
     if (!so.by_column || nnz < 2 || !p->perm || p->store.consecutive || !p->blocks.empty() ||
         !p->cols_sorted)
@@ -401,18 +530,24 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
     std::string err;
     HostPlan meta;
     DevPlanArrays arr;
-    int rc = build_device_plan(dev_stream(p->ctx), ncols, nrows, nnz, d_jj, d_ii, po, meta, arr, err);
+    PlanOpts whole = po;
+    whole.keep_counts = wants_hub_tiles(p->dtype, nnz, opts, po);
+    int rc = build_device_plan(dev_stream(p->ctx), ncols, nrows, nnz, d_jj, d_ii, whole, meta, arr, err);
     if (rc)
         return optional_path(fail(rc, err));
+    KeptCounts counts(p->ctx, arr);
     spc3d_plan *q = nullptr;
     rc = adopt_device_plan(p->ctx, p->dtype, meta, arr, 0 /* never runs SpMM */, &q);
     if (!rc)
         rc = add_store_staging(q, so);
     if (!rc)
         rc = add_hot_rows(q, po.hot_row_bytes / (uint32_t)elem_size(p->dtype));
+    if (!rc && (!q->perm || q->store.consecutive))
+        rc = add_hub_tiles(q, counts.source(q, meta, d_ii), po, opts);
     if (rc || (q->perm && !q->store.consecutive)) { // no better than what there is
         if (q) {
             const std::string keep = g_err;
+            drop_hub_tiles(q);
             plan_free_device(q);
             q->magic = 0;
             delete q;
@@ -695,10 +830,12 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     DevPlanArrays arr;
     std::string err;
     const bool blocks = opts && opts->col_blocks > 1; // (for certain: choose_col_blocks follows the caller)
-    int rc = build_device_plan(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj,
-                               blocks ? without_hot_rows(po) : po, meta, arr, err);
+    PlanOpts whole = blocks ? without_hot_rows(po) : po;
+    whole.keep_counts = wants_hub_tiles(dtype, nnz, opts, po);
+    int rc = build_device_plan(dev_stream(ctx), nrows, ncols, nnz, d_ii, d_jj, whole, meta, arr, err);
     if (rc != SPC3D_OK)
         return fail(rc, err);
+    KeptCounts counts(ctx, arr);
     spc3d_plan *p = nullptr;
     rc = adopt_device_plan(ctx, dtype, meta, arr, planned_k(opts), &p);
     if (rc)
@@ -730,11 +867,13 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     if (!rc && nb <= 1)
         rc = add_store_staging(p, so);
     if (!rc && nb <= 1)
-        rc = add_sddmm_companion(p, nrows, ncols, nnz, d_ii, d_jj, po, so);
+        rc = add_sddmm_companion(p, nrows, ncols, nnz, d_ii, d_jj, po, so, opts);
     if (!rc && nb <= 1)
         rc = add_two_pass(p, so);
     if (!rc && nb <= 1)
         rc = add_tiles(p, nrows, ncols, nnz, d_ii, d_jj, po, opts);
+    if (!rc && nb <= 1)
+        rc = add_hub_tiles(p, counts.source(p, meta, d_jj), po, opts);
     if (rc || nb <= 1) {
         if (rc) {
             const std::string keep = g_err;
@@ -1131,18 +1270,18 @@ int spc3d_plan_destroy(spc3d_plan *plan)
         plan->tiles = nullptr;
     }
     if (plan->by_col) {
+        drop_hub_tiles(plan->by_col);
         plan_free_device(plan->by_col);
         plan->by_col->magic = 0;
         delete plan->by_col;
         plan->by_col = nullptr;
     }
+    drop_hub_tiles(plan);
     plan_free_device(plan);
     plan->magic = 0;
     delete plan;
     return SPC3D_OK;
 }
-
-
 
 // The values at `vals` (device, the caller's order) into every part of the plan but other_k.
 static hipError_t gather_values(spc3d_plan *plan, const void *vals)
@@ -1163,6 +1302,10 @@ static hipError_t gather_values(spc3d_plan *plan, const void *vals)
     }
     if (e == hipSuccess && plan->tiles)
         e = gather_values(plan->tiles, vals);
+    for (const spc3d_plan *part : {(const spc3d_plan *)plan, (const spc3d_plan *)plan->by_col})
+        if (e == hipSuccess && part && part->hub.n) // (from the plan's own, in whose order neighbours are near)
+            e = launch_gather_vals(plan->dtype, part->hub_by_kernel ? part->sval : vals, part->hub.perm, part->hub_sval,
+                                   part->hub.n, plan->ctx->stream);
     if (e == hipSuccess)
         plan->has_values = true;
     return e;
@@ -1179,7 +1322,8 @@ int spc3d_plan_set_values(spc3d_plan *plan, const void *vv_host)
     if (rc)
         return rc;
     const size_t bytes = (size_t)nnz * elem_size(plan->dtype);
-    if (plan->blocks.empty() && !plan->perm && !plan->by_col && !plan->sweep.n && !plan->tiles) {
+    if (plan->blocks.empty() && !plan->perm && !plan->by_col && !plan->sweep.n && !plan->tiles &&
+        !plan->hub.n) {
         rc = send_h2d(plan->ctx, plan->sval, vv_host, bytes);
     } else {
         void *tmp = nullptr;
@@ -1234,6 +1378,12 @@ static int probe_columns_of(spc3d_plan *p, int mode, uint32_t modulus)
     // the columns, the calls do without.  (Nothing is freed: recordings of the plan's calls may use it.)
     const int rc = p->hot_rows ? name_hot_columns(p) : SPC3D_OK;
     p->hot_stale = rc != SPC3D_OK;
+    if (!p->hub.n)
+        return rc;
+    // (plain columns from now on, which the kernels of the hot form take as well)
+    HIP_TRY(launch_probe_cols(p->hub.col, p->hub.n, (uint32_t)mode, 0, modulus, p->info.ncols, p->ctx->stream));
+    HIP_TRY(launch_first_cols(p->hub.rest, p->hub.nrest, p->hot_rows && !p->hot_stale ? p->hot_col : p->col,
+                              p->hub_first_cols, p->ctx->stream));
     return rc;
 }
 
@@ -1295,6 +1445,15 @@ static uint64_t own_device_bytes(const spc3d_plan *p)
     if (p->store.perm2) b += nnz * 4;
     if (p->store.n) b += (uint64_t)p->store.n * (8 + w); // dst, src, staged results
     if (p->two.n) b += nnz * (2 + 4 + 2) + 2 * nnz * w;  // l1, dst1, l2; c_stage, c_mid
+    if (p->hub.n) {
+        const HubTiles &t = p->hub;
+        b += nnz * (2 * 4 + 2) + t.n * w; // col, perm, lrow; values
+        if (t.src)
+            b += nnz * (2 * 4) + t.n * w; // src, dst; staged results
+        b += ((uint64_t)t.ntiles * t.nblocks + 1) * 4 + (uint64_t)t.ntiles * sweep_rows_per_tile(p->hub_lanes) * 8;
+        b += t.split_cap * sizeof(SplitRow) + (uint64_t)t.nslots * p->hub_k * w;
+        b += (uint64_t)p->info.nsegments_padded * sizeof(Seg) + (uint64_t)t.nrest * kFirstCols * 4;
+    }
     if (p->sweep.n) {
         const uint64_t n = p->sweep.n, rest = nnz - n;
         b += n * (4 + 2 + w) + nnz * 4; // col, lrow, values; perm

@@ -45,6 +45,7 @@ struct DevPlanView {
     void *hot_rows = nullptr;
     const uint32_t *hot_col = nullptr, *hot_first_cols = nullptr;
     uint32_t ref_at = 0, hot_at = 0; // set for a launch that gathers from there
+    bool hot_copied = false;         // the call has copied the rows already
 };
 
 // The context's stream, plus an auxiliary stream of the same (default) priority
@@ -86,6 +87,13 @@ struct SweepView {
     uint32_t lanes = 0;                  // lanes per dense row the plan was made for: 16, 32 or 64
     uint32_t per_launch = 0;             // tiles per generation (the GPU's CU count)
     uint32_t K = 0;                      // reals of a dense row, at most lanes * 16 bytes of them
+    // tiles of a sliced plan (HubTiles): [ntiles * rows_per_tile] partial-sum row of each place, kWholeRow for
+    // whole rows (null: all are), and the partial-sum rows
+    const uint32_t *slot = nullptr;
+    void *partial = nullptr;
+    uint32_t ref_at = 0, hot_at = 0;     // as in DevPlanView
+    const uint32_t *src = nullptr, *dst = nullptr; // [n] result src[h] of SDDMM goes to dst[h]
+    uint64_t rest_entries = 0;           // of the plan's other rows
 };
 // Lanes per dense row of K reals when the sweep kernels take that width (dense rows of 256,
 // 512 or 1024 bytes), else 0; lane groups per workgroup, rows of a tile, and the most column
@@ -102,6 +110,16 @@ uint32_t sweep_max_blocks(uint32_t lanes);
 hipError_t launch_sweep_sddmm(int dtype, const SweepView &S, const void *A, const void *B, void *C,
                               hipStream_t stream);
 hipError_t launch_sweep_spmm(int dtype, const SweepView &S, const void *X, void *Y, hipStream_t stream);
+// The same over the tiles of a sliced plan, and beside them the segments of its other rows (P).  SDDMM: results
+// to their places in `out` (P's positions; S.pos, or S.dst by way of stage[0 .. n)).  SpMM: pieces of cut rows to
+// S.partial.  hipErrorNotSupported, before anything is launched: the copy of P's hot rows, which the tiles'
+// columns name, is out of reach of the operand.
+hipError_t launch_hub_sddmm(int dtype, const DevPlanView &P, const SweepView &S, const void *A, const void *B,
+                            void *out, void *stage, const Streams &streams);
+hipError_t launch_hub_spmm(int dtype, const DevPlanView &P, const SweepView &S, const void *X, void *Y,
+                           const Streams &streams);
+// Y[row,:] += the partial sums of the rows in P.splits, P.partial's rows being K wide.
+hipError_t launch_split_sums(int dtype, const DevPlanView &P, void *Y, uint32_t K, hipStream_t stream);
 // first_cols[s * kFirstCols + u] = column of entry min(u, len - 1) of segment segs[s], s < n
 hipError_t launch_first_cols(const Seg *segs, uint32_t n, const uint32_t *col, uint32_t *first_cols,
                              hipStream_t stream);

@@ -1418,11 +1418,19 @@ constexpr uint32_t kSweepPtrWords = 1028;       // nb + 1 range bounds of a tile
 // at element alignment; as in the "odd" variants above, the lane that holds the row's end takes
 // the 16 bytes that END there and the lanes past it the same ones, and what is not a lane's to
 // count is left out of dot products and stores.  A tile's rows stay LPR * 16 bytes apart in LDS.
-template <typename T, int LPR, bool ANY> struct SweepLane {
+// HOT: rows that fill the lanes, and gathers from the operand or from the copy of its hot rows (RG == -1 above:
+// `ref` turns a column into a count of kHotUnit bytes from a base below both).
+enum SweepRows { kExact, kAny, kHot };
+struct HotAt {
+    uint32_t at = 0, hot_at = 0;
+};
+template <typename T, int LPR, int ROWS> struct SweepLane {
     using V = typename Vec<T>::type;
+    static constexpr bool ANY = ROWS == kAny;
     uint32_t sub, off = 0, bytes = LPR * 16;
+    HotAt hot;
     bool keep[Vec<T>::N], all = true;
-    __device__ __forceinline__ SweepLane(uint32_t lane, uint32_t K) : sub(lane)
+    __device__ __forceinline__ SweepLane(uint32_t lane, uint32_t K, HotAt h) : sub(lane), hot(h)
     {
         if constexpr (ANY) {
             bytes = K * (uint32_t)sizeof(T);
@@ -1444,6 +1452,21 @@ template <typename T, int LPR, bool ANY> struct SweepLane {
             return loose_load<T>(at(base, row));
         else
             return reinterpret_cast<const V *>(base)[(uint64_t)row * LPR + sub];
+    }
+    // what `gather` takes of a column, and the lane's part of that dense row
+    __device__ __forceinline__ uint32_t ref(uint32_t c) const
+    {
+        if constexpr (ROWS == kHot)
+            return c * (LPR * 16 / kHotUnit) + ((c & kHotRow) ? hot.hot_at : hot.at);
+        else
+            return c;
+    }
+    __device__ __forceinline__ V gather(const T *base, uint32_t r) const
+    {
+        if constexpr (ROWS == kHot)
+            return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + (uint64_t)r * kHotUnit + sub * 16);
+        else
+            return load(base, r);
     }
     __device__ __forceinline__ V load_once(const T *base, uint32_t row) const
     {
@@ -1484,13 +1507,13 @@ template <typename T> struct SweepIdx {
     T val = (T)0;
 };
 
-template <typename T, int LPR, int UB, bool ANY>
+template <typename T, int LPR, int UB, int ROWS>
 __global__ void __launch_bounds__(kSweepBlock)
 sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ tile_rows,
                    const uint32_t *__restrict__ col, const uint16_t *__restrict__ lrow,
                    const T *__restrict__ sval, const uint32_t *__restrict__ pos,
                    const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, uint32_t nb,
-                   uint32_t R, uint32_t tile0, uint32_t K)
+                   uint32_t R, uint32_t tile0, uint32_t K, HotAt hot)
 {
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
@@ -1498,13 +1521,13 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
     __shared__ V tile_a[kSweepRowBytes / 16];
     const uint32_t tile = tile0 + blockIdx.x;
     const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
-    const SweepLane<T, LPR, ANY> lane(sub, K);
+    const SweepLane<T, LPR, ROWS> lane(sub, K, hot);
     for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock) { // i % LPR == sub
         const uint32_t g = tile_rows[(uint64_t)tile * R + i / LPR];
         V v{};
         if (g != 0xFFFFFFFFu)
             v = lane.load_once(A, g);
-        if constexpr (ANY) {
+        if constexpr (ROWS == kAny) {
 #pragma unroll
             for (int j = 0; j < Vec<T>::N; ++j)
                 v[j] = lane.keep[j] ? v[j] : (T)0;
@@ -1523,7 +1546,7 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
         x.n = hi - q < (uint32_t)UB ? hi - q : (uint32_t)UB;
         uint32_t e = sub & (UB - 1);
         e = e < x.n ? e : x.n - 1;
-        x.col = nt_load(col + q + e);
+        x.col = lane.ref(nt_load(col + q + e));
         x.row = nt_load(lrow + q + e);
         x.val = (wlane && uo < x.n) ? nt_load(sval + q + uo) : (T)0;
         if (pos)
@@ -1542,7 +1565,7 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
         V bv[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u)
-            bv[u] = lane.load(B, bcast(cur.col, u));
+            bv[u] = lane.gather(B, bcast(cur.col, u));
         __builtin_amdgcn_sched_barrier(0); // all gathers in flight before the first use
         T part[UB];
 #pragma unroll
@@ -1560,13 +1583,13 @@ sweep_sddmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict_
     }
 }
 
-template <typename T, int LPR, int UB, bool ANY>
+template <typename T, int LPR, int UB, int ROWS>
 __global__ void __launch_bounds__(kSweepBlock)
 sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ tile_rows,
                   const uint32_t *__restrict__ col, const uint16_t *__restrict__ lrow,
                   const T *__restrict__ sval, const uint32_t *__restrict__ vpos,
                   const T *__restrict__ X, T *__restrict__ Y, uint32_t nb, uint32_t R, uint32_t tile0,
-                  uint32_t K)
+                  uint32_t K, HotAt hot, const uint32_t *__restrict__ slot, T *__restrict__ partial)
 {
     using V = typename Vec<T>::type;
     constexpr uint32_t G = kSweepBlock / LPR;
@@ -1583,13 +1606,13 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         lptr[i] = ptr[(uint64_t)tile * nb + i];
     __syncthreads();
     const uint32_t grp = threadIdx.x / LPR, sub = threadIdx.x % LPR;
-    const SweepLane<T, LPR, ANY> lane(sub, K);
+    const SweepLane<T, LPR, ROWS> lane(sub, K, hot);
     auto fetch = [&](uint32_t q, uint32_t qhi) {
         SweepIdx<T> x;
         x.n = qhi - q < (uint32_t)UB ? qhi - q : (uint32_t)UB;
         uint32_t e = sub & (UB - 1);
         e = e < x.n ? e : x.n - 1;
-        x.col = nt_load(col + q + e);
+        x.col = lane.ref(nt_load(col + q + e));
         x.row = nt_load(lrow + q + e);
         x.val = vpos ? sval[nt_load(vpos + q + e)] : nt_load(sval + q + e);
         if ((sub & (UB - 1)) >= x.n)
@@ -1635,7 +1658,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
             V xv[UB];
 #pragma unroll
             for (int u = 0; u < UB; ++u)
-                xv[u] = lane.load(X, bcast.entry(cur.col, u));
+                xv[u] = lane.gather(X, bcast.entry(cur.col, u));
             __builtin_amdgcn_sched_barrier(0);
             // where a row begins: lane u of a group holds entry u and sees entry u - 1 (lane 0 the row
             // that is being summed); the wavefront steps aside only where one of its groups needs it.
@@ -1691,8 +1714,49 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
     }
     for (uint32_t i = threadIdx.x; i < R * LPR; i += kSweepBlock) {
         const uint32_t g = tile_rows[(uint64_t)tile * R + i / LPR];
-        if (g != 0xFFFFFFFFu)
+        if (g == 0xFFFFFFFFu)
+            continue;
+        const uint32_t part = slot ? slot[(uint64_t)tile * R + i / LPR] : kWholeRow;
+        if (part == kWholeRow)
             lane.store(lane.load_once(Y, g) + tile_y[i], Y, g);
+        else // a piece of a cut row
+            lane.store(tile_y[i], partial, part);
+    }
+}
+
+// The tiles' results to their places: out[dst[h]] = stage[src[h]], the h-th entry of a tile counted place after
+// place.  What a tile's entries read lies anywhere in the tile's results (0.4 MB), so the workgroups of a tile
+// run on one XCD, as its results were written, and meet them in its L2; what they write are whole rows.
+// (13 M results beside the segments of the other rows: 118 us in fp64, 85 in fp32.)
+constexpr uint32_t kHomePieces = 8; // workgroups of a tile
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+hub_home_kernel(const uint32_t *__restrict__ ptr, uint32_t nb, uint32_t ntiles, const uint32_t *__restrict__ src,
+                const uint32_t *__restrict__ dst, const T *__restrict__ stage, T *__restrict__ out)
+{
+    const uint32_t j = blockIdx.x >> 3, tile = j / kHomePieces * 8 + (blockIdx.x & 7u), piece = j % kHomePieces;
+    if (tile >= ntiles)
+        return;
+    const uint32_t lo = ptr[(uint64_t)tile * nb], n = ptr[(uint64_t)(tile + 1) * nb] - lo;
+    const uint32_t h0 = (uint32_t)((uint64_t)n * piece / kHomePieces);
+    const uint32_t h1 = (uint32_t)((uint64_t)n * (piece + 1) / kHomePieces);
+    constexpr uint32_t U = 8;
+    for (uint32_t h = h0 + threadIdx.x; h < h1; h += U * kBlock) {
+        uint32_t s[U], d[U];
+        T v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t at = lo + (h + u * kBlock < h1 ? h + u * kBlock : h);
+            s[u] = nt_load(src + at);
+            d[u] = nt_load(dst + at);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            v[u] = stage[s[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (h + u * kBlock < h1)
+                out[d[u]] = v[u];
     }
 }
 
@@ -2473,7 +2537,7 @@ hipError_t run_spmm(const DevPlanView &P, const T *X, T *Y, const Streams &S, ui
 inline bool hot_view(const DevPlanView &P, size_t elem, const void *dense, uint32_t row_bytes,
                      DevPlanView &out, const void **base, hipStream_t st, hipError_t *e)
 {
-    if (!P.nhot || row_bytes > P.hot_row_bytes || !hot_rows_pay(P.nnz, row_bytes))
+    if (!P.nhot || row_bytes > P.hot_row_bytes || (!P.hot_copied && !hot_rows_pay(P.nnz, row_bytes)))
         return false;
     // the buffer has kHotUnit bytes to spare, so that both lie a whole number of units apart
     const uintptr_t d = reinterpret_cast<uintptr_t>(dense);
@@ -2486,8 +2550,9 @@ inline bool hot_view(const DevPlanView &P, size_t elem, const void *dense, uint3
     RowMapView rows;
     rows.rows = P.hot_cols;
     rows.nslots = P.nhot;
-    *e = launch_rows(0, elem == 8 ? 1 : 0, const_cast<void *>(dense), rows, row_bytes / (uint32_t)elem,
-                     reinterpret_cast<void *>(h), st);
+    *e = P.hot_copied ? hipSuccess
+                      : launch_rows(0, elem == 8 ? 1 : 0, const_cast<void *>(dense), rows,
+                                    row_bytes / (uint32_t)elem, reinterpret_cast<void *>(h), st);
     out = P;
     out.col = P.hot_col;
     out.first_cols = P.hot_first_cols;
@@ -2769,21 +2834,34 @@ uint32_t sweep_rows_per_tile(uint32_t lanes) { return lanes ? kSweepRowBytes / (
 uint32_t sweep_max_blocks(uint32_t lanes) { return lanes ? kSweepPtrWords - 1 : 0; }
 
 namespace {
-template <typename T, int LPR, bool ANY>
+template <typename T, int LPR, int ROWS>
 void sweep_launch(bool spmm, const SweepView &S, const T *A, const T *B, T *out, uint32_t tile0,
                   uint32_t ntiles, hipStream_t stream)
 {
+    const HotAt hot = {S.ref_at, S.hot_at};
     if (spmm)
-        hipLaunchKernelGGL((sweep_spmm_kernel<T, LPR, 16, ANY>), dim3(ntiles), dim3(kSweepBlock), 0,
+        hipLaunchKernelGGL((sweep_spmm_kernel<T, LPR, 16, ROWS>), dim3(ntiles), dim3(kSweepBlock), 0,
                            stream, S.ptr, S.tile_rows, S.col, S.lrow, (const T *)S.sval, S.pos, B,
-                           out, S.nblocks, S.rows_per_tile, tile0, S.K);
+                           out, S.nblocks, S.rows_per_tile, tile0, S.K, hot, S.slot, (T *)S.partial);
     else
-        hipLaunchKernelGGL((sweep_sddmm_kernel<T, LPR, 16, ANY>), dim3(ntiles), dim3(kSweepBlock), 0,
+        hipLaunchKernelGGL((sweep_sddmm_kernel<T, LPR, 16, ROWS>), dim3(ntiles), dim3(kSweepBlock), 0,
                            stream, S.ptr, S.tile_rows, S.col, S.lrow, (const T *)S.sval, S.pos, A,
-                           B, out, S.nblocks, S.rows_per_tile, tile0, S.K);
+                           B, out, S.nblocks, S.rows_per_tile, tile0, S.K, hot);
+}
+template <typename T, int LPR>
+void sweep_launch_rows(SweepRows rows, bool spmm, const SweepView &S, const T *A, const T *B, T *out,
+                       uint32_t tile0, uint32_t ntiles, hipStream_t stream)
+{
+    if (rows == kExact)
+        sweep_launch<T, LPR, kExact>(spmm, S, A, B, out, tile0, ntiles, stream);
+    else if (rows == kAny)
+        sweep_launch<T, LPR, kAny>(spmm, S, A, B, out, tile0, ntiles, stream);
+    else
+        sweep_launch<T, LPR, kHot>(spmm, S, A, B, out, tile0, ntiles, stream);
 }
 template <typename T>
-hipError_t sweep_run(bool spmm, const SweepView &S, const T *A, const T *B, T *out, hipStream_t stream)
+hipError_t sweep_run(bool spmm, const SweepView &S, const T *A, const T *B, T *out, hipStream_t stream,
+                     bool hot = false)
 {
     if (S.ntiles == 0)
         return hipSuccess;
@@ -2791,22 +2869,60 @@ hipError_t sweep_run(bool spmm, const SweepView &S, const T *A, const T *B, T *o
     if ((S.lanes != 16 && S.lanes != 32 && S.lanes != 64) || S.per_launch == 0 ||
         S.rows_per_tile * S.lanes * 16 > kSweepRowBytes ||
         (uint64_t)S.nblocks + 1 > kSweepPtrWords || S.K * sizeof(T) < 16 ||
-        S.K * sizeof(T) > S.lanes * 16)
+        S.K * sizeof(T) > S.lanes * 16 || (hot && S.K * sizeof(T) != S.lanes * 16))
         return hipErrorInvalidValue;
-    const bool any = S.K * sizeof(T) != S.lanes * 16;
+    const SweepRows rows = S.K * sizeof(T) != S.lanes * 16 ? kAny : (hot ? kHot : kExact);
     for (uint32_t t0 = 0; t0 < S.ntiles; t0 += S.per_launch) { // one generation per launch
         const uint32_t n = S.ntiles - t0 < S.per_launch ? S.ntiles - t0 : S.per_launch;
         if (S.lanes == 16)
-            any ? sweep_launch<T, 16, true>(spmm, S, A, B, out, t0, n, stream)
-                : sweep_launch<T, 16, false>(spmm, S, A, B, out, t0, n, stream);
+            sweep_launch_rows<T, 16>(rows, spmm, S, A, B, out, t0, n, stream);
         else if (S.lanes == 32)
-            any ? sweep_launch<T, 32, true>(spmm, S, A, B, out, t0, n, stream)
-                : sweep_launch<T, 32, false>(spmm, S, A, B, out, t0, n, stream);
+            sweep_launch_rows<T, 32>(rows, spmm, S, A, B, out, t0, n, stream);
         else
-            any ? sweep_launch<T, 64, true>(spmm, S, A, B, out, t0, n, stream)
-                : sweep_launch<T, 64, false>(spmm, S, A, B, out, t0, n, stream);
+            sweep_launch_rows<T, 64>(rows, spmm, S, A, B, out, t0, n, stream);
     }
     return hipGetLastError();
+}
+// The tiles of a sliced plan: their columns are named as the plan's hot form names them, where it has one.
+// The other rows' segments run beside the tiles: the tiles wait for the L2s and leave the fabric idle,
+// short rows are the other way round, and a tile's workgroup leaves each SIMD registers for a wavefront of the
+// short-segment launch.  That starts a few microseconds after the tiles, which need a CU each.
+template <typename T>
+hipError_t hub_run(bool spmm, DevPlanView P, const SweepView &S, const T *A, const T *B, T *out, T *stage,
+                   const Streams &streams)
+{
+    SweepView v = S;
+    const void *base = B;
+    const bool hot = P.nhot != 0;
+    if (hot) {
+        DevPlanView H;
+        hipError_t e = hipSuccess;
+        if (!hot_view(P, sizeof(T), B, S.K * (uint32_t)sizeof(T), H, &base, streams.main, &e))
+            return e != hipSuccess ? e : hipErrorNotSupported;
+        P.hot_copied = true;
+        v.ref_at = H.ref_at;
+        v.hot_at = H.hot_at;
+    }
+    P.nnz = S.rest_entries;
+    const bool beside = P.nseg && fork_aux(streams);
+    const bool staged = !spmm && !S.pos;
+    hipError_t e = sweep_run<T>(spmm, v, A, static_cast<const T *>(base), staged ? stage : out, streams.main, hot);
+    if (P.nseg) {
+        Streams own = streams;
+        if (beside) {
+            own.main = streams.aux;
+            own.aux = nullptr;
+        }
+        const hipError_t r = spmm ? spmm_typed<T>(P, B, out, S.K, own)
+                                  : sddmm_typed<T, 0>(P, A, B, out, nullptr, S.K, own);
+        e = e == hipSuccess ? r : e;
+    }
+    if (e == hipSuccess && staged)
+        hipLaunchKernelGGL((hub_home_kernel<T>), dim3((S.ntiles + 7) / 8 * 8 * kHomePieces), dim3(kBlock), 0,
+                           streams.main, S.ptr, S.nblocks, S.ntiles, S.src, S.dst, (const T *)stage, out);
+    const hipError_t launched = hipGetLastError();
+    const hipError_t joined = beside ? join_aux(streams) : hipSuccess;
+    return e != hipSuccess ? e : (launched != hipSuccess ? launched : joined);
 }
 } // namespace
 
@@ -2821,6 +2937,28 @@ hipError_t launch_sweep_spmm(int dtype, const SweepView &S, const void *X, void 
 {
     return dtype == 1 ? sweep_run<double>(true, S, nullptr, (const double *)X, (double *)Y, stream)
                       : sweep_run<float>(true, S, nullptr, (const float *)X, (float *)Y, stream);
+}
+
+hipError_t launch_hub_sddmm(int dtype, const DevPlanView &P, const SweepView &S, const void *A, const void *B,
+                            void *out, void *stage, const Streams &streams)
+{
+    return dtype == 1 ? hub_run<double>(false, P, S, (const double *)A, (const double *)B, (double *)out,
+                                        (double *)stage, streams)
+                      : hub_run<float>(false, P, S, (const float *)A, (const float *)B, (float *)out,
+                                       (float *)stage, streams);
+}
+
+hipError_t launch_hub_spmm(int dtype, const DevPlanView &P, const SweepView &S, const void *X, void *Y,
+                           const Streams &streams)
+{
+    return dtype == 1 ? hub_run<double>(true, P, S, nullptr, (const double *)X, (double *)Y, nullptr, streams)
+                      : hub_run<float>(true, P, S, nullptr, (const float *)X, (float *)Y, nullptr, streams);
+}
+
+hipError_t launch_split_sums(int dtype, const DevPlanView &P, void *Y, uint32_t K, hipStream_t stream)
+{
+    return dtype == 1 ? launch_fixup<double>(P, (double *)Y, K, stream)
+                      : launch_fixup<float>(P, (float *)Y, K, stream);
 }
 
 hipError_t launch_first_cols(const Seg *segs, uint32_t n, const uint32_t *col, uint32_t *first_cols,

@@ -22,6 +22,8 @@ struct DevPlanArrays {
     uint32_t nsplit = 0;
     uint32_t *hot_cols = nullptr; // [nhot] the hottest columns where their rows crowd (hot_rows_crowd)
     uint32_t nhot = 0;
+    // PlanOpts::keep_counts: [nrows + 1] first kernel position of every row, [ncols] entries of every column
+    uint32_t *rowptr = nullptr, *coldeg = nullptr;
 };
 
 // d_ii, d_jj: device arrays of nnz entries.  On success fills `meta` (every
@@ -124,6 +126,52 @@ int build_sweep(const DevStream &stream, uint32_t nrows, uint32_t ncols, uint64_
                 const uint32_t *d_ii, const uint32_t *d_jj, uint32_t lanes, uint32_t rows_per_tile,
                 uint32_t nblocks, uint32_t min_row, uint32_t per_launch, SweepPlan &out,
                 std::string &err);
+// ---- row tiles over skewed columns -----------------------------------------------------
+// The longest rows of a sliced plan once more as tiles for the sweep kernels (kernels.hip says what they gain).
+// Rows of at least min_row entries, those of more than nnz / (per_launch * kTileParts) cut into pieces that
+// take every np-th entry, are ranked longest first and dealt to the tiles of one launch there and back, so
+// that they carry the same load to a few percent.
+// A tile's entries are sorted by (block of columns, place), the source's order kept inside a place's run.
+//   col, lrow   column and place in the tile of entry k                                      [n]
+//   perm        its position in the source                                                   [n]
+//   ptr         range bounds per (tile, block)                                               [ntiles * nblocks + 1]
+//   tile_rows   row of place l of tile t, 0xFFFFFFFF where there is none                     [ntiles * rows_per_tile]
+//   slot        partial-sum row of a piece, kWholeRow for a whole row                        [ntiles * rows_per_tile]
+//   splits      the cut rows and their slots                                                 [nsplit]
+//   src, dst    result k = src[h] goes to dst[h], ascending inside a place; null where `direct`: results go
+//               straight to perm                                                             [n]
+//   rest        the plan's segments of the other rows, in its queues, none of them a part    [nrest]
+// (room for nnz of what has n, for all the plan's segments, and for split_cap of splits)
+struct HubTiles {
+    uint32_t *col = nullptr, *perm = nullptr, *ptr = nullptr, *tile_rows = nullptr, *slot = nullptr;
+    uint32_t *src = nullptr, *dst = nullptr;
+    uint16_t *lrow = nullptr;
+    SplitRow *splits = nullptr;
+    Seg *rest = nullptr;
+    uint64_t n = 0, split_cap = 0;
+    bool direct = false;
+    uint32_t ntiles = 0, nblocks = 0, nsplit = 0, nslots = 0, nrest = 0;
+};
+struct HubSource {
+    uint32_t nrows = 0, ncols = 0;
+    uint64_t nnz = 0;
+    // the entries by row: row r's are rowptr[r] .. rowptr[r + 1), entry p in column col[p] and at the
+    // caller's position pos[p] (null: p); results go to the caller's position (by_pos) or to p
+    const uint32_t *rowptr = nullptr, *coldeg = nullptr, *col = nullptr, *pos = nullptr;
+    bool by_pos = true, results = true; // (results: SDDMM runs over the tiles)
+    const Seg *segs = nullptr; // the plan's, in kSlices queues
+    uint32_t nseg = 0;
+    const uint32_t *hot_cols = nullptr; // [nhot] `col` names these by rank (kHotRow | rank)
+    uint32_t nhot = 0;
+    uint32_t rows_per_tile = 0, per_launch = 0, min_row = 0;
+    uint32_t must = 0; // rows of so many entries, and cut ones, are all in the tiles, or there are no tiles
+    uint64_t row_bytes = 0, block_bytes = 0;
+    uint32_t min_blocks = 0, max_blocks = 0;
+};
+// n == 0 (and nothing to free): the pattern has no such tiles.  The arrays belong to the receiver (blocks of
+// the stream's pool).  Synchronous.
+int build_hub_tiles(const DevStream &stream, const HubSource &in, HubTiles &out, std::string &err);
+
 // The pattern back from a plan: d_ii / d_jj at the caller's positions of the entries of a
 // sweep, and of a plan in segments (d_perm null: its kernel order is the caller's).
 // Asynchronous on `stream`.

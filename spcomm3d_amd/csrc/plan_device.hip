@@ -1274,7 +1274,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         return SPC3D_OK;
     }
 
-    // One block for everything whose size is known now: ten arrays per row, five and
+    // One block for everything whose size is known now: nine arrays per row, four and
     // a class byte per column, the sorted column ids, two keys and an index per entry,
     // the primitives' scratch.
     Arena arena(st);
@@ -1289,10 +1289,11 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     HIP_OK(hipMemsetAsync(&dC.p->first_bad, 0xFF, sizeof(uint32_t), st));
 
     // ---- histograms, validation ------------------------------------------------
-    SBuf<uint32_t> rowcnt, rowptr, coldeg;
+    SBuf<uint32_t> rowcnt;
+    DBuf<uint32_t> rowptr, coldeg;
     HIP_OK(rowcnt.alloc(arena, (size_t)nrows + 1));
-    HIP_OK(rowptr.alloc(arena, (size_t)nrows + 1));
-    HIP_OK(coldeg.alloc(arena, ncols));
+    HIP_OK(rowptr.alloc(st, (size_t)nrows + 1));
+    HIP_OK(coldeg.alloc(st, ncols));
     HIP_OK(hipMemsetAsync(rowcnt.p, 0, ((size_t)nrows + 1) * sizeof(uint32_t), st));
     HIP_OK(hipMemsetAsync(coldeg.p, 0, (size_t)ncols * sizeof(uint32_t), st));
     LAUNCH_SMALL(check_k, nnz, d_ii, d_jj, nnz, nrows, ncols, dC.p);
@@ -1309,6 +1310,8 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     }
     const bool rows_unsorted = hC.rows_unsorted != 0;
     P.cols_sorted = hC.cols_unsorted == 0;
+    P.rows_sorted = !rows_unsorted;
+    P.row_runs = hC.row_changes + 1; // (nnz > 0)
     const bool by_column = rows_unsorted && !opts.keep_entry_order;
     const int col_bits = bits_for(ncols ? ncols - 1 : 0);
     P.by_column_in_rows = by_column;
@@ -1564,6 +1567,10 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     out.splits = splits.release();
     out.nsplit = nsplit;
     out.hot_cols = hot.release();
+    if (opts.keep_counts && slices) {
+        out.rowptr = rowptr.release();
+        out.coldeg = coldeg.release();
+    }
     meta = std::move(P);
     return SPC3D_OK;
 }
@@ -2381,6 +2388,498 @@ int build_sweep(const DevStream &st, uint32_t nrows, uint32_t ncols, uint64_t nn
     out.lanes = lanes;
     out.per_launch = P;
     out.nrows_in = nin;
+    return SPC3D_OK;
+}
+
+// ---- row tiles over skewed columns ----------------------------------------------------
+struct HubCounters {
+    uint32_t nsplit, nslots; // cut rows; partial-sum rows, gaps included
+    uint32_t left_out;       // segments of rows without a place that need one
+    uint32_t rest[kSlices];  // segments of other rows per queue
+    uint32_t adjacent;       // entries of a tile that follow their predecessor in the caller's order too (at least)
+};
+
+// What the scan adds up: [0, ncols] how much of an L2 a column takes on average, in 1/1024 of its dense row (the
+// tiles of an XCD are an eighth of all, and meet a column of d entries with probability 1 - (7/8)^d); and from
+// ncols + 1 on, per row of at least min_row entries, its pieces.  And what starts as nothing.
+__global__ void hub_start_k(const uint32_t *__restrict__ deg, uint64_t ncols, const uint32_t *__restrict__ rowptr,
+                            uint64_t nrows, uint32_t min_row, uint32_t cut, uint64_t nplaces, uint32_t *sums,
+                            uint8_t *row_in, uint32_t *tile_rows, TilePlace *place, HubCounters *C)
+{
+    const uint64_t n = ncols + nrows + 2 > nplaces ? ncols + nrows + 2 : nplaces;
+    GRID_STRIDE(i, n)
+    {
+        if (i <= ncols) {
+            uint32_t miss = 1024; // of 1024, rounded down at every step
+            const uint32_t d = i < ncols ? (deg[i] < 52 ? deg[i] : 52u) : 0u;
+            for (uint32_t k = 0; k < d; ++k)
+                miss = miss * 7 / 8;
+            sums[i] = 1024 - miss;
+        } else if (i < ncols + nrows + 2) {
+            const uint64_t r = i - ncols - 1;
+            const uint32_t len = r < nrows ? rowptr[r + 1] - rowptr[r] : 0u;
+            sums[i] = len >= min_row ? (len + cut - 1) / cut : 0u;
+            if (r < nrows)
+                row_in[r] = 0;
+        }
+        if (i < nplaces) {
+            tile_rows[i] = 0xFFFFFFFFu;
+            place[i] = TilePlace{0, 0, 0};
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *C = HubCounters{};
+}
+// Of every column its block, and no rank.
+__global__ void hub_blocks_k(const uint32_t *__restrict__ before, uint64_t ncols, uint32_t per_block, uint32_t nb,
+                             uint16_t *block, uint16_t *rank)
+{
+    GRID_STRIDE(c, ncols)
+    {
+        const uint32_t b = before[c] / per_block;
+        block[c] = (uint16_t)(b < nb ? b : nb - 1);
+        if (rank)
+            rank[c] = 0xFFFFu;
+    }
+}
+// The pieces, a row's together, under a sort key that is the length to an eighth of an octave.
+__global__ void hub_pieces_k(const uint32_t *__restrict__ rowptr, uint64_t nrows, const uint32_t *__restrict__ first,
+                             uint32_t base, uint32_t *key, uint32_t *id, uint32_t *row)
+{
+    GRID_STRIDE(r, nrows)
+    {
+        const uint32_t at = first[r] - base, np = first[r + 1] - first[r];
+        if (!np)
+            continue;
+        const uint32_t len = (rowptr[r + 1] - rowptr[r]) / np, e = 31 - __clz((int)len);
+        const uint32_t k = e * 8 + (uint32_t)(((unsigned long long)len << 3 >> e) & 7);
+        for (uint32_t i = 0; i < np; ++i) {
+            key[at + i] = k;
+            id[at + i] = at + i;
+            row[at + i] = (uint32_t)r;
+        }
+    }
+}
+
+// The piece of rank j (longest first) goes to tile j mod P, there and back.  A cut row's
+// pieces have neighbouring ranks; its partial sums are the slots of those numbers.  A row has places for
+// all its pieces or for none.
+__global__ void hub_places_k(const uint32_t *__restrict__ order, const uint32_t *__restrict__ row_of,
+                             uint64_t npc, const uint32_t *__restrict__ rowptr,
+                             const uint32_t *__restrict__ first, uint32_t base, uint32_t P,
+                             uint32_t R, TilePlace *place, uint32_t *tile_rows, uint32_t *slot,
+                             uint8_t *row_in, SplitRow *splits, HubCounters *C)
+{
+    GRID_STRIDE(j, npc)
+    {
+        const uint32_t pc = order[j], row = row_of[pc], np = first[row + 1] - first[row], i = pc - (first[row] - base);
+        if (j - i + np > (uint64_t)P * R)
+            continue;
+        const uint32_t l = (uint32_t)j / P, x = (uint32_t)j % P;
+        const uint64_t at = (uint64_t)(l & 1 ? P - 1 - x : x) * R + l;
+        const uint32_t start = rowptr[row], len = rowptr[row + 1] - start;
+        const uint32_t groups = (len + kTileGroup - 1) / kTileGroup, mine = (groups - i + np - 1) / np * kTileGroup;
+        place[at] = TilePlace{start + i * kTileGroup, np * kTileGroup,
+                              mine - ((groups - 1) % np == i ? groups * kTileGroup - len : 0)};
+        tile_rows[at] = row;
+        slot[at] = np > 1 ? (uint32_t)j : kWholeRow;
+        row_in[row] = 1;
+        if (np > 1 && i == 0) {
+            splits[atomicAdd(&C->nsplit, 1u)] = SplitRow{row, (uint32_t)j, np, 0};
+            atomicMax(&C->nslots, (uint32_t)j + np);
+        }
+    }
+}
+
+// One workgroup per tile: entries before each of its places, and in all.
+__global__ void __launch_bounds__(kTileMaxRows)
+hub_offsets_k(const TilePlace *__restrict__ place, uint32_t R, uint32_t *off, uint32_t *tile_n)
+{
+    __shared__ uint32_t sum[kTileMaxRows / 64];
+    const uint32_t l = threadIdx.x, lane = l & 63u, wave = l >> 6;
+    const uint64_t at = (uint64_t)blockIdx.x * R + l;
+    const uint32_t len = l < R ? place[at].len : 0u;
+    uint32_t upto = len;
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(upto, d, 64);
+        upto += lane >= d ? v : 0u;
+    }
+    if (lane == 63)
+        sum[wave] = upto;
+    __syncthreads();
+    uint32_t total = 0, before = 0;
+    for (uint32_t w = 0; w < kTileMaxRows / 64; ++w) {
+        before += w < wave ? sum[w] : 0u;
+        total += sum[w];
+    }
+    if (l < R)
+        off[at] = before + upto - len;
+    if (l == 0)
+        tile_n[blockIdx.x] = total;
+}
+
+// One workgroup per tile: its entries by block, in a block by place, in a place in the order of the source.
+// They are counted by block first, then taken in the order of the places, kFillRound at a time: every wavefront
+// counts its own by block, a thread per block adds those up, and the wavefronts lay theirs out from there.  All
+// wavefronts write near the same few places of every block, so that lines are full when they leave the L2:
+// R-MAT 20, 13 M entries, 241 us (266 without a round's loads under way during the one before); 277 with a sixteenth
+// of the tile to every wavefront, and 500 for a device-wide radix sort on (tile, block, place) and the gathers after it.
+constexpr int kFillTB = 1024;
+constexpr uint32_t kFillBlocks = 1027; // at most
+struct HubFill {
+    const uint32_t *col, *pos; // the source; pos (may be null): caller's position of entry p
+    const uint16_t *block, *hot; // of a column: its block, and its rank where it is hot (null: none is)
+    const TilePlace *place;
+    const uint32_t *off, *tptr;
+    uint32_t R, nb;
+    bool by_pos; // results go to the caller's position, else to the entry's in the source
+    uint32_t *where; // scratch: place << 16 | block of every entry
+    uint32_t *ptr, *out_col, *out_perm, *src, *dst;
+    uint16_t *lrow;
+    HubCounters *C;
+};
+__device__ __forceinline__ uint32_t place_at(uint32_t start, uint32_t step, uint32_t y)
+{
+    return start + y / kTileGroup * step + y % kTileGroup;
+}
+__global__ void __launch_bounds__(kFillTB) hub_fill_k(HubFill F)
+{
+    constexpr uint32_t kWaves = kFillTB / 64;
+    __shared__ uint32_t first[kTileMaxRows + 1], start[kTileMaxRows], step[kTileMaxRows];
+    __shared__ uint32_t counts[kWaves * kFillBlocks], next[kFillBlocks];
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    volatile uint32_t *count = counts + w * kFillBlocks;
+    const uint32_t t = blockIdx.x, lo = F.tptr[t], n = F.tptr[t + 1] - lo;
+    for (uint32_t l = threadIdx.x; l <= F.R; l += kFillTB) {
+        const uint64_t at = (uint64_t)t * F.R + l;
+        first[l] = l < F.R ? F.off[at] : n;
+        if (l < F.R) {
+            start[l] = F.place[at].start;
+            step[l] = F.place[at].step;
+        }
+    }
+    for (uint32_t k = lane; k < F.nb; k += 64)
+        count[k] = 0;
+    __syncthreads();
+        constexpr int V = 8; // entries of a lane at a time, here
+    for (uint32_t y0 = w * V * 64; y0 < n; y0 += kWaves * V * 64) {
+        // the place of the first, and from there of the others: few places end among 256 entries
+        uint32_t at = 0, up = F.R;
+        while (up - at > 1) {
+            const uint32_t mid = (at + up) / 2;
+            if (first[mid] <= y0)
+                at = mid;
+            else
+                up = mid;
+        }
+        uint32_t l[V], c[V];
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const uint32_t y = y0 + u * 64 + lane < n ? y0 + u * 64 + lane : n - 1;
+            l[u] = u ? l[u ? u - 1 : 0] : at;
+            while (__any(first[l[u] + 1] <= y)) // (first[R] == n: no lane goes past the last place)
+                l[u] += first[l[u] + 1] <= y;
+            c[u] = F.col[place_at(start[l[u]], step[l[u]], y - first[l[u]])];
+        }
+#pragma unroll
+        for (int u = 0; u < V; ++u)
+            c[u] = F.block[c[u]];
+#pragma unroll
+        for (int u = 0; u < V; ++u)
+            if (y0 + u * 64 + lane < n) {
+                atomicAdd(const_cast<uint32_t *>(&count[c[u]]), 1u);
+                F.where[lo + y0 + u * 64 + lane] = l[u] << 16 | c[u];
+            }
+    }
+    __syncthreads();
+    if (w == 0) { // where the blocks begin
+        uint32_t run = 0;
+        for (uint32_t k0 = 0; k0 < F.nb; k0 += 64) {
+            const uint32_t k = k0 + lane;
+            uint32_t sum = 0;
+            if (k < F.nb)
+                for (uint32_t v = 0; v < kWaves; ++v)
+                    sum += counts[v * kFillBlocks + k];
+            uint32_t upto = sum;
+            for (uint32_t d = 1; d < 64; d <<= 1) {
+                const uint32_t o = __shfl_up(upto, d, 64);
+                upto += lane >= d ? o : 0u;
+            }
+            if (k < F.nb) {
+                next[k] = run + upto - sum;
+                F.ptr[(uint64_t)t * F.nb + k] = lo + run + upto - sum;
+            }
+            run += __shfl(upto, 63, 64);
+        }
+        if (lane == 0 && t + 1 == gridDim.x)
+            F.ptr[(uint64_t)(t + 1) * F.nb] = lo + n;
+    }
+    int bits = 1;
+    while ((F.nb - 1) >> bits)
+        ++bits;
+    uint32_t adjacent = 0;
+    constexpr int U = 4; // and here
+    constexpr uint32_t kFillRound = kWaves * U * 64;
+    // The loads of a round are under way while the one before is laid out.
+    uint32_t next_at[U], next_col[U], next_pos[U];
+    auto where_of = [&](uint32_t r0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t y = r0 + w * U * 64 + u * 64 + lane;
+            next_at[u] = F.where[lo + (y < n ? y : n - 1)];
+        }
+    };
+    auto source_of = [&](uint32_t r0, int u) {
+        const uint32_t y = r0 + w * U * 64 + u * 64 + lane, l = next_at[u] >> 16;
+        return place_at(start[l], step[l], (y < n ? y : n - 1) - first[l]);
+    };
+    if (n) {
+        where_of(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            next_col[u] = F.col[source_of(0, u)];
+        if (F.pos)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                next_pos[u] = F.pos[source_of(0, u)];
+    }
+    for (uint32_t r0 = 0; r0 < n; r0 += kFillRound) {
+        const uint32_t y0 = r0 + w * U * 64;
+        uint32_t l[U], p[U], c[U], h[U], blk[U], e[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            p[u] = source_of(r0, u);
+            l[u] = next_at[u] >> 16;
+            blk[u] = next_at[u] & 0xFFFFu;
+            c[u] = next_col[u];
+            e[u] = F.pos ? next_pos[u] : p[u];
+            h[u] = F.hot ? F.hot[c[u]] : 0xFFFFu;
+        }
+        const bool more = r0 + kFillRound < n;
+        if (more)
+            where_of(r0 + kFillRound);
+        __syncthreads(); // the round before has laid its entries out (the first: the blocks' beginnings are there)
+        for (uint32_t k = lane; k < F.nb; k += 64)
+            count[k] = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (y0 + u * 64 + lane < n)
+                atomicAdd(const_cast<uint32_t *>(&count[blk[u]]), 1u);
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < F.nb; k += kFillTB) {
+            uint32_t m[kWaves], at = next[k];
+#pragma unroll
+            for (uint32_t v = 0; v < kWaves; ++v)
+                m[v] = counts[v * kFillBlocks + k];
+#pragma unroll
+            for (uint32_t v = 0; v < kWaves; ++v) {
+                counts[v * kFillBlocks + k] = at;
+                at += m[v];
+            }
+            next[k] = at;
+        }
+        if (more) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                next_col[u] = F.col[source_of(r0 + kFillRound, u)];
+            if (F.pos)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    next_pos[u] = F.pos[source_of(r0 + kFillRound, u)];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool on = y0 + u * 64 + lane < n;
+            const uint32_t e0 = __shfl_up(e[u], 1, 64), blk0 = __shfl_up(blk[u], 1, 64);
+            adjacent += (uint32_t)__popcll(__ballot(on && lane && e0 + 1 == e[u] && blk0 == blk[u]));
+            unsigned long long same = __ballot(on); // lanes with an entry of this block
+            for (int k = 0; k < bits; ++k) {
+                const unsigned long long m = __ballot((blk[u] >> k & 1) != 0);
+                same &= (blk[u] >> k & 1) ? m : ~m;
+            }
+            if (on) {
+                const uint32_t rank = (uint32_t)__popcll(same & ((1ull << lane) - 1));
+                const uint32_t base = count[blk[u]];
+                if (rank == 0)
+                    count[blk[u]] = base + (uint32_t)__popcll(same);
+                const uint32_t at = lo + base + rank;
+                F.out_col[at] = h[u] == 0xFFFFu ? c[u] : kHotRow | h[u];
+                F.lrow[at] = (uint16_t)l[u];
+                F.out_perm[at] = p[u];
+                if (F.src) {
+                    F.src[lo + y0 + u * 64 + lane] = at;
+                    F.dst[lo + y0 + u * 64 + lane] = F.by_pos ? e[u] : p[u];
+                }
+            }
+        }
+    }
+    if (lane == 0 && adjacent)
+        atomicAdd(&F.C->adjacent, adjacent);
+}
+
+// The segments of the other rows, queue by queue in their order: flag[i] for the i-th of queue 0, 1, ...  None of
+// them may be a part of a row, or of `must` entries and more.
+__global__ void rest_flags_k(const Seg *__restrict__ segs, uint32_t nseg, const uint8_t *__restrict__ row_in,
+                             uint32_t must, uint32_t *flag, Seg *__restrict__ out, HubCounters *C)
+{
+    const uint32_t per_queue = nseg / kSlices, q = blockIdx.y;
+    uint32_t mine = 0;
+    bool left = false;
+    for (uint32_t i = blockIdx.x * kTB + threadIdx.x; i < per_queue; i += gridDim.x * kTB) {
+        const uint32_t s = (i / kChunk * kSlices + q) * kChunk + i % kChunk;
+        const Seg g = segs[s];
+        const bool rest = g.len && !row_in[g.row];
+        flag[q * per_queue + i] = rest;
+        out[s] = Seg{0, 0, 0, kWholeRow};
+        mine += rest;
+        left |= rest && (g.slot != kWholeRow || g.len >= must);
+    }
+    mine = block_sum(mine);
+    if (threadIdx.x == 0 && mine)
+        atomicAdd(&C->rest[q], mine);
+    if (__syncthreads_or(left) && threadIdx.x == 0)
+        atomicOr(&C->left_out, 1u);
+}
+__global__ void rest_segs_k(const Seg *__restrict__ segs, uint32_t nseg, const uint32_t *__restrict__ flag,
+                            const uint32_t *__restrict__ at, Seg *__restrict__ out)
+{
+    const uint32_t per_queue = nseg / kSlices, q = blockIdx.y;
+    for (uint32_t i = blockIdx.x * kTB + threadIdx.x; i < per_queue; i += gridDim.x * kTB) {
+        if (!flag[q * per_queue + i])
+            continue;
+        const uint32_t j = at[q * per_queue + i] - at[q * per_queue];
+        out[(j / kChunk * kSlices + q) * kChunk + j % kChunk] = segs[(i / kChunk * kSlices + q) * kChunk + i % kChunk];
+    }
+}
+
+int build_hub_tiles(const DevStream &st, const HubSource &in, HubTiles &out, std::string &err)
+{
+    out = HubTiles();
+    const uint32_t R = in.rows_per_tile, P = in.per_launch, nrows = in.nrows, ncols = in.ncols;
+    const uint64_t nnz = in.nnz, nplaces = (uint64_t)P * R;
+    if (nnz == 0 || R == 0 || R > kTileMaxRows || P == 0 || in.nseg % (kSlices * kChunk) ||
+        (uint64_t)ncols * 1024 + nnz >= (1ull << 32) || in.block_bytes < in.row_bytes)
+        return SPC3D_OK;
+    // From here to the entries the device waits for launches more than it works, so there are few of them.
+    Arena arena(st);
+    HIP_OK(arena.reserve(((size_t)nrows + 1) * 9 + ((size_t)ncols + 1) * 12 + (size_t)in.nseg * 8 + nplaces * 16 +
+                         (size_t)nnz * 4 + ((size_t)8 << 20)));
+    Temp tmp(arena);
+    const uint32_t cut = (uint32_t)std::max<uint64_t>(64, nnz / ((uint64_t)P * kTileParts));
+    SBuf<uint32_t> sums, before;
+    SBuf<uint16_t> block, hot;
+    SBuf<uint8_t> row_in;
+    SBuf<HubCounters> dC;
+    SBuf<TilePlace> place;
+    DBuf<uint32_t> tile_rows, slot, col, perm, src, dst, ptr;
+    DBuf<uint16_t> lrow;
+    DBuf<SplitRow> splits;
+    DBuf<Seg> rest;
+    const size_t nsums = (size_t)ncols + nrows + 2;
+    HIP_OK(sums.alloc(arena, nsums));
+    HIP_OK(before.alloc(arena, nsums));
+    HIP_OK(row_in.alloc(arena, nrows));
+    HIP_OK(block.alloc(arena, ncols));
+    HIP_OK(dC.alloc(arena, 1));
+    HIP_OK(place.alloc(arena, nplaces));
+    HIP_OK(tile_rows.alloc(st, nplaces));
+    HIP_OK(slot.alloc(st, nplaces));
+    LAUNCH(hub_start_k, std::max<uint64_t>(nsums, nplaces), in.coldeg, (uint64_t)ncols, in.rowptr, (uint64_t)nrows,
+           std::max(1u, in.min_row), cut, nplaces, sums.p, row_in.p, tile_rows.p, place.p, dC.p);
+    TRY(exclusive_sum(tmp, sums.p, before.p, nsums, st, err));
+    const uint32_t *first = before.p + ncols + 1; // of every row its first piece, from total_weight on
+    uint32_t upto = 0, total_weight = 0;
+    TRY(fetch_all(st, {{&upto, first + nrows, sizeof upto}, {&total_weight, before.p + ncols, sizeof total_weight}},
+                  err));
+    const uint32_t npc = upto - total_weight;
+    // Blocks of columns by number (hot and cold ones mixed: gathers that hit and gathers that miss overlap)
+    // whose dense rows take block_bytes of every L2.
+    const uint32_t per_block = (uint32_t)std::min<uint64_t>(0xFFFFFFFFull, in.block_bytes / in.row_bytes * 1024);
+    const uint32_t nb = total_weight / per_block + 1;
+    if (npc == 0 || nb < in.min_blocks || nb > std::min(kFillBlocks, in.max_blocks))
+        return SPC3D_OK;
+    if (in.nhot)
+        HIP_OK(hot.alloc(arena, ncols));
+    LAUNCH(hub_blocks_k, ncols, before.p, (uint64_t)ncols, per_block, nb, block.p, in.nhot ? hot.p : nullptr);
+    if (in.nhot)
+        LAUNCH(hot_ranks_k, in.nhot, in.hot_cols, (uint64_t)in.nhot, hot.p);
+    // ---- places ----
+    HIP_OK(arena.reserve((size_t)npc * 20 + ((size_t)4 << 20)));
+    SBuf<uint32_t> key, row_of, id, key_sorted, order, off, tile_n, tptr;
+    HIP_OK(key.alloc(arena, npc));
+    HIP_OK(row_of.alloc(arena, npc));
+    HIP_OK(id.alloc(arena, npc));
+    HIP_OK(key_sorted.alloc(arena, npc));
+    HIP_OK(order.alloc(arena, npc));
+    HIP_OK(off.alloc(arena, nplaces));
+    HIP_OK(tile_n.alloc(arena, (size_t)P + 1));
+    HIP_OK(tptr.alloc(arena, (size_t)P + 1));
+    // cut rows have more than `cut` entries each
+    out.split_cap = nnz / cut + 1;
+    HIP_OK(splits.alloc(st, out.split_cap));
+    LAUNCH(hub_pieces_k, nrows, in.rowptr, (uint64_t)nrows, first, total_weight, key.p, id.p, row_of.p);
+    TRY(sort_pairs<uint32_t>(tmp, key.p, key_sorted.p, id.p, order.p, npc, 8, true, st, err));
+    LAUNCH(hub_places_k, npc, order.p, row_of.p, (uint64_t)npc, in.rowptr, first, total_weight, P, R,
+           place.p, tile_rows.p, slot.p, row_in.p, splits.p, dC.p);
+    hipLaunchKernelGGL(hub_offsets_k, dim3(P), dim3(kTileMaxRows), 0, st, place.p, R, off.p, tile_n.p);
+    TRY(exclusive_sum(tmp, tile_n.p, tptr.p, (size_t)P + 1, st, err));
+    // ---- the other rows' segments ----
+    SBuf<uint32_t> flag, at;
+    HIP_OK(flag.alloc(arena, in.nseg));
+    HIP_OK(at.alloc(arena, in.nseg));
+    HIP_OK(rest.alloc(st, in.nseg));
+    const dim3 seg_grid((in.nseg / kSlices + kTB * 4 - 1) / (kTB * 4), kSlices);
+    hipLaunchKernelGGL(rest_flags_k, seg_grid, dim3(kTB), 0, st, in.segs, in.nseg, row_in.p, in.must, flag.p, rest.p,
+                       dC.p);
+    TRY(exclusive_sum(tmp, flag.p, at.p, in.nseg, st, err));
+    hipLaunchKernelGGL(rest_segs_k, seg_grid, dim3(kTB), 0, st, in.segs, in.nseg, flag.p, at.p, rest.p);
+    // ---- entries (room for all: how many are in the tiles is known when they are) ----
+    HIP_OK(col.alloc(st, nnz));
+    HIP_OK(perm.alloc(st, nnz));
+    if (in.results) {
+        HIP_OK(src.alloc(st, nnz));
+        HIP_OK(dst.alloc(st, nnz));
+    }
+    HIP_OK(lrow.alloc(st, nnz));
+    HIP_OK(ptr.alloc(st, (size_t)P * nb + 1));
+    SBuf<uint32_t> where;
+    HIP_OK(where.alloc(arena, nnz));
+    const HubFill F = {in.col, in.pos, block.p, in.nhot ? hot.p : nullptr, place.p, off.p, tptr.p, R, nb, in.by_pos,
+                       where.p, ptr.p, col.p, perm.p, src.p, dst.p, lrow.p, dC.p};
+    hipLaunchKernelGGL(hub_fill_k, dim3(P), dim3(kFillTB), 0, st, F);
+    uint32_t n = 0;
+    HubCounters hC;
+    TRY(fetch_all(st, {{&n, tptr.p + P, sizeof n}, {&hC, dC.p, sizeof hC}}, err));
+    if ((uint64_t)n * 2 < nnz || hC.left_out) // (little gained; or the rest is not of short rows alone)
+        return SPC3D_OK;
+    uint32_t chunks = 0;
+    for (uint32_t q = 0; q < kSlices; ++q)
+        chunks = std::max(chunks, (hC.rest[q] + kChunk - 1) / kChunk);
+    // Results whose neighbours in the tile are mostly their neighbours in the caller's order go straight there:
+    // pieces of lines that the same workgroup completes a few blocks later.  (R-MAT 20, rows and columns sorted,
+    // three in four, fp64 / fp32 705 -> 685 us and 363 -> 357; a block of R-MAT 24, one in six, 491 -> 546.)
+    out.direct = in.results && !in.pos && (uint64_t)hC.adjacent * 5 >= (uint64_t)n * 3;
+    if (out.direct) {
+        src.reset();
+        dst.reset();
+    }
+    out.col = col.release();
+    out.perm = perm.release();
+    out.src = src.release();
+    out.dst = dst.release();
+    out.lrow = lrow.release();
+    out.ptr = ptr.release();
+    out.tile_rows = tile_rows.release();
+    out.slot = slot.release();
+    out.splits = splits.release();
+    out.rest = rest.release();
+    out.n = n;
+    out.ntiles = P;
+    out.nblocks = nb;
+    out.nsplit = hC.nsplit;
+    out.nslots = hC.nslots;
+    out.nrest = chunks * kSlices * kChunk;
     return SPC3D_OK;
 }
 

@@ -45,6 +45,17 @@ struct SplitRow {
 constexpr uint32_t kSweepRound = 1024;
 inline bool sweep_fits(uint64_t nnz) { return nnz + kSweepRound <= (1ull << 32); }
 
+constexpr uint32_t kTileMaxRows = 512;
+// A row, or a piece of one, in the arrays a tile is made of: kTileGroup entries from start on, as many from
+// start + step on, ..., len in all.  (A line of columns and more, so that a piece reads whole lines, and every piece of
+// a row has columns of all blocks.)
+constexpr uint32_t kTileGroup = 16;
+struct TilePlace {
+    uint32_t start, step, len;
+};
+// Rows of more than this part of a tile's share are cut into pieces (build_hub_tiles).
+constexpr uint32_t kTileParts = 32;
+
 // ---- hot rows that crowd ---------------------------------------------------------
 // Dense rows a power of two apart whose numbers share their low bits (the hubs of an R-MAT graph,
 // whose numbers have few one-bits) share channels and sets of every L2, and the hottest of them carry
@@ -105,6 +116,8 @@ struct PlanOpts {
     bool slice_affinity = true;
     // the plan serves one call: no row tiles beside it, which take several to repay their making
     bool one_call = false;
+    // GPU builder: DevPlanArrays::rowptr and coldeg are wanted of a sliced plan
+    bool keep_counts = false;
 };
 
 struct HostPlan {
@@ -114,6 +127,8 @@ struct HostPlan {
     uint32_t max_row_nnz = 0;
     uint64_t row_sq = 0;           // sum over rows of length * min(length, 2048) (GPU builder)
     bool cols_sorted = false;      // the caller's columns never step down (GPU builder)
+    bool rows_sorted = false;      // nor do the rows (GPU builder)
+    uint32_t row_runs = 0;         // runs of equal rows in the caller's order (GPU builder)
     uint32_t seg_max = 0;
     bool seg_shortened = false;    // by default, and for the width: under seg_max_by_entries
     uint32_t nslots = 0;
