@@ -2010,15 +2010,19 @@ scatter_kernel(const T *__restrict__ in, const uint32_t *__restrict__ perm, T *_
         out[perm ? perm[i] : i] = in[i];
 }
 
-// out[i] = in[pos[i]], four results per lane: positions and results move as 16-byte
-// vectors, streaming; the reads in between are whatever `pos` makes them (runs, for the
-// staged results of a plan kept in column blocks).
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
+// out[i] = in[pos[i]], four results per lane and step, U steps in flight: positions and results move as
+// 16-byte vectors, streaming; the reads in between are whatever `pos` makes them (runs, for the staged results
+// of a plan kept in column blocks).  Where a row's columns are in no order they go to and fro among the row's
+// runs (one per block of columns): a lane waits for them, and their lines are met again while the first level
+// holds them, so a wavefront takes whole rows, one after the other, with many reads under way.  572 M results
+// of rows of up to 1024, fp32, the whole SDDMM call: workgroups of 256 and one step 17.38 ms, two 17.03, four 16.86;
+// of 64 and 4 steps 16.77, 8 16.70, 16 17.17; of 1024 and one 17.76.  Of 86 M: 3302 us -> 3258 (64 and 4), 3330 (8).
+template <typename T, int BLOCK, int U>
+__global__ void __launch_bounds__(BLOCK)
 gather4_kernel(const T *__restrict__ in, const uint32_t *__restrict__ pos, T *__restrict__ out,
                uint64_t n)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock * 4;
+    const uint64_t stride = (uint64_t)gridDim.x * BLOCK * 4 * U;
     const uint64_t nfull = n / 4 * 4;
     // Workgroups are dealt to the XCDs in turn: workgroup b takes the chunk that gives every
     // XCD a contiguous eighth of each round of chunks, so that neighbours in `out`, whose
@@ -2026,18 +2030,28 @@ gather4_kernel(const T *__restrict__ in, const uint32_t *__restrict__ pos, T *__
     uint32_t chunk = blockIdx.x;
     if (gridDim.x % 8 == 0)
         chunk = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-    for (uint64_t i = ((uint64_t)chunk * kBlock + threadIdx.x) * 4; i < nfull; i += stride) {
-        const u32x4 p = nt_load(reinterpret_cast<const u32x4 *>(pos + i));
+    for (uint64_t i = ((uint64_t)chunk * BLOCK * U + threadIdx.x) * 4; i < nfull; i += stride) {
+        u32x4 p[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const uint64_t at = i + (uint64_t)k * BLOCK * 4;
+            p[k] = nt_load(reinterpret_cast<const u32x4 *>(pos + (at < nfull ? at : i)));
+        }
         using V = typename Vec<T>::type; // 16 bytes: 4 floats or 2 doubles
-        V v[4 / Vec<T>::N];
+        V v[U][4 / Vec<T>::N];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            v[u / Vec<T>::N][u % Vec<T>::N] = in[p[u]];
+        for (int k = 0; k < U; ++k)
 #pragma unroll
-        for (int u = 0; u < 4 / Vec<T>::N; ++u)
-            nt_store(v[u], reinterpret_cast<V *>(out + i) + u);
+            for (int u = 0; u < 4; ++u)
+                v[k][u / Vec<T>::N][u % Vec<T>::N] = in[p[k][u]];
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (i + (uint64_t)k * BLOCK * 4 < nfull)
+#pragma unroll
+                for (int u = 0; u < 4 / Vec<T>::N; ++u)
+                    nt_store(v[k][u], reinterpret_cast<V *>(out + i + (uint64_t)k * BLOCK * 4) + u);
     }
-    const uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    const uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (t < n - nfull)
         out[nfull + t] = in[pos[nfull + t]];
 }
@@ -2972,18 +2986,32 @@ hipError_t launch_first_cols(const Seg *segs, uint32_t n, const uint32_t *col, u
     return hipGetLastError();
 }
 
+namespace {
+// Fewer results than this do not fill the chip with wavefronts of 1024 of them (6 M: the call 214 -> 217 us;
+// level at 8.6 M, 2 % faster at 28 M).
+constexpr uint64_t kGatherDeep = (uint64_t)8 << 20;
+template <typename T>
+void gather4_run(const void *in, const uint32_t *pos, void *out, uint64_t n, hipStream_t st)
+{
+    constexpr uint64_t deep = 64 * 4 * 4; // results of a deep workgroup's step
+    if (n >= kGatherDeep)
+        hipLaunchKernelGGL((gather4_kernel<T, 64, 4>), dim3((uint32_t)std::min<uint64_t>((n + deep - 1) / deep, 32768)),
+                           dim3(64), 0, st, (const T *)in, pos, (T *)out, n);
+    else
+        hipLaunchKernelGGL((gather4_kernel<T, kBlock, 1>), dim3(stream_grid((n + 3) / 4)), dim3(kBlock), 0, st,
+                           (const T *)in, pos, (T *)out, n);
+}
+} // namespace
+
 hipError_t launch_unstage(int dtype, const void *in, const uint32_t *pos, void *out, uint64_t n,
                           hipStream_t stream)
 {
     if (n == 0)
         return hipSuccess;
-    const uint32_t grid = stream_grid((n + 3) / 4);
     if (dtype == 1)
-        hipLaunchKernelGGL((gather4_kernel<double>), dim3(grid), dim3(kBlock), 0, stream,
-                           (const double *)in, pos, (double *)out, n);
+        gather4_run<double>(in, pos, out, n, stream);
     else
-        hipLaunchKernelGGL((gather4_kernel<float>), dim3(grid), dim3(kBlock), 0, stream,
-                           (const float *)in, pos, (float *)out, n);
+        gather4_run<float>(in, pos, out, n, stream);
     return hipGetLastError();
 }
 

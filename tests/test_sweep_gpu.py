@@ -240,3 +240,25 @@ def test_random_shapes_differential(ctx):
         if want and nb > 1:  # (1 leaves the number of blocks to the rule)
             assert info.ncol_blocks == min(nb, n)
         check(out, *case)
+
+
+@pytest.mark.parametrize("dtype,k", [(np.float32, 64), (np.float64, 32)])
+@pytest.mark.parametrize("nnz", [(8 << 20) - 1, 8 << 20, (8 << 20) + 1027, 34000103])
+def test_results_of_many_entries_come_home(ctx, dtype, k, nnz):
+    # either side of the number of results from which the pass home has wavefronts of 1024, parts of a vector,
+    # of a wavefront's share and of a round of workgroups at the end.  Integers: exact in any order.
+    rng = np.random.default_rng(nnz)
+    m, n = nnz // 1000 + 1, 60000
+    ii = (np.arange(nnz, dtype=np.uint64) // 1000).astype(np.uint32)
+    jj = rng.integers(0, n, nnz, dtype=np.uint32)  # in draw order inside a row
+    vv = rng.integers(1, 1 << 15, nnz).astype(dtype)
+    a, b = (rng.integers(-1, 2, (7, k)) for _ in range(2))
+    A, B = a[np.arange(m) % 7].astype(dtype), b[np.arange(n) % 7].astype(dtype)
+    S = ctx.plan(m, n, ii, jj, vv, k_hint=k, sweep=True, sweep_min_row=12, col_blocks=7)
+    assert S.info.staged_entries == nnz
+    dA, dB, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.vals(nnz, dtype)
+    dC.fill(-7.5)
+    ctx.sddmm(S, dA, dB, dC)
+    assert np.array_equal(dC.download(), vv * (a @ b.T).astype(dtype)[ii % 7, jj % 7])
+    for h in (S, dA, dB, dC):
+        h.close()
