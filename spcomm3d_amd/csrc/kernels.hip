@@ -1777,7 +1777,13 @@ hub_home_kernel(const uint32_t *__restrict__ ptr, uint32_t nb, uint32_t ntiles, 
 // each over its own panel: a real per lane with a division per real took 76 / 89 / 135 us, this
 // 50 / 50 / 69 (a row of 200 bytes at any alignment touches 2.6 lines of 128; repeated alone, on a
 // panel of which much stays in the Infinity Cache, 45 / 85 / 129 and 39 / 40 / 62).  Over panels that
-// change from pass to pass the three take 298 and 202 us together.
+// change from pass to pass the three took 298 and 202 us together.
+// What is met again is cached and what is not streams: a panel's rows are read (by a sum) and written once, so they
+// stream and leave the caches to the buffer, whose rows share lines with their neighbours, which other workgroups
+// read, and which has just been written.  The other way round before; the three together, fp32 K = 50, 500 k slots of
+// 1 M rows 202 -> 155 us, K = 64, 1 M slots 277 -> 244 (fp64 545 -> 494), fp64 K = 8 137 -> 104, fp32 K = 130, 1.5 M of
+// 2 M 1100 -> 988, fp64 K = 256, 20 k of 60 k 54 -> 48.  (Streaming only the stores 157, 264, 527, 106, 986, 51; a
+// pack that streams the rows it reads 160, 254, 517, 104, 1013, 48, one that caches what it writes 5 % slower.)
 enum RowUnit { kVec, kLoose, kElem };
 constexpr int kRowsAhead = 4;    // of a copy
 // Fewer workgroups than this (8 per CU) do not fill the chip: one row at a time then, which
@@ -1905,9 +1911,9 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
             typename A::V x[U], y[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                x[u] = A::load_nt(buf + (uint64_t)d[u][ADD ? 1 : 2] * bytes + off);
+                x[u] = A::load(buf + (uint64_t)d[u][ADD ? 1 : 2] * bytes + off);
                 if constexpr (ADD)
-                    y[u] = A::load(panel + (uint64_t)d[u][0] * bytes + off);
+                    y[u] = A::load_nt(panel + (uint64_t)d[u][0] * bytes + off);
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (ADD) {
@@ -1922,7 +1928,7 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
                         slot[j] = slots[d[0][3] + (t + j < left ? t + j : left)];
 #pragma unroll
                     for (int j = 0; j < D; ++j)
-                        z[j] = A::load_nt(buf + (uint64_t)slot[j] * bytes + off);
+                        z[j] = A::load(buf + (uint64_t)slot[j] * bytes + off);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int j = 0; j < D; ++j)
@@ -1936,7 +1942,7 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
                     continue;
                 char *to = panel + (uint64_t)d[u][0] * bytes + off;
                 if constexpr (!ADD) {
-                    A::store(x[u], to);
+                    A::store_nt(x[u], to);
                 } else {
                     if constexpr (UNIT == kLoose) {
                         const uint32_t skip = (uint32_t)((uint64_t)v * 16 - off) / (uint32_t)sizeof(T);
@@ -1949,7 +1955,7 @@ rows_unpack_kernel(char *__restrict__ panel, const u32x4 *__restrict__ dests,
                             continue;
                         }
                     }
-                    A::store(y[u], to);
+                    A::store_nt(y[u], to);
                 }
             }
         }
