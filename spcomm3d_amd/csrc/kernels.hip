@@ -1394,8 +1394,9 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // between 6 % faster, 256- and 1024-byte rows, and 5 % slower here; not kept.)
 // SpMM, with a barrier per block (one per batch measured 12 % slower), cuts every block's range into batches
 // of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum
-// of a row's run of entries is kept in registers, from the row's sum in LDS on, and stored there when the run
-// ends.  A row's entries are contiguous, so a row is shared between lane groups only
+// of a row's run of entries is kept in registers and added to the row's sum in LDS, read when the run begins,
+// when it ends (a run's sum of its own: carried on from the row's, fp32 rows of up to 1024 were three times as far
+// from 64 bits, 4.8e-7 against 1.5e-7).  A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
 // goes to the row's sum by that lane group), the later parts each BEGIN a chunk.  The
 // first run of every chunk therefore goes to an edge slot of its lane group instead, and
@@ -1645,7 +1646,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
         if (sub == 0)
             edge_row[grp] = row;
         // the run that is being summed, and where its sum goes: the chunk's first to the edge slot
-        V acc{};
+        V acc{}, base{};
         uint32_t to = kEdge + threadIdx.x;
         while (p < hi) {
             const uint32_t np = p + UB;
@@ -1683,8 +1684,9 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
                 if (any >> u & 1) {
                     const uint32_t l = bcast.entry(cur.row, u) * LPR + sub;
                     if (mine >> u & 1) {
-                        tile_y[to] = acc;
-                        acc = tile_y[l];
+                        tile_y[to] = base + acc;
+                        base = tile_y[l];
+                        acc = V{};
                         to = l;
                     }
                 }
@@ -1695,7 +1697,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
             cur = nxt;
         }
         if (had)
-            tile_y[to] = acc;
+            tile_y[to] = base + acc;
         p = p_nb;
         hi = hi_nb;
         if (!had && p < hi)
