@@ -317,7 +317,6 @@ __global__ void run_lengths_k(const uint32_t *__restrict__ start, uint64_t nbins
 
 // How often every id comes (count_ids): the ids lie in buckets of 1 << low by their upper bits, which are cut
 // into parts of at most `part` entries; a workgroup counts a part in LDS.
-constexpr uint32_t kCountBits = 14; // 64 KiB of counters, two workgroups to a CU
 constexpr int kCountTB = 1024;
 
 // The first of n keys, ascending in key >> low, that is `bucket` or above there.  By a wavefront, 64 probes at a time.
@@ -348,7 +347,7 @@ __global__ void bucket_parts_k(const uint32_t *__restrict__ key, uint32_t n, uin
     const uint32_t hi = b < nbuckets ? bucket_start(key, n, low, b + 1) : n;
     if ((threadIdx.x & 63u) == 0) {
         start[b] = lo;
-        parts[b] = (hi - lo + part - 1) / part;
+        parts[b] = parts_of(hi - lo, part);
     }
 }
 __global__ void __launch_bounds__(kCountTB)
@@ -1083,10 +1082,8 @@ int count_ids(Temp &tmp, Arena &arena, const uint32_t *ids, uint32_t n, uint32_t
               uint32_t *cnt, const DevStream &st, std::string &err)
 {
     const uint32_t bits = (uint32_t)bits_for(nbins ? nbins - 1 : 0);
-    const uint32_t low = bits <= kCountBits ? bits : std::min(kCountBits, bits - 8); // (a digit has 8 bits)
-    const uint32_t nbuckets = ((nbins ? nbins - 1 : 0) >> low) + 1;
-    const uint32_t part = std::max(n / 64, 1u << 16);
-    const uint32_t most = n / part + nbuckets; // parts
+    const CountSizes sizes = count_sizes(n, nbins);
+    const uint32_t low = sizes.low, nbuckets = sizes.nbuckets, part = sizes.part, most = sizes.most;
     if (low < bits) {
         size_t bytes = 0;
         HIP_OK(rocprim::radix_sort_keys<SortConfig>(nullptr, bytes, ids, scratch, (size_t)n, low, bits, st));

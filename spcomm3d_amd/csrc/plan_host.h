@@ -1,6 +1,7 @@
 // Host-side construction of the kernel-order form of a COO pattern.
 // Pure C++ (no HIP): testable and usable without a GPU.
 #pragma once
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -36,6 +37,29 @@ struct SplitRow {
     uint32_t nslots;
     uint32_t pad;
 };
+
+// ---- how often every id comes (count_ids) ------------------------------------------
+// Parts of at most `part` into which n entries are cut.  (Not n + part - 1: n is any 32-bit count, and one bucket
+// may hold nearly all entries of a pattern near 2^32.)
+constexpr uint32_t parts_of(uint32_t n, uint32_t part) { return n / part + (n % part != 0); }
+// n ids below 2^bits lie in buckets of 1 << low by their upper bits; a bucket's ids are cut into parts.
+constexpr uint32_t kCountBits = 14; // 64 KiB of counters in LDS, two workgroups to a CU
+struct CountSizes {
+    uint32_t low, nbuckets, part, most; // most: parts of all buckets together, at most
+};
+inline CountSizes count_sizes(uint32_t n, uint32_t nbins)
+{
+    const uint32_t last = nbins ? nbins - 1 : 0;
+    uint32_t bits = 1;
+    while (bits < 32 && last >> bits)
+        ++bits;
+    CountSizes s;
+    s.low = bits <= kCountBits ? bits : std::min(kCountBits, bits - 8); // (a digit of a sort has 8 bits)
+    s.nbuckets = (last >> s.low) + 1;
+    s.part = std::max(n / 64, 1u << 16);
+    s.most = n / s.part + s.nbuckets;
+    return s;
+}
 
 // ---- row tiles -------------------------------------------------------------------
 // SDDMM over a tile's entries runs in rounds of at most kSweepRound of them, and asks for a round's

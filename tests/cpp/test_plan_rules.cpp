@@ -62,8 +62,31 @@ static void row_tiles_near_the_end_of_32_bits()
     CHECK(!walk(0xFFFFFFFFu - 100, 0xFFFFFFFFu, 64));
 }
 
+// The parts of a bucket cover its ids, each of them once and none past its end, as bucket_count_k takes them, in a
+// pattern of n entries that all lie in that bucket or in all of them alike.
+static void counts_near_the_end_of_32_bits()
+{
+    const uint32_t most_entries = 0xFFFFFFFFu;
+    for (uint32_t n : {1u, 65535u, 65536u, 65537u, 1u << 22, (1u << 22) + 1, 4228000000u, 4230000000u, most_entries - 63,
+                       most_entries - 1, most_entries})
+        for (uint32_t nbins : {1u, 2u, 1u << 14, (1u << 14) + 1, 1u << 22, (1u << 22) + 1, 1u << 26}) {
+            const CountSizes s = count_sizes(n, nbins);
+            CHECK(s.low <= kCountBits && ((uint64_t)s.nbuckets << s.low) >= nbins);
+            const uint32_t g = parts_of(n, s.part); // all in one bucket
+            CHECK(g >= 1 && g <= s.most);
+            CHECK((uint64_t)(g - 1) * s.part < n && (uint64_t)g * s.part >= n);
+            CHECK((uint64_t)(g - 1) * s.part <= most_entries); // where the last one begins
+            const uint32_t each = n / s.nbuckets, extra = n % s.nbuckets; // all alike
+            const uint64_t all = (uint64_t)extra * parts_of(each + 1, s.part) +
+                                 (uint64_t)(s.nbuckets - extra) * parts_of(each, s.part);
+            CHECK(all <= s.most);
+        }
+    CHECK(parts_of(0, 1 << 16) == 0);
+}
+
 int main()
 {
+    counts_near_the_end_of_32_bits();
     row_tiles_near_the_end_of_32_bits();
     std::printf(g_fail ? "%d checks FAILED\n" : "PASSED\n", g_fail);
     return g_fail != 0;
