@@ -1396,7 +1396,8 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum
 // of a row's run of entries is kept in registers and added to the row's sum in LDS, read when the run begins,
 // when it ends (a run's sum of its own: carried on from the row's, fp32 rows of up to 1024 were three times as far
-// from 64 bits, 4.8e-7 against 1.5e-7).  A row's entries are contiguous, so a row is shared between lane groups only
+// from 64 bits, 4.8e-7 against 1.5e-7), and after every kRunBatches batches of a chunk: a tile may hold tens of
+// thousands of a row's entries in one block.  A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
 // goes to the row's sum by that lane group), the later parts each BEGIN a chunk.  The
 // first run of every chunk therefore goes to an edge slot of its lane group instead, and
@@ -1413,6 +1414,7 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // Every lane group with rows of its own, without edges or a barrier per block: a tenth faster with every
 // gather a hit, and 9 % slower, at 65 % hits and not 88: chance makes the groups drift by half a block.)
 constexpr int kSweepBlock = 1024;
+constexpr uint32_t kRunBatches = 128; // of 16: no sum goes over more than 2048 terms, as in the segments
 constexpr uint32_t kSweepRowBytes = 128u << 10; // of LDS for the tile's rows
 constexpr uint32_t kSweepPtrWords = 1028;       // nb + 1 range bounds of a tile, in LDS too
 // A lane's 16 bytes of a dense row.  ANY: rows of K reals, at least 16 bytes and at most LPR * 16,
@@ -1647,7 +1649,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
             edge_row[grp] = row;
         // the run that is being summed, and where its sum goes: the chunk's first to the edge slot
         V acc{}, base{};
-        uint32_t to = kEdge + threadIdx.x;
+        uint32_t to = kEdge + threadIdx.x, batch = 0;
         while (p < hi) {
             const uint32_t np = p + UB;
             SweepIdx<T> nxt;
@@ -1691,6 +1693,10 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
                     }
                 }
                 acc += xv[u] * bcast.entry(cur.val, u);
+            }
+            if (++batch % kRunBatches == 0) {
+                base += acc;
+                acc = V{};
             }
             row = bcast.entry(cur.row, UB - 1);
             p = np;

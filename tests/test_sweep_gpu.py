@@ -262,3 +262,27 @@ def test_results_of_many_entries_come_home(ctx, dtype, k, nnz):
     assert np.array_equal(dC.download(), vv * (a @ b.T).astype(dtype)[ii % 7, jj % 7])
     for h in (S, dA, dB, dC):
         h.close()
+
+
+@pytest.mark.parametrize("k", [64, 128, 256])
+def test_no_sum_goes_over_more_terms_than_in_a_segment(ctx, k):
+    # A row of 1.2 M entries in two column blocks: a lane group's share of a block is 9375 to 37500 of them.  One
+    # value is 2^24 and the others 1, which a sum that carries the 2^24 loses one by one (ties to even): as many as
+    # are added up in one go, at most 2048 with the 2^24 itself.  Elsewhere partial sums are whole numbers up to
+    # 2^25, each addition off by at most 1: the chunks' (64 per block at most, one of them cut at the 2^24) and Y's.
+    n, long = 3000, 1200000
+    ii = np.repeat(np.arange(5, dtype=np.uint32), [long, 40, 40, 3, 40])
+    jj = np.random.default_rng(k).integers(0, n, ii.size).astype(np.uint32)
+    vv = np.ones(ii.size, dtype=np.float32)
+    vv[np.flatnonzero(jj < n // 2)[0]] = 1 << 24
+    S = ctx.plan(5, n, ii, jj, vv, k_hint=k, sweep=True, sweep_min_row=12, col_blocks=2)
+    assert S.info.sweep_entries >= long and S.info.ncol_blocks == 2
+    dB, dY = ctx.panel_from(np.ones((n, k), dtype=np.float32)), ctx.panel_from(np.zeros((5, k), dtype=np.float32))
+    ctx.spmm(S, dB, dY)
+    Y = dY.download().astype(np.float64)
+    want = np.bincount(ii, weights=vv.astype(np.float64))[:, None]
+    assert np.array_equal(Y[1:], np.broadcast_to(want[1:], (4, k)))
+    # (20 more where a chunk takes its share in up to 19 sums)
+    assert np.abs(Y[0] - want[0]).max() <= 2047 + 2 * 64 + 20 + 4
+    for h in (S, dB, dY):
+        h.close()
