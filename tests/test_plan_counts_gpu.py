@@ -73,3 +73,14 @@ def test_rows_in_order(ctx, lengths, hub_min):
     P = both(ctx, len(lengths), n, ii, jj, xcd_slices=8, l2_hot_bytes=256, hub_min=hub_min, k_hint=4, seg_max=500)
     assert P["info"].nqueues == 8 and P["info"].hub_rows == sum(v >= hub_min for v in lengths)
     both(ctx, len(lengths), n, ii, jj, xcd_slices=1)
+
+
+# the longest row that is placed without a sort, and the shortest that makes the plan sort its entries
+@pytest.mark.parametrize("longest", [1 << 24, (1 << 24) + 1])
+def test_longest_row_in_order(ctx, longest):
+    lengths = [3, 700, longest, 1, 200000, 64]
+    ii = np.repeat(np.arange(len(lengths), dtype=np.uint32), lengths)
+    n = 4000
+    jj = np.minimum(np.random.default_rng(5).pareto(0.6, ii.size) * 4, n - 1).astype(np.uint32)
+    P = both(ctx, len(lengths), n, ii, jj, xcd_slices=8, l2_hot_bytes=256, hub_min=64, k_hint=4)
+    assert P["info"].nqueues == 8 and P["info"].hub_rows == 4
