@@ -1274,13 +1274,7 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
         return SPC3D_OK;
     }
 
-    // One block for everything whose size is known now: nine arrays per row, four and
-    // a class byte per column, the sorted column ids, two keys and an index per entry,
-    // the primitives' scratch.
     Arena arena(st);
-    const size_t key_bytes = bits_for(nrows ? nrows - 1 : 0) + 4 > 32 ? 8 : 4;
-    HIP_OK(arena.reserve(((size_t)nrows + 1) * 40 + (size_t)ncols * 17 + (size_t)std::max(nrows, ncols) * 4 +
-                         (size_t)nnz * (2 * key_bytes + 8) + (size_t)nnz / 2 + ((size_t)8 << 20)));
     Temp tmp(arena);
     SBuf<Counters> dC;
     Counters hC;
@@ -1289,13 +1283,6 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     HIP_OK(hipMemsetAsync(&dC.p->first_bad, 0xFF, sizeof(uint32_t), st));
 
     // ---- histograms, validation ------------------------------------------------
-    SBuf<uint32_t> rowcnt;
-    DBuf<uint32_t> rowptr, coldeg;
-    HIP_OK(rowcnt.alloc(arena, (size_t)nrows + 1));
-    HIP_OK(rowptr.alloc(st, (size_t)nrows + 1));
-    HIP_OK(coldeg.alloc(st, ncols));
-    HIP_OK(hipMemsetAsync(rowcnt.p, 0, ((size_t)nrows + 1) * sizeof(uint32_t), st));
-    HIP_OK(hipMemsetAsync(coldeg.p, 0, (size_t)ncols * sizeof(uint32_t), st));
     LAUNCH_SMALL(check_k, nnz, d_ii, d_jj, nnz, nrows, ncols, dC.p);
     TRY(fetch(st, &hC, dC.p, sizeof hC, err));
     if (hC.first_bad != 0xFFFFFFFFu) {
@@ -1315,22 +1302,43 @@ int build_device_plan(const DevStream &st, uint32_t nrows, uint32_t ncols, uint6
     const bool by_column = rows_unsorted && !opts.keep_entry_order;
     const int col_bits = bits_for(ncols ? ncols - 1 : 0);
     P.by_column_in_rows = by_column;
+    // Rows that come in runs are counted run by run (hist_sorted_k), which eight per run already pay for.
+    const bool count_rows = rows_unsorted && (uint64_t)hC.row_changes * 8 > nnz;
+    const CountSizes of_rows = count_sizes((uint32_t)nnz, nrows), of_cols = count_sizes((uint32_t)nnz, ncols);
+    const bool sort_ids = by_column || of_cols.nbuckets > 1 || (count_rows && of_rows.nbuckets > 1);
+    // One block for what is known to be needed: seven arrays of words and two of bytes per row, four and a byte per
+    // column, the scratch of the columns' sort; per entry, where rows are sorted, the ids and the scratch of a sort of
+    // theirs, with the counters of the ids, elsewhere two keys and two orders (the scratch of their sorts comes on top).
+    {
+        const size_t key_bytes = bits_for(nrows ? nrows - 1 : 0) + 4 > 32 ? 8 : 4;
+        const size_t per_entry = rows_unsorted ? 2 * key_bytes + 8 : (sort_ids ? 8 : 0);
+        const size_t counters = rows_unsorted ? 0 : (size_t)of_cols.most << of_cols.low;
+        HIP_OK(arena.reserve(((size_t)nrows + 1) * 34 + (size_t)ncols * 26 + counters * 4 + (size_t)nnz * per_entry +
+                             (size_t)nnz / 2 + ((size_t)8 << 20)));
+    }
+    SBuf<uint32_t> rowcnt;
+    DBuf<uint32_t> rowptr, coldeg;
+    HIP_OK(rowcnt.alloc(arena, (size_t)nrows + 1));
+    HIP_OK(rowptr.alloc(st, (size_t)nrows + 1));
+    HIP_OK(coldeg.alloc(st, ncols));
+    HIP_OK(hipMemsetAsync(rowcnt.p, 0, ((size_t)nrows + 1) * sizeof(uint32_t), st));
+    HIP_OK(hipMemsetAsync(coldeg.p, 0, (size_t)ncols * sizeof(uint32_t), st));
     DBuf<uint32_t> perm, col;
     SBuf<uint32_t> visit;
     HIP_OK(perm.alloc(st, nnz));
     HIP_OK(col.alloc(st, nnz));
     {
         SBuf<uint32_t> sorted, start;
-        HIP_OK(sorted.alloc(arena, nnz));
-        HIP_OK(start.alloc(arena, ncols));
-        // Rows that come in runs are counted run by run (hist_sorted_k), which eight per run already pay for.
-        if (rows_unsorted && (uint64_t)hC.row_changes * 8 > nnz) {
+        if (sort_ids)
+            HIP_OK(sorted.alloc(arena, nnz));
+        if (count_rows) {
             TRY(count_ids(tmp, arena, d_ii, (uint32_t)nnz, nrows, sorted.p, rowcnt.p, st, err));
         } else {
             LAUNCH(hist_sorted_k, nnz, d_ii, nnz, rowcnt.p);
         }
         if (by_column) { // the visiting order of order_entries; its sorted columns in `col`
             HIP_OK(visit.alloc(arena, nnz));
+            HIP_OK(start.alloc(arena, ncols));
             LAUNCH(iota_k, nnz, sorted.p, nnz);
             TRY(sort_pairs<uint32_t>(tmp, d_jj, col.p, sorted.p, visit.p, (uint32_t)nnz, col_bits,
                                      false, st, err));

@@ -1,5 +1,7 @@
 """Column and row counts, and the order of staged results, as the device builder makes them, at the edges of
 their buckets, parts and tiles, against the host builder and against unstaged stores."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,29 @@ def test_longest_row_in_order(ctx, longest):
     jj = np.minimum(np.random.default_rng(5).pareto(0.6, ii.size) * 4, n - 1).astype(np.uint32)
     P = both(ctx, len(lengths), n, ii, jj, xcd_slices=8, l2_hot_bytes=256, hub_min=64, k_hint=4)
     assert P["info"].nqueues == 8 and P["info"].hub_rows == 4
+
+
+def test_scratch_of_a_pattern_in_order():
+    # The pool of a fresh context keeps what making a plan took.  Per entry that is the ids and the scratch of one
+    # digit of their sort (8 bytes), half a byte for the primitives, and the kernel order, which is the caller's and
+    # goes back (4): less than 14.  Rows, columns and counters: under 64 MiB.
+    n, deg = 1 << 17, 512
+    jj = np.random.default_rng(0).integers(0, n, n * deg, dtype=np.uint32)
+    with device.Context(0) as c:
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+        def used():
+            c.sync()
+            assert c._lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            return total.value - free.value
+
+        dii, djj = c.vals(jj.size, np.float32), c.vals(jj.size, np.float32)
+        dii.upload(np.repeat(np.arange(n, dtype=np.uint32), deg).view(np.float32))
+        djj.upload(jj.view(np.float32))
+        small = device.Plan.from_device(c, n, n, dii, djj, 1000, np.float32)
+        before = used()
+        S = device.Plan.from_device(c, n, n, dii, djj, jj.size, np.float32, col_blocks=1, sweep=False)
+        assert S.info.order_is_identity and S.info.nqueues == 1
+        assert used() - before - S.info.device_bytes <= jj.size * 14 + (64 << 20)
+        for h in (S, small, dii, djj):
+            h.close()
