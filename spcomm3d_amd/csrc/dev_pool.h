@@ -57,8 +57,9 @@ class DevPool {
         registry() = this;
     }
 
-    // A block of at least `bytes`; a kept one when its size is within a quarter of that.
-    hipError_t get(void **out, size_t bytes)
+    // A block of at least `bytes`; a kept one when it is larger by no more than `spare` (a quarter).
+    hipError_t get(void **out, size_t bytes) { return get(out, bytes, bytes / 4); }
+    hipError_t get(void **out, size_t bytes, size_t spare)
     {
         *out = nullptr;
         if (bytes == 0)
@@ -69,7 +70,7 @@ class DevPool {
         try {
             std::lock_guard<std::mutex> lock(mu_);
             auto it = kept_.lower_bound(bytes);
-            if (it != kept_.end() && it->first <= bytes + bytes / 4) {
+            if (it != kept_.end() && it->first - bytes <= spare) {
                 void *p = it->second.p;
                 sizes_.emplace(p, it->first);
                 kept_bytes_ -= it->first;

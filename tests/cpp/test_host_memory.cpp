@@ -191,9 +191,35 @@ static void pools_give_way()
     CHECK(g_device.empty());
 }
 
+// A kept block serves what is smaller by up to the caller's spare, by a quarter unless it says otherwise.
+static void kept_blocks_serve_smaller_ones()
+{
+    g_device_room = 400 << 10;
+    {
+        DevPool a;
+        a.open(0, 400 << 10);
+        void *p = nullptr, *q = nullptr;
+        CHECK(a.get(&p, 100 << 10) == hipSuccess);
+        a.put(p);
+        CHECK(a.get(&q, 80 << 10) == hipSuccess && q == p);
+        a.put(q);
+        CHECK(a.get(&q, (80 << 10) - 512) == hipSuccess && q != p);
+        a.put(q); // (kept: 100 KiB and half a KiB less than 80)
+        CHECK(a.get(&q, 50 << 10, 50 << 10) == hipSuccess && q != p); // the smaller of two that would do
+        void *r = nullptr;
+        CHECK(a.get(&r, 50 << 10, (50 << 10) - 1) == hipSuccess && r != p && r != q);
+        a.put(r);
+        CHECK(a.get(&r, 51 << 10, 49 << 10) == hipSuccess && r == p);
+        a.put(r);
+        a.put(q);
+    }
+    CHECK(g_device.empty());
+}
+
 int main()
 {
     pools_give_way();
+    kept_blocks_serve_smaller_ones();
     for (unsigned threads : {1u, 3u})
         for (size_t room : {(size_t)0, (size_t)1 << 20, (size_t)2 << 20, (size_t)13 << 20, (size_t)30 << 20,
                             (size_t)1 << 30})
