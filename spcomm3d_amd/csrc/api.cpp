@@ -750,7 +750,7 @@ static void *staged_out(const spc3d_plan *parent, const spc3d_plan *)
 static hipError_t single_sddmm(const spc3d_plan *S, const void *A, const void *B, void *C, uint32_t K)
 {
     const Streams st = streams_of(S->ctx);
-    if (S->hub.n && K == S->hub_k && (S->hub.direct || S->hub_stage)) {
+    if (S->hub_sddmm && K == S->hub_k) {
         SweepView v = hub_view_of(S);
         if (S->hub.direct)
             v.pos = S->hub.perm;
@@ -765,7 +765,7 @@ static hipError_t single_sddmm(const spc3d_plan *S, const void *A, const void *B
 static hipError_t single_spmm(const spc3d_plan *S, const DevPlanView &view, const void *X, void *Y, uint32_t K)
 {
     const Streams st = streams_of(S->ctx);
-    if (S->hub.n && K == S->hub_k) {
+    if (S->hub_spmm && K == S->hub_k) {
         DevPlanView v = rest_view_of(S);
         const hipError_t e = launch_hub_spmm(S->dtype, v, hub_view_of(S), X, Y, st);
         if (e != hipErrorNotSupported) {

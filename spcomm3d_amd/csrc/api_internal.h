@@ -218,6 +218,7 @@ struct spc3d_plan {
     // form where the plan has one).
     HubTiles hub;
     uint32_t hub_k = 0, hub_lanes = 0;
+    bool hub_sddmm = false, hub_spmm = false; // the calls that run over them
     bool hub_by_pos = true; // SDDMM's results go to the caller's positions, else to the kernel's (two)
     bool hub_by_kernel = false; // hub.perm counts in kernel order, else in the caller's
     uint32_t *hub_first_cols = nullptr;

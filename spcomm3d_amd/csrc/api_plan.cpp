@@ -346,6 +346,7 @@ static void drop_hub_tiles(spc3d_plan *p)
         *a = nullptr;
     }
     p->hub_k = p->hub_lanes = 0;
+    p->hub_sddmm = p->hub_spmm = false;
 }
 
 static void destroy_blocks(spc3d_plan *p)
@@ -420,8 +421,14 @@ constexpr uint64_t kHubGather = (uint64_t)5 << 29;
 // Of an L2's 4 MiB; the tiles of an XCD are not in the same block at the same moment, so more of it is too much and
 // less only adds barriers (R-MAT 20, fp64: 3.5 - 7 MiB level within 1 %, 10 MiB 4 % slower).
 constexpr uint64_t kHubBlock = (uint64_t)5 << 20;
-// With fewer the panel nearly fits the L2s.
-constexpr uint32_t kHubMinBlocks = 4;
+// With fewer the panel nearly fits the L2s, and what does not costs less than the tiles' barriers and, at 64 lanes, their
+// one entry per wavefront.  SDDMM + SpMM in fp64, us over the segments / over the tiles, rows in order, in runs and
+// arbitrary: 32 lanes, 6 blocks 260 + 220 / 232 + 232, 285 + 219 / 283 + 232, 289 + 220 / 306 + 230, 7 blocks 300 + 242 /
+// 237 + 247, 323 + 234 / 281 + 231, 335 + 242 / 306 + 247; 64 lanes, 5 blocks 292 + 258 / 319 + 277, 320 + 258 / 368 + 275,
+// 322 + 258 / 389 + 276, 8 blocks 235 + 226 / 236 + 228, 255 + 231 / 255 + 229, 251 + 226 / 268 + 227, 9 blocks 303 + 289 /
+// 292 + 278, 327 + 292 / 323 + 281, 323 + 289 / 332 + 278, 10 blocks 295 + 280 / 245 + 255, 307 + 274 / 260 + 242,
+// 313 + 279 / 269 + 254.  (So at 64 lanes results that two passes bring home in fp64 need ten.)
+constexpr uint32_t kHubMinBlocks = 7, kHubMinBlocksWide = 8, kHubMinBlocksTwoPass = 10;
 // Rows of fewer entries gain nothing from a place in a tile (8 and 12 level, 16 up to 3 % slower, 4 fills more tiles).
 constexpr uint32_t kHubMinRow = 8;
 static bool wants_hub_tiles(int dtype, uint64_t nnz, const spc3d_plan_opts *opts, const PlanOpts &po)
@@ -463,8 +470,18 @@ struct KeptCounts {
 };
 
 // Row tiles beside a finished sliced plan `p` (spc3d_plan::hub) of the pattern that `in` gives by row, for its
-// longest rows.
-static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const spc3d_plan_opts *opts)
+// longest rows, and for those of its calls (`sddmm`, `spmm`: what it is there for) that are faster over them.
+// R-MAT patterns of 2^18 to 2^20 rows, us over the segments / over the tiles:
+//  - SpMM adds a row's sums up once per block, in all lanes.  Rows that fill two thirds of them and less: fp64 K = 40
+//    559 / 573, fp32 K = 70 571 / 578; fp32 K = 90 684 / 645.  At 64 lanes level (K = 67 405 / 395, 481 / 479, 1040 / 981).
+//    fp64 rows of up to 256 bytes: K = 32 394 / 405 and 473 / 481 where hot rows are copied, elsewhere 270 / 255 and, in
+//    a block of R-MAT 24, 532 / 498, which is little without SDDMM's gain.
+//  - SDDMM whose results two passes bring home in fp64 pays for a pass more.  K = 40 729 / 749, K = 66 632 / 666, K = 80
+//    469 / 500; rows over two thirds: K = 64 948 / 854, K = 97 696 / 631.
+//  - fp64 rows of up to 256 bytes that do not come in order: K = 32 in runs 532 / 478, arbitrary 568 / 575, beside
+//    500 us for the plan.  (In order 461 / 380; fp32 K = 64 453 / 394, 467 / 438 and 426 / 351.)
+static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const spc3d_plan_opts *opts, bool sddmm,
+                         bool spmm)
 {
     const spc3d_plan_info &I = p->info;
     if (!wants_hub_tiles(p->dtype, I.nnz, opts, po) || I.nqueues != kSlices || !in.rowptr || (p->store.n && in.pos))
@@ -472,6 +489,11 @@ static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const 
     const uint32_t lanes = sweep_lanes_any(p->dtype, opts->k_hint);
     const uint64_t w = elem_size(p->dtype), row_bytes = (uint64_t)opts->k_hint * w;
     if (!lanes)
+        return SPC3D_OK;
+    const bool f64 = w == 8, narrow = lanes == 16, filled = row_bytes * 3 > (uint64_t)lanes * 16 * 2;
+    sddmm = sddmm && !(f64 && (narrow ? in.pos != nullptr : !in.by_pos && !filled));
+    spmm = spmm && (filled || lanes == 64) && !(f64 && narrow && (!sddmm || p->hot_rows));
+    if (!sddmm && !spmm)
         return SPC3D_OK;
     spc3d_ctx *ctx = p->ctx;
     in.segs = p->segs;
@@ -482,12 +504,14 @@ static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const 
     }
     in.rows_per_tile = sweep_rows_per_tile(lanes);
     in.per_launch = (uint32_t)std::max(1, ctx->cu_count);
-    in.results = !p->by_col;
+    in.results = sddmm;
+    in.sums = spmm;
     in.min_row = opts->sweep_min_row ? opts->sweep_min_row : kHubMinRow;
     in.must = std::min(po.hub_min ? po.hub_min : kDefaultHubMin, I.seg_max + 1);
     in.row_bytes = row_bytes;
     in.block_bytes = kHubBlock;
-    in.min_blocks = kHubMinBlocks;
+    in.min_blocks = lanes == 64 ? kHubMinBlocksWide : kHubMinBlocks;
+    in.min_blocks_results = lanes == 64 && f64 && !in.by_pos ? kHubMinBlocksTwoPass : 0;
     in.max_blocks = sweep_max_blocks(lanes);
     std::string err;
     int rc = build_hub_tiles(dev_stream(ctx), in, p->hub, err);
@@ -498,11 +522,13 @@ static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const 
         return SPC3D_OK;
     p->hub_k = opts->k_hint;
     p->hub_lanes = lanes;
+    p->hub_sddmm = t.direct || t.src;
+    p->hub_spmm = spmm;
     p->hub_by_pos = in.by_pos;
     p->hub_by_kernel = in.col == p->col;
     rc = ctx_alloc_bytes(ctx, &p->hub_sval, (size_t)t.n * w);
     if (!rc && t.src) rc = ctx_alloc_bytes(ctx, &p->hub_stage, (size_t)t.n * w);
-    if (!rc) rc = ctx_alloc_bytes(ctx, &p->hub_partial, (size_t)t.nslots * row_bytes);
+    if (!rc && spmm) rc = ctx_alloc_bytes(ctx, &p->hub_partial, (size_t)t.nslots * row_bytes);
     if (!rc) rc = ctx_alloc(ctx, &p->hub_first_cols, (size_t)t.nrest * kFirstCols);
     if (!rc) {
         const hipError_t e = launch_first_cols(t.rest, t.nrest, p->hot_rows ? p->hot_col : p->col, p->hub_first_cols,
@@ -543,7 +569,7 @@ static int add_sddmm_companion(spc3d_plan *p, uint32_t nrows, uint32_t ncols, ui
     if (!rc)
         rc = add_hot_rows(q, po.hot_row_bytes / (uint32_t)elem_size(p->dtype));
     if (!rc && (!q->perm || q->store.consecutive))
-        rc = add_hub_tiles(q, counts.source(q, meta, d_ii), po, opts);
+        rc = add_hub_tiles(q, counts.source(q, meta, d_ii), po, opts, true, false);
     if (rc || (q->perm && !q->store.consecutive)) { // no better than what there is
         if (q) {
             const std::string keep = g_err;
@@ -873,7 +899,7 @@ static int build_from_device(spc3d_ctx *ctx, int dtype, uint32_t nrows, uint32_t
     if (!rc && nb <= 1)
         rc = add_tiles(p, nrows, ncols, nnz, d_ii, d_jj, po, opts);
     if (!rc && nb <= 1)
-        rc = add_hub_tiles(p, counts.source(p, meta, d_jj), po, opts);
+        rc = add_hub_tiles(p, counts.source(p, meta, d_jj), po, opts, !p->by_col, true);
     if (rc || nb <= 1) {
         if (rc) {
             const std::string keep = g_err;
@@ -1451,7 +1477,7 @@ static uint64_t own_device_bytes(const spc3d_plan *p)
         if (t.src)
             b += nnz * (2 * 4) + t.n * w; // src, dst; staged results
         b += ((uint64_t)t.ntiles * t.nblocks + 1) * 4 + (uint64_t)t.ntiles * sweep_rows_per_tile(p->hub_lanes) * 8;
-        b += t.split_cap * sizeof(SplitRow) + (uint64_t)t.nslots * p->hub_k * w;
+        b += t.split_cap * sizeof(SplitRow) + (p->hub_spmm ? (uint64_t)t.nslots * p->hub_k * w : 0);
         b += (uint64_t)p->info.nsegments_padded * sizeof(Seg) + (uint64_t)t.nrest * kFirstCols * 4;
     }
     if (p->sweep.n) {

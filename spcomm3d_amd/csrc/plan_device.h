@@ -138,8 +138,8 @@ int build_sweep(const DevStream &stream, uint32_t nrows, uint32_t ncols, uint64_
 //   tile_rows   row of place l of tile t, 0xFFFFFFFF where there is none                     [ntiles * rows_per_tile]
 //   slot        partial-sum row of a piece, kWholeRow for a whole row                        [ntiles * rows_per_tile]
 //   splits      the cut rows and their slots                                                 [nsplit]
-//   src, dst    result k = src[h] goes to dst[h], ascending inside a place; null where `direct`: results go
-//               straight to perm                                                             [n]
+//   src, dst    result k = src[h] goes to dst[h], ascending inside a place; null without results, and where
+//               `direct`: they go straight to perm                                                             [n]
 //   rest        the plan's segments of the other rows, in its queues, none of them a part    [nrest]
 // (room for nnz of what has n, for all the plan's segments, and for split_cap of splits)
 struct HubTiles {
@@ -158,7 +158,7 @@ struct HubSource {
     // the entries by row: row r's are rowptr[r] .. rowptr[r + 1), entry p in column col[p] and at the
     // caller's position pos[p] (null: p); results go to the caller's position (by_pos) or to p
     const uint32_t *rowptr = nullptr, *coldeg = nullptr, *col = nullptr, *pos = nullptr;
-    bool by_pos = true, results = true; // (results: SDDMM runs over the tiles)
+    bool by_pos = true, results = true, sums = true; // (results, sums: SDDMM, SpMM runs over the tiles)
     const Seg *segs = nullptr; // the plan's, in kSlices queues
     uint32_t nseg = 0;
     const uint32_t *hot_cols = nullptr; // [nhot] `col` names these by rank (kHotRow | rank)
@@ -166,7 +166,7 @@ struct HubSource {
     uint32_t rows_per_tile = 0, per_launch = 0, min_row = 0;
     uint32_t must = 0; // rows of so many entries, and cut ones, are all in the tiles, or there are no tiles
     uint64_t row_bytes = 0, block_bytes = 0;
-    uint32_t min_blocks = 0, max_blocks = 0;
+    uint32_t min_blocks = 0, max_blocks = 0, min_blocks_results = 0; // (results: none from fewer than these)
 };
 // n == 0 (and nothing to free): the pattern has no such tiles.  The arrays belong to the receiver (blocks of
 // the stream's pool).  Synchronous.

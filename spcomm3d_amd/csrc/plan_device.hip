@@ -2811,6 +2811,9 @@ int build_hub_tiles(const DevStream &st, const HubSource &in, HubTiles &out, std
     const uint32_t nb = total_weight / per_block + 1;
     if (npc == 0 || nb < in.min_blocks || nb > std::min(kFillBlocks, in.max_blocks))
         return SPC3D_OK;
+    const bool results = in.results && nb >= in.min_blocks_results;
+    if (!results && !in.sums)
+        return SPC3D_OK;
     if (in.nhot)
         HIP_OK(hot.alloc(arena, ncols));
     LAUNCH(hub_blocks_k, ncols, before.p, (uint64_t)ncols, per_block, nb, block.p, in.nhot ? hot.p : nullptr);
@@ -2849,7 +2852,7 @@ int build_hub_tiles(const DevStream &st, const HubSource &in, HubTiles &out, std
     // ---- entries (room for all: how many are in the tiles is known when they are) ----
     HIP_OK(col.alloc(st, nnz));
     HIP_OK(perm.alloc(st, nnz));
-    if (in.results) {
+    if (results) {
         HIP_OK(src.alloc(st, nnz));
         HIP_OK(dst.alloc(st, nnz));
     }
@@ -2871,7 +2874,7 @@ int build_hub_tiles(const DevStream &st, const HubSource &in, HubTiles &out, std
     // Results whose neighbours in the tile are mostly their neighbours in the caller's order go straight there:
     // pieces of lines that the same workgroup completes a few blocks later.  (R-MAT 20, rows and columns sorted,
     // three in four, fp64 / fp32 705 -> 685 us and 363 -> 357; a block of R-MAT 24, one in six, 491 -> 546.)
-    out.direct = in.results && !in.pos && (uint64_t)hC.adjacent * 5 >= (uint64_t)n * 3;
+    out.direct = results && !in.pos && (uint64_t)hC.adjacent * 5 >= (uint64_t)n * 3;
     if (out.direct) {
         src.reset();
         dst.reset();

@@ -6,6 +6,7 @@ import pytest
 from spcomm3d_amd import _capi as capi
 from spcomm3d_amd import device
 from spcomm3d_amd import workloads as W
+from tests._launches import launches
 from tests.test_parity_gpu import check_sddmm, check_spmm
 
 pytestmark = pytest.mark.gpu
@@ -22,10 +23,10 @@ def patterns():
     made = {}
 
     def get(scale, edges, order):
-        if scale not in made:
+        if (scale, edges) not in made:
             made.clear()
-            made[scale] = W.rmat(scale, edges, 1)
-        w = made[scale]
+            made[scale, edges] = W.rmat(scale, edges, 1)
+        w = made[scale, edges]
         ii, jj = w.ii, w.jj
         rng = np.random.default_rng(scale)
         if order == "runs":      # every row's entries lie together, rows and columns renumbered
@@ -159,3 +160,46 @@ def test_where_there_are_none(ctx, patterns):
     assert size["tiles"] > size["none"]
     assert size["less"] == size["less_none"] and size["kept"] == size["kept_none"]
     assert size["cut"] == size["cut_none"]
+
+
+# Which calls run over the tiles, on either side of every line of the rule: few blocks of columns, rows that leave a
+# third of their lanes idle, rows of up to 256 bytes and results of two passes in fp64 (A: SDDMM, B: SpMM).
+RULE = [(np.float64, 80, 16, 120, {o: "" for o in ("sorted", "runs", "shuffled", "column")}),
+        (np.float64, 100, 17, 40, {"sorted": "AB", "runs": "AB", "shuffled": "B", "column": "AB"}),
+        (np.float64, 120, 17, 40, {"shuffled": "AB"}),
+        (np.float32, 200, 17, 40, {"sorted": "AB", "shuffled": "AB"}),
+        (np.float64, 67, 18, 32, {"sorted": "AB", "runs": "AB", "shuffled": "B", "column": "AB"}),
+        (np.float32, 134, 18, 32, {"shuffled": "AB"}),
+        (np.float64, 42, 19, 24, {"sorted": "A", "runs": "A", "shuffled": "", "column": "A"}),
+        (np.float64, 43, 19, 24, {"sorted": "AB", "shuffled": "AB"}),
+        (np.float32, 85, 19, 24, {"sorted": "A", "shuffled": "A"}),
+        (np.float64, 32, 19, 24, {"sorted": "AB", "runs": "", "shuffled": "", "column": "A"}),
+        (np.float32, 64, 19, 24, {"runs": "AB", "column": "AB"}),
+        (np.float64, 32, 19, 28, {"sorted": "A"}),  # from 3 GiB on hot rows are copied
+        (np.float32, 64, 19, 28, {"sorted": "AB"})]
+
+
+@pytest.mark.parametrize("dtype,k,scale,edges,order,over", [(*c, o, over) for *c, orders in RULE
+                                                            for o, over in orders.items()])
+def test_calls_that_run_over_tiles(ctx, patterns, dtype, k, scale, edges, order, over):
+    m, ii, jj = patterns(scale, edges, order)
+    nnz = ii.size
+    assert nnz * k * np.dtype(dtype).itemsize >= 5 << 29
+    rng = np.random.default_rng(k)
+    vv = rng.uniform(0.5, 1, nnz).astype(dtype)
+    A, B, Y0 = (rng.uniform(-1, 1, (m, k)).astype(dtype) for _ in range(3))
+    S, plain = ctx.plan(m, m, ii, jj, vv, k_hint=k), ctx.plan(m, m, ii, jj, vv, k_hint=k, sweep=False)
+    assert (S.info.device_bytes > plain.info.device_bytes) == (over != "")
+    dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(nnz, dtype)
+    dC.fill(-5.0)
+    ctx.sddmm(S, dA, dB, dC)
+    ctx.spmm(S, dB, dY)
+    rows, at, sub = some_rows(ii, m)
+    check_sddmm(A[rows], B, sub, jj[at], vv[at], dC.download()[at])
+    check_spmm(B, sub, jj[at], vv[at], Y0[rows], dY.download()[rows])
+    ctx.sddmm(plain, dA, dB, dC)
+    ctx.spmm(plain, dB, dY)
+    for name, call in (("A", lambda P: ctx.sddmm(P, dA, dB, dC)), ("B", lambda P: ctx.spmm(P, dB, dY))):
+        assert (launches(ctx, lambda: call(S)) != launches(ctx, lambda: call(plain))) == (name in over), name
+    for h in (S, plain, dA, dB, dY, dC):
+        h.close()
