@@ -429,6 +429,9 @@ constexpr uint64_t kHubBlock = (uint64_t)5 << 20;
 // 292 + 278, 327 + 292 / 323 + 281, 323 + 289 / 332 + 278, 10 blocks 295 + 280 / 245 + 255, 307 + 274 / 260 + 242,
 // 313 + 279 / 269 + 254.  (So at 64 lanes results that two passes bring home in fp64 need ten.)
 constexpr uint32_t kHubMinBlocks = 7, kHubMinBlocksWide = 8, kHubMinBlocksTwoPass = 10;
+// Where they give a call less (add_hub_tiles): from so many blocks, or bytes of gathered rows, on.
+constexpr uint32_t kHubFewBlocks = 19, kHubMinBlocksF64 = 17;
+constexpr uint64_t kHubGatherIdle = (uint64_t)3 << 30;
 // Rows of fewer entries gain nothing from a place in a tile (8 and 12 level, 16 up to 3 % slower, 4 fills more tiles).
 constexpr uint32_t kHubMinRow = 8;
 static bool wants_hub_tiles(int dtype, uint64_t nnz, const spc3d_plan_opts *opts, const PlanOpts &po)
@@ -476,10 +479,19 @@ struct KeptCounts {
 //    559 / 573, fp32 K = 70 571 / 578; fp32 K = 90 684 / 645.  At 64 lanes level (K = 67 405 / 395, 481 / 479, 1040 / 981).
 //    fp64 rows of up to 256 bytes: K = 32 394 / 405 and 473 / 481 where hot rows are copied, elsewhere 270 / 255 and, in
 //    a block of R-MAT 24, 532 / 498, which is little without SDDMM's gain.
-//  - SDDMM whose results two passes bring home in fp64 pays for a pass more.  K = 40 729 / 749, K = 66 632 / 666, K = 80
-//    469 / 500; rows over two thirds: K = 64 948 / 854, K = 97 696 / 631.
+//  - SDDMM whose results two passes bring home pays for a pass more.  fp64 K = 40 729 / 749, K = 66 632 / 666, K = 80
+//    469 / 500; fp32 K = 80 634 / 627, 428 / 416, 446 / 450, and at 64 lanes K = 134, 10 to 17 blocks, 432 / 457,
+//    488 / 500, 580 / 591, 688 / 710 (19 blocks and more 575 / 577, 748 / 720, 681 / 640); rows over two thirds: fp64
+//    K = 64 948 / 854, K = 97 696 / 631.  fp64 at 32 lanes SDDMM + SpMM, 8 to 17 blocks 363 + 289 / 365 + 286, 387 + 303 /
+//    362 + 306, 420 + 373 / 405 + 368, 602 + 502 / 585 + 505, 582 + 530 / 549 + 488: from kHubMinBlocksF64 on.
 //  - fp64 rows of up to 256 bytes that do not come in order: K = 32 in runs 532 / 478, arbitrary 568 / 575, beside
 //    500 us for the plan.  (In order 461 / 380; fp32 K = 64 453 / 394, 467 / 438 and 426 / 351.)
+//  - A plan of fewer than kHubFewBlocks that does not come in order and has them for one of its calls takes 11 to 28 calls of
+//    that one to repay its making (22 us per million entries): SDDMM K = 80 in runs 643 / 603, 436 / 401, 455 / 421 at
+//    17, 14 and 11 blocks, 741 / 670 and 842 / 751 at 22 and 27; SpMM of patterns in column order fp32 K = 64 391 / 376,
+//    267 / 249 and 438 / 412 at 13, 9 and 18, 522 / 474 at 22, K = 128 498 / 470 at 17.
+//  - 64 lanes, a third of them idle, gathers of up to 3 GiB: SDDMM + SpMM, fp64 K = 80 298 + 271 / 307 + 286, fp32
+//    K = 150 297 + 285 / 290 + 298 and K = 168 283 + 260 / 290 + 265; from 3.1 GiB on K = 168 313 + 304 / 300 + 301.
 static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const spc3d_plan_opts *opts, bool sddmm,
                          bool spmm)
 {
@@ -491,7 +503,9 @@ static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const 
     if (!lanes)
         return SPC3D_OK;
     const bool f64 = w == 8, narrow = lanes == 16, filled = row_bytes * 3 > (uint64_t)lanes * 16 * 2;
-    sddmm = sddmm && !(f64 && (narrow ? in.pos != nullptr : !in.by_pos && !filled));
+    if (lanes == 64 && !filled && I.nnz * row_bytes < kHubGatherIdle)
+        return SPC3D_OK;
+    sddmm = sddmm && !(f64 && narrow && in.pos) && !(!in.by_pos && !filled && (f64 || lanes < 64));
     spmm = spmm && (filled || lanes == 64) && !(f64 && narrow && (!sddmm || p->hot_rows));
     if (!sddmm && !spmm)
         return SPC3D_OK;
@@ -510,8 +524,11 @@ static int add_hub_tiles(spc3d_plan *p, HubSource in, const PlanOpts &po, const 
     in.must = std::min(po.hub_min ? po.hub_min : kDefaultHubMin, I.seg_max + 1);
     in.row_bytes = row_bytes;
     in.block_bytes = kHubBlock;
-    in.min_blocks = lanes == 64 ? kHubMinBlocksWide : kHubMinBlocks;
-    in.min_blocks_results = lanes == 64 && f64 && !in.by_pos ? kHubMinBlocksTwoPass : 0;
+    const bool one_call = in.pos && (!sddmm || (!spmm && lanes == 32));
+    in.min_blocks = lanes == 64 ? kHubMinBlocksWide
+                                : (one_call ? kHubFewBlocks : (f64 && !in.by_pos ? kHubMinBlocksF64 : kHubMinBlocks));
+    if (lanes == 64 && !in.by_pos)
+        in.min_blocks_results = !filled ? kHubFewBlocks : (f64 ? kHubMinBlocksTwoPass : 0);
     in.max_blocks = sweep_max_blocks(lanes);
     std::string err;
     int rc = build_hub_tiles(dev_stream(ctx), in, p->hub, err);

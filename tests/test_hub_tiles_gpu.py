@@ -163,20 +163,27 @@ def test_where_there_are_none(ctx, patterns):
 
 
 # Which calls run over the tiles, on either side of every line of the rule: few blocks of columns, rows that leave a
-# third of their lanes idle, rows of up to 256 bytes and results of two passes in fp64 (A: SDDMM, B: SpMM).
+# third of their lanes idle, rows of up to 256 bytes, results of two passes, and plans that have them for one call only
+# (A: SDDMM, B: SpMM).
 RULE = [(np.float64, 80, 16, 120, {o: "" for o in ("sorted", "runs", "shuffled", "column")}),
         (np.float64, 100, 17, 40, {"sorted": "AB", "runs": "AB", "shuffled": "B", "column": "AB"}),
         (np.float64, 120, 17, 40, {"shuffled": "AB"}),
         (np.float32, 200, 17, 40, {"sorted": "AB", "shuffled": "AB"}),
         (np.float64, 67, 18, 32, {"sorted": "AB", "runs": "AB", "shuffled": "B", "column": "AB"}),
-        (np.float32, 134, 18, 32, {"shuffled": "AB"}),
-        (np.float64, 42, 19, 24, {"sorted": "A", "runs": "A", "shuffled": "", "column": "A"}),
-        (np.float64, 43, 19, 24, {"sorted": "AB", "shuffled": "AB"}),
-        (np.float32, 85, 19, 24, {"sorted": "A", "shuffled": "A"}),
+        (np.float32, 134, 18, 32, {"runs": "AB", "shuffled": "B"}),
+        (np.float64, 80, 18, 20, {"sorted": "", "shuffled": ""}),  # gathers of less than 3 GiB
+        (np.float32, 168, 19, 20, {"shuffled": "AB"}),             # blocks enough for results of two passes
+        (np.float64, 42, 19, 24, {"sorted": "A", "runs": "", "shuffled": "", "column": "A"}),
+        (np.float64, 43, 19, 24, {"sorted": "AB", "runs": "AB", "shuffled": ""}),
+        (np.float64, 64, 19, 28, {"shuffled": "AB"}),
+        (np.float32, 85, 19, 24, {"sorted": "A", "runs": "", "shuffled": "", "column": "A"}),
+        (np.float32, 86, 19, 24, {"runs": "AB", "shuffled": "AB", "column": "A"}),
         (np.float64, 32, 19, 24, {"sorted": "AB", "runs": "", "shuffled": "", "column": "A"}),
-        (np.float32, 64, 19, 24, {"runs": "AB", "column": "AB"}),
+        (np.float32, 64, 19, 24, {"runs": "AB", "column": "A"}),
         (np.float64, 32, 19, 28, {"sorted": "A"}),  # from 3 GiB on hot rows are copied
-        (np.float32, 64, 19, 28, {"sorted": "AB"})]
+        (np.float32, 64, 19, 28, {"sorted": "AB"}),
+        (np.float32, 128, 20, 12, {"column": "AB"}),  # blocks enough for one call alone
+        (np.float32, 85, 20, 26, {"runs": "A"})]
 
 
 @pytest.mark.parametrize("dtype,k,scale,edges,order,over", [(*c, o, over) for *c, orders in RULE
