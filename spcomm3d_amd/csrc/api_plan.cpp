@@ -1424,7 +1424,8 @@ static int probe_columns_of(spc3d_plan *p, int mode, uint32_t modulus)
     if (!p->hub.n)
         return rc;
     // (plain columns from now on, which the kernels of the hot form take as well)
-    HIP_TRY(launch_probe_cols(p->hub.col, p->hub.n, (uint32_t)mode, 0, modulus, p->info.ncols, p->ctx->stream));
+    HIP_TRY(launch_probe_cols(p->hub.col, p->hub.n, (uint32_t)mode, 0, modulus, p->info.ncols, p->ctx->stream,
+                              p->hot_rows ? p->hot_cols : nullptr));
     HIP_TRY(launch_first_cols(p->hub.rest, p->hub.nrest, p->hot_rows && !p->hot_stale ? p->hot_col : p->col,
                               p->hub_first_cols, p->ctx->stream));
     return rc;

@@ -1983,15 +1983,16 @@ __global__ void __launch_bounds__(64) xcc_probe_kernel(uint32_t *__restrict__ ou
 // Measurement aid (launch_probe_cols): the column of every kernel-order entry replaced so
 // that the launches keep their instruction stream, segments and queues while every gather
 // hits (mode 1: base + (c - base) % modulus, a table of `modulus` dense rows) or nearly
-// every gather misses (mode 2: a hash of the entry's position, uniform over ncols).
+// every gather misses (mode 2: a hash of the entry's position, uniform over ncols).  hot (may be
+// null): the columns that `col` names by rank.
 __global__ void __launch_bounds__(kBlock)
 probe_cols_kernel(uint32_t *__restrict__ col, uint64_t n, uint32_t mode, uint32_t base,
-                  uint32_t modulus, uint32_t ncols)
+                  uint32_t modulus, uint32_t ncols, const uint32_t *__restrict__ hot)
 {
     const uint64_t stride = (uint64_t)gridDim.x * kBlock;
     for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
         if (mode == 1) {
-            const uint32_t c = col[i];
+            const uint32_t c = hot && (col[i] & kHotRow) ? hot[col[i] & ~kHotRow] : col[i];
             col[i] = c >= base ? base + (c - base) % modulus : c % modulus;
         } else {
             uint64_t x = (i + 1) * 0x9E3779B97F4A7C15ull; // splitmix64 finaliser
@@ -3207,12 +3208,12 @@ hipError_t launch_xcc_probe(uint32_t *out, uint32_t nblocks, hipStream_t stream)
 }
 
 hipError_t launch_probe_cols(uint32_t *col, uint64_t n, uint32_t mode, uint32_t base,
-                             uint32_t modulus, uint32_t ncols, hipStream_t stream)
+                             uint32_t modulus, uint32_t ncols, hipStream_t stream, const uint32_t *hot)
 {
     if (n == 0)
         return hipSuccess;
     hipLaunchKernelGGL(probe_cols_kernel, dim3(stream_grid(n)), dim3(kBlock), 0, stream, col, n,
-                       mode, base, modulus, ncols);
+                       mode, base, modulus, ncols, hot);
     return hipGetLastError();
 }
 

@@ -210,3 +210,41 @@ def test_calls_that_run_over_tiles(ctx, patterns, dtype, k, scale, edges, order,
         assert (launches(ctx, lambda: call(S)) != launches(ctx, lambda: call(plain))) == (name in over), name
     for h in (S, plain, dA, dB, dY, dC):
         h.close()
+
+
+@pytest.mark.parametrize("dtype,k,scale,edges,order", [(np.float64, 64, 19, 28, "sorted"), (np.float32, 128, 19, 28, "shuffled"),
+                                                       (np.float32, 64, 19, 24, "runs"), (np.float64, 64, 19, 24, "column")])
+def test_probed_columns(ctx, patterns, dtype, k, scale, edges, order):
+    """spc3d_plan_probe_columns on a plan that holds tiles, hot rows copied and not: its calls run over them as before,
+    and compute the pattern (ii, jj % modulus), or one of columns that are all there."""
+    m, ii, jj = patterns(scale, edges, order)
+    nnz, modulus = ii.size, 997
+    rng = np.random.default_rng(5)
+    vv = rng.uniform(0.5, 1, nnz).astype(dtype)
+    A, B, Y0 = (rng.uniform(-1, 1, (m, k)).astype(dtype) for _ in range(3))
+    S = ctx.plan(m, m, ii, jj, vv, k_hint=k)
+    dA, dB, dY, dC = ctx.panel_from(A), ctx.panel_from(B), ctx.panel_from(Y0), ctx.vals(nnz, dtype)
+    calls = (lambda: ctx.sddmm(S, dA, dB, dC), lambda: ctx.spmm(S, dB, dY))
+    for call in calls:
+        call()
+    before, held = [launches(ctx, call) for call in calls], S.info.device_bytes
+    rows, at, sub = some_rows(ii, m)
+    for again in range(2):
+        S.probe_columns("all_hit", modulus)
+        dY.upload(Y0)
+        for call in calls:
+            call()
+        if order != "column":
+            check_sddmm(A[rows], B, sub, (jj[at] % modulus).astype(np.uint32), vv[at], dC.download()[at])
+        else:  # SDDMM exchanges rows and columns: it is the rows that are taken modulo
+            check_sddmm(A, B[jj[at]], (ii[at] % modulus).astype(np.uint32), np.arange(at.size, dtype=np.uint32), vv[at],
+                        dC.download()[at])
+        check_spmm(B, sub, (jj[at] % modulus).astype(np.uint32), vv[at], Y0[rows], dY.download()[rows])
+        assert [launches(ctx, call) for call in calls] == before and S.info.device_bytes == held
+    S.probe_columns("all_miss")
+    dY.upload(Y0)
+    for call in calls:
+        call()
+    assert np.isfinite(dC.download()).all() and np.isfinite(dY.download()).all()
+    for h in (S, dA, dB, dY, dC):
+        h.close()
