@@ -148,3 +148,8 @@ def test_shim_without_the_cache_of_the_one_shot_calls():
     env = dict(os.environ, SPC3D_HOST_CACHE="0")
     r = subprocess.run([_binary("test_shim_f64")], capture_output=True, text=True, timeout=300, env=env)
     assert r.returncode == 0 and "PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-3000:]
+
+
+@pytest.mark.gpu
+def test_tiles_of_the_longest_rows_at_their_edges():
+    _run("test_hub_tiles")

@@ -183,7 +183,12 @@ RULE = [(np.float64, 80, 16, 120, {o: "" for o in ("sorted", "runs", "shuffled",
         (np.float64, 32, 19, 28, {"sorted": "A"}),  # from 3 GiB on hot rows are copied
         (np.float32, 64, 19, 28, {"sorted": "AB"}),
         (np.float32, 128, 20, 12, {"column": "AB"}),  # blocks enough for one call alone
-        (np.float32, 85, 20, 26, {"runs": "A"})]
+        (np.float32, 85, 20, 26, {"runs": "A"}),
+        # 512 and 1024 bytes, hot rows copied and (their numbers drawn anew) not
+        (np.float64, 64, 19, 28, {"sorted": "AB", "runs": "AB"}),
+        (np.float32, 128, 19, 28, {"sorted": "AB", "runs": "AB"}),
+        (np.float64, 128, 18, 28, {"runs": "AB"}),
+        (np.float32, 256, 18, 28, {"sorted": "AB", "runs": "AB"})]
 
 
 @pytest.mark.parametrize("dtype,k,scale,edges,order,over", [(*c, o, over) for *c, orders in RULE
