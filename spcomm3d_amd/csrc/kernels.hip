@@ -1396,8 +1396,9 @@ spmm_fixup_kernel(const SplitRow *__restrict__ splits, uint32_t nsplit, const U 
 // of its own: lane group g takes the contiguous batches [g per, (g + 1) per), per = ceil(nbat / G).  The sum
 // of a row's run of entries is kept in registers and added to the row's sum in LDS, read when the run begins,
 // when it ends (a run's sum of its own: carried on from the row's, fp32 rows of up to 1024 were three times as far
-// from 64 bits, 4.8e-7 against 1.5e-7), and after every kRunBatches batches of a chunk: a tile may hold tens of
-// thousands of a row's entries in one block.  A row's entries are contiguous, so a row is shared between lane groups only
+// from 64 bits, 4.8e-7 against 1.5e-7; the fp64 step of R-MAT 20 takes 1401 us for it and not 1365, others are level),
+// and after every kRunBatches batches of a chunk: a tile may hold tens of thousands of a row's entries in one block.
+// A row's entries are contiguous, so a row is shared between lane groups only
 // where a boundary between two chunks falls inside it: its first part then ends a chunk (and
 // goes to the row's sum by that lane group), the later parts each BEGIN a chunk.  The
 // first run of every chunk therefore goes to an edge slot of its lane group instead, and
@@ -1735,7 +1736,7 @@ sweep_spmm_kernel(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__
 // The tiles' results to their places: out[dst[h]] = stage[src[h]], the h-th entry of a tile counted place after
 // place.  What a tile's entries read lies anywhere in the tile's results (0.4 MB), so the workgroups of a tile
 // run on one XCD, as its results were written, and meet them in its L2; what they write are whole rows.
-// (13 M results beside the segments of the other rows: 118 us in fp64, 85 in fp32.)
+// (13 M results beside the segments of the other rows: 117 us in fp64, 76 in fp32.)
 constexpr uint32_t kHomePieces = 8; // workgroups of a tile
 template <typename T>
 __global__ void __launch_bounds__(kBlock)

@@ -2573,9 +2573,9 @@ __global__ void __launch_bounds__(kFillTB) hub_fill_k(HubFill F)
     for (uint32_t k = lane; k < F.nb; k += 64)
         count[k] = 0;
     __syncthreads();
-        constexpr int V = 8; // entries of a lane at a time, here
+    constexpr int V = 8; // entries of a lane at a time, here
     for (uint32_t y0 = w * V * 64; y0 < n; y0 += kWaves * V * 64) {
-        // the place of the first, and from there of the others: few places end among 256 entries
+        // the place of the first, and from there of the others: few places end among 512 entries
         uint32_t at = 0, up = F.R;
         while (up - at > 1) {
             const uint32_t mid = (at + up) / 2;
