@@ -185,18 +185,25 @@ typedef struct {
                               SPC3D_PLAN_KEEP_ENTRY_ORDER: they add block after block.  They
                               make the plan 0.76 to 1.05 ms slower at 6 to 10 M entries, which
                               three to five steps repay: for a plan of fewer calls, sweep = 1.
-                              Where its columns are skewed (XCD slices) and a call gathers
-                              2.5 GiB and more, it holds tiles of its longest rows, one to a
-                              CU (device_bytes only; none where seg_max is given): spc3d_sddmm, spc3d_spmm and
-                              spc3d_spmm_noalloc at K = k_hint run over them and the segments
-                              of the other rows.  They make the plan 0.4 to 0.5 ms slower at
-                              16 M entries (one step of fp64, K = 64, repays that; of fp32,
-                              ten).
+                              Where its columns are skewed (XCD slices), k_hint is given and a
+                              call gathers 2.5 GiB and more, it holds tiles of its longest
+                              rows, one to a CU (device_bytes only; none where seg_max is
+                              given): those of spc3d_sddmm, spc3d_spmm and spc3d_spmm_noalloc
+                              at K = k_hint that are faster so run over them and the segments
+                              of the other rows.  They make the plan slower by 22 to 30 us per
+                              million entries (0.4 to 0.5 ms at 16 M; twice that for a pattern
+                              sorted by column).  SDDMM + SpMM steps that repay it, R-MAT 20:
+                              two to four in fp64, K = 64; in fp32, K = 64, six where rows
+                              come in order, ten in runs, sixteen in an arbitrary order;
+                              other patterns mostly one to six at rows of 400 bytes and more,
+                              four to fourteen below.  For a plan of fewer steps, and for one of
+                              spc3d_sddmm_spmm alone, which does not run over them, sweep = 1.
                               0 (default): as described; 1: never; 2: whenever k_hint has such
                               a width, whatever the pattern (col_blocks, if given, is the
                               number of blocks) */
     uint32_t sweep_min_row; /* shortest row kept in the tiles (default 64; in the tiles
-                              of an ordinary plan 16 to 64, by the number of blocks) */
+                              of an ordinary plan 16 to 64, by the number of blocks, in
+                              those of its longest rows 8) */
     uint32_t reserved[1];  /* must be 0 */
 } spc3d_plan_opts;
 /* spc3d_plan_opts.flags.  The first three keep spc3d_sddmm's plain stores where the plan
