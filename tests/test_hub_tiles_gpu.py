@@ -188,7 +188,10 @@ RULE = [(np.float64, 80, 16, 120, {o: "" for o in ("sorted", "runs", "shuffled",
         (np.float64, 64, 19, 28, {"sorted": "AB", "runs": "AB"}),
         (np.float32, 128, 19, 28, {"sorted": "AB", "runs": "AB"}),
         (np.float64, 128, 18, 28, {"runs": "AB"}),
-        (np.float32, 256, 18, 28, {"sorted": "AB", "runs": "AB"})]
+        (np.float32, 256, 18, 28, {"sorted": "AB", "runs": "AB"}),
+        # the workload of the benchmark, planned for its width
+        (np.float64, 64, 20, 16, {"sorted": "AB", "runs": "AB", "shuffled": "AB", "column": "AB"}),
+        (np.float32, 64, 20, 16, {"sorted": "AB", "shuffled": "AB", "column": "A"})]
 
 
 @pytest.mark.parametrize("dtype,k,scale,edges,order,over", [(*c, o, over) for *c, orders in RULE
